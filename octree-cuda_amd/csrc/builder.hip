@@ -630,7 +630,7 @@ void OctreeBuilder::mergeLevels()
     // leaf data blocks (A4): exclusive scan of the block sizes in id order
     scanExclusive<uint32_t>(m, ArrayIn{itsNodeAux.as<uint32_t>()}, ExclusiveToArray{itsNodeAux.as<uint32_t>()},
                             itsScanScratch.as<uint32_t>(), reinterpret_cast<uint32_t*>(sc + SC_LEAF_TOTAL),
-                            itsStream);
+                            itsStream, true);
     OC_LAUNCH_CHECK();
     kLeafDataIdx<<<gridFor(m), BLOCK, 0, itsStream>>>(itsM, itsProc.mergingThreshold, itsNodeAux.as<uint32_t>(),
                                                        itsNodeFlags.as<uint8_t>(), itsNodeChild.as<int32_t>(),

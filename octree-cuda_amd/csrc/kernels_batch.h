@@ -29,6 +29,7 @@ constexpr uint32_t MAX_BATCH      = 1024;   // clouds per batched launch
 constexpr uint32_t HIST_CHUNK     = 16384;  // points per work item of the batched bucket histogram
 constexpr uint32_t DIST_CHUNK     = 1024;   // sorted points per work item of the batched distribution
 constexpr uint32_t BATCH_SCAN_X   = 256;    // workgroups per cloud of a batched multi-workgroup scan
+static_assert(BATCH_SCAN_X <= SCAN_THREADS, "a workgroup reads one range sum per thread");
 constexpr uint32_t ERR_OVERFLOW   = 4u;     // N + I > E (A14)
 
 // per-cloud scalar slots (u64)
@@ -218,7 +219,7 @@ struct WordCount  // bitmap words of the level's internal nodes
 };
 
 // ------------------------------------------------------------------------------------------------
-// Batched exclusive scans: one independent scan per cloud, grid (BATCH_SCAN_X, B), in the three
+// Batched exclusive scans: one independent scan per cloud, grid (BATCH_SCAN_X, B), in the two
 // launches of scanExclusive. A job binds cloud c to {in, out, n, total, sums}.
 // ------------------------------------------------------------------------------------------------
 
@@ -245,32 +246,14 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kScanReduceB(Job job)
 }
 
 template <typename V, typename Job>
-static __global__ __launch_bounds__(SCAN_THREADS) void kScanTilesB(Job job, uint32_t blocks)
-{
-    __shared__ V lds[SCAN_ITEMS * SCAN_WAVES];
-    const auto j = job.bind(blockIdx.y);
-    V* sums      = reinterpret_cast<V*>(j.sums);
-    V carry      = 0;
-    for (uint64_t base = 0; base < blocks; base += SCAN_TILE)
-    {
-        V v[SCAN_ITEMS], pre[SCAN_ITEMS];
-        loadTile<V>([sums](uint64_t i) { return sums[i]; }, base, blocks, v);
-        const V chunk = tileExclusiveScan(v, pre, lds);
-        storeTile<V>([sums](uint64_t i, V p, V) { sums[i] = p; }, base, blocks, v, pre, carry);
-        carry += chunk;
-    }
-    if (threadIdx.x == 0)
-        j.setTotal(carry);
-}
-
-template <typename V, typename Job>
 static __global__ __launch_bounds__(SCAN_THREADS) void kScanDownB(Job job)
 {
     __shared__ V lds[SCAN_ITEMS * SCAN_WAVES];
     const auto j = job.bind(blockIdx.y);
     uint64_t first, last;
     tileRange(scanTiles(j.n), first, last);
-    V carry = reinterpret_cast<const V*>(j.sums)[blockIdx.x];
+    const V* sums = reinterpret_cast<const V*>(j.sums);
+    V carry       = blockSum(threadIdx.x < blockIdx.x ? sums[threadIdx.x] : V(0), lds);
     for (uint64_t tile = first; tile < last; ++tile)
     {
         V v[SCAN_ITEMS], pre[SCAN_ITEMS];
@@ -279,6 +262,8 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kScanDownB(Job job)
         storeTile<V>(j.out, tile * SCAN_TILE, j.n, v, pre, carry);
         carry += chunk;
     }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+        j.setTotal(carry);
 }
 
 // maxItems: an upper bound of any cloud's item count; it sizes the workgroups per cloud (each at
@@ -295,7 +280,6 @@ void scanBatch(Job job, uint32_t B, uint64_t maxItems, hipStream_t stream)
     const uint32_t X = scanWidth(maxItems);
     const dim3 grid(X, B);
     kScanReduceB<V, Job><<<grid, SCAN_THREADS, 0, stream>>>(job);
-    kScanTilesB<V, Job><<<dim3(1, B), SCAN_THREADS, 0, stream>>>(job, X);
     kScanDownB<V, Job><<<grid, SCAN_THREADS, 0, stream>>>(job);
 }
 

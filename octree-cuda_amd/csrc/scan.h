@@ -1,9 +1,10 @@
 // Device-wide exclusive prefix sum for the builder (sparse ids, leaf blocks, table slices, slots).
 //
-// Reduce-then-scan in three launches with no inter-workgroup waiting: (1) each workgroup reduces
-// its contiguous range of tiles of SCAN_TILE items, (2) one workgroup scans the per-workgroup sums,
-// (3) each workgroup rescans its tiles in order from its offset and hands (index, exclusive prefix,
-// value) to an output functor.
+// Reduce-then-scan in two launches with no inter-workgroup waiting: (1) each workgroup reduces its
+// contiguous range of tiles of SCAN_TILE items, (2) each workgroup adds up the sums of the ranges
+// before its own (at most SCAN_GRID values, one or a few per thread, from L2), rescans its tiles in
+// order from there and hands (index, exclusive prefix, value) to an output functor. A launch in
+// between that scans the sums took 4-10 us per scan, 28 to 116 us per build.
 // A tile is held striped: thread t holds items k * SCAN_THREADS + t (k < SCAN_ITEMS), so each load
 // and store instruction of a wave covers 64 consecutive items, and a full tile is read with no
 // bounds test, all SCAN_ITEMS loads in flight at once. Its scan is SCAN_ITEMS row scans (row k =
@@ -11,9 +12,9 @@
 // all rows through LDS, one barrier. Inputs and outputs are functors so the flags / values are
 // generated and consumed in the same pass as the scan (e.g. occupancy flags straight from the
 // counting grid); an output functor is called once per item, in no particular order, and may
-// write the item's own input (in-place scans). Inputs of at most SCAN_SINGLE_TILES tiles take one
-// launch of a single workgroup instead (small builds make many small scans, and every launch is a
-// runtime call).
+// write the item's own input (in-place scans). Out-of-place scans of at most SCAN_DIRECT_TILES tiles
+// take one launch (small builds make many small scans): one workgroup per tile, which reduces the
+// tiles before its own by itself.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -173,32 +174,26 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kScanReduce(In in, uint64
         blockSums[blockIdx.x] = total;
 }
 
-// exclusive scan of the per-workgroup sums, in place
+// Sum of v over the workgroup, in every thread. Contains barriers.
 template <typename T>
-static __global__ __launch_bounds__(SCAN_THREADS) void kScanTiles(T* tileSums, uint64_t tiles, T* total)
+__device__ __forceinline__ T blockSum(T v, T* lds)
 {
-    __shared__ T lds[SCAN_ITEMS * SCAN_WAVES];
-    T carry = 0;
-    for (uint64_t base = 0; base < tiles; base += SCAN_TILE)
-    {
-        T v[SCAN_ITEMS], pre[SCAN_ITEMS];
-        loadTile<T>([tileSums](uint64_t i) { return tileSums[i]; }, base, tiles, v);
-        const T chunk = tileExclusiveScan(v, pre, lds);
-        storeTile<T>([tileSums](uint64_t i, T p, T) { tileSums[i] = p; }, base, tiles, v, pre, carry);
-        carry += chunk;
-    }
-    if (threadIdx.x == 0 && total)
-        *total = carry;
+    T total;
+    (void)blockExclusiveScan(v, total, lds);
+    return total;
 }
 
 template <typename T, typename In, typename Out>
-static __global__ __launch_bounds__(SCAN_THREADS) void kScanDown(In in, Out out, uint64_t n, const T* blockOffsets,
-                                                          uint64_t tiles)
+static __global__ __launch_bounds__(SCAN_THREADS) void kScanDown(In in, Out out, uint64_t n, const T* blockSums,
+                                                          uint64_t tiles, T* total)
 {
     __shared__ T lds[SCAN_ITEMS * SCAN_WAVES];
     uint64_t first, last;
     tileRange(tiles, first, last);
-    T carry = blockOffsets[blockIdx.x];
+    T before = 0;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += SCAN_THREADS)
+        before += blockSums[b];
+    T carry = blockSum(before, lds);
     for (uint64_t tile = first; tile < last; ++tile)
     {
         T v[SCAN_ITEMS], pre[SCAN_ITEMS];
@@ -207,6 +202,48 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kScanDown(In in, Out out,
         storeTile<T>(out, tile * SCAN_TILE, n, v, pre, carry);
         carry += chunk;
     }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && total)
+        *total = carry;
+}
+
+// One launch, workgroup b for tile b: the sum of the tiles before it (two tiles' loads in flight),
+// then its own tile. The input is read while other workgroups write their outputs, so an output
+// must not write what the input reads.
+template <typename T, typename In, typename Out>
+static __global__ __launch_bounds__(SCAN_THREADS) void kScanDirect(In in, Out out, uint64_t n, T* total)
+{
+    __shared__ T lds[SCAN_ITEMS * SCAN_WAVES];
+    const uint64_t own = static_cast<uint64_t>(blockIdx.x) * SCAN_TILE;
+    T v[SCAN_ITEMS], pre[SCAN_ITEMS];
+    loadTile<T>(in, own, n, v);
+    T before = 0;
+    constexpr uint64_t STEP = 2 * SCAN_ITEMS * SCAN_THREADS;
+    uint64_t i              = threadIdx.x;
+    for (; i - threadIdx.x + STEP <= own; i += STEP)
+    {
+        T w[2 * SCAN_ITEMS];
+#pragma unroll
+        for (int k = 0; k < 2 * SCAN_ITEMS; ++k)
+            w[k] = in(i + static_cast<uint64_t>(k) * SCAN_THREADS);
+#pragma unroll
+        for (int k = 0; k < 2 * SCAN_ITEMS; ++k)
+            before += w[k];
+    }
+    if (i < own)  // an odd tile: own is a whole number of tiles
+    {
+        T w[SCAN_ITEMS];
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; ++k)
+            w[k] = in(i + static_cast<uint64_t>(k) * SCAN_THREADS);
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; ++k)
+            before += w[k];
+    }
+    const T carry = blockSum(before, lds);
+    const T chunk = tileExclusiveScan(v, pre, lds);
+    storeTile<T>(out, own, n, v, pre, carry);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && total)
+        *total = carry + chunk;
 }
 
 // Small inputs: one workgroup walks the tiles in order with a running carry. All SCAN_THREADS
@@ -228,37 +265,33 @@ __device__ __forceinline__ void blockScanAll(In in, Out out, uint64_t n, T* tota
         *total = carry;
 }
 
-// the same as one launch
-template <typename T, typename In, typename Out>
-static __global__ __launch_bounds__(SCAN_THREADS) void kScanSingle(In in, Out out, uint64_t n, T* total)
-{
-    __shared__ T lds[SCAN_ITEMS * SCAN_WAVES];
-    blockScanAll<T>(in, out, n, total, lds);
-}
-
 __host__ __device__ inline uint64_t scanTiles(uint64_t n)
 {
     return (n + SCAN_TILE - 1) / SCAN_TILE;
 }
 
-// Inputs up to this many tiles are scanned by kScanSingle.
-constexpr uint64_t SCAN_SINGLE_TILES = 16;
+// Out-of-place inputs up to this many tiles are scanned by kScanDirect: its last workgroup reads
+// all of them, SCAN_DIRECT_TILES / 2 dependent rounds of loads (16 tiles: ~6 us; one workgroup
+// walking them took ~25 us, two launches take ~9 us).
+constexpr uint64_t SCAN_DIRECT_TILES = 16;
+// Workgroups of a two-launch scan: eight of 256 threads fill each of 256 compute units.
+constexpr uint64_t SCAN_GRID = 2048;
 
 // Exclusive scan of in(0..n-1); out(i, prefix, value) for each i; *total (device) = sum.
-// tileScratch must hold scanTiles(n) values (unused for inputs of at most SCAN_SINGLE_TILES tiles).
+// tileScratch must hold scanTiles(n) values. inPlace: out writes what in reads.
 template <typename T, typename In, typename Out>
-void scanExclusive(uint64_t n, In in, Out out, T* tileScratch, T* total, hipStream_t stream)
+void scanExclusive(uint64_t n, In in, Out out, T* tileScratch, T* total, hipStream_t stream, bool inPlace = false)
 {
-    uint64_t tiles = scanTiles(n);
-    if (tiles <= SCAN_SINGLE_TILES)
+    const uint64_t tiles = scanTiles(n);
+    if (tiles <= (inPlace ? 1 : SCAN_DIRECT_TILES))
     {
-        kScanSingle<T, In, Out><<<1, SCAN_THREADS, 0, stream>>>(in, out, n, total);
+        kScanDirect<T, In, Out><<<static_cast<unsigned>(tiles ? tiles : 1), SCAN_THREADS, 0, stream>>>(in, out, n,
+                                                                                                       total);
         return;
     }
-    unsigned grid = static_cast<unsigned>(tiles < 8192 ? tiles : 8192);
+    const unsigned grid = static_cast<unsigned>(tiles < SCAN_GRID ? tiles : SCAN_GRID);
     kScanReduce<T, In><<<grid, SCAN_THREADS, 0, stream>>>(in, n, tileScratch, tiles);
-    kScanTiles<T><<<1, SCAN_THREADS, 0, stream>>>(tileScratch, grid, total);
-    kScanDown<T, In, Out><<<grid, SCAN_THREADS, 0, stream>>>(in, out, n, tileScratch, tiles);
+    kScanDown<T, In, Out><<<grid, SCAN_THREADS, 0, stream>>>(in, out, n, tileScratch, tiles, total);
 }
 
 }  // namespace oc

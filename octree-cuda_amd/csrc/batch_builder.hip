@@ -86,6 +86,7 @@ BatchLevels levelsOf(uint32_t G)
     L.lc      = std::min<uint32_t>(MAX_COARSE_LEVEL, L.depth > 3 ? L.depth - 3 : 0);
     const uint32_t bg = G >> L.lc;
     L.buckets = bg * bg * bg;
+    L.marked  = L.lc == MAX_COARSE_LEVEL ? L.offset[BIT_LEVELS] : 0;
     return L;
 }
 
@@ -165,6 +166,7 @@ void carveCloud(Carver& cv, BatchCloud<T>& cc, const BatchRequest& r, const Clou
     }
     cv.take(cc.count, L.dense);
     cv.take(cc.denseToSparse, L.dense);
+    cv.take(cc.occ, (static_cast<uint64_t>(L.dense) + 31) / 32);
     cv.take(cc.nodeKey, s.mBound);
     cv.take(cc.nodeCount, s.mBound);
     cv.take(cc.scanSums, BATCH_SCAN_X);
@@ -509,7 +511,7 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
 
     // ---- segment 1: count, pyramid, canonical ids, level starts ---------------------------------
     auto segment1 = [&]() {
-    kBatchInit<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B0, L.buckets);
+    kBatchInit<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B0, L);
     OC_LAUNCH_CHECK();
     const uint32_t fineBits = 3 * L.lc;
     kBucketHistB<T><<<LG.sortGrid, HIST_THREADS, 0, s>>>(ctx, B0, slot(P_HIST), fineBits, L.buckets);
@@ -518,14 +520,14 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
     OC_LAUNCH_CHECK();
     kBucketScatterB<T><<<LG.sortGrid, SCATTER_THREADS, 0, s>>>(ctx, B0, slot(P_SCATTER), fineBits);
     OC_LAUNCH_CHECK();
-    kFineSortB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, fp, L.buckets);
+    kFineSortB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, fp, L.buckets, L.marked != 0);
     OC_LAUNCH_CHECK();
     if (split)
     {
         kSplitChunksB<T><<<std::min<uint32_t>(B0, 1024), SCAN_THREADS, 0, s>>>(ctx, B0, L.buckets);
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(ScalarCount<T>{ctx, BS_SPLIT, false}, B0, slot(P_SPLIT));
         kFineChunkHistB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), L.lc);
-        kFineSplitScanB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), fp);
+        kFineSplitScanB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), fp, L.marked != 0);
         kFineChunkPermB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), L.lc);
         OC_LAUNCH_CHECK();
     }
@@ -536,7 +538,9 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
                                                         L.grid[l - 1]);
         OC_LAUNCH_CHECK();
     }
-    scanBatch<uint32_t>(OccupancyJob<T>{ctx, L.dense}, B0, L.dense, s);
+    kOccupancyBitsB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B0, L);
+    const uint64_t words = (static_cast<uint64_t>(L.dense) + 31) / 32;
+    scanBatch<uint32_t>(OccupancyJob<T>{ctx, words}, B0, words, s);
     OC_LAUNCH_CHECK();
     kLevelStartsB<T><<<B0, 64, 0, s>>>(ctx, lo);
     OC_LAUNCH_CHECK();

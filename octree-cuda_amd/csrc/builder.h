@@ -123,8 +123,8 @@ private:
     template <typename T>
     void countPoints();
     void mergeLevels();
-    // whether the fine sort writes the level-0 occupancy bits (a bucket's level-0 rows are 32 cells)
-    bool levelZeroBits() const;
+    // whether the fine sort writes the occupancy bits of the BIT_LEVELS lowest levels
+    bool fineSortBits() const;
     template <typename T>
     void distributePoints();
     template <typename T>

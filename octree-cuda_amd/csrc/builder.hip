@@ -424,9 +424,7 @@ void OctreeBuilder::generate()
 template <typename T>
 void OctreeBuilder::generateTyped()
 {
-    uint64_t* sc = itsScalars.as<uint64_t>();
-    kFill64<<<1, BLOCK, 0, itsStream>>>(sc, SC_COUNT, 0);
-    OC_LAUNCH_CHECK();
+    uint64_t* sc  = itsScalars.as<uint64_t>();
     itsBatchesRun = 0;
 
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_START], itsStream));
@@ -482,7 +480,10 @@ void OctreeBuilder::countPoints()
     Gridding g{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2], itsCloud.bbMax[0] - itsCloud.bbMin[0],
                itsProc.chunkingGrid};
     itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(nb) + 1));
-    kFill32<<<gridFor(nb + 1), BLOCK, 0, itsStream>>>(bucketCount, nb + 1, 0);
+    uint32_t* occ = fineSortBits() ? itsOccupancy.as<uint32_t>() : nullptr;
+    const uint64_t marked = occ ? itsLevelOffset[BIT_LEVELS] : 0;
+    kBuildInit<<<gridFor(std::max<uint64_t>(nb, marked / 32), 2048), BLOCK, 0, itsStream>>>(
+            sc, bucketCount, nb + 1, occ, marked / 32, itsCount.as<uint32_t>(), marked, occ ? itsDense : 0);
     OC_LAUNCH_CHECK();
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_COUNT_BEGIN], itsStream));
 
@@ -508,10 +509,8 @@ void OctreeBuilder::countPoints()
         fp.levelOffset[l] = itsLevelOffset[l];
         fp.levelGrid[l]   = itsLevelGrid[l];
     }
-    // the level-0 occupancy bits with the counts where a bucket row is a whole bitmap word
-    uint32_t* occ0 = levelZeroBits() ? itsOccupancy.as<uint32_t>() : nullptr;
     kFineSort<<<nb, SORT_THREADS, 0, itsStream>>>(itsFineCode.as<uint16_t>(), bucketStart, fp,
-                                                  itsCount.as<uint32_t>(), itsPerm.as<uint32_t>(), occ0);
+                                                  itsCount.as<uint32_t>(), itsPerm.as<uint32_t>(), occ);
     OC_LAUNCH_CHECK();
     if (n > FINE_SPLIT)
     {
@@ -530,7 +529,7 @@ void OctreeBuilder::countPoints()
         OC_LAUNCH_CHECK();
         kFineSplitScan<<<grid, SORT_THREADS, 0, itsStream>>>(bucketStart, itsSplitChunks.as<uint64_t>(), chunkCount,
                                                              fp, itsCount.as<uint32_t>(), itsSplitHist.as<uint32_t>(),
-                                                             occ0);
+                                                             occ);
         OC_LAUNCH_CHECK();
         kFineChunkPerm<<<grid, SORT_THREADS, 0, itsStream>>>(itsFineCode.as<uint16_t>(), bucketStart,
                                                              itsSplitChunks.as<uint64_t>(), chunkCount, fp.lc,
@@ -540,10 +539,10 @@ void OctreeBuilder::countPoints()
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_COUNT_END], itsStream));  // the records move with the distribution
 }
 
-bool OctreeBuilder::levelZeroBits() const
+bool OctreeBuilder::fineSortBits() const
 {
-    // 32-cell rows starting at multiples of 32, and level 1 starting at a multiple of 64
-    return itsCoarse == MAX_COARSE_LEVEL && itsProc.chunkingGrid % 64 == 0;
+    // 32^3-cell buckets: chunking grids of 256 and 512, whose levels also start at multiples of 64
+    return itsCoarse == MAX_COARSE_LEVEL;
 }
 
 void OctreeBuilder::mergeLevels()
@@ -560,7 +559,7 @@ void OctreeBuilder::mergeLevels()
     // occupancy bits of the levels the fine sort has not marked, then sparse ids (A2) + node keys /
     // counts + first id of every level, by one scan over the bitmap's words
     uint32_t* occ         = itsOccupancy.as<uint32_t>();
-    const uint64_t marked = levelZeroBits() ? itsLevelOffset[1] : 0;
+    const uint64_t marked = fineSortBits() ? itsLevelOffset[BIT_LEVELS] : 0;
     kOccupancyBits<<<gridFor(itsDense - marked), BLOCK, 0, itsStream>>>(count, marked, itsDense, occ);
     OC_LAUNCH_CHECK();
     uint32_t* levelStart = reinterpret_cast<uint32_t*>(sc + SC_LEVEL_START);
@@ -621,7 +620,7 @@ void OctreeBuilder::mergeLevels()
     lp.depth     = itsDepth;
     lp.threshold = itsProc.mergingThreshold;
     kNodeLinks<<<gridFor(m), BLOCK, 0, itsStream>>>(
-            itsM, lp, itsNodeKey.as<uint32_t>(), itsNodeCount.as<uint32_t>(), count, itsDenseToSparse.as<int32_t>(),
+            itsM, lp, itsNodeKey.as<uint32_t>(), itsNodeCount.as<uint32_t>(), itsDenseToSparse.as<int32_t>(),
             itsNodePoints.as<uint32_t>(), itsNodeData.as<uint64_t>(), itsNodeParent.as<int32_t>(),
             itsNodeChild.as<int32_t>(), itsNodeFlags.as<uint8_t>(), itsNodeAux.as<uint32_t>(),
             itsNodeSub.as<uint32_t>(), occ);

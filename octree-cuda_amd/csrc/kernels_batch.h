@@ -77,6 +77,7 @@ struct BatchCloud
     uint32_t* splitHist;
     uint32_t* count;
     int32_t* denseToSparse;
+    uint32_t* occ;  // one bit per dense cell
     uint32_t *nodeKey, *nodeCount;  // bounded by min(D, (depth + 1) N)
     // nodes
     uint32_t* nodePoints;
@@ -130,6 +131,7 @@ struct BatchLevels
     uint32_t grid[MAX_LEVELS];
     uint32_t nodes[MAX_LEVELS];
     uint32_t dense;
+    uint32_t marked;  // cells of the levels whose occupancy bits the fine sort writes (0: none)
 };
 
 // The cloud of item i: the last c with prefix[c] <= i (prefix[B] = total > i).
@@ -315,12 +317,13 @@ template <typename T>
 struct OccupancyJob
 {
     const BatchCloud<T>* ctx;
-    uint64_t dense;
+    uint64_t words;
     __device__ auto bind(uint32_t c) const
     {
         const BatchCloud<T>& cc = ctx[c];
-        return bound(OccupiedIn{cc.count}, OccupiedOut{cc.denseToSparse, cc.nodeKey, cc.nodeCount, cc.count}, dense,
-                     cc.scanSums, cc.sc + BS_M);
+        return bound(OccupiedWordIn{cc.occ},
+                     OccupiedWordOut{cc.occ, cc.denseToSparse, cc.nodeKey, cc.nodeCount, cc.count}, words, cc.scanSums,
+                     cc.sc + BS_M);
     }
 };
 
@@ -444,19 +447,51 @@ struct PlacedChunkJob
 // Count stage
 // ------------------------------------------------------------------------------------------------
 
-// zero scalars and bucket counts of every cloud
+// What every cloud starts from: zero scalars and bucket counts, and with the fine sort's occupancy
+// bits the bitmap of the levels it marks and the counts of the others (as kBuildInit).
 template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kBatchInit(const BatchCloud<T>* __restrict__ ctx, uint32_t B, uint32_t buckets)
+static __global__ __launch_bounds__(BLOCK) void kBatchInit(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
+                                                     BatchLevels L)
 {
-    const uint64_t per = BS_SLOTS + buckets + 1;
+    const uint32_t words = L.marked / 32, counts = L.marked ? L.dense - L.marked : 0;
+    const uint64_t per = BS_SLOTS + L.buckets + 1 + words + counts;
     for (uint64_t i = globalThread(); i < per * B; i += globalStride())
     {
         const BatchCloud<T>& cc = ctx[i / per];
-        const uint32_t k        = static_cast<uint32_t>(i % per);
+        uint32_t k              = static_cast<uint32_t>(i % per);
         if (k < BS_SLOTS)
+        {
             cc.sc[k] = (k == BS_CURSOR) ? cc.n : 0;
+            continue;
+        }
+        k -= BS_SLOTS;
+        if (k <= L.buckets)
+        {
+            cc.bucketCount[k] = 0;
+            continue;
+        }
+        k -= L.buckets + 1;
+        if (k < words)
+            cc.occ[k] = 0;
         else
-            cc.bucketCount[k - BS_SLOTS] = 0;
+            cc.count[L.marked + (k - words)] = 0;
+    }
+}
+
+// Occupancy bits of the levels the fine sort has not marked, from their counts (as kOccupancyBits:
+// whole waves of 64 consecutive cells, two words).
+template <typename T>
+static __global__ __launch_bounds__(BLOCK) void kOccupancyBitsB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
+                                                          BatchLevels L)
+{
+    const uint64_t per = (static_cast<uint64_t>(L.dense) - L.marked + 63) / 64 * 64;
+    for (uint64_t i = globalThread(); i < per * B; i += globalStride())
+    {
+        const BatchCloud<T>& cc = ctx[i / per];
+        const uint64_t d        = L.marked + i % per;
+        const uint64_t bits     = __ballot(d < L.dense && cc.count[d] != 0);
+        if ((threadIdx.x & 31) == 0 && d < L.dense)
+            cc.occ[d >> 5] = static_cast<uint32_t>(bits >> (threadIdx.x & 32));
     }
 }
 
@@ -535,7 +570,7 @@ static __global__ __launch_bounds__(SCATTER_THREADS) void kBucketScatterB(const 
 // items: (cloud, bucket)
 template <typename T>
 static __global__ __launch_bounds__(SORT_THREADS) void kFineSortB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                            FineSortParams fp, uint32_t buckets)
+                                                            FineSortParams fp, uint32_t buckets, bool bits)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS + 1];
     __shared__ uint32_t scratch[SORT_WAVES];
@@ -543,7 +578,8 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineSortB(const BatchClo
     for (uint32_t item = blockIdx.x; item < total; item += gridDim.x)
     {
         const BatchCloud<T>& cc = ctx[item / buckets];
-        fineSortBucket(item % buckets, cc.fineCode, cc.bucketStart, fp, cc.count, cc.perm, h, scratch);
+        fineSortBucket(item % buckets, cc.fineCode, cc.bucketStart, fp, cc.count, cc.perm, h, scratch,
+                       bits ? cc.occ : nullptr);
         __syncthreads();
     }
 }
@@ -585,7 +621,7 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineChunkHistB(const Bat
 template <typename T>
 static __global__ __launch_bounds__(SORT_THREADS) void kFineSplitScanB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
                                                                  const uint32_t* __restrict__ prefix,
-                                                                 FineSortParams fp)
+                                                                 FineSortParams fp, bool bits)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS + 1];
     __shared__ uint32_t scratch[SORT_WAVES];
@@ -597,7 +633,8 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineSplitScanB(const Bat
         const uint32_t chunk    = item - prefix[c];
         if (static_cast<uint32_t>(cc.splitChunks[chunk]) != 0)
             continue;  // not the first chunk of its bucket (uniform over the workgroup)
-        fineSplitScan(chunk, cc.bucketStart, cc.splitChunks, fp, cc.count, cc.splitHist, h, scratch);
+        fineSplitScan(chunk, cc.bucketStart, cc.splitChunks, fp, cc.count, cc.splitHist, h, scratch,
+                      bits ? cc.occ : nullptr);
         __syncthreads();
     }
 }
@@ -666,8 +703,8 @@ static __global__ __launch_bounds__(BLOCK) void kNodeLinksB(const BatchCloud<T>*
         const uint32_t c        = findCloud(wp, B, static_cast<uint32_t>(i));
         const BatchCloud<T>& cc = ctx[c];
         const uint32_t id       = static_cast<uint32_t>(i) - wp[c];
-        nodeLinksOf(id, levelParams(L, cc.threshold), cc.nodeKey, cc.nodeCount, cc.count, cc.denseToSparse, cc.nodePoints,
-                    cc.nodeData, cc.nodeParent, cc.nodeChild, cc.nodeFlags, cc.nodeAux, cc.nodeSub);
+        nodeLinksOf(id, levelParams(L, cc.threshold), cc.nodeKey, cc.nodeCount, cc.denseToSparse, cc.nodePoints,
+                    cc.nodeData, cc.nodeParent, cc.nodeChild, cc.nodeFlags, cc.nodeAux, cc.nodeSub, cc.occ);
         cc.keyOut[id]   = cc.nodeKey[id];
         cc.countOut[id] = cc.nodeCount[id];
     }

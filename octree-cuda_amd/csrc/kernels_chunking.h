@@ -49,6 +49,24 @@ static __global__ __launch_bounds__(BLOCK) void kFill64(uint64_t* p, uint64_t n,
         p[i] = v;
 }
 
+// What a build starts from, cleared in one launch: the scalars, the bucket counts, and with the fine
+// sort's occupancy bits the bitmap words [0, words) and the counts [first, last) of the levels whose
+// bits come from the counts.
+static __global__ __launch_bounds__(BLOCK) void kBuildInit(uint64_t* __restrict__ sc, uint32_t* __restrict__ bucketCount,
+                                                     uint32_t buckets, uint32_t* __restrict__ occ, uint64_t words,
+                                                     uint32_t* __restrict__ count, uint64_t first, uint64_t last)
+{
+    const uint64_t i = globalThread();
+    if (i < SC_COUNT)
+        sc[i] = 0;
+    for (uint64_t b = i; b < buckets; b += globalStride())
+        bucketCount[b] = 0;
+    for (uint64_t w = i; w < words; w += globalStride())
+        occ[w] = 0;
+    for (uint64_t d = first + i; d < last; d += globalStride())
+        count[d] = 0;
+}
+
 // K2 (counts only): kernelPropagatePointCounts (point_count_propagation.cuh:34-86). Child slot k
 // of parent (x, y, z) is (2x + (k>>2 & 1), 2y + (k>>1 & 1), 2z + (k & 1)).
 __device__ __forceinline__ void propagateOne(uint32_t idx, uint32_t* __restrict__ count, uint32_t offset,
@@ -87,7 +105,8 @@ static __global__ __launch_bounds__(BLOCK) void kOccupancyBits(const uint32_t* _
 }
 
 // Sparse ids (A2) from the occupancy bitmap, one scan item per word: the exclusive rank of an
-// occupied dense cell; its node key and dense count are written in the same pass.
+// occupied dense cell; its node key and dense count are written in the same pass. denseToSparse is
+// written for occupied cells only: an array of D entries is never filled with -1.
 struct OccupiedWordIn
 {
     const uint32_t* occ;
@@ -112,33 +131,6 @@ struct OccupiedWordOut
             nodeKey[prefix]   = static_cast<uint32_t>(d);
             nodeCount[prefix] = count[d];
             ++prefix;
-        }
-    }
-};
-
-struct OccupiedIn
-{
-    const uint32_t* count;
-    __device__ uint32_t operator()(uint64_t d) const { return count[d] ? 1u : 0u; }
-};
-
-// Sparse id = exclusive rank of the occupied dense cell (A2); the node's key and dense count are
-// written in the same pass.
-// denseToSparse is written for occupied cells only (a cell is occupied where its dense count is
-// not zero): an array of D entries is never filled with -1.
-struct OccupiedOut
-{
-    int32_t* denseToSparse;
-    uint32_t* nodeKey;
-    uint32_t* nodeCount;
-    const uint32_t* count;
-    __device__ void operator()(uint64_t d, uint32_t prefix, uint32_t v) const
-    {
-        if (v)
-        {
-            denseToSparse[d]  = static_cast<int32_t>(prefix);
-            nodeKey[prefix]   = static_cast<uint32_t>(d);
-            nodeCount[prefix] = count[d];
         }
     }
 };
@@ -200,12 +192,11 @@ __device__ __forceinline__ uint32_t levelOfKey(uint32_t key, const LevelParams& 
 // and the size of the leaf data block an internal node hands out to its leaf children.
 __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, const uint32_t* __restrict__ nodeKey,
                                             const uint32_t* __restrict__ nodeCount,
-                                            const uint32_t* __restrict__ denseCount,
                                             const int32_t* __restrict__ denseToSparse,
                                             uint32_t* __restrict__ pointCount, uint64_t* __restrict__ dataIdx,
                                             int32_t* __restrict__ parent, int32_t* __restrict__ children,
                                             uint8_t* __restrict__ flags, uint32_t* __restrict__ blockSize,
-                                            uint32_t* __restrict__ subtree, const uint32_t* __restrict__ occ = nullptr)
+                                            uint32_t* __restrict__ subtree, const uint32_t* __restrict__ occ)
 {
     {
         uint32_t key = nodeKey[id];
@@ -232,9 +223,9 @@ __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, 
             {
                 uint32_t cx = 2 * x + ((k >> 2) & 1), cy = 2 * y + ((k >> 1) & 1), cz = 2 * z + (k & 1);
                 const uint32_t cd = lp.offset[l - 1] + cx + cy * cg + cz * cg * cg;
-                // occupancy from the bitmap where there is one (level-0 counts of empty cells are
-                // not written then); denseToSparse is set for occupied cells only
-                const bool occupied = occ ? ((occ[cd >> 5] >> (cd & 31)) & 1u) != 0 : denseCount[cd] != 0;
+                // occupancy from the bitmap (the counts of empty cells of the lowest levels are not
+                // written); denseToSparse is set for occupied cells only
+                const bool occupied = ((occ[cd >> 5] >> (cd & 31)) & 1u) != 0;
                 int32_t c           = occupied ? denseToSparse[cd] : -1;
                 children[8 * static_cast<uint64_t>(id) + k] = c;
                 if (internal && c >= 0)
@@ -262,7 +253,6 @@ __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, 
 
 static __global__ __launch_bounds__(BLOCK) void kNodeLinks(uint32_t m, LevelParams lp, const uint32_t* __restrict__ nodeKey,
                                                      const uint32_t* __restrict__ nodeCount,
-                                                     const uint32_t* __restrict__ denseCount,
                                                      const int32_t* __restrict__ denseToSparse,
                                                      uint32_t* __restrict__ pointCount, uint64_t* __restrict__ dataIdx,
                                                      int32_t* __restrict__ parent,
@@ -271,7 +261,7 @@ static __global__ __launch_bounds__(BLOCK) void kNodeLinks(uint32_t m, LevelPara
                                                      uint32_t* __restrict__ subtree, const uint32_t* __restrict__ occ)
 {
     for (uint64_t i = globalThread(); i < m; i += globalStride())
-        nodeLinksOf(static_cast<uint32_t>(i), lp, nodeKey, nodeCount, denseCount, denseToSparse, pointCount, dataIdx,
+        nodeLinksOf(static_cast<uint32_t>(i), lp, nodeKey, nodeCount, denseToSparse, pointCount, dataIdx,
                     parent, children, flags, blockSize, subtree, occ);
 }
 

@@ -318,13 +318,18 @@ struct FineSortParams
     uint32_t levelGrid[MAX_LEVELS];
 };
 
+// Levels whose occupancy bits the fine sort writes when it gets the bitmap (lc = 5, chunking grid
+// >= 256): a bucket's rows of levels 0, 1 and 2 are 32, 16 and 8 cells from a multiple of that, one
+// word, half-word and byte of the bitmap, so each row is stored whole by one lane, no atomics.
+constexpr uint32_t BIT_LEVELS = 3;
+
 // Dense counts of bucket b's cells on levels 0..lc (kernelPropagatePointCounts,
 // point_count_propagation.cuh:34-86, as differences of the Morton prefix h over the bucket's
-// fine cells; h null: an empty bucket, all zero). With occ and 32-cell rows (lc = 5), the
-// level-0 occupancy bits instead of the level-0 zero counts: a wave writes two whole rows, 32
-// consecutive cells from a multiple of 32, so each row is one word of the bitmap, written whole,
-// no atomics; the count of a level-0 cell is then written only where it is not zero (the later
-// passes read level-0 counts of occupied cells only, and test occupancy on the bitmap).
+// fine cells; h null: an empty bucket, all zero). With occ, the occupancy bits of levels 0..2 as
+// well, and only what is not zero: the bitmap of those levels and the counts of the others have
+// been cleared, and the later passes read the counts of levels 0..2 for occupied cells only
+// (storing those levels' zero counts was 77 MB per 512^3 build whatever the cloud's size: the fine
+// sort and kOccupancyBits took 147 + 35 us of a 200K-point build, now 108 + 4 after 6 us of clearing).
 __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& fp, const uint32_t* h,
                                              uint32_t* __restrict__ count, uint32_t* __restrict__ occ = nullptr)
 {
@@ -335,18 +340,6 @@ __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& f
         const uint32_t n3     = side * side * side;
         const uint64_t gk     = fp.levelGrid[k];
         const uint64_t offset = fp.levelOffset[k];
-        const bool bits       = k == 0 && occ && side == 32;
-        if (bits && !h)
-        {
-            // an empty bucket: its 32 x 32 rows of level 0 are zero words
-            for (uint32_t r = threadIdx.x; r < side * side; r += SORT_THREADS)
-            {
-                const uint64_t gy = static_cast<uint64_t>(by) * side + (r % side),
-                               gz = static_cast<uint64_t>(bz) * side + (r / side);
-                occ[(offset + static_cast<uint64_t>(bx) * side + gy * gk + gz * gk * gk) >> 5] = 0;
-            }
-            continue;
-        }
         for (uint32_t j = threadIdx.x; j < n3; j += SORT_THREADS)
         {
             const uint32_t lx = j & (side - 1), ly = (j >> (fp.lc - k)) & (side - 1), lz = j >> (2 * (fp.lc - k));
@@ -359,13 +352,20 @@ __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& f
             const uint64_t gx = static_cast<uint64_t>(bx) * side + lx, gy = static_cast<uint64_t>(by) * side + ly,
                            gz = static_cast<uint64_t>(bz) * side + lz;
             const uint64_t d = offset + gx + gy * gk + gz * gk * gk;
-            if (!bits || v)
+            if (!occ || v)
                 count[d] = v;
-            if (bits)  // uniform; every lane of the wave is here (n3 % SORT_THREADS == 0)
+            if (occ && k < BIT_LEVELS)  // uniform; every lane of the wave is here (n3 is a multiple of 64)
             {
-                const uint64_t set = __ballot(v != 0);
-                if ((threadIdx.x & 31) == 0)
-                    occ[d >> 5] = static_cast<uint32_t>(set >> (threadIdx.x & 32));
+                const uint64_t set = __ballot(v != 0) >> (threadIdx.x & (64 - side) & 63);
+                if (lx == 0 && (set & ((1ull << side) - 1)))
+                {
+                    if (k == 0)
+                        occ[d >> 5] = static_cast<uint32_t>(set);
+                    else if (k == 1)
+                        reinterpret_cast<uint16_t*>(occ)[d >> 4] = static_cast<uint16_t>(set);
+                    else
+                        reinterpret_cast<uint8_t*>(occ)[d >> 3] = static_cast<uint8_t>(set);
+                }
             }
         }
     }
@@ -488,7 +488,8 @@ __device__ __forceinline__ void fineSortBucket(uint32_t b, const uint16_t* __res
     if (lo == hi)
     {
         // an empty bucket (most of them in a sparse cloud): zero counts, no histogram, no scan
-        bucketCounts(b, fp, nullptr, count, occ);
+        if (!occ)
+            bucketCounts(b, fp, nullptr, count);
         return;
     }
 

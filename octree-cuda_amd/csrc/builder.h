@@ -187,7 +187,7 @@ private:
             itsNodeSorted, itsNodeAux, itsNodeStage, itsNodeSub, itsNodeRegion;
 
     // Morton bucket sort of the cloud
-    DeviceBuffer itsBucketed, itsSorted, itsFineCode, itsPerm, itsBucketCount, itsBucketStart, itsBucketCursor;
+    DeviceBuffer itsBucketed, itsSorted, itsFineCode, itsPerm, itsBucketCount, itsBucketStart, itsBucketCursor, itsBucketList;
     DeviceBuffer itsSplitChunks, itsSplitHist;  // the fine sort's split buckets: chunk list, per-chunk histograms
 
     // output region [0, E) (lut: point index, out: 18-byte record): leaf points at [0, N), internal

@@ -217,6 +217,7 @@ void OctreeBuilder::setup(const CloudInfo& cloud, const ProcessingInfo& proc, co
     itsBucketCount.ensure(sizeof(uint32_t) * (itsBuckets + 1));
     itsBucketStart.ensure(sizeof(uint32_t) * (itsBuckets + 1));
     itsBucketCursor.ensure(sizeof(uint32_t) * (itsBuckets + 1));
+    itsBucketList.ensure(sizeof(uint32_t) * itsBuckets);
     itsStLut.ensure(sizeof(uint32_t) * stagedCap);
     itsStOut.ensure(sizeof(OutRecord) * stagedCap);
     itsStPts.ensure(coordBytes * stagedCap);
@@ -242,7 +243,7 @@ std::vector<DeviceBuffer*> OctreeBuilder::arena()
             &itsNodeData,    &itsNodeParent,  &itsNodeChild,     &itsNodeFlags,    &itsNodeSorted,  &itsNodeAux,
             &itsNodeStage,   &itsNodeSub,     &itsNodeRegion,    &itsBucketed,     &itsSorted,      &itsFineCode,
             &itsPerm,
-            &itsBucketCount, &itsBucketStart, &itsBucketCursor,  &itsLut,          &itsOut,
+            &itsBucketCount, &itsBucketStart, &itsBucketCursor,  &itsBucketList,  &itsLut,          &itsOut,
             &itsStLut,       &itsStOut,       &itsStPts,         &itsStRgb,        &itsInternalList, &itsSegCount,    &itsSegSrc,
             &itsSegTile,     &itsSegInput,    &itsNodeGrid,      &itsTileList,     &itsBitmap,      &itsPrefix,
             &itsNodeFirst,   &itsWin,         &itsColor,         &itsCellCnt,      &itsCellStart,   &itsCellKey,
@@ -482,8 +483,8 @@ void OctreeBuilder::countPoints()
     itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(nb) + 1));
     uint32_t* occ = fineSortBits() ? itsOccupancy.as<uint32_t>() : nullptr;
     const uint64_t marked = occ ? itsLevelOffset[BIT_LEVELS] : 0;
-    kBuildInit<<<gridFor(std::max<uint64_t>(nb, marked / 32), 2048), BLOCK, 0, itsStream>>>(
-            sc, bucketCount, nb + 1, occ, marked / 32, itsCount.as<uint32_t>(), marked, occ ? itsDense : 0);
+    kBuildInit<<<gridFor(std::max<uint64_t>({nb, marked / 32, itsDense - marked}), 2048), BLOCK, 0, itsStream>>>(
+            sc, bucketCount, nb + 1, occ, marked / 32, itsCount.as<uint32_t>(), marked, itsDense);
     OC_LAUNCH_CHECK();
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_COUNT_BEGIN], itsStream));
 
@@ -492,8 +493,14 @@ void OctreeBuilder::countPoints()
                                                                3 * itsCoarse, nb, bucketCount,
                                                                reinterpret_cast<uint32_t*>(sc + SC_ERROR));
     OC_LAUNCH_CHECK();
-    scanExclusive<uint32_t>(nb, ArrayIn{bucketCount}, BucketStartOut{bucketStart, bucketCursor},
-                            itsScanScratch.as<uint32_t>(), bucketStart + nb, itsStream);
+    // buckets above FINE_SPLIT points, a chunk per workgroup (at most 2 n / FINE_SPLIT chunks)
+    const uint64_t chunkBound = 2ull * n / FINE_SPLIT + 1;
+    itsSplitChunks.ensure(sizeof(uint64_t) * chunkBound);
+    const uint64_t* totals = sc + SC_BUCKETS;
+    scanExclusive<uint64_t>(nb, BucketIn{bucketCount},
+                            BucketTablesOut{bucketStart, bucketCursor, itsBucketList.as<uint32_t>(),
+                                            itsSplitChunks.as<uint64_t>(), nb},
+                            itsScanScratch.as<uint64_t>(), sc + SC_BUCKETS, itsStream);
     OC_LAUNCH_CHECK();
     const unsigned scatterBlocks = static_cast<unsigned>((static_cast<uint64_t>(n) + STAGE_CHUNK - 1) / STAGE_CHUNK);
     kBucketScatter<T><<<scatterBlocks, SCATTER_THREADS, 0, itsStream>>>(itsCloudDevice, n, itsCloud.dataStride, g,
@@ -509,30 +516,25 @@ void OctreeBuilder::countPoints()
         fp.levelOffset[l] = itsLevelOffset[l];
         fp.levelGrid[l]   = itsLevelGrid[l];
     }
-    kFineSort<<<nb, SORT_THREADS, 0, itsStream>>>(itsFineCode.as<uint16_t>(), bucketStart, fp,
-                                                  itsCount.as<uint32_t>(), itsPerm.as<uint32_t>(), occ);
+    kFineSort<<<std::min<uint32_t>(nb, COMPUTE_UNITS), SORT_THREADS, 0, itsStream>>>(
+            itsFineCode.as<uint16_t>(), bucketStart, itsBucketList.as<uint32_t>(), totals,
+            reinterpret_cast<uint32_t*>(sc + SC_NEXT_BUCKET), fp, itsCount.as<uint32_t>(), itsPerm.as<uint32_t>(),
+            occ);
     OC_LAUNCH_CHECK();
     if (n > FINE_SPLIT)
     {
-        // buckets above FINE_SPLIT points, a chunk per workgroup (at most 2 n / FINE_SPLIT chunks)
-        const uint64_t bound = 2ull * n / FINE_SPLIT + 1;
-        itsSplitChunks.ensure(sizeof(uint64_t) * bound);
-        itsSplitHist.ensure(sizeof(uint32_t) * MAX_FINE_CELLS * bound);
-        uint32_t* chunkCount = reinterpret_cast<uint32_t*>(itsScalars.as<uint64_t>() + SC_SPLIT);
-        scanExclusive<uint32_t>(nb, SplitChunksIn{bucketStart}, SplitChunksOut{itsSplitChunks.as<uint64_t>()},
-                                itsScanScratch.as<uint32_t>(), chunkCount, itsStream);
-        OC_LAUNCH_CHECK();
-        const unsigned grid = static_cast<unsigned>((bound + XCD_COUNT - 1) / XCD_COUNT * XCD_COUNT);
+        itsSplitHist.ensure(sizeof(uint32_t) * MAX_FINE_CELLS * chunkBound);
+        const unsigned grid = static_cast<unsigned>((chunkBound + XCD_COUNT - 1) / XCD_COUNT * XCD_COUNT);
         kFineChunkHist<<<grid, SORT_THREADS, 0, itsStream>>>(itsFineCode.as<uint16_t>(), bucketStart,
-                                                             itsSplitChunks.as<uint64_t>(), chunkCount, fp.lc,
+                                                             itsSplitChunks.as<uint64_t>(), totals, fp.lc,
                                                              itsSplitHist.as<uint32_t>());
         OC_LAUNCH_CHECK();
-        kFineSplitScan<<<grid, SORT_THREADS, 0, itsStream>>>(bucketStart, itsSplitChunks.as<uint64_t>(), chunkCount,
+        kFineSplitScan<<<grid, SORT_THREADS, 0, itsStream>>>(bucketStart, itsSplitChunks.as<uint64_t>(), totals,
                                                              fp, itsCount.as<uint32_t>(), itsSplitHist.as<uint32_t>(),
                                                              occ);
         OC_LAUNCH_CHECK();
         kFineChunkPerm<<<grid, SORT_THREADS, 0, itsStream>>>(itsFineCode.as<uint16_t>(), bucketStart,
-                                                             itsSplitChunks.as<uint64_t>(), chunkCount, fp.lc,
+                                                             itsSplitChunks.as<uint64_t>(), totals, fp.lc,
                                                              itsSplitHist.as<uint32_t>(), itsPerm.as<uint32_t>());
         OC_LAUNCH_CHECK();
     }

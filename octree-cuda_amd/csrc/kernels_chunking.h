@@ -21,7 +21,8 @@ enum ScalarSlot : int
     SC_LEAF_TOTAL  = 2,
     SC_SEG_TOTAL   = 3,  // packed (tiles << 32 | inputs)
     SC_TABLE_TOTAL = 4,
-    SC_SPLIT       = 5,  // chunks of the fine sort's split buckets
+    SC_BUCKETS     = 5,  // totals of the bucket tables (BucketIn)
+    SC_NEXT_BUCKET = 6,  // the fine sort's next occupied bucket
     SC_LEVEL_START = 8,  // u32[MAX_LEVELS + 1] packed into the following slots
     SC_COUNT       = 16
 };
@@ -49,9 +50,9 @@ static __global__ __launch_bounds__(BLOCK) void kFill64(uint64_t* p, uint64_t n,
         p[i] = v;
 }
 
-// What a build starts from, cleared in one launch: the scalars, the bucket counts, and with the fine
-// sort's occupancy bits the bitmap words [0, words) and the counts [first, last) of the levels whose
-// bits come from the counts.
+// What a build starts from, cleared in one launch: the scalars, the bucket counts, the bitmap words
+// [0, words) of the levels whose occupancy bits the fine sort writes (none for small grids) and the
+// counts [first, last) of the other levels.
 static __global__ __launch_bounds__(BLOCK) void kBuildInit(uint64_t* __restrict__ sc, uint32_t* __restrict__ bucketCount,
                                                      uint32_t buckets, uint32_t* __restrict__ occ, uint64_t words,
                                                      uint32_t* __restrict__ count, uint64_t first, uint64_t last)

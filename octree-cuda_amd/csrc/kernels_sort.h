@@ -41,6 +41,7 @@ constexpr int SCATTER_THREADS       = 1024;
 constexpr int STAGE_ITEMS           = 4;
 constexpr uint32_t STAGE_CHUNK      = SCATTER_THREADS * STAGE_ITEMS;   // points per scatter workgroup
 constexpr int HIST_THREADS          = 512;
+constexpr uint32_t COMPUTE_UNITS    = 256;
 constexpr uint32_t XCD_COUNT        = 8;  // workgroup b runs on XCD b mod 8, each XCD with its own L2
 
 // The item of a work list of `count` entries that this workgroup takes when XCD x is to take the
@@ -193,6 +194,51 @@ struct BucketStartOut
     }
 };
 
+// Buckets above FINE_SPLIT points are sorted by several workgroups (kFineChunkHist,
+// kFineSplitScan, kFineChunkPerm): one workgroup's time grows with its bucket, and a dense
+// cluster puts more than a million points in one bucket while the median holds a quarter of that.
+constexpr uint32_t FINE_SPLIT = 196608;
+
+__device__ __forceinline__ uint32_t splitChunksOf(uint32_t points)
+{
+    return points > FINE_SPLIT ? (points + FINE_SPLIT - 1) / FINE_SPLIT : 0u;
+}
+
+// The bucket tables in one scan: per bucket its points (low 32 bits), whether it holds any (bits
+// 32-47) and its chunks in the split path (bits 48-63; at most 2 n / FINE_SPLIT + 1 in all).
+struct BucketIn
+{
+    const uint32_t* count;
+    __device__ uint64_t operator()(uint64_t b) const
+    {
+        const uint32_t c = count[b];
+        return (static_cast<uint64_t>(splitChunksOf(c)) << 48) | (c ? 1ull << 32 : 0ull) | c;
+    }
+};
+
+// starts, scatter cursors, the list of the buckets that hold points, and the split chunks (entry:
+// bucket << 32 | part)
+struct BucketTablesOut
+{
+    uint32_t* start;  // buckets + 1
+    uint32_t* cursor;
+    uint32_t* occupied;
+    uint64_t* chunks;
+    uint32_t buckets;
+    __device__ void operator()(uint64_t b, uint64_t prefix, uint64_t v) const
+    {
+        const uint32_t first = static_cast<uint32_t>(prefix), points = static_cast<uint32_t>(v);
+        start[b]  = first;
+        cursor[b] = first;
+        if (b + 1 == buckets)
+            start[buckets] = first + points;
+        if (points)
+            occupied[(prefix >> 32) & 0xFFFF] = static_cast<uint32_t>(b);
+        for (uint32_t k = 0; k < (v >> 48); ++k)
+            chunks[(prefix >> 48) + k] = (b << 32) | k;
+    }
+};
+
 // Each workgroup takes a chunk of STAGE_CHUNK consecutive points, ranks them per bucket in LDS,
 // reserves one range per occupied bucket with a single global atomic, stages the records in LDS
 // in bucket order and writes them out so that consecutive lanes write consecutive records of one
@@ -318,6 +364,14 @@ struct FineSortParams
     uint32_t levelGrid[MAX_LEVELS];
 };
 
+// Place of fine cell c in the LDS histogram: the five bits that choose the bank take in the ten above
+// them. The counts are read along x, whose bits lie three apart in a Morton code, so unswizzled a
+// wave's 64 reads fell in 4 banks on level 0 and in one on the levels above.
+__device__ __forceinline__ uint32_t fineSlot(uint32_t c)
+{
+    return c ^ (((c >> 5) ^ (c >> 10)) & 31u);
+}
+
 // Levels whose occupancy bits the fine sort writes when it gets the bitmap (lc = 5, chunking grid
 // >= 256): a bucket's rows of levels 0, 1 and 2 are 32, 16 and 8 cells from a multiple of that, one
 // word, half-word and byte of the bitmap, so each row is stored whole by one lane, no atomics.
@@ -329,7 +383,7 @@ constexpr uint32_t BIT_LEVELS = 3;
 // well, and only what is not zero: the bitmap of those levels and the counts of the others have
 // been cleared, and the later passes read the counts of levels 0..2 for occupied cells only
 // (storing those levels' zero counts was 77 MB per 512^3 build whatever the cloud's size: the fine
-// sort and kOccupancyBits took 147 + 35 us of a 200K-point build, now 108 + 4 after 6 us of clearing).
+// sort and kOccupancyBits took 147 + 35 us of a 200K-point build, now 60 + 4 after 6 us of clearing).
 __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& fp, const uint32_t* h,
                                              uint32_t* __restrict__ count, uint32_t* __restrict__ occ = nullptr)
 {
@@ -347,7 +401,7 @@ __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& f
             if (h)
             {
                 const uint32_t m = morton3(lx, ly, lz);
-                v                = h[(m + 1) << (3 * k)] - h[m << (3 * k)];
+                v                = h[fineSlot((m + 1) << (3 * k))] - h[fineSlot(m << (3 * k))];
             }
             const uint64_t gx = static_cast<uint64_t>(bx) * side + lx, gy = static_cast<uint64_t>(by) * side + ly,
                            gz = static_cast<uint64_t>(bz) * side + lz;
@@ -371,66 +425,50 @@ __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& f
     }
 }
 
-// In place: the exclusive prefix of h[0 .. cells), the total in h[cells]. All threads; cells is a
-// power of two (8^lc). Each thread scans a run of R = cells / SORT_THREADS consecutive entries
-// around one workgroup scan of the runs' sums (a workgroup scan per SORT_THREADS entries would
-// take 32 of them, 64 barriers, per 32^3-cell bucket). A thread walks its run starting at entry
-// t mod R, so the lanes of a wave read different banks (runs of 32 words start in one bank).
+// In place: the exclusive prefix of the histogram h of `cells` cells (entries at fineSlot), the total
+// in entry `cells`. All threads; cells is a power of two (8^lc). Each thread scans a run of
+// R = cells / SORT_THREADS consecutive entries around one workgroup scan of the runs' sums (a
+// workgroup scan per SORT_THREADS entries would take 32 of them, 64 barriers, per 32^3-cell
+// bucket); fineSlot puts the lanes' k-th entries in different banks.
 __device__ __forceinline__ void bucketScan(uint32_t* h, uint32_t cells, uint32_t* scratch)
 {
     if (cells <= SORT_THREADS)
     {
         const uint32_t c = threadIdx.x;
-        const uint32_t v = c < cells ? h[c] : 0u;
+        const uint32_t v = c < cells ? h[fineSlot(c)] : 0u;
         uint32_t total;
         const uint32_t ex = sortBlockExclusiveScan(v, total, scratch);
         if (c < cells)
-            h[c] = ex;
+            h[fineSlot(c)] = ex;
         if (threadIdx.x == 0)
-            h[cells] = total;
+            h[fineSlot(cells)] = total;
         __syncthreads();
         return;
     }
-    const uint32_t R    = cells / SORT_THREADS;
-    uint32_t* run       = h + threadIdx.x * R;
-    const uint32_t from = threadIdx.x & (R - 1);
-    // the run's sum, and the sum of its entries before `from` (read last)
-    uint32_t sum = 0, before = 0;
+    const uint32_t R     = cells / SORT_THREADS;
+    const uint32_t first = threadIdx.x * R;
+    uint32_t sum         = 0;
     for (uint32_t k = 0; k < R; ++k)
-    {
-        const uint32_t i = (from + k) & (R - 1);
-        const uint32_t v = run[i];
-        sum += v;
-        before += i < from ? v : 0u;
-    }
+        sum += h[fineSlot(first + k)];
     uint32_t total;
-    const uint32_t off = sortBlockExclusiveScan(sum, total, scratch);
-    // the same walk: entries from `from` on start at off + before, the wrapped ones at off
-    uint32_t acc = off + before;
+    uint32_t acc = sortBlockExclusiveScan(sum, total, scratch);
     for (uint32_t k = 0; k < R; ++k)
     {
-        const uint32_t i = (from + k) & (R - 1);
-        if (i == 0)
-            acc = off;
-        const uint32_t v = run[i];
-        run[i]           = acc;
+        const uint32_t i = fineSlot(first + k);
+        const uint32_t v = h[i];
+        h[i]             = acc;
         acc += v;
     }
     if (threadIdx.x == 0)
-        h[cells] = total;
+        h[fineSlot(cells)] = total;
     __syncthreads();
 }
-
-// Buckets above FINE_SPLIT points are sorted by several workgroups (kFineChunkHist,
-// kFineSplitScan, kFineChunkPerm): one workgroup's time grows with its bucket, and a dense
-// cluster puts more than a million points in one bucket while the median holds a quarter of that.
-constexpr uint32_t FINE_SPLIT = 196608;
 
 // Fine codes per thread and step of the fine-sort loops: all of a step's loads are in flight
 // before its LDS atomics (a load -> atomic -> load chain waits out the memory latency per code).
 constexpr uint32_t FINE_ITEMS = 8;
 
-// LDS histogram of fineCode[lo, hi) into h.
+// LDS histogram of fineCode[lo, hi) into h (at fineSlot).
 __device__ __forceinline__ void fineHistogram(const uint16_t* __restrict__ fineCode, uint32_t lo, uint32_t hi,
                                               uint32_t* h)
 {
@@ -443,13 +481,13 @@ __device__ __forceinline__ void fineHistogram(const uint16_t* __restrict__ fineC
             c[k] = fineCode[i + k * SORT_THREADS];
 #pragma unroll
         for (uint32_t k = 0; k < FINE_ITEMS; ++k)
-            atomicAdd(h + c[k], 1u);
+            atomicAdd(h + fineSlot(c[k]), 1u);
     }
     for (; i < hi; i += SORT_THREADS)
-        atomicAdd(h + fineCode[i], 1u);
+        atomicAdd(h + fineSlot(fineCode[i]), 1u);
 }
 
-// perm[base + slot] = i for every i in [lo, hi), slot taken from the running starts h[code].
+// perm[base + slot] = i for every i in [lo, hi), slot taken from the running starts at h[fineSlot(code)].
 __device__ __forceinline__ void finePermute(const uint16_t* __restrict__ fineCode, uint32_t lo, uint32_t hi,
                                             uint32_t* h, uint32_t base, uint32_t* __restrict__ perm)
 {
@@ -463,14 +501,14 @@ __device__ __forceinline__ void finePermute(const uint16_t* __restrict__ fineCod
         uint32_t slot[FINE_ITEMS];
 #pragma unroll
         for (uint32_t k = 0; k < FINE_ITEMS; ++k)
-            slot[k] = atomicAdd(h + c[k], 1u);
+            slot[k] = atomicAdd(h + fineSlot(c[k]), 1u);
 #pragma unroll
         for (uint32_t k = 0; k < FINE_ITEMS; ++k)
             perm[base + slot[k]] = i + k * SORT_THREADS;
     }
     for (; i < hi; i += SORT_THREADS)
     {
-        const uint32_t slot = atomicAdd(h + fineCode[i], 1u);
+        const uint32_t slot = atomicAdd(h + fineSlot(fineCode[i]), 1u);
         perm[base + slot]   = i;
     }
 }
@@ -506,26 +544,39 @@ __device__ __forceinline__ void fineSortBucket(uint32_t b, const uint16_t* __res
     finePermute(fineCode, lo, hi, h, lo, perm);
 }
 
+// The occupied buckets (list of `totals` bits 32-47), a workgroup per compute unit taking the next
+// one from a counter: with its 132 KB of LDS one workgroup fits a compute unit, and a grid over all
+// buckets spent 16 rounds of launches on the empty ones (512^3 grid: 4096, a few hundred occupied).
 static __global__ __launch_bounds__(SORT_THREADS) void kFineSort(const uint16_t* __restrict__ fineCode,
-                                                           const uint32_t* __restrict__ bucketStart, FineSortParams fp,
+                                                           const uint32_t* __restrict__ bucketStart,
+                                                           const uint32_t* __restrict__ occupied,
+                                                           const uint64_t* __restrict__ totals,
+                                                           uint32_t* __restrict__ next, FineSortParams fp,
                                                            uint32_t* __restrict__ count, uint32_t* __restrict__ perm,
                                                            uint32_t* __restrict__ occ)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS + 1];
     __shared__ uint32_t scratch[SORT_WAVES];
-    fineSortBucket(blockIdx.x, fineCode, bucketStart, fp, count, perm, h, scratch, occ);
+    __shared__ uint32_t mine;
+    const uint32_t buckets = static_cast<uint32_t>(*totals >> 32) & 0xFFFF;
+    for (;;)
+    {
+        if (threadIdx.x == 0)
+            mine = atomicAdd(next, 1u);
+        __syncthreads();
+        const uint32_t i = mine;
+        if (i >= buckets)
+            return;
+        fineSortBucket(occupied[i], fineCode, bucketStart, fp, count, perm, h, scratch, occ);
+        __syncthreads();
+    }
 }
 
-// chunks of the buckets above FINE_SPLIT points: entry = first chunk of the bucket's points,
-// bucket << 32 | part
+// chunks of the buckets above FINE_SPLIT points: entry = bucket << 32 | part
 struct SplitChunksIn
 {
     const uint32_t* bucketStart;
-    __device__ uint32_t operator()(uint64_t b) const
-    {
-        const uint32_t n = bucketStart[b + 1] - bucketStart[b];
-        return n > FINE_SPLIT ? (n + FINE_SPLIT - 1) / FINE_SPLIT : 0u;
-    }
+    __device__ uint32_t operator()(uint64_t b) const { return splitChunksOf(bucketStart[b + 1] - bucketStart[b]); }
 };
 
 struct SplitChunksOut
@@ -556,17 +607,17 @@ __device__ __forceinline__ void fineChunkHist(uint32_t chunk, const uint16_t* __
     __syncthreads();
     uint32_t* dst = chunkHist + static_cast<uint64_t>(chunk) * MAX_FINE_CELLS;
     for (uint32_t c = threadIdx.x; c < cells; c += SORT_THREADS)
-        dst[c] = h[c];
+        dst[c] = h[fineSlot(c)];
 }
 
 static __global__ __launch_bounds__(SORT_THREADS) void kFineChunkHist(const uint16_t* __restrict__ fineCode,
                                                                 const uint32_t* __restrict__ bucketStart,
                                                                 const uint64_t* __restrict__ chunks,
-                                                                const uint32_t* __restrict__ chunkCount, uint32_t lc,
+                                                                const uint64_t* __restrict__ totals, uint32_t lc,
                                                                 uint32_t* __restrict__ chunkHist)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS];
-    if (blockIdx.x >= *chunkCount)
+    if (blockIdx.x >= *totals >> 48)
         return;  // the whole workgroup
     fineChunkHist(blockIdx.x, fineCode, bucketStart, chunks, lc, chunkHist, h);
 }
@@ -593,22 +644,22 @@ __device__ __forceinline__ void fineSplitScan(uint32_t chunk, const uint32_t* __
         uint32_t v = 0;
         for (uint32_t k = 0; k < parts; ++k)
             v += first[static_cast<uint64_t>(k) * MAX_FINE_CELLS + c];
-        h[c] = v;
+        h[fineSlot(c)] = v;
     }
     __syncthreads();
     bucketScan(h, cells, scratch);  // every chunk histogram has been read
     bucketCounts(b, fp, h, count, occ);
     for (uint32_t c = threadIdx.x; c < cells; c += SORT_THREADS)
-        first[c] = h[c];
+        first[c] = h[fineSlot(c)];
     for (uint32_t k = 1 + threadIdx.x; k < parts; k += SORT_THREADS)
     {
-        // the first cell c with h[c] >= k * FINE_SPLIT (k * FINE_SPLIT < h[cells], so c <= cells)
+        // the first cell c with h[c] >= k * FINE_SPLIT (k * FINE_SPLIT < the total, so c <= cells)
         const uint32_t target = k * FINE_SPLIT;
         uint32_t lo = 0, hi = cells;
         while (lo < hi)
         {
             const uint32_t mid = (lo + hi) >> 1;
-            if (h[mid] < target)
+            if (h[fineSlot(mid)] < target)
                 lo = mid + 1;
             else
                 hi = mid;
@@ -619,14 +670,14 @@ __device__ __forceinline__ void fineSplitScan(uint32_t chunk, const uint32_t* __
 
 static __global__ __launch_bounds__(SORT_THREADS) void kFineSplitScan(const uint32_t* __restrict__ bucketStart,
                                                                 const uint64_t* __restrict__ chunks,
-                                                                const uint32_t* __restrict__ chunkCount,
+                                                                const uint64_t* __restrict__ totals,
                                                                 FineSortParams fp, uint32_t* __restrict__ count,
                                                                 uint32_t* __restrict__ chunkHist,
                                                                 uint32_t* __restrict__ occ)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS + 1];
     __shared__ uint32_t scratch[SORT_WAVES];
-    if (blockIdx.x >= *chunkCount || static_cast<uint32_t>(chunks[blockIdx.x]) != 0)
+    if (blockIdx.x >= *totals >> 48 || static_cast<uint32_t>(chunks[blockIdx.x]) != 0)
         return;  // the whole workgroup: not the first chunk of a bucket
     fineSplitScan(blockIdx.x, bucketStart, chunks, fp, count, chunkHist, h, scratch, occ);
 }
@@ -675,13 +726,13 @@ __device__ __forceinline__ void fineChunkPerm(uint32_t chunk, const uint16_t* __
 static __global__ __launch_bounds__(SORT_THREADS) void kFineChunkPerm(const uint16_t* __restrict__ fineCode,
                                                                 const uint32_t* __restrict__ bucketStart,
                                                                 const uint64_t* __restrict__ chunks,
-                                                                const uint32_t* __restrict__ chunkCount, uint32_t lc,
+                                                                const uint64_t* __restrict__ totals, uint32_t lc,
                                                                 const uint32_t* __restrict__ chunkHist,
                                                                 uint32_t* __restrict__ perm)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS];
     // the partitions of one bucket read the same fine codes: on one XCD, from one L2
-    const uint32_t chunk = xcdItem(*chunkCount);
+    const uint32_t chunk = xcdItem(static_cast<uint32_t>(*totals >> 48));
     if (chunk == ~0u)
         return;  // the whole workgroup
     fineChunkPerm(chunk, fineCode, bucketStart, chunks, lc, chunkHist, perm, h);

@@ -49,13 +49,11 @@ enum PrefixSlot : uint32_t
     P_DIST,
     P_SPLIT,
     P_NODES,
-    P_LEVEL0,
     P_LEAFCHUNK,
     P_K,
     P_SEG,
     P_TILES,
     P_WORDS,
-    P_K1,
     P_CELLS,
     P_LIVE_TILES,
     P_PLACE,
@@ -188,7 +186,6 @@ void carveCloud(Carver& cv, BatchCloud<T>& cc, const BatchRequest& r, const Clou
     cv.take(cc.tileList, s.tileBound);
     cv.take(cc.bitmap, s.kBound * s.wordsPerNode);
     cv.take(cc.prefix, s.kBound * s.wordsPerNode + 1);
-    cv.take(cc.nodeFirst, s.kBound + 1);
     cv.take(cc.cellOf, s.E);
     cv.take(cc.cellKey, s.E);
     cv.take(cc.cellNode, s.E);
@@ -221,7 +218,6 @@ void carveNodes(Carver& cv, BatchCloud<T>& cc, uint64_t m, const CloudSizes& s)
     cv.take(cc.nodeChild, 8 * m);
     cv.take(cc.nodeFlags, m);
     cv.take(cc.nodeSorted, m);
-    cv.take(cc.nodeAux, m + 1);
     cv.take(cc.nodeStage, m);
     cv.take(cc.nodeSub, m);
     cv.take(cc.nodeRegion, m);
@@ -499,10 +495,6 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
         fp.levelOffset[l] = L.offset[l];
         fp.levelGrid[l]   = L.grid[l];
     }
-    LevelOffsets lo{};
-    for (uint32_t l = 0; l <= L.depth; ++l)
-        lo.offset[l] = L.offset[l];
-    lo.levels = L.depth + 1;
     const bool graphs = itsUseGraphs;
     auto mark         = [&](int k) {
         if (!graphs)
@@ -532,17 +524,11 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
         OC_LAUNCH_CHECK();
     }
     mark(1);
-    for (uint32_t l = L.lc + 1; l <= L.depth; ++l)
-    {
-        kPropagateB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B0, L.offset[l], L.grid[l], L.offset[l - 1],
-                                                        L.grid[l - 1]);
-        OC_LAUNCH_CHECK();
-    }
-    kOccupancyBitsB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B0, L);
+    kPropagateTopB<T><<<B0, TOP_THREADS, 0, s>>>(ctx, L);
     const uint64_t words = (static_cast<uint64_t>(L.dense) + 31) / 32;
-    scanBatch<uint32_t>(OccupancyJob<T>{ctx, words}, B0, words, s);
-    OC_LAUNCH_CHECK();
-    kLevelStartsB<T><<<B0, 64, 0, s>>>(ctx, lo);
+    const dim3 wordGrid(scanWidth(words), B0);
+    kScanReduceB<uint32_t><<<wordGrid, SCAN_THREADS, 0, s>>>(OccupancyJob<T>{ctx, L.marked, L.dense});
+    kOccupiedIdsB<T><<<wordGrid, SCAN_THREADS, 0, s>>>(ctx, L);
     OC_LAUNCH_CHECK();
     };
     OC_HIP_CHECK(hipEventRecord(itsEvents[0], s));
@@ -611,7 +597,6 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
     hostPrefix(P_POINTS, B, [&](uint32_t j) { return liveSizes[j].n; });
     hostPrefix(P_DIST, B, [&](uint32_t j) { return (liveSizes[j].n + DIST_CHUNK - 1) / DIST_CHUNK; });
     hostPrefix(P_NODES, B, [&](uint32_t j) { return table[j].m; });
-    hostPrefix(P_LEVEL0, B, [&](uint32_t j) { return lsOf(j)[1]; });
     for (uint32_t l = 1; l <= L.depth; ++l)
         hostPrefix(P_LEVEL + l, B, [&](uint32_t j) { return lsOf(j)[l + 1] - lsOf(j)[l]; });
     uploadTables(B);
@@ -621,13 +606,10 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
     kNodeLinksB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_NODES), L);
     OC_LAUNCH_CHECK();
     scanBatch<uint32_t>(LeafBlockJob<T>{ctx}, B, maxM, s);
-    kLeafDataIdxB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_NODES));
-    kCellLeafB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_LEVEL0));
     OC_LAUNCH_CHECK();
     mark(2);
 
     // ---- distribution: leaf and cell order of the sorted clouds, then the leaf blocks ----------
-    kSortedStartB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_NODES), L);
     scanBatch<uint32_t>(LeafChunkJob<T>{ctx}, B, maxM, s);
     kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(ScalarCount<T>{ctx, BS_TABLE_TOTAL, false}, B, slot(P_LEAFCHUNK));
     kLeafCellOrderB<T><<<LG.sortGrid, LEAF_THREADS, 0, s>>>(ctx, B, slot(P_LEAFCHUNK), L);
@@ -780,10 +762,10 @@ void BatchBuilder::subsampleGroup(uint32_t B, const BatchLevels& L, const BatchB
     for (uint32_t l = 1; l <= depth; ++l)
     {
         scanBatch<uint32_t>(InternalJob<T>{ctx, l}, B, bounds.levelNodes[l], s);
-        kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(LevelNodeCount<T>{ctx, 1, 0}, B, slot(P_K));
+        kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(LevelNodeCount<T>{ctx, 1}, B, slot(P_K));
         kSegmentsB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_K), L, l);
         scanBatch<uint64_t>(SegmentJob<T>{ctx}, B, bounds.segments, s);
-        kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(LevelNodeCount<T>{ctx, 8, 0}, B, slot(P_SEG));
+        kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(LevelNodeCount<T>{ctx, 8}, B, slot(P_SEG));
         kTileListB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_SEG));
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(TileCount<T>{ctx}, B, slot(P_TILES));
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(WordCount<T>{ctx}, B, slot(P_WORDS));
@@ -791,8 +773,7 @@ void BatchBuilder::subsampleGroup(uint32_t B, const BatchLevels& L, const BatchB
         kMarkB<T><<<LG.tileGrid, TILE, 0, s>>>(ctx, B, slot(P_TILES));
         scanBatch<uint32_t>(PopcountJob<T>{ctx}, B, bounds.words, s);
         kLevelCellsB<T><<<(B + 255) / 256, 256, 0, s>>>(ctx, B);
-        kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(LevelNodeCount<T>{ctx, 1, 1}, B, slot(P_K1));
-        kBatchNodesB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_K1));
+        kBatchNodesB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_K));
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(ScalarCount<T>{ctx, BS_CELLS, true}, B, slot(P_CELLS));
         kClearCellsB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_CELLS), MODE);
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(TileCount<T>{ctx}, B, slot(P_LIVE_TILES));

@@ -123,23 +123,25 @@ private:
     template <typename T>
     void countPoints();
     void mergeLevels();
+    uint64_t nodeBound() const;  // sparse nodes: at most min(D, levels * N)
+    struct LevelParams levelParams() const;
+    struct ChildSlots childSlots(uint32_t firstInternal) const;
+    struct LeafOrderParams leafTables();
+    uint32_t stepNodes() const;
+    uint32_t planSteps();
+    uint64_t leafChunkBound() const;
+    uint64_t placeChunkBound() const;
     // whether the fine sort writes the occupancy bits of the BIT_LEVELS lowest levels
     bool fineSortBits() const;
     template <typename T>
     void distributePoints();
     template <typename T>
-    bool orderLeafPoints();
-    template <typename T>
     void subsampleLevels();
     void placeInternalNodes();
-    void placeLevelByLevel();
 
     void syncStream();
     void progress();
     void waitForSnapshotOnStream();
-    template <typename V>
-    V readDevice(const V* devicePtr);
-    std::array<uint64_t, 2> readDevicePair(const uint64_t* devicePtr);
     void waitMailbox(uint64_t seq);
 
     int itsDevice;
@@ -149,7 +151,7 @@ private:
     hipEvent_t itsCopiedEvent         = nullptr;  // the snapshot's last copy
     hipEvent_t itsUploadedEvent       = nullptr;  // the cloud upload of the current setup
     bool itsSnapshotPending           = false;    // copies enqueued that the build stream has not waited for
-    // Size readbacks: a one-thread kernel publishes {value, value, sequence} into coherent pinned
+    // Readbacks: a small kernel publishes its values and then a sequence number into coherent pinned
     // host memory and the host spins on the sequence (no staging copy, no blocking-sync wake-up).
     uint64_t* itsMailbox  = nullptr;
     uint64_t itsMailSeq   = 0;
@@ -175,6 +177,8 @@ private:
     uint64_t itsE          = 0;
     uint64_t itsUsed       = 0;
     uint32_t itsLevelStart[MAX_LEVELS + 1] = {};
+    uint32_t itsInner[MAX_LEVELS + 1]      = {};  // internal nodes before each level; [depth + 1]: all
+    uint32_t itsSteps                      = 0;   // subsampling steps (batches of a level's nodes)
     std::vector<float> itsTimings;
 
     // cloud
@@ -184,7 +188,7 @@ private:
     // dense pyramid and sparse nodes
     DeviceBuffer itsCount, itsDenseToSparse, itsOccupancy;  // dense counts, sparse ids, occupancy bits
     DeviceBuffer itsNodeKey, itsNodeCount, itsNodePoints, itsNodeData, itsNodeParent, itsNodeChild, itsNodeFlags,
-            itsNodeSorted, itsNodeAux, itsNodeStage, itsNodeSub, itsNodeRegion;
+            itsNodeSorted, itsNodeStage, itsNodeSub;
 
     // Morton bucket sort of the cloud
     DeviceBuffer itsBucketed, itsSorted, itsFineCode, itsPerm, itsBucketCount, itsBucketStart, itsBucketCursor, itsBucketList;
@@ -199,7 +203,7 @@ private:
     // occupancy bitmaps with their popcount prefix, per-cell (dense index) state, per-input state
     DeviceBuffer itsLeafList, itsInternalList, itsSegCount, itsSegSrc, itsSegTile, itsSegInput, itsNodeGrid,
             itsTileList;
-    DeviceBuffer itsBitmap, itsPrefix, itsNodeFirst;
+    DeviceBuffer itsBitmap, itsPrefix, itsCursors;
     DeviceBuffer itsWin, itsColor, itsCellCnt, itsCellStart, itsCellKey, itsCellNode;
     DeviceBuffer itsCellOf, itsRankOf, itsPayload;
 

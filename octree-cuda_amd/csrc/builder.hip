@@ -108,6 +108,24 @@ size_t DeviceBuffer::peakAllocated()
 // Bytes of bitmap + prefix the nodes of one subsampling batch may use.
 static constexpr uint64_t kBitmapBudget = 6ull << 30;
 
+// Bitmap words up to which the popcount scan also resets the cells (a launch less; its threads walk
+// the cells of their words, which costs more than a pass of its own on large levels).
+static constexpr uint64_t CLEAR_IN_SCAN_WORDS = 1u << 20;
+
+// words of the host mailbox
+enum MailSlot
+{
+    MAIL_SEQ,
+    MAIL_ERROR,
+    MAIL_NODES,
+    MAIL_INTERNAL,
+    MAIL_USED,
+    MAIL_INPUTS,
+    MAIL_LEVEL = 8,                        // first node of every level
+    MAIL_INNER = MAIL_LEVEL + MAX_LEVELS,  // first internal node of every level
+    MAIL_WORDS = MAIL_INNER + MAX_LEVELS
+};
+
 static uint32_t octreeDepth(uint32_t grid)  // tools.cu:63-88
 {
     for (uint32_t d = 1; d <= 9; ++d)
@@ -126,10 +144,8 @@ OctreeBuilder::OctreeBuilder(int device) : itsDevice(device)
     OC_HIP_CHECK(hipEventCreateWithFlags(&itsUploadedEvent, hipEventDisableTiming));
     for (auto& ev : itsEvents)
         OC_HIP_CHECK(hipEventCreate(&ev));
-    OC_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&itsMailbox), 3 * sizeof(uint64_t), hipHostMallocCoherent));
-    itsMailbox[0] = 0;
-    itsMailbox[1] = 0;
-    itsMailbox[2] = 0;
+    OC_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&itsMailbox), MAIL_WORDS * sizeof(uint64_t), hipHostMallocCoherent));
+    std::fill(itsMailbox, itsMailbox + MAIL_WORDS, 0);
 }
 
 OctreeBuilder::OctreeBuilder(int device, const CloudInfo& cloud, const ProcessingInfo& proc,
@@ -193,7 +209,7 @@ void OctreeBuilder::setup(const CloudInfo& cloud, const ProcessingInfo& proc, co
     itsCount.ensure(sizeof(uint32_t) * static_cast<uint64_t>(itsDense));
     itsDenseToSparse.ensure(sizeof(int32_t) * static_cast<uint64_t>(itsDense));
     itsOccupancy.ensure(sizeof(uint32_t) * ((static_cast<uint64_t>(itsDense) + 31) / 32));
-    uint64_t mBound = std::min<uint64_t>(itsDense, static_cast<uint64_t>(itsDepth + 1) * cloud.pointAmount);
+    const uint64_t mBound = nodeBound();
     // The previous build's snapshot copies may still read the node keys and counts, the LUT and
     // the output: growing one of them frees it, so those copies are waited for first. (The other
     // arrays a snapshot reads are grown by the merge, after its stream has waited for the copies
@@ -240,13 +256,13 @@ std::vector<DeviceBuffer*> OctreeBuilder::arena()
 {
     return {&itsCloudOwned,  &itsCount,       &itsDenseToSparse, &itsOccupancy,
             &itsNodeKey,     &itsNodeCount,   &itsNodePoints,
-            &itsNodeData,    &itsNodeParent,  &itsNodeChild,     &itsNodeFlags,    &itsNodeSorted,  &itsNodeAux,
-            &itsNodeStage,   &itsNodeSub,     &itsNodeRegion,    &itsBucketed,     &itsSorted,      &itsFineCode,
+            &itsNodeData,    &itsNodeParent,  &itsNodeChild,     &itsNodeFlags,    &itsNodeSorted,
+            &itsNodeStage,   &itsNodeSub,     &itsBucketed,     &itsSorted,      &itsFineCode,
             &itsPerm,
             &itsBucketCount, &itsBucketStart, &itsBucketCursor,  &itsBucketList,  &itsLut,          &itsOut,
             &itsStLut,       &itsStOut,       &itsStPts,         &itsStRgb,        &itsInternalList, &itsSegCount,    &itsSegSrc,
             &itsSegTile,     &itsSegInput,    &itsNodeGrid,      &itsTileList,     &itsBitmap,      &itsPrefix,
-            &itsNodeFirst,   &itsWin,         &itsColor,         &itsCellCnt,      &itsCellStart,   &itsCellKey,
+            &itsCursors,     &itsWin,         &itsColor,         &itsCellCnt,      &itsCellStart,   &itsCellKey,
             &itsCellNode,    &itsCellOf,      &itsRankOf,        &itsPayload,      &itsScalars,
             &itsScanScratch, &itsLeafList,   &itsSplitChunks,   &itsSplitHist};
 }
@@ -295,10 +311,10 @@ uint64_t OctreeBuilder::estimateFootprint(const CloudInfo& cloud, const Processi
     if (proc.useInterCellAvg && proc.useWeightingFunction && !proc.useIntraCellAvg)
         bytes += 4 * staged;                                // staged colours of the weighted filter
     // per-level work: inputs (cell, then its dense index; rank; payload) and cells (winner, colour sum,
-    // count, start, key, node), both bounded by E; the occupancy bitmaps and their prefix
+    // count, start, key, node), both bounded by N and with it by E; the occupancy bitmaps and their prefix
     const uint64_t wordsPerNode = (rowsPerNode(proc.subsamplingGrid) * proc.subsamplingGrid + 31) / 32;
     const uint64_t levelNodes   = std::min<uint64_t>(mBound, n / std::max<uint32_t>(1, proc.mergingThreshold) + 8);
-    bytes += (8 + sizeof(WeightPayload) + sizeof(uint64_t)) * e + 32 * staged;
+    bytes += std::max<uint64_t>((8 + sizeof(WeightPayload) + sizeof(uint64_t)) * e + 32 * staged, 48 * n);
     bytes += std::min<uint64_t>(kBitmapBudget, 8 * wordsPerNode * levelNodes);
     return bytes;
 }
@@ -349,64 +365,82 @@ void OctreeBuilder::syncStream()
     OC_HIP_CHECK(hipStreamSynchronize(itsStream));
 }
 
-// Publishes a device value to the host mailbox: the value first, then (after a system-scope
-// release) the sequence number the host waits for.
-template <typename V>
-__global__ void kPublish(const V* __restrict__ src, uint64_t* box, uint64_t seq)
+// The sizes after the merge, to the host mailbox: the nodes, the error flags, the internal nodes,
+// and the first node and first internal node of every level. The values first, then (after a
+// system-scope release) the sequence number the host waits for.
+__global__ __launch_bounds__(64) void kPublishMerge(const uint64_t* __restrict__ sc, const uint32_t* __restrict__ internal,
+                                                    uint32_t levels, uint64_t* box, uint64_t seq)
+{
+    const uint32_t l     = threadIdx.x;
+    const uint32_t inner = static_cast<uint32_t>(sc[SC_INTERNAL]);
+    auto post            = [&](uint32_t at, uint64_t v) {
+        __hip_atomic_store(box + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    };
+    if (l < levels)
+    {
+        const uint32_t start = reinterpret_cast<const uint32_t*>(sc + SC_LEVEL_START)[l];
+        uint32_t a = 0, b = inner;  // the first internal node at or after the level's first node
+        while (a < b)
+        {
+            const uint32_t mid = a + (b - a) / 2;
+            if (internal[mid] < start)
+                a = mid + 1;
+            else
+                b = mid;
+        }
+        post(MAIL_LEVEL + l, start);
+        post(MAIL_INNER + l, a);
+    }
+    if (l == 0)
+    {
+        post(MAIL_NODES, sc[SC_M]);
+        post(MAIL_ERROR, sc[SC_ERROR]);
+        post(MAIL_INTERNAL, inner);
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (l == 0)
+        __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// (tiles << 32 | inputs) of a level
+__global__ void kPublishInputs(const uint64_t* __restrict__ segTotal, uint64_t* box, uint64_t seq)
 {
     if (threadIdx.x != 0)
         return;
-    __hip_atomic_store(box, static_cast<uint64_t>(*src), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(box + 2, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(box + MAIL_INPUTS, *segTotal & 0xFFFFFFFFull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Two consecutive device words through the mailbox (one wait for two sizes).
-__global__ void kPublishPair(const uint64_t* __restrict__ src, uint64_t* box, uint64_t seq)
+// The end of a build: the error flags and the used output records (the last cursor).
+__global__ void kPublishEnd(const uint64_t* __restrict__ sc, const uint64_t* __restrict__ cursor, uint64_t* box,
+                            uint64_t seq)
 {
     if (threadIdx.x != 0)
         return;
-    __hip_atomic_store(box, src[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(box + 1, src[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(box + 2, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(box + MAIL_ERROR, sc[SC_ERROR], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(box + MAIL_USED, *cursor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// A size the host needs to size the next launches. The stream is drained up to the publish: the
+// Sizes the host needs from the device. The stream is drained up to the publish: the
 // host spins on the mailbox for up to 2 ms (the common case: the value is ready within microseconds
 // of the last kernel) and then falls back to a blocking synchronisation, which also reports a
 // failed kernel instead of waiting forever.
 void OctreeBuilder::waitMailbox(uint64_t seq)
 {
     const auto start = std::chrono::steady_clock::now();
-    while (__atomic_load_n(itsMailbox + 2, __ATOMIC_ACQUIRE) != seq)
+    while (__atomic_load_n(itsMailbox + MAIL_SEQ, __ATOMIC_ACQUIRE) != seq)
     {
         __builtin_ia32_pause();
         if (std::chrono::steady_clock::now() - start > std::chrono::milliseconds(2))
         {
             OC_HIP_CHECK(hipStreamSynchronize(itsStream));
-            if (__atomic_load_n(itsMailbox + 2, __ATOMIC_ACQUIRE) != seq)
+            if (__atomic_load_n(itsMailbox + MAIL_SEQ, __ATOMIC_ACQUIRE) != seq)
                 throw std::runtime_error("device value was not published");
             break;
         }
     }
-}
-
-template <typename V>
-V OctreeBuilder::readDevice(const V* devicePtr)
-{
-    const uint64_t seq = ++itsMailSeq;
-    kPublish<V><<<1, 64, 0, itsStream>>>(devicePtr, itsMailbox, seq);
-    OC_LAUNCH_CHECK();
-    waitMailbox(seq);
-    return static_cast<V>(__atomic_load_n(itsMailbox, __ATOMIC_ACQUIRE));
-}
-
-std::array<uint64_t, 2> OctreeBuilder::readDevicePair(const uint64_t* devicePtr)
-{
-    const uint64_t seq = ++itsMailSeq;
-    kPublishPair<<<1, 64, 0, itsStream>>>(devicePtr, itsMailbox, seq);
-    OC_LAUNCH_CHECK();
-    waitMailbox(seq);
-    return {__atomic_load_n(itsMailbox, __ATOMIC_ACQUIRE), __atomic_load_n(itsMailbox + 1, __ATOMIC_ACQUIRE)};
 }
 
 void OctreeBuilder::generate()
@@ -425,7 +459,6 @@ void OctreeBuilder::generate()
 template <typename T>
 void OctreeBuilder::generateTyped()
 {
-    uint64_t* sc  = itsScalars.as<uint64_t>();
     itsBatchesRun = 0;
 
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_START], itsStream));
@@ -440,11 +473,19 @@ void OctreeBuilder::generateTyped()
     subsampleLevels<T>();
     placeInternalNodes();
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_END], itsStream));
+    const uint64_t seq = ++itsMailSeq;
+    kPublishEnd<<<1, 64, 0, itsStream>>>(itsScalars.as<uint64_t>(), itsCursors.as<uint64_t>() + itsSteps, itsMailbox, seq);
+    OC_LAUNCH_CHECK();
+    waitMailbox(seq);
     syncStream();
 
-    uint32_t err = static_cast<uint32_t>(readDevice(sc + SC_ERROR));
+    const uint64_t err = itsMailbox[MAIL_ERROR];
+    if (err & ERR_OVERFLOW)  // A14
+        throw std::runtime_error("the subsampled points exceed the estimated output size (N + I > E); "
+                                 "raise the output factor");
     if (err & ERR_OUTSIDE)
         throw std::runtime_error("a point lies outside the cubic bounding box");
+    itsUsed = itsMailbox[MAIL_USED];
     if (err & ERR_CAPACITY)
         throw std::runtime_error("a node has more than 2^31 input points");
 
@@ -547,56 +588,76 @@ bool OctreeBuilder::fineSortBits() const
     return itsCoarse == MAX_COARSE_LEVEL;
 }
 
+LevelParams OctreeBuilder::levelParams() const
+{
+    LevelParams lp{};
+    for (uint32_t l = 0; l <= itsDepth; ++l)
+    {
+        lp.offset[l] = itsLevelOffset[l];
+        lp.grid[l]   = itsLevelGrid[l];
+    }
+    lp.depth     = itsDepth;
+    lp.threshold = itsProc.mergingThreshold;
+    return lp;
+}
+
 void OctreeBuilder::mergeLevels()
 {
     uint64_t* sc    = itsScalars.as<uint64_t>();
     uint32_t* count = itsCount.as<uint32_t>();
-    for (uint32_t l = itsCoarse + 1; l <= itsDepth; ++l)  // levels 0..coarse come from the fine sort
-    {
-        kPropagate<<<gridFor(itsLevelNodes[l]), BLOCK, 0, itsStream>>>(count, itsLevelOffset[l], itsLevelGrid[l],
-                                                                        itsLevelOffset[l - 1], itsLevelGrid[l - 1]);
-        OC_LAUNCH_CHECK();
-    }
-
-    // occupancy bits of the levels the fine sort has not marked, then sparse ids (A2) + node keys /
-    // counts + first id of every level, by one scan over the bitmap's words
-    uint32_t* occ         = itsOccupancy.as<uint32_t>();
-    const uint64_t marked = fineSortBits() ? itsLevelOffset[BIT_LEVELS] : 0;
-    kOccupancyBits<<<gridFor(itsDense - marked), BLOCK, 0, itsStream>>>(count, marked, itsDense, occ);
-    OC_LAUNCH_CHECK();
-    uint32_t* levelStart = reinterpret_cast<uint32_t*>(sc + SC_LEVEL_START);
-    const uint64_t words = (static_cast<uint64_t>(itsDense) + 31) / 32;
-    itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(words) + 1));
-    OccupiedWordOut occOut{};
-    occOut.occ           = occ;
-    occOut.denseToSparse = itsDenseToSparse.as<int32_t>();
-    occOut.nodeKey       = itsNodeKey.as<uint32_t>();
-    occOut.nodeCount     = itsNodeCount.as<uint32_t>();
-    occOut.count         = count;
-    scanExclusive<uint32_t>(words, OccupiedWordIn{occ}, occOut, itsScanScratch.as<uint32_t>(),
-                            reinterpret_cast<uint32_t*>(sc + SC_M), itsStream);
-    OC_LAUNCH_CHECK();
     LevelOffsets lo{};
     for (uint32_t l = 0; l <= itsDepth; ++l)
         lo.offset[l] = itsLevelOffset[l];
     lo.levels = itsDepth + 1;
-    kLevelStarts<<<1, 64, 0, itsStream>>>(itsNodeKey.as<uint32_t>(), reinterpret_cast<uint32_t*>(sc + SC_M), lo,
-                                          levelStart);
+    // levels 0..coarse come from the fine sort
+    kPropagateTop<<<1, TOP_THREADS, 0, itsStream>>>(count, lo, itsCoarse, itsProc.chunkingGrid);
     OC_LAUNCH_CHECK();
 
-    uint32_t hostStart[MAX_LEVELS + 1] = {};
-    OC_HIP_CHECK(hipMemcpyAsync(hostStart, levelStart, sizeof(uint32_t) * (itsDepth + 1), hipMemcpyDeviceToHost,
-                                itsStream));
-    uint64_t mRaw = 0, errRaw = 0;
-    OC_HIP_CHECK(hipMemcpyAsync(&mRaw, sc + SC_M, sizeof(uint64_t), hipMemcpyDeviceToHost, itsStream));
-    OC_HIP_CHECK(hipMemcpyAsync(&errRaw, sc + SC_ERROR, sizeof(uint64_t), hipMemcpyDeviceToHost, itsStream));
-    syncStream();
-    if (errRaw & ERR_OUTSIDE)
+    // occupancy bits of the levels the fine sort has not marked, sparse ids (A2) + node keys / counts
+    // + first id of every level by a scan over the bitmap's words, and the list of internal nodes
+    uint32_t* occ         = itsOccupancy.as<uint32_t>();
+    const uint64_t marked = fineSortBits() ? itsLevelOffset[BIT_LEVELS] / 32 : 0;
+    uint32_t* levelStart  = reinterpret_cast<uint32_t*>(sc + SC_LEVEL_START);
+    uint32_t* nodes       = reinterpret_cast<uint32_t*>(sc + SC_M);
+    const uint64_t words  = (static_cast<uint64_t>(itsDense) + 31) / 32;
+    const uint64_t bound  = nodeBound();
+    // at most N / threshold internal nodes on a level (they hold disjoint point sets), and at most
+    // as many as nodes above level 0
+    uint64_t inner = 0;
+    for (uint32_t l = 1; l <= itsDepth; ++l)
+        inner += std::min<uint64_t>(std::min<uint64_t>(itsLevelNodes[l], itsCloud.pointAmount),
+                                    itsCloud.pointAmount / std::max<uint32_t>(1, itsProc.mergingThreshold));
+    itsInternalList.ensure(sizeof(uint32_t) * std::max<uint64_t>(1, inner));
+    itsScanScratch.ensure(sizeof(uint64_t) * SCAN_GRID);
+    uint32_t* sums = itsScanScratch.as<uint32_t>();
+    const unsigned wordGrid = static_cast<unsigned>(std::min<uint64_t>(scanTiles(words), SCAN_GRID));
+    kScanReduce<uint32_t><<<wordGrid, SCAN_THREADS, 0, itsStream>>>(OccupancyIn{occ, count, marked, itsDense},
+                                                                    HostCount{words}, sums);
+    OC_LAUNCH_CHECK();
+    const IdTables ids{occ, count, itsDenseToSparse.as<int32_t>(), itsNodeKey.as<uint32_t>(),
+                       itsNodeCount.as<uint32_t>(), levelStart, lo};
+    kOccupiedIds<<<wordGrid, SCAN_THREADS, 0, itsStream>>>(ids, words, sums, nodes);
+    OC_LAUNCH_CHECK();
+    uint32_t* internal = itsInternalList.as<uint32_t>();
+    scanExclusive<uint32_t>(DeviceCount{nodes, levelStart + 1}, bound,
+                            InternalNodeIn{itsNodeCount.as<uint32_t>(), levelStart, itsProc.mergingThreshold},
+                            InternalNodeOut{internal, levelStart}, sums, reinterpret_cast<uint32_t*>(sc + SC_INTERNAL),
+                            itsStream);
+    OC_LAUNCH_CHECK();
+    const uint64_t seq = ++itsMailSeq;
+    kPublishMerge<<<1, 64, 0, itsStream>>>(sc, internal, itsDepth + 1, itsMailbox, seq);
+    OC_LAUNCH_CHECK();
+    waitMailbox(seq);
+    if (itsMailbox[MAIL_ERROR] & ERR_OUTSIDE)
         throw std::runtime_error("a point lies outside the cubic bounding box");
-    itsM = static_cast<uint32_t>(mRaw);
+    itsM = static_cast<uint32_t>(itsMailbox[MAIL_NODES]);
     for (uint32_t l = 0; l <= itsDepth; ++l)
-        itsLevelStart[l] = hostStart[l];
+    {
+        itsLevelStart[l] = static_cast<uint32_t>(itsMailbox[MAIL_LEVEL + l]);
+        itsInner[l]      = static_cast<uint32_t>(itsMailbox[MAIL_INNER + l]);
+    }
     itsLevelStart[itsDepth + 1] = itsM;
+    itsInner[itsDepth + 1]      = static_cast<uint32_t>(itsMailbox[MAIL_INTERNAL]);
     if (itsM == 0)
         throw std::runtime_error("the cloud has no points inside the bounding box");
 
@@ -607,40 +668,71 @@ void OctreeBuilder::mergeLevels()
     itsNodeChild.ensure(sizeof(int32_t) * 8 * m);
     itsNodeFlags.ensure(m);
     itsNodeSorted.ensure(sizeof(uint32_t) * m);
-    itsNodeAux.ensure(sizeof(uint32_t) * (m + 1));
     itsNodeStage.ensure(sizeof(uint32_t) * m);
     itsNodeSub.ensure(sizeof(uint32_t) * m);
-    itsNodeRegion.ensure(sizeof(uint32_t) * m);
-    itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(m) + 1));
+    itsCursors.ensure(sizeof(uint64_t) * (planSteps() + 1));
+    kNodeLinks<<<gridFor(m), BLOCK, 0, itsStream>>>(
+            itsM, levelParams(), itsNodeKey.as<uint32_t>(), itsNodeCount.as<uint32_t>(),
+            itsDenseToSparse.as<int32_t>(), occ, itsNodePoints.as<uint32_t>(), itsNodeData.as<uint64_t>(),
+            itsNodeParent.as<int32_t>(), itsNodeChild.as<int32_t>(), itsNodeFlags.as<uint8_t>(),
+            itsNodeSub.as<uint32_t>(), itsCoarse, itsBucketStart.as<uint32_t>(), itsNodeSorted.as<uint32_t>(), count,
+            itsCursors.as<uint64_t>(), itsCloud.pointAmount);
+    OC_LAUNCH_CHECK();
+}
 
-    LevelParams lp{};
+uint64_t OctreeBuilder::nodeBound() const
+{
+    return std::min<uint64_t>(itsDense, static_cast<uint64_t>(itsDepth + 1) * itsCloud.pointAmount);
+}
+
+ChildSlots OctreeBuilder::childSlots(uint32_t firstInternal) const
+{
+    return ChildSlots{itsInternalList.as<uint32_t>() + firstInternal, itsNodeFlags.as<uint8_t>(),
+                      itsNodeChild.as<int32_t>(), itsNodeCount.as<uint32_t>()};
+}
+
+// Leaf data blocks (A4) and leaf chunks.
+LeafOrderParams OctreeBuilder::leafTables()
+{
+    uint64_t* sc             = itsScalars.as<uint64_t>();
+    const uint32_t nodes     = itsInner[itsDepth + 1];
+    const double cubicSize   = itsCloud.bbMax[0] - itsCloud.bbMin[0];  // metadata.cuh:66-69
+    LeafOrderParams p{};
+    for (int a = 0; a < 3; ++a)
+        p.cubicMin[a] = itsCloud.bbMin[a];
     for (uint32_t l = 0; l <= itsDepth; ++l)
     {
-        lp.offset[l] = itsLevelOffset[l];
-        lp.grid[l]   = itsLevelGrid[l];
+        p.side[l]     = cubicSize / std::pow(2.0, static_cast<double>(itsDepth - l));  // rp_subsampling.cu:17-18
+        p.sideHalf[l] = p.side[l] / 2.0;
     }
-    lp.depth     = itsDepth;
-    lp.threshold = itsProc.mergingThreshold;
-    kNodeLinks<<<gridFor(m), BLOCK, 0, itsStream>>>(
-            itsM, lp, itsNodeKey.as<uint32_t>(), itsNodeCount.as<uint32_t>(), itsDenseToSparse.as<int32_t>(),
-            itsNodePoints.as<uint32_t>(), itsNodeData.as<uint64_t>(), itsNodeParent.as<int32_t>(),
-            itsNodeChild.as<int32_t>(), itsNodeFlags.as<uint8_t>(), itsNodeAux.as<uint32_t>(),
-            itsNodeSub.as<uint32_t>(), occ);
+    p.lp                = levelParams();
+    p.g                 = itsProc.subsamplingGrid;
+    const uint32_t h    = p.g > 1 ? p.g / 2 : 1;  // cells per axis of a leaf's octant, as kLeafCellOrder
+    const uint64_t keys = rowsPerNode(h) * ((h + 31) / 32);
+    while (((keys - 1) >> p.keyShift) >= LEAF_KEYS)
+        ++p.keyShift;
+    if (nodes == 0)
+        return p;
+    const uint64_t slots = 8ull * nodes;
+    // one list for the leaf chunks here and the placement chunks at the end
+    itsLeafList.ensure(sizeof(uint64_t) * std::max<uint64_t>(leafChunkBound(), placeChunkBound()));
+    const ChildSlots cs = childSlots(0);
+    scanExclusive<uint64_t>(slots, LeafSlotIn{cs},
+                            LeafSlotOut{cs, itsNodeData.as<uint64_t>(), itsLeafList.as<uint64_t>()},
+                            itsScanScratch.as<uint64_t>(), sc + SC_LEAF_TOTAL, itsStream);
     OC_LAUNCH_CHECK();
+    return p;
+}
 
-    // leaf data blocks (A4): exclusive scan of the block sizes in id order
-    scanExclusive<uint32_t>(m, ArrayIn{itsNodeAux.as<uint32_t>()}, ExclusiveToArray{itsNodeAux.as<uint32_t>()},
-                            itsScanScratch.as<uint32_t>(), reinterpret_cast<uint32_t*>(sc + SC_LEAF_TOTAL),
-                            itsStream, true);
-    OC_LAUNCH_CHECK();
-    kLeafDataIdx<<<gridFor(m), BLOCK, 0, itsStream>>>(itsM, itsProc.mergingThreshold, itsNodeAux.as<uint32_t>(),
-                                                       itsNodeFlags.as<uint8_t>(), itsNodeChild.as<int32_t>(),
-                                                       itsNodePoints.as<uint32_t>(), itsNodeData.as<uint64_t>());
-    OC_LAUNCH_CHECK();
-    kCellLeaf<<<gridFor(itsLevelStart[1]), BLOCK, 0, itsStream>>>(itsLevelStart[1], itsNodeKey.as<uint32_t>(),
-                                                                   itsNodeFlags.as<uint8_t>(),
-                                                                   itsNodeParent.as<int32_t>(), count);
-    OC_LAUNCH_CHECK();
+// chunks of leaves: at most N / LEAF_CHUNK plus one per leaf, and a leaf is a child of an internal node
+uint64_t OctreeBuilder::leafChunkBound() const
+{
+    return itsCloud.pointAmount / LEAF_CHUNK + std::min<uint64_t>(8ull * itsInner[itsDepth + 1], itsM);
+}
+
+uint64_t OctreeBuilder::placeChunkBound() const
+{
+    return (itsE - itsCloud.pointAmount) / PLACE_CHUNK + itsInner[itsDepth + 1];
 }
 
 template <typename T>
@@ -650,30 +742,22 @@ void OctreeBuilder::distributePoints()
                itsProc.chunkingGrid};
     // octree_chunking.cu:108-112
     double sx = 1.0 / itsCloud.scale[0], sy = 1.0 / itsCloud.scale[1], sz = 1.0 / itsCloud.scale[2];
-    LevelParams lp{};
-    for (uint32_t l = 0; l <= itsDepth; ++l)
-    {
-        lp.offset[l] = itsLevelOffset[l];
-        lp.grid[l]   = itsLevelGrid[l];
-    }
-    lp.depth     = itsDepth;
-    lp.threshold = itsProc.mergingThreshold;
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_DIST_BEGIN], itsStream));
-    kSortedStart<<<gridFor(itsM), BLOCK, 0, itsStream>>>(itsM, lp, itsNodeKey.as<uint32_t>(),
-                                                         itsNodeCount.as<uint32_t>(), itsNodeFlags.as<uint8_t>(),
-                                                         itsNodeParent.as<int32_t>(), itsNodeChild.as<int32_t>(),
-                                                         itsNodeSorted.as<uint32_t>());
-    OC_LAUNCH_CHECK();
-    // the records move to the sorted cloud: leaf and cell order when there are internal nodes,
-    // plain Morton order otherwise; then the leaf data blocks are copied from it
+    const LeafOrderParams p = leafTables();
+    // the records move to the sorted cloud: leaf and cell order when there are internal nodes and
+    // more than one cell to a node's grid, plain Morton order otherwise; then the leaf data blocks are
+    // copied from it
     const uint32_t n = itsCloud.pointAmount;
-    if (!orderLeafPoints<T>())
-    {
+    if (itsInner[itsDepth + 1] > 0 && p.g >= 2)
+        kLeafCellOrder<T><<<static_cast<unsigned>(leafChunkBound()), LEAF_THREADS, 0, itsStream>>>(
+                itsLeafList.as<uint64_t>(), itsScalars.as<uint64_t>() + SC_LEAF_TOTAL, p, itsNodeKey.as<uint32_t>(),
+                itsNodeParent.as<int32_t>(), itsNodeCount.as<uint32_t>(), itsNodeSorted.as<uint32_t>(),
+                itsBucketed.as<SortedPoint<T>>(), itsPerm.as<uint32_t>(), itsSorted.as<SortedPoint<T>>());
+    else
         kGatherSorted<T><<<gatherGrid(n), BLOCK, 0, itsStream>>>(itsBucketed.as<SortedPoint<T>>(),
                                                                      itsPerm.as<uint32_t>(), n,
                                                                      itsSorted.as<SortedPoint<T>>());
-        OC_LAUNCH_CHECK();
-    }
+    OC_LAUNCH_CHECK();
     kDistributeSorted<T><<<gridFor(n, 16384), BLOCK, 0, itsStream>>>(
             itsSorted.as<SortedPoint<T>>(), n, g, itsCount.as<uint32_t>(), itsNodeSorted.as<uint32_t>(),
             itsNodeData.as<uint64_t>(), itsLut.as<uint32_t>(), itsOut.as<OutRecord>(), sx, sy, sz);
@@ -681,70 +765,35 @@ void OctreeBuilder::distributePoints()
     OC_HIP_CHECK(hipEventRecord(itsEvents[EV_DIST_END], itsStream));
 }
 
-template <typename T, uint32_t MODE>
-static void launchAccumulate(bool random, unsigned blocks, hipStream_t s, uint32_t tileBase, uint32_t nodeBase,
-                             uint64_t words, const uint32_t* tileList, const uint32_t* segTile,
-                             const uint32_t* segCount, const uint32_t* segSrc, const uint32_t* segInput,
-                             const NodeGrid* nodeGrid, const uint32_t* bitmap, const uint32_t* prefix,
-                             uint32_t* cellOf, const PointStore<T>& ps, uint64_t* win, uint64_t* color,
-                             uint32_t* cellCnt, uint32_t* cellKey, uint32_t* cellNode, uint32_t* rankOf)
+// Nodes of one subsampling step: their bitmaps and prefixes fit kBitmapBudget.
+uint32_t OctreeBuilder::stepNodes() const
 {
-    if (random)
-        kAccumulate<T, MODE, true><<<blocks, TILE, 0, s>>>(tileBase, nodeBase, words, tileList, segTile, segCount,
-                                                            segSrc, segInput, nodeGrid, bitmap, prefix, cellOf, ps,
-                                                            win, color, cellCnt, cellKey, cellNode, rankOf);
-    else
-        kAccumulate<T, MODE, false><<<blocks, TILE, 0, s>>>(tileBase, nodeBase, words, tileList, segTile, segCount,
-                                                             segSrc, segInput, nodeGrid, bitmap, prefix, cellOf, ps,
-                                                             win, color, cellCnt, cellKey, cellNode, rankOf);
+    const uint64_t words = (rowsPerNode(itsProc.subsamplingGrid) * itsProc.subsamplingGrid + 31) / 32;
+    return static_cast<uint32_t>(std::max<uint64_t>(1, kBitmapBudget / (2 * sizeof(uint32_t) * words)));
 }
 
-
-// The sorted cloud in leaf and cell order (kLeafCellOrder): false when no leaf has a parent (the
-// root is the only leaf), so nothing is subsampled and plain Morton order serves.
-template <typename T>
-bool OctreeBuilder::orderLeafPoints()
+// Subsampling steps of the build (batches of a level's nodes).
+uint32_t OctreeBuilder::planSteps()
 {
-    if (itsProc.subsamplingGrid < 2 || itsM < 2)
-        return false;
-    uint64_t* sc = itsScalars.as<uint64_t>();
-    // chunks per leaf are at most N / LEAF_CHUNK + (number of leaves) in total
-    itsLeafList.ensure(sizeof(uint64_t) * (itsM + itsCloud.pointAmount / LEAF_CHUNK + 1));
-    itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(itsM) + 1));
-    scanExclusive<uint32_t>(itsM, LeafIn{itsNodeFlags.as<uint8_t>(), itsNodeParent.as<int32_t>(),
-                                         itsNodeCount.as<uint32_t>()},
-                            LeafOut{itsLeafList.as<uint64_t>()}, itsScanScratch.as<uint32_t>(),
-                            reinterpret_cast<uint32_t*>(sc + SC_TABLE_TOTAL), itsStream);
-    OC_LAUNCH_CHECK();
-    const uint32_t chunks = static_cast<uint32_t>(readDevice(sc + SC_TABLE_TOTAL));
-    if (chunks == 0)
-        return false;  // the root is the only leaf: nothing is subsampled
-    const double cubicSize = itsCloud.bbMax[0] - itsCloud.bbMin[0];  // metadata.cuh:66-69
-    LeafOrderParams p{};
-    for (int a = 0; a < 3; ++a)
-        p.cubicMin[a] = itsCloud.bbMin[a];
-    for (uint32_t l = 0; l <= itsDepth; ++l)
-    {
-        p.side[l]      = cubicSize / std::pow(2.0, static_cast<double>(itsDepth - l));  // rp_subsampling.cu:17-18
-        p.sideHalf[l]  = p.side[l] / 2.0;
-        p.lp.offset[l] = itsLevelOffset[l];
-        p.lp.grid[l]   = itsLevelGrid[l];
-    }
-    p.lp.depth     = itsDepth;
-    p.lp.threshold = itsProc.mergingThreshold;
-    p.g            = itsProc.subsamplingGrid;
-    const uint32_t h    = p.g > 1 ? p.g / 2 : 1;  // cells per axis of a leaf's octant, as kLeafCellOrder
-    const uint64_t keys = rowsPerNode(h) * ((h + 31) / 32);
-    while (((keys - 1) >> p.keyShift) >= LEAF_KEYS)
-        ++p.keyShift;
-    kLeafCellOrder<T><<<chunks, LEAF_THREADS, 0, itsStream>>>(
-            itsLeafList.as<uint64_t>(), p, itsNodeKey.as<uint32_t>(), itsNodeParent.as<int32_t>(),
-            itsNodeCount.as<uint32_t>(), itsNodeSorted.as<uint32_t>(), itsBucketed.as<SortedPoint<T>>(),
-            itsPerm.as<uint32_t>(), itsSorted.as<SortedPoint<T>>());
-    OC_LAUNCH_CHECK();
-    return true;
+    itsSteps = 0;
+    for (uint32_t l = 1; l <= itsDepth; ++l)
+        itsSteps += (itsInner[l + 1] - itsInner[l] + stepNodes() - 1) / stepNodes();
+    return itsSteps;
 }
 
+// Points from which the host reads a level's inputs back to size its launches.
+static constexpr uint32_t READ_INPUTS_POINTS = 1u << 24;
+
+// The levels bottom-up, a step per batch of a level's nodes. The merge has told the host the internal
+// nodes of every level; inputs, tiles, occupied cells and the output cursor stay on the device, the
+// launches are sized by bounds (a level's inputs are distinct points, so there are at most N of them,
+// and no more cells than inputs), and a step that does not fit the output leaves itself and the later
+// ones without work. So the host waits for nothing: with two readbacks a level, each of which drains
+// the GPU for ~15 us, small builds spent a third of their time waiting. From READ_INPUTS_POINTS points
+// on, one readback a level costs less than the empty workgroups of the upper levels (a 120M-point
+// bound is 470K of them, ~30 us a launch, three or four launches a level). Grids that stride over
+// the work instead were slower on large levels (payload scatter 3.9 -> 4.9 ms, emit 11.0 -> 11.9 ms at
+// 119.7M points): workgroups drift apart and no longer share cache lines while they are in L2.
 template <typename T>
 void OctreeBuilder::subsampleLevels()
 {
@@ -755,11 +804,9 @@ void OctreeBuilder::subsampleLevels()
     const double cubicSize   = itsCloud.bbMax[0] - itsCloud.bbMin[0];  // metadata.cuh:66-69
     const uint64_t cellsPerNode = rowsPerNode(g) * g;
     const uint64_t wordsPerNode = (cellsPerNode + 31) / 32;
-    const uint32_t batchNodes   = static_cast<uint32_t>(
-            std::max<uint64_t>(1, kBitmapBudget / (2 * sizeof(uint32_t) * wordsPerNode)));
+    const uint32_t batchNodes   = stepNodes();
     const bool packed   = itsColorMode == COLOR_INTRA || itsColorMode == COLOR_INTER;
     const bool weighted = itsColorMode == COLOR_INTER_WEIGHTED;
-    uint64_t cursor     = N;
     PointStore<T> ps{};
     ps.sorted = itsSorted.as<SortedPoint<T>>();
     ps.stLut  = itsStLut.as<uint32_t>();
@@ -781,331 +828,223 @@ void OctreeBuilder::subsampleLevels()
     sp.g     = g;
     sp.seed  = itsProc.seed;
 
+    // sizes over all levels
+    uint32_t levelMost = 0;
+    for (uint32_t l = 1; l <= itsDepth; ++l)
+        levelMost = std::max(levelMost, itsInner[l + 1] - itsInner[l]);
+    uint64_t* cursors = itsCursors.as<uint64_t>();
+    if (levelMost == 0)
+        return;
+    const uint64_t segMost  = 8ull * levelMost;
+    const uint64_t tileMost = N / TILE + segMost;
+    const uint64_t wordMost = std::min(levelMost, batchNodes) * wordsPerNode;
+    itsSegCount.ensure(sizeof(uint32_t) * segMost);
+    itsSegSrc.ensure(sizeof(uint32_t) * segMost);
+    itsSegTile.ensure(sizeof(uint32_t) * segMost);
+    itsSegInput.ensure(sizeof(uint32_t) * segMost);
+    itsNodeGrid.ensure(sizeof(NodeGrid) * levelMost);
+    itsTileList.ensure(sizeof(uint32_t) * tileMost);
+    itsBitmap.ensure(sizeof(uint32_t) * wordMost);
+    itsPrefix.ensure(sizeof(uint32_t) * (wordMost + 1));
+    itsCellOf.ensure(sizeof(uint32_t) * N);
+    itsCellKey.ensure(sizeof(uint32_t) * N);
+    itsCellNode.ensure(sizeof(uint32_t) * N);
+    if (weighted)
+    {
+        itsRankOf.ensure(sizeof(uint32_t) * N);
+        itsPayload.ensure((sizeof(WeightPayload) + sizeof(uint64_t)) * N);  // payloads, then winner keys
+        itsCellCnt.ensure(sizeof(uint32_t) * N);
+        itsCellStart.ensure(sizeof(uint32_t) * (static_cast<uint64_t>(N) + 1));
+    }
+    else  // the weighted filter takes its winners from the payload keys
+        itsWin.ensure(sizeof(uint64_t) * N);
+    if (packed)
+        itsColor.ensure(sizeof(uint64_t) * N);
+    uint64_t* winKey =
+            weighted ? reinterpret_cast<uint64_t*>(itsPayload.as<uint8_t>() + sizeof(WeightPayload) * N) : nullptr;
+    uint64_t* win     = weighted ? nullptr : itsWin.as<uint64_t>();
+    uint64_t* color   = packed ? itsColor.as<uint64_t>() : nullptr;
+    uint32_t* cellCnt = weighted ? itsCellCnt.as<uint32_t>() : nullptr;
+    uint32_t* bitmap  = itsBitmap.as<uint32_t>();
+    uint32_t* prefix  = itsPrefix.as<uint32_t>();
+
+    uint32_t stepAt = 0;
     for (uint32_t l = 1; l <= itsDepth; ++l)
     {
-        const uint32_t ls          = itsLevelStart[l];
-        const uint32_t levelNodes  = itsLevelStart[l + 1] - ls;
-        if (levelNodes == 0)
+        const uint32_t K = itsInner[l + 1] - itsInner[l];
+        if (K == 0)
             continue;
+        const ChildSlots cs        = childSlots(itsInner[l]);
+        NodeGrid* nodeGrid         = itsNodeGrid.as<NodeGrid>();
+        scanExclusive<uint64_t>(8ull * K, LevelSegmentIn{cs, itsNodePoints.as<uint32_t>()},
+                                LevelSegmentOut{cs, itsNodeSorted.as<uint32_t>(), itsNodeStage.as<uint32_t>(),
+                                                itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(),
+                                                itsSegTile.as<uint32_t>(), itsSegInput.as<uint32_t>()},
+                                itsScanScratch.as<uint64_t>(), sc + SC_SEG_TOTAL, itsStream);
+        OC_LAUNCH_CHECK();
+        uint64_t inputMost = N;
+        if (N >= READ_INPUTS_POINTS)
+        {
+            const uint64_t seq = ++itsMailSeq;
+            kPublishInputs<<<1, 64, 0, itsStream>>>(sc + SC_SEG_TOTAL, itsMailbox, seq);
+            OC_LAUNCH_CHECK();
+            waitMailbox(seq);
+            inputMost = itsMailbox[MAIL_INPUTS];
+        }
+        const uint32_t tileGrid = xcdRunGrid(inputMost / TILE + 8ull * K, XCD_TILE_RUN);
         sp.level       = l;
         sp.levelOffset = itsLevelOffset[l];
         sp.levelGrid   = itsLevelGrid[l];
         sp.side        = cubicSize / std::pow(2.0, static_cast<double>(itsDepth - l));  // rp_subsampling.cu:17-18
 
-        // the internal nodes of the level, their input segments and griddings, the segment scan
-        // and the tile list: one workgroup and one readback for small levels, four launches and
-        // two readbacks otherwise (inputs <= cursor: leaf points plus everything subsampled so far)
-        const bool smallLevel = levelNodes <= SMALL_LEVEL_NODES && cursor <= SMALL_LEVEL_POINTS;
-        itsInternalList.ensure(sizeof(uint32_t) * levelNodes);
-        itsSegCount.ensure(sizeof(uint32_t) * 8 * levelNodes);
-        itsSegSrc.ensure(sizeof(uint32_t) * 8 * levelNodes);
-        itsSegTile.ensure(sizeof(uint32_t) * 8 * levelNodes);
-        itsSegInput.ensure(sizeof(uint32_t) * 8 * levelNodes);
-        itsNodeGrid.ensure(sizeof(NodeGrid) * levelNodes);
-        auto tables = [&]() {
-            return LevelTables{itsNodeKey.as<uint32_t>(),     itsNodeFlags.as<uint8_t>(),   itsNodeChild.as<int32_t>(),
-                               itsNodePoints.as<uint32_t>(),  itsNodeSorted.as<uint32_t>(), itsNodeStage.as<uint32_t>(),
-                               itsInternalList.as<uint32_t>(), itsSegCount.as<uint32_t>(),  itsSegSrc.as<uint32_t>(),
-                               itsSegTile.as<uint32_t>(),     itsSegInput.as<uint32_t>(),   itsTileList.as<uint32_t>(),
-                               itsNodeGrid.as<NodeGrid>()};
-        };
-        uint32_t K        = 0;
-        uint64_t segTotal = 0;
-        if (smallLevel)
-        {
-            itsTileList.ensure(sizeof(uint32_t) * (cursor / TILE + 8ull * levelNodes + 1));
-            kLevelSetup<<<1, SCAN_THREADS, 0, itsStream>>>(ls, levelNodes, sp, tables(),
-                                                           reinterpret_cast<uint32_t*>(sc + SC_TABLE_TOTAL),
-                                                           sc + SC_SEG_TOTAL);
-            OC_LAUNCH_CHECK();
-            const auto v = readDevicePair(sc + SC_SEG_TOTAL);  // segment total, internal-node count
-            segTotal     = v[0];
-            K            = static_cast<uint32_t>(v[1]);
-            if (K == 0)
-                continue;
-        }
-        else
-        {
-            itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(8ull * levelNodes) + 1));
-            scanExclusive<uint32_t>(levelNodes, InternalIn{itsNodeFlags.as<uint8_t>(), ls},
-                                    InternalOut{itsInternalList.as<uint32_t>(), ls}, itsScanScratch.as<uint32_t>(),
-                                    reinterpret_cast<uint32_t*>(sc + SC_TABLE_TOTAL), itsStream);
-            OC_LAUNCH_CHECK();
-            K = static_cast<uint32_t>(readDevice(sc + SC_TABLE_TOTAL));
-            if (K == 0)
-                continue;
-            kSegments<<<gridFor(K), BLOCK, 0, itsStream>>>(K, sp, tables());
-            OC_LAUNCH_CHECK();
-            scanExclusive<uint64_t>(8ull * K, SegmentIn{itsSegCount.as<uint32_t>()},
-                                    SegmentOut{itsSegTile.as<uint32_t>(), itsSegInput.as<uint32_t>()},
-                                    itsScanScratch.as<uint64_t>(), sc + SC_SEG_TOTAL, itsStream);
-            OC_LAUNCH_CHECK();
-            segTotal = readDevice(sc + SC_SEG_TOTAL);
-            itsTileList.ensure(sizeof(uint32_t) * (segTotal >> 32));
-            kTileList<<<gridFor(8ull * K), BLOCK, 0, itsStream>>>(8ull * K, itsSegCount.as<uint32_t>(),
-                                                                  itsSegTile.as<uint32_t>(), itsTileList.as<uint32_t>());
-            OC_LAUNCH_CHECK();
-        }
-        const uint32_t tiles  = static_cast<uint32_t>(segTotal >> 32);
-        const uint32_t inputs = static_cast<uint32_t>(segTotal);
-        if (inputs == 0)
-            continue;
-
-        itsCellOf.ensure(sizeof(uint32_t) * inputs);
-        if (weighted)
-        {
-            itsRankOf.ensure(sizeof(uint32_t) * inputs);
-            itsPayload.ensure((sizeof(WeightPayload) + sizeof(uint64_t)) * inputs);  // payloads, then winner keys
-        }
-        uint64_t* winKey =
-                weighted ? reinterpret_cast<uint64_t*>(itsPayload.as<uint8_t>() + sizeof(WeightPayload) * inputs) : nullptr;
-
         for (uint32_t k0 = 0; k0 < K; k0 += batchNodes)
         {
             const uint32_t k1 = std::min<uint32_t>(K, k0 + batchNodes);
             const uint32_t Kb = k1 - k0;
-            uint32_t tileLo = 0, tileHi = tiles;
-            if (k0 > 0)
-                tileLo = readDevice(itsSegTile.as<uint32_t>() + 8ull * k0);
-            if (k1 < K)
-                tileHi = readDevice(itsSegTile.as<uint32_t>() + 8ull * k1);
-            const unsigned blocks = tileHi - tileLo;
-            const uint64_t words  = static_cast<uint64_t>(Kb) * wordsPerNode;
-            itsBitmap.ensure(sizeof(uint32_t) * words);
-            itsPrefix.ensure(sizeof(uint32_t) * (words + 1));
-            itsNodeFirst.ensure(sizeof(uint32_t) * (Kb + 1));
-            itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(words) + 1));
-            uint32_t* bitmap = itsBitmap.as<uint32_t>();
-            uint32_t* prefix = itsPrefix.as<uint32_t>();
+            const uint64_t words = static_cast<uint64_t>(Kb) * wordsPerNode;
+            const uint64_t cellMost = std::min<uint64_t>(inputMost, 32 * words);
+            const TileRange tiles{k0 > 0 ? itsSegTile.as<uint32_t>() + 8ull * k0 : nullptr,
+                                  k1 < K ? itsSegTile.as<uint32_t>() + 8ull * k1
+                                         : reinterpret_cast<uint32_t*>(sc + SC_SEG_TOTAL) + 1};
+            const StepSizes step{cursors + stepAt, cursors + stepAt + 1, prefix + words, itsE};
+            ++stepAt;
             std::array<hipEvent_t, 4> none{};
             auto& ev         = itsDetailedTimings ? batchEvents() : none;
 
-            kFill32<<<gridFor(words), BLOCK, 0, itsStream>>>(bitmap, words, 0);
+            kLevelPrepare<<<gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384), BLOCK, 0, itsStream>>>(
+                    K, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
+                    sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap);
             OC_LAUNCH_CHECK();
             if (itsDetailedTimings)
                 OC_HIP_CHECK(hipEventRecord(ev[0], itsStream));
-            if (blocks > 0)
-            {
-                kMark<T><<<xcdRunGrid(blocks, XCD_TILE_RUN), TILE, 0, itsStream>>>(
-                        tileLo, blocks, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                        itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(),
-                        itsNodeGrid.as<NodeGrid>(), ps, bitmap, itsCellOf.as<uint32_t>(), err);
-                OC_LAUNCH_CHECK();
-            }
-            // per-cell state, reset for the occupied cells: by the scan itself on small levels
-            // (arrays sized by the inputs, an upper bound of the cells), else by kClearCompact
-            auto sizeCells = [&](uint64_t n) {
-                if (!weighted)  // the weighted filter takes its winners from the payload keys
-                    itsWin.ensure(sizeof(uint64_t) * n);
-                itsCellKey.ensure(sizeof(uint32_t) * n);
-                itsCellNode.ensure(sizeof(uint32_t) * n);
-                if (packed)
-                    itsColor.ensure(sizeof(uint64_t) * n);
-                if (weighted)
-                {
-                    itsCellCnt.ensure(sizeof(uint32_t) * n);
-                    itsCellStart.ensure(sizeof(uint32_t) * (n + 1));
-                    itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(n) + 1));
-                }
-            };
-            if (smallLevel)
-            {
-                sizeCells(inputs);
-                scanExclusive<uint32_t>(words, PopcountIn{bitmap},
-                                        PrefixClearOut{prefix, weighted ? nullptr : itsWin.as<uint64_t>(),
-                                                       packed ? itsColor.as<uint64_t>() : nullptr,
-                                                       weighted ? itsCellCnt.as<uint32_t>() : nullptr},
+            kMark<T><<<tileGrid, TILE, 0, itsStream>>>(
+                    tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                    itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid, ps,
+                    bitmap, itsCellOf.as<uint32_t>(), err);
+            OC_LAUNCH_CHECK();
+            // per-cell state, reset for the occupied cells: by the scan itself on small levels, else
+            // by kClearCompact
+            const bool clearInScan = words <= CLEAR_IN_SCAN_WORDS;
+            if (clearInScan)
+                scanExclusive<uint32_t>(words, PopcountIn{bitmap}, PrefixClearOut{prefix, win, color, cellCnt},
                                         itsScanScratch.as<uint32_t>(), prefix + words, itsStream);
-            }
             else
                 scanExclusive<uint32_t>(words, PopcountIn{bitmap}, ExclusiveToArray{prefix},
                                         itsScanScratch.as<uint32_t>(), prefix + words, itsStream);
             OC_LAUNCH_CHECK();
-            kBatchNodes<<<gridFor(Kb + 1), BLOCK, 0, itsStream>>>(
-                    k0, Kb, wordsPerNode, itsNodeGrid.as<NodeGrid>(), prefix, static_cast<uint32_t>(cursor),
-                    itsNodePoints.as<uint32_t>(), itsNodeStage.as<uint32_t>(), itsNodeFirst.as<uint32_t>());
-            OC_LAUNCH_CHECK();
-            const uint32_t cells = readDevice(prefix + words);
-            if (cursor + cells > itsE)  // A14
-                throw std::runtime_error("the subsampled points exceed the estimated output size (N + I > E); "
-                                         "raise the output factor");
-            if (cells == 0)
-                continue;
-            if (!smallLevel)
+            if (!clearInScan)
             {
-                sizeCells(cells);
-                kClearCompact<<<gridFor(cells), BLOCK, 0, itsStream>>>(
-                        cells, weighted ? nullptr : itsWin.as<uint64_t>(), packed ? itsColor.as<uint64_t>() : nullptr,
-                        weighted ? itsCellCnt.as<uint32_t>() : nullptr);
+                kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(prefix + words, win, color, cellCnt);
                 OC_LAUNCH_CHECK();
             }
-            uint64_t* color   = packed ? itsColor.as<uint64_t>() : nullptr;
-            uint32_t* cellCnt = weighted ? itsCellCnt.as<uint32_t>() : nullptr;
 
-
-            if (blocks > 0)
-            {
-                switch (itsColorMode)
-                {
-#define OC_ACC(M)                                                                                                      \
-    launchAccumulate<T, M>(itsProc.useRandomSubsampling, blocks, itsStream, tileLo, k0, wordsPerNode,                 \
-                           itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(), itsSegCount.as<uint32_t>(),         \
-                           itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), itsNodeGrid.as<NodeGrid>(), bitmap,  \
-                           prefix, itsCellOf.as<uint32_t>(), ps, itsWin.as<uint64_t>(), color, cellCnt,               \
-                           itsCellKey.as<uint32_t>(), itsCellNode.as<uint32_t>(),                                     \
-                        weighted ? itsRankOf.as<uint32_t>() : nullptr)
-                case COLOR_NONE: OC_ACC(COLOR_NONE); break;
-                case COLOR_INTRA: OC_ACC(COLOR_INTRA); break;
-                case COLOR_INTER: OC_ACC(COLOR_INTER); break;
-                default: OC_ACC(COLOR_INTER_WEIGHTED); break;
-#undef OC_ACC
-                }
+            auto accumulate = [&](auto kernel) {
+                kernel<<<tileGrid, TILE, 0, itsStream>>>(
+                        tiles, step, k0, Kb, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                        itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
+                        bitmap, prefix, itsCellOf.as<uint32_t>(), ps, win, color, cellCnt, itsCellKey.as<uint32_t>(),
+                        itsCellNode.as<uint32_t>(), weighted ? itsRankOf.as<uint32_t>() : nullptr,
+                        itsNodePoints.as<uint32_t>(), itsNodeStage.as<uint32_t>(), itsNodeSub.as<uint32_t>(),
+                        itsNodeFlags.as<uint8_t>(), itsNodeChild.as<int32_t>(), err);
                 OC_LAUNCH_CHECK();
+            };
+            const bool random = itsProc.useRandomSubsampling;
+            switch (itsColorMode)
+            {
+            case COLOR_NONE: accumulate(random ? kAccumulate<T, COLOR_NONE, true> : kAccumulate<T, COLOR_NONE, false>); break;
+            case COLOR_INTRA:
+                accumulate(random ? kAccumulate<T, COLOR_INTRA, true> : kAccumulate<T, COLOR_INTRA, false>);
+                break;
+            case COLOR_INTER:
+                accumulate(random ? kAccumulate<T, COLOR_INTER, true> : kAccumulate<T, COLOR_INTER, false>);
+                break;
+            default:
+                accumulate(random ? kAccumulate<T, COLOR_INTER_WEIGHTED, true>
+                                  : kAccumulate<T, COLOR_INTER_WEIGHTED, false>);
+                break;
             }
             if (itsDetailedTimings)
                 OC_HIP_CHECK(hipEventRecord(ev[1], itsStream));
 
             if (weighted)
             {
-                scanExclusive<uint32_t>(cells, ArrayIn{cellCnt}, ExclusiveToArray{itsCellStart.as<uint32_t>()},
-                                        itsScanScratch.as<uint32_t>(), itsCellStart.as<uint32_t>() + cells,
-                                        itsStream);
+                scanExclusive<uint32_t>(DeviceCount{step.cells, nullptr}, cellMost, ArrayIn{cellCnt},
+                                        ExclusiveWithTotal{itsCellStart.as<uint32_t>(), step.cells},
+                                        itsScanScratch.as<uint32_t>(), static_cast<uint32_t*>(nullptr), itsStream);
                 OC_LAUNCH_CHECK();
-                if (blocks > 0)
-                {
-                    if (itsProc.useRandomSubsampling)
-                        kScatterPayload<T, true><<<xcdRunGrid(blocks, XCD_TILE_RUN), TILE, 0, itsStream>>>(
-                                tileLo, blocks, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                                itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(),
-                                itsNodeGrid.as<NodeGrid>(), itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(),
-                                itsCellStart.as<uint32_t>(), itsCellOf.as<uint32_t>(), ps,
-                                itsPayload.as<WeightPayload>(), winKey);
-                    else
-                        kScatterPayload<T, false><<<xcdRunGrid(blocks, XCD_TILE_RUN), TILE, 0, itsStream>>>(
-                                tileLo, blocks, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                                itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(),
-                                itsNodeGrid.as<NodeGrid>(), itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(),
-                                itsCellStart.as<uint32_t>(), itsCellOf.as<uint32_t>(), ps,
-                                itsPayload.as<WeightPayload>(), winKey);
+                auto scatter = [&](auto kernel) {
+                    kernel<<<tileGrid, TILE, 0, itsStream>>>(
+                            tiles, step, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                            itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
+                            itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(), itsCellStart.as<uint32_t>(),
+                            itsCellOf.as<uint32_t>(), ps, itsPayload.as<WeightPayload>(), winKey);
                     OC_LAUNCH_CHECK();
-                }
+                };
+                scatter(random ? kScatterPayload<T, true> : kScatterPayload<T, false>);
             }
 
             if (itsDetailedTimings)
                 OC_HIP_CHECK(hipEventRecord(ev[2], itsStream));
             if (weighted)
-            {
-                const uint32_t emitBlocks = xcdRunGrid((cells + BLOCK - 1) / BLOCK, EMIT_CHUNK);
-                kEmitWeighted<T><<<emitBlocks, BLOCK, 0, itsStream>>>(
-                        cells, k0, wordsPerNode, static_cast<uint32_t>(cursor), itsNodeGrid.as<NodeGrid>(), bitmap,
-                        prefix, itsCellKey.as<uint32_t>(), itsCellNode.as<uint32_t>(), itsCellStart.as<uint32_t>(),
-                        itsPayload.as<WeightPayload>(), winKey, ps);
-                OC_LAUNCH_CHECK();
-            }
+                kEmitWeighted<T><<<xcdRunGrid((cellMost + BLOCK - 1) / BLOCK, EMIT_CHUNK), BLOCK, 0, itsStream>>>(
+                        step, k0, wordsPerNode, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
+                        itsCellNode.as<uint32_t>(), itsCellStart.as<uint32_t>(), itsPayload.as<WeightPayload>(), winKey,
+                        ps);
             else
             {
+                auto emit = [&](auto kernel) {
+                    kernel<<<gridFor(cellMost), BLOCK, 0, itsStream>>>(
+                            step, k0, wordsPerNode, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
+                            itsCellNode.as<uint32_t>(), win, color, ps);
+                };
                 switch (itsColorMode)
                 {
-#define OC_EMIT(M)                                                                                                     \
-    kEmit<T, M><<<gridFor(cells), BLOCK, 0, itsStream>>>(cells, k0, wordsPerNode, static_cast<uint32_t>(cursor),      \
-                                                         itsNodeGrid.as<NodeGrid>(), bitmap, prefix,                  \
-                                                         itsCellKey.as<uint32_t>(), itsCellNode.as<uint32_t>(),       \
-                                                         itsWin.as<uint64_t>(), itsColor.as<uint64_t>(), ps)
-                case COLOR_NONE: OC_EMIT(COLOR_NONE); break;
-                case COLOR_INTRA: OC_EMIT(COLOR_INTRA); break;
-                default: OC_EMIT(COLOR_INTER); break;
-#undef OC_EMIT
+                case COLOR_NONE: emit(kEmit<T, COLOR_NONE>); break;
+                case COLOR_INTRA: emit(kEmit<T, COLOR_INTRA>); break;
+                default: emit(kEmit<T, COLOR_INTER>); break;
                 }
-                OC_LAUNCH_CHECK();
             }
+            OC_LAUNCH_CHECK();
             if (itsDetailedTimings)
                 OC_HIP_CHECK(hipEventRecord(ev[3], itsStream));
-            cursor += cells;
         }
         progress();
     }
-    itsUsed = cursor;
 }
-
-// Trees up to this many nodes are placed by one workgroup in one launch.
-static constexpr uint32_t kPlaceOneGroupNodes = 1u << 16;
 
 void OctreeBuilder::placeInternalNodes()
 {
-    const uint32_t N      = itsCloud.pointAmount;
-    const uint64_t staged = itsUsed - N;
-    if (itsM <= kPlaceOneGroupNodes)
-    {
-        PlaceParams pp{};
-        for (uint32_t l = 0; l <= itsDepth + 1 && l <= MAX_LEVELS; ++l)
-            pp.levelStart[l] = itsLevelStart[l];
-        pp.depth = itsDepth;
-        pp.m     = itsM;
-        pp.root  = itsM - 1;
-        pp.N     = N;
-        kPlaceLevels<<<1, PLACE_THREADS, 0, itsStream>>>(pp, itsNodeFlags.as<uint8_t>(), itsNodeChild.as<int32_t>(),
-                                                          itsNodePoints.as<uint32_t>(), itsNodeSub.as<uint32_t>(),
-                                                          itsNodeRegion.as<uint32_t>(), itsNodeData.as<uint64_t>());
-        OC_LAUNCH_CHECK();
-    }
-    else
-        placeLevelByLevel();
-    if (staged > 0)
-    {
-        // (internal node, chunk) work items; the leaf chunk list is free again after the distribution
-        uint64_t* sc = itsScalars.as<uint64_t>();
-        itsLeafList.ensure(sizeof(uint64_t) * (itsM + staged / PLACE_CHUNK + 1));
-        itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(itsM) + 1));
-        scanExclusive<uint32_t>(itsM, PlacedChunksIn{itsNodeFlags.as<uint8_t>(), itsNodePoints.as<uint32_t>()},
-                                LeafOut{itsLeafList.as<uint64_t>()}, itsScanScratch.as<uint32_t>(),
-                                reinterpret_cast<uint32_t*>(sc + SC_TABLE_TOTAL), itsStream);
-        OC_LAUNCH_CHECK();
-        const uint32_t chunks = static_cast<uint32_t>(readDevice(sc + SC_TABLE_TOTAL));
-        if (chunks == 0)
-            return;
-        const Gridding cubic{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
-                             itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid};
-        const double sx = 1.0 / itsCloud.scale[0], sy = 1.0 / itsCloud.scale[1], sz = 1.0 / itsCloud.scale[2];
-        const uint32_t* rgb = itsColorMode == COLOR_INTER_WEIGHTED ? itsStRgb.as<uint32_t>() : nullptr;
-        if (itsCloud.cloudType == CLOUD_FLOAT_UINT8_T)
-            kPermute<float><<<chunks, BLOCK, 0, itsStream>>>(
-                    itsLeafList.as<uint64_t>(), N, itsNodeStage.as<uint32_t>(), itsNodeData.as<uint64_t>(),
-                    itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(), itsStOut.as<OutRecord>(),
-                    itsStPts.as<float>(), rgb, cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
-        else
-            kPermute<double><<<chunks, BLOCK, 0, itsStream>>>(
-                    itsLeafList.as<uint64_t>(), N, itsNodeStage.as<uint32_t>(), itsNodeData.as<uint64_t>(),
-                    itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(), itsStOut.as<OutRecord>(),
-                    itsStPts.as<double>(), rgb, cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
-        OC_LAUNCH_CHECK();
-    }
-}
-
-void OctreeBuilder::placeLevelByLevel()
-{
-    const uint32_t N = itsCloud.pointAmount;
-    kFill32<<<gridFor(itsM), BLOCK, 0, itsStream>>>(itsNodeSub.as<uint32_t>(), itsM, 0);
+    const uint32_t N     = itsCloud.pointAmount;
+    const uint32_t nodes = itsInner[itsDepth + 1];
+    if (nodes == 0)
+        return;
+    const uint32_t* list = itsInternalList.as<uint32_t>();
+    kPlaceNodes<<<std::min<uint32_t>((nodes + 63) / 64, 4096), 64, 0, itsStream>>>(
+            list, nodes, N, itsNodeParent.as<int32_t>(), itsNodeChild.as<int32_t>(), itsNodePoints.as<uint32_t>(),
+            itsNodeSub.as<uint32_t>(), itsNodeData.as<uint64_t>());
     OC_LAUNCH_CHECK();
-    for (uint32_t l = 1; l <= itsDepth; ++l)
-    {
-        uint32_t ls = itsLevelStart[l], nodes = itsLevelStart[l + 1] - ls;
-        if (nodes == 0)
-            continue;
-        kSubtree<<<gridFor(nodes), BLOCK, 0, itsStream>>>(ls, nodes, itsNodeFlags.as<uint8_t>(),
-                                                          itsNodeChild.as<int32_t>(), itsNodePoints.as<uint32_t>(),
-                                                          itsNodeSub.as<uint32_t>());
-        OC_LAUNCH_CHECK();
-    }
-    for (uint32_t l = itsDepth; l >= 1; --l)
-    {
-        uint32_t ls = itsLevelStart[l], nodes = itsLevelStart[l + 1] - ls;
-        if (nodes == 0)
-            continue;
-        kRegion<<<gridFor(nodes), BLOCK, 0, itsStream>>>(ls, nodes, itsM - 1, N, itsNodeFlags.as<uint8_t>(),
-                                                         itsNodeChild.as<int32_t>(), itsNodeSub.as<uint32_t>(),
-                                                         itsNodeRegion.as<uint32_t>(), itsNodeData.as<uint64_t>());
-        OC_LAUNCH_CHECK();
-    }
+    // (internal node, chunk) work items; the leaf chunk list is free again after the distribution
+    uint32_t* chunks = reinterpret_cast<uint32_t*>(itsScalars.as<uint64_t>() + SC_TABLE_TOTAL);
+    scanExclusive<uint32_t>(nodes, PlacedListIn{list, itsNodePoints.as<uint32_t>()},
+                            PlacedListOut{list, itsLeafList.as<uint64_t>()}, itsScanScratch.as<uint32_t>(), chunks,
+                            itsStream);
+    OC_LAUNCH_CHECK();
+    const Gridding cubic{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
+                         itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid};
+    const double sx = 1.0 / itsCloud.scale[0], sy = 1.0 / itsCloud.scale[1], sz = 1.0 / itsCloud.scale[2];
+    const uint32_t* rgb = itsColorMode == COLOR_INTER_WEIGHTED ? itsStRgb.as<uint32_t>() : nullptr;
+    const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(placeChunkBound(), 1u << 20));
+    if (itsCloud.cloudType == CLOUD_FLOAT_UINT8_T)
+        kPermute<float><<<grid, BLOCK, 0, itsStream>>>(
+                itsLeafList.as<uint64_t>(), chunks, N, itsNodeStage.as<uint32_t>(), itsNodeData.as<uint64_t>(),
+                itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(), itsStOut.as<OutRecord>(),
+                itsStPts.as<float>(), rgb, cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
+    else
+        kPermute<double><<<grid, BLOCK, 0, itsStream>>>(
+                itsLeafList.as<uint64_t>(), chunks, N, itsNodeStage.as<uint32_t>(), itsNodeData.as<uint64_t>(),
+                itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(), itsStOut.as<OutRecord>(),
+                itsStPts.as<double>(), rgb, cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
+    OC_LAUNCH_CHECK();
 }
 
 // Copies go through the builder's own stream, so slots of a build service copy concurrently.

@@ -172,6 +172,33 @@ __device__ __forceinline__ V runScan(V v, const WaveRun& r, Op op)
     return v;
 }
 
+// Bit interleaving for coordinates below 2^10 (part1by2 / compact1by2).
+__host__ __device__ __forceinline__ uint32_t spread3(uint32_t v)
+{
+    v &= 0x000003FFu;
+    v = (v ^ (v << 16)) & 0xFF0000FFu;
+    v = (v ^ (v << 8)) & 0x0300F00Fu;
+    v = (v ^ (v << 4)) & 0x030C30C3u;
+    v = (v ^ (v << 2)) & 0x09249249u;
+    return v;
+}
+
+__host__ __device__ __forceinline__ uint32_t compact3(uint32_t v)
+{
+    v &= 0x09249249u;
+    v = (v ^ (v >> 2)) & 0x030C30C3u;
+    v = (v ^ (v >> 4)) & 0x0300F00Fu;
+    v = (v ^ (v >> 8)) & 0xFF0000FFu;
+    v = (v ^ (v >> 16)) & 0x000003FFu;
+    return v;
+}
+
+// Morton code whose 3-bit groups are child slots (x -> 4, y -> 2, z -> 1).
+__host__ __device__ __forceinline__ uint32_t morton3(uint32_t x, uint32_t y, uint32_t z)
+{
+    return (spread3(x) << 2) | (spread3(y) << 1) | spread3(z);
+}
+
 // grid-stride helpers
 __device__ __forceinline__ uint64_t globalThread()
 {

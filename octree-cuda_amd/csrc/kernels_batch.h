@@ -30,7 +30,6 @@ constexpr uint32_t HIST_CHUNK     = 16384;  // points per work item of the batch
 constexpr uint32_t DIST_CHUNK     = 1024;   // sorted points per work item of the batched distribution
 constexpr uint32_t BATCH_SCAN_X   = 256;    // workgroups per cloud of a batched multi-workgroup scan
 static_assert(BATCH_SCAN_X <= SCAN_THREADS, "a workgroup reads one range sum per thread");
-constexpr uint32_t ERR_OVERFLOW   = 4u;     // N + I > E (A14)
 
 // per-cloud scalar slots (u64)
 enum BatchSlot : int
@@ -84,7 +83,7 @@ struct BatchCloud
     uint64_t* nodeData;
     int32_t *nodeParent, *nodeChild;
     uint8_t* nodeFlags;
-    uint32_t *nodeSorted, *nodeAux, *nodeStage, *nodeSub, *nodeRegion;
+    uint32_t *nodeSorted, *nodeStage, *nodeSub, *nodeRegion;
     uint32_t *keyOut, *countOut;  // packed copies of the node keys and dense counts for the result
     uint64_t* chunkList;
     // output and staging
@@ -97,7 +96,7 @@ struct BatchCloud
     // per-level work
     uint32_t *internalList, *segCount, *segSrc, *segTile, *segInput, *tileList;
     NodeGrid* nodeGrid;
-    uint32_t *bitmap, *prefix, *nodeFirst;
+    uint32_t *bitmap, *prefix;
     uint64_t *win, *color;
     uint32_t *cellCnt, *cellStart, *cellKey, *cellNode, *cellOf, *rankOf;
     WeightPayload* payload;
@@ -196,16 +195,16 @@ struct TileCount  // tiles of the current level (high half of BS_SEG_TOTAL), 0 o
 };
 
 template <typename T>
-struct LevelNodeCount  // internal nodes x factor (+ extra), 0 once failed
+struct LevelNodeCount  // internal nodes x factor, 0 once failed
 {
     const BatchCloud<T>* ctx;
-    uint32_t factor, extra;
+    uint32_t factor;
     __device__ uint32_t operator()(uint64_t c) const
     {
         const BatchCloud<T>& cc = ctx[c];
         if (cc.dead())
             return 0u;
-        return static_cast<uint32_t>(cc.sc[BS_TABLE_TOTAL]) * factor + extra;
+        return static_cast<uint32_t>(cc.sc[BS_TABLE_TOTAL]) * factor;
     }
 };
 
@@ -279,8 +278,7 @@ inline uint32_t scanWidth(uint64_t maxItems)
 template <typename V, typename Job>
 void scanBatch(Job job, uint32_t B, uint64_t maxItems, hipStream_t stream)
 {
-    const uint32_t X = scanWidth(maxItems);
-    const dim3 grid(X, B);
+    const dim3 grid(scanWidth(maxItems), B);
     kScanReduceB<V, Job><<<grid, SCAN_THREADS, 0, stream>>>(job);
     kScanDownB<V, Job><<<grid, SCAN_THREADS, 0, stream>>>(job);
 }
@@ -312,22 +310,21 @@ __device__ __forceinline__ BoundScan<In, Out> bound(In in, Out out, uint64_t n, 
     return BoundScan<In, Out>{in, out, n, sums, total, total32};
 }
 
-// canonical sparse ids over the dense pyramid (A2)
+// occupancy bits and their number per range of words, for the canonical sparse ids (kOccupiedIdsB)
 template <typename T>
 struct OccupancyJob
 {
     const BatchCloud<T>* ctx;
-    uint64_t words;
+    uint64_t marked, dense;
     __device__ auto bind(uint32_t c) const
     {
         const BatchCloud<T>& cc = ctx[c];
-        return bound(OccupiedWordIn{cc.occ},
-                     OccupiedWordOut{cc.occ, cc.denseToSparse, cc.nodeKey, cc.nodeCount, cc.count}, words, cc.scanSums,
-                     cc.sc + BS_M);
+        const OccupancyIn in{cc.occ, cc.count, marked / 32, dense};
+        return bound(in, 0, (dense + 31) / 32, cc.scanSums, cc.sc + BS_M);
     }
 };
 
-// leaf data blocks (A4): scan of the block sizes in id order, in place
+// leaf data blocks (A4): scan of the block sizes in id order
 template <typename T>
 struct LeafBlockJob
 {
@@ -335,7 +332,8 @@ struct LeafBlockJob
     __device__ auto bind(uint32_t c) const
     {
         const BatchCloud<T>& cc = ctx[c];
-        return bound(ArrayIn{cc.nodeAux}, ExclusiveToArray{cc.nodeAux}, cc.m, cc.scanSums, cc.sc + BS_LEAF_TOTAL);
+        const LeafBlockIn in{cc.nodeFlags, cc.nodeChild, cc.nodePoints};
+        return bound(in, LeafBlockOut{in, cc.nodeData}, cc.m, cc.scanSums, cc.sc + BS_LEAF_TOTAL);
     }
 };
 
@@ -475,23 +473,6 @@ static __global__ __launch_bounds__(BLOCK) void kBatchInit(const BatchCloud<T>* 
             cc.occ[k] = 0;
         else
             cc.count[L.marked + (k - words)] = 0;
-    }
-}
-
-// Occupancy bits of the levels the fine sort has not marked, from their counts (as kOccupancyBits:
-// whole waves of 64 consecutive cells, two words).
-template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kOccupancyBitsB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                          BatchLevels L)
-{
-    const uint64_t per = (static_cast<uint64_t>(L.dense) - L.marked + 63) / 64 * 64;
-    for (uint64_t i = globalThread(); i < per * B; i += globalStride())
-    {
-        const BatchCloud<T>& cc = ctx[i / per];
-        const uint64_t d        = L.marked + i % per;
-        const uint64_t bits     = __ballot(d < L.dense && cc.count[d] != 0);
-        if ((threadIdx.x & 31) == 0 && d < L.dense)
-            cc.occ[d >> 5] = static_cast<uint32_t>(bits >> (threadIdx.x & 32));
     }
 }
 
@@ -658,24 +639,39 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineChunkPermB(const Bat
 // Merge
 // ------------------------------------------------------------------------------------------------
 
-template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kPropagateB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                      uint32_t offset, uint32_t grid, uint32_t childOffset,
-                                                      uint32_t childGrid)
+__device__ __forceinline__ LevelOffsets levelOffsets(const BatchLevels& L)
 {
-    const uint64_t per = static_cast<uint64_t>(grid) * grid * grid;
-    for (uint64_t i = globalThread(); i < per * B; i += globalStride())
-        propagateOne(static_cast<uint32_t>(i % per), ctx[i / per].count, offset, grid, childOffset, childGrid);
+    LevelOffsets lo;
+    for (uint32_t l = 0; l < MAX_LEVELS; ++l)
+        lo.offset[l] = L.offset[l];
+    lo.levels = L.depth + 1;
+    return lo;
 }
 
+// the levels above the bucket level, a workgroup per cloud
 template <typename T>
-static __global__ void kLevelStartsB(const BatchCloud<T>* __restrict__ ctx, LevelOffsets lo)
+static __global__ __launch_bounds__(TOP_THREADS) void kPropagateTopB(const BatchCloud<T>* __restrict__ ctx, BatchLevels L)
 {
-    const BatchCloud<T>& cc = ctx[blockIdx.x];
-    const uint32_t* m       = reinterpret_cast<const uint32_t*>(cc.sc + BS_M);
-    kLevelStartsBody(cc.nodeKey, m, lo, cc.levelStart());
-    if (threadIdx.x == 0)
-        cc.levelStart()[lo.levels] = *m;  // the end of the top level
+    propagateTop(ctx[blockIdx.x].count, levelOffsets(L), L.lc, L.grid[0]);
+}
+
+// canonical sparse ids over the occupancy bitmap (A2), second pass: grid (scanWidth, B)
+template <typename T>
+static __global__ __launch_bounds__(SCAN_THREADS) void kOccupiedIdsB(const BatchCloud<T>* __restrict__ ctx, BatchLevels L)
+{
+    __shared__ IdLds lds;
+    const BatchCloud<T>& cc = ctx[blockIdx.y];
+    const IdTables t{cc.occ, cc.count, cc.denseToSparse, cc.nodeKey, cc.nodeCount, cc.levelStart(), levelOffsets(L)};
+    const uint64_t words = (static_cast<uint64_t>(L.dense) + 31) / 32;
+    uint64_t first, last;
+    tileRange(scanTiles(words), first, last);
+    const uint32_t before = sumBefore(reinterpret_cast<const uint32_t*>(cc.scanSums), lds.scan);
+    const uint32_t next   = occupiedIds(t, words, first, last, before, lds);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+    {
+        cc.sc[BS_M]                     = next;
+        cc.levelStart()[L.depth + 1] = next;  // the end of the top level
+    }
 }
 
 __device__ __forceinline__ LevelParams levelParams(const BatchLevels& L, uint32_t threshold)
@@ -703,61 +699,17 @@ static __global__ __launch_bounds__(BLOCK) void kNodeLinksB(const BatchCloud<T>*
         const uint32_t c        = findCloud(wp, B, static_cast<uint32_t>(i));
         const BatchCloud<T>& cc = ctx[c];
         const uint32_t id       = static_cast<uint32_t>(i) - wp[c];
-        nodeLinksOf(id, levelParams(L, cc.threshold), cc.nodeKey, cc.nodeCount, cc.denseToSparse, cc.nodePoints,
-                    cc.nodeData, cc.nodeParent, cc.nodeChild, cc.nodeFlags, cc.nodeAux, cc.nodeSub, cc.occ);
+        nodeLinksOf(id, levelParams(L, cc.threshold), cc.nodeKey, cc.nodeCount, cc.denseToSparse, cc.occ, cc.nodePoints,
+                    cc.nodeData, cc.nodeParent, cc.nodeChild, cc.nodeFlags, cc.nodeSub, L.lc, cc.bucketStart, cc.nodeSorted,
+                    cc.count);
         cc.keyOut[id]   = cc.nodeKey[id];
         cc.countOut[id] = cc.nodeCount[id];
-    }
-}
-
-template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kLeafDataIdxB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                        const uint32_t* __restrict__ prefix)
-{
-    __shared__ uint32_t wp[MAX_BATCH + 1];
-    loadPrefix(prefix, B, wp);
-    for (uint64_t i = globalThread(); i < wp[B]; i += globalStride())
-    {
-        const uint32_t c        = findCloud(wp, B, static_cast<uint32_t>(i));
-        const BatchCloud<T>& cc = ctx[c];
-        leafDataIdxOf(static_cast<uint32_t>(i) - wp[c], cc.m, cc.nodeAux, cc.nodeFlags, cc.nodeChild, cc.nodePoints,
-                      cc.nodeData);
-    }
-}
-
-// items: level-0 nodes of all clouds
-template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kCellLeafB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                     const uint32_t* __restrict__ prefix)
-{
-    __shared__ uint32_t wp[MAX_BATCH + 1];
-    loadPrefix(prefix, B, wp);
-    for (uint64_t i = globalThread(); i < wp[B]; i += globalStride())
-    {
-        const uint32_t c        = findCloud(wp, B, static_cast<uint32_t>(i));
-        const BatchCloud<T>& cc = ctx[c];
-        cellLeafOf(static_cast<uint32_t>(i) - wp[c], cc.nodeKey, cc.nodeFlags, cc.nodeParent, cc.count);
     }
 }
 
 // ------------------------------------------------------------------------------------------------
 // Distribution
 // ------------------------------------------------------------------------------------------------
-
-template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kSortedStartB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                        const uint32_t* __restrict__ prefix, BatchLevels L)
-{
-    __shared__ uint32_t wp[MAX_BATCH + 1];
-    loadPrefix(prefix, B, wp);
-    for (uint64_t i = globalThread(); i < wp[B]; i += globalStride())
-    {
-        const uint32_t c        = findCloud(wp, B, static_cast<uint32_t>(i));
-        const BatchCloud<T>& cc = ctx[c];
-        sortedStartOf(static_cast<uint32_t>(i) - wp[c], levelParams(L, cc.threshold), cc.nodeKey, cc.nodeCount,
-                      cc.nodeFlags, cc.nodeParent, cc.nodeChild, cc.nodeSorted);
-    }
-}
 
 // items: leaf chunks of all clouds (prefix over the clouds' chunk counts)
 template <typename T>
@@ -948,7 +900,7 @@ static __global__ void kLevelCellsB(const BatchCloud<T>* __restrict__ ctx, uint3
     }
 }
 
-// items: internal nodes + 1 per cloud
+// items: internal nodes
 template <typename T>
 static __global__ __launch_bounds__(BLOCK) void kBatchNodesB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
                                                        const uint32_t* __restrict__ prefix)
@@ -959,9 +911,8 @@ static __global__ __launch_bounds__(BLOCK) void kBatchNodesB(const BatchCloud<T>
     {
         const uint32_t c        = findCloud(wp, B, static_cast<uint32_t>(i));
         const BatchCloud<T>& cc = ctx[c];
-        const uint32_t K        = static_cast<uint32_t>(cc.sc[BS_TABLE_TOTAL]);
-        batchNodeOf(static_cast<uint32_t>(i) - wp[c], 0, K, cc.wordsPerNode, cc.nodeGrid, cc.prefix,
-                    static_cast<uint32_t>(cc.sc[BS_CURSOR]), cc.nodePoints, cc.nodeStage, cc.nodeFirst);
+        batchNodeOf(static_cast<uint32_t>(i) - wp[c], 0, cc.wordsPerNode, cc.nodeGrid, cc.prefix,
+                    static_cast<uint32_t>(cc.sc[BS_CURSOR]), cc.nodePoints, cc.nodeStage);
     }
 }
 

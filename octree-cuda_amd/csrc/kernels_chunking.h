@@ -7,6 +7,7 @@
 #include <cstdint>
 
 #include "device_common.h"
+#include "scan.h"
 #include "types.h"
 
 namespace oc {
@@ -18,17 +19,19 @@ enum ScalarSlot : int
 {
     SC_ERROR       = 0,
     SC_M           = 1,
-    SC_LEAF_TOTAL  = 2,
+    SC_LEAF_TOTAL  = 2,  // packed (leaf chunks << 32 | leaf points)
     SC_SEG_TOTAL   = 3,  // packed (tiles << 32 | inputs)
     SC_TABLE_TOTAL = 4,
     SC_BUCKETS     = 5,  // totals of the bucket tables (BucketIn)
     SC_NEXT_BUCKET = 6,  // the fine sort's next occupied bucket
+    SC_INTERNAL    = 7,  // internal nodes
     SC_LEVEL_START = 8,  // u32[MAX_LEVELS + 1] packed into the following slots
     SC_COUNT       = 16
 };
 
 constexpr uint32_t ERR_OUTSIDE  = 1u;
 constexpr uint32_t ERR_CAPACITY = 2u;
+constexpr uint32_t ERR_OVERFLOW = 4u;  // N + I > E (A14)
 
 inline unsigned gridFor(uint64_t n, uint64_t cap = 65536)
 {
@@ -38,17 +41,6 @@ inline unsigned gridFor(uint64_t n, uint64_t cap = 65536)
     return static_cast<unsigned>(b < cap ? b : cap);
 }
 
-static __global__ __launch_bounds__(BLOCK) void kFill32(uint32_t* p, uint64_t n, uint32_t v)
-{
-    for (uint64_t i = globalThread(); i < n; i += globalStride())
-        p[i] = v;
-}
-
-static __global__ __launch_bounds__(BLOCK) void kFill64(uint64_t* p, uint64_t n, uint64_t v)
-{
-    for (uint64_t i = globalThread(); i < n; i += globalStride())
-        p[i] = v;
-}
 
 // What a build starts from, cleared in one launch: the scalars, the bucket counts, the bitmap words
 // [0, words) of the levels whose occupancy bits the fine sort writes (none for small grids) and the
@@ -82,90 +74,156 @@ __device__ __forceinline__ void propagateOne(uint32_t idx, uint32_t* __restrict_
     count[offset + idx] = sum;
 }
 
-static __global__ __launch_bounds__(BLOCK) void kPropagate(uint32_t* __restrict__ count, uint32_t offset, uint32_t grid,
-                                                     uint32_t childOffset, uint32_t childGrid)
-{
-    const uint64_t n = static_cast<uint64_t>(grid) * grid * grid;
-    for (uint64_t i = globalThread(); i < n; i += globalStride())
-        propagateOne(static_cast<uint32_t>(i), count, offset, grid, childOffset, childGrid);
-}
-
-// Occupancy bitmap of the dense cells [from, dense) from their counts (bit d: cell d holds
-// points). `from` is a multiple of 64 and every wave covers 64 consecutive cells, two whole words.
-static __global__ __launch_bounds__(BLOCK) void kOccupancyBits(const uint32_t* __restrict__ count, uint64_t from,
-                                                         uint64_t dense, uint32_t* __restrict__ occ)
-{
-    const uint64_t n = (dense - from + 63) / 64 * 64;  // whole waves: the loop is uniform per wave
-    for (uint64_t i = globalThread(); i < n; i += globalStride())
-    {
-        const uint64_t d    = from + i;
-        const uint64_t bits = __ballot(d < dense && count[d] != 0);
-        if ((threadIdx.x & 31) == 0 && d < dense)
-            occ[d >> 5] = static_cast<uint32_t>(bits >> (threadIdx.x & 32));
-    }
-}
-
-// Sparse ids (A2) from the occupancy bitmap, one scan item per word: the exclusive rank of an
-// occupied dense cell; its node key and dense count are written in the same pass. denseToSparse is
-// written for occupied cells only: an array of D entries is never filled with -1.
-struct OccupiedWordIn
-{
-    const uint32_t* occ;
-    __device__ uint32_t operator()(uint64_t w) const { return __popc(occ[w]); }
-};
-
-struct OccupiedWordOut
-{
-    const uint32_t* occ;
-    int32_t* denseToSparse;
-    uint32_t* nodeKey;
-    uint32_t* nodeCount;
-    const uint32_t* count;
-    __device__ void operator()(uint64_t w, uint32_t prefix, uint32_t v) const
-    {
-        uint32_t bits = v ? occ[w] : 0u;
-        while (bits)
-        {
-            const uint64_t d  = 32 * w + static_cast<uint32_t>(__builtin_ctz(bits));
-            bits &= bits - 1u;
-            denseToSparse[d]  = static_cast<int32_t>(prefix);
-            nodeKey[prefix]   = static_cast<uint32_t>(d);
-            nodeCount[prefix] = count[d];
-            ++prefix;
-        }
-    }
-};
-
 struct LevelOffsets
 {
     uint32_t offset[MAX_LEVELS];
     uint32_t levels;
 };
 
-// First sparse id of every level: ids ascend with the dense index and a level is one dense range,
-// so it is the number of node keys below the level's dense offset (a lower bound over the m keys).
-__device__ __forceinline__ void kLevelStartsBody(const uint32_t* __restrict__ nodeKey, const uint32_t* __restrict__ m,
-                                                 const LevelOffsets& lo, uint32_t* __restrict__ levelStart)
+// The levels above the bucket level, at most 8^3 + 4^3 + 2^3 + 1 cells: one workgroup, one launch.
+constexpr int TOP_THREADS = 512;
+
+__device__ __forceinline__ void propagateTop(uint32_t* count, const LevelOffsets& lo, uint32_t lc,
+                                             uint32_t chunkingGrid)
 {
-    const uint32_t l = threadIdx.x;
-    if (l >= lo.levels)
-        return;
-    uint32_t a = 0, b = *m;
-    while (a < b)
+    for (uint32_t l = lc + 1; l < lo.levels; ++l)
     {
-        const uint32_t mid = a + (b - a) / 2;
-        if (nodeKey[mid] < lo.offset[l])
-            a = mid + 1;
-        else
-            b = mid;
+        const uint32_t grid = chunkingGrid >> l;
+        for (uint32_t i = threadIdx.x; i < grid * grid * grid; i += TOP_THREADS)
+            propagateOne(i, count, lo.offset[l], grid, lo.offset[l - 1], 2 * grid);
+        __syncthreads();
     }
-    levelStart[l] = a;
 }
 
-static __global__ void kLevelStarts(const uint32_t* __restrict__ nodeKey, const uint32_t* __restrict__ m,
-                             LevelOffsets lo, uint32_t* __restrict__ levelStart)
+static __global__ __launch_bounds__(TOP_THREADS) void kPropagateTop(uint32_t* count, LevelOffsets lo, uint32_t lc,
+                                                             uint32_t chunkingGrid)
 {
-    kLevelStartsBody(nodeKey, m, lo, levelStart);
+    propagateTop(count, lo, lc, chunkingGrid);
+}
+
+// Occupancy bitmap (bit d: dense cell d holds points), one scan item per word: the words of the
+// levels that the fine sort has marked as they are, the others made from their counts and stored.
+struct OccupancyIn
+{
+    uint32_t* occ;
+    const uint32_t* count;
+    uint64_t marked;  // words
+    uint64_t dense;   // cells
+    __device__ uint32_t operator()(uint64_t w) const
+    {
+        if (w < marked)
+            return __popc(occ[w]);
+        uint32_t bits    = 0;
+        const uint64_t d = 32 * w;
+        if (d + 32 <= dense)
+        {
+            const uint4* c = reinterpret_cast<const uint4*>(count + d);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+            {
+                const uint4 v = c[k];
+                bits |= ((v.x ? 1u : 0u) | (v.y ? 2u : 0u) | (v.z ? 4u : 0u) | (v.w ? 8u : 0u)) << (4 * k);
+            }
+        }
+        else
+            for (uint32_t k = 0; k < dense - d; ++k)
+                bits |= (count[d + k] ? 1u : 0u) << k;
+        occ[w] = bits;
+        return __popc(bits);
+    }
+};
+
+// Sparse ids (A2): the exclusive rank of an occupied dense cell; its node key and dense count are
+// written in the same pass, and the first id of every level (ids ascend with the dense index and a
+// level is one dense range). denseToSparse is written for occupied cells only: an array of D
+// entries is never filled with -1.
+struct IdTables
+{
+    const uint32_t* occ;
+    const uint32_t* count;
+    int32_t* denseToSparse;
+    uint32_t* nodeKey;
+    uint32_t* nodeCount;
+    uint32_t* levelStart;
+    LevelOffsets levels;
+};
+
+// Set bits of a tile that are listed in LDS at a time.
+constexpr uint32_t ID_LIST = 8192;
+
+struct IdLds
+{
+    uint32_t scan[SCAN_ITEMS * SCAN_WAVES];
+    uint16_t list[ID_LIST];
+};
+
+// The tiles [first, last) of the bitmap's words from id `carry` on (all threads); returns the next
+// id. A tile's set bits are listed in LDS in order and then written one per thread, coalesced: a
+// thread walking the bits of its own words wrote every node from one lane, 40 us of a 200K-point
+// build and 284 us of a 7.3M-node one, now 15 and 166.
+__device__ __forceinline__ uint32_t occupiedIds(const IdTables& t, uint64_t words, uint64_t first, uint64_t last,
+                                                uint32_t carry, IdLds& lds)
+{
+    for (uint64_t tile = first; tile < last; ++tile)
+    {
+        uint32_t w[SCAN_ITEMS], v[SCAN_ITEMS], pre[SCAN_ITEMS];
+        loadTile<uint32_t>([&t](uint64_t i) { return t.occ[i]; }, tile * SCAN_TILE, words, w);
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; ++k)
+            v[k] = __popc(w[k]);
+        const uint32_t ids  = sparseTileScan(v, pre, lds.scan);
+        const uint64_t cell = 32 * tile * SCAN_TILE;  // of the tile's first bit
+        for (uint32_t l = 0; l < t.levels.levels; ++l)
+        {
+            const uint32_t d = t.levels.offset[l];
+            if (d < cell || d - cell >= 32 * SCAN_TILE)
+                continue;
+            const uint32_t item = static_cast<uint32_t>(d - cell) >> 5;
+#pragma unroll
+            for (int k = 0; k < SCAN_ITEMS; ++k)
+                if (item == k * SCAN_THREADS + threadIdx.x)
+                    t.levelStart[l] = carry + pre[k] + __popc(w[k] & ((1u << (d & 31)) - 1u));
+        }
+        for (uint32_t base = 0; base < ids; base += ID_LIST)
+        {
+#pragma unroll
+            for (int k = 0; k < SCAN_ITEMS; ++k)
+            {
+                uint32_t at = pre[k] - base;  // wraps below the listed range
+                if (v[k] == 0 || pre[k] >= base + ID_LIST || pre[k] + v[k] <= base)
+                    continue;
+                for (uint32_t bits = w[k]; bits; bits &= bits - 1u, ++at)
+                    if (at < ID_LIST)
+                        lds.list[at] = static_cast<uint16_t>(32 * (k * SCAN_THREADS + threadIdx.x) +
+                                                             static_cast<uint32_t>(__builtin_ctz(bits)));
+            }
+            __syncthreads();
+            const uint32_t n = ids - base < ID_LIST ? ids - base : ID_LIST;
+            for (uint32_t j = threadIdx.x; j < n; j += SCAN_THREADS)
+            {
+                const uint64_t d      = cell + lds.list[j];
+                const uint32_t id     = carry + base + j;
+                t.nodeKey[id]         = static_cast<uint32_t>(d);
+                t.nodeCount[id]       = t.count[d];
+                t.denseToSparse[d]    = static_cast<int32_t>(id);
+            }
+            __syncthreads();
+        }
+        carry += ids;
+    }
+    return carry;
+}
+
+// second pass of the id scan; *m: the number of nodes
+static __global__ __launch_bounds__(SCAN_THREADS) void kOccupiedIds(IdTables t, uint64_t words, const uint32_t* sums,
+                                                             uint32_t* __restrict__ m)
+{
+    __shared__ IdLds lds;
+    uint64_t first, last;
+    tileRange(scanTiles(words), first, last);
+    const uint32_t next = occupiedIds(t, words, first, last, sumBefore(sums, lds.scan), lds);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+        *m = next;
 }
 
 struct LevelParams
@@ -185,86 +243,147 @@ __device__ __forceinline__ uint32_t levelOfKey(uint32_t key, const LevelParams& 
     return l;
 }
 
+// The leaf of a level-0 cell (the first finished ancestor-or-self, point_distributing.cuh:56-60): the
+// first node on the way up whose parent is internal, or the root.
+__device__ __forceinline__ uint32_t leafOfCell(uint32_t id, uint32_t x, uint32_t y, uint32_t z, const LevelParams& lp,
+                                               const uint32_t* __restrict__ nodeCount,
+                                               const int32_t* __restrict__ denseToSparse)
+{
+    for (uint32_t l = 1; l <= lp.depth; ++l)
+    {
+        const uint32_t g = lp.grid[l];
+        const uint32_t p = static_cast<uint32_t>(denseToSparse[lp.offset[l] + (x >> l) + (y >> l) * g + (z >> l) * g * g]);
+        if (nodeCount[p] >= lp.threshold)
+            return id;
+        id = p;
+    }
+    return id;
+}
+
+// Start of a node's range in the sorted cloud (full Morton order of the level-0 cells): the points of
+// all buckets before its own, which are numbered in Morton order, and below the bucket level lc those
+// of the lower-slot siblings of the node and of its ancestors inside the bucket.
+__device__ __forceinline__ uint32_t sortedStartOf(uint32_t l, uint32_t x, uint32_t y, uint32_t z, uint32_t lc,
+                                                  const LevelParams& lp, const uint32_t* __restrict__ bucketStart,
+                                                  const uint32_t* __restrict__ occ,
+                                                  const int32_t* __restrict__ denseToSparse,
+                                                  const uint32_t* __restrict__ nodeCount)
+{
+    uint32_t start = 0;
+    for (; l < lc; ++l)
+    {
+        const uint32_t g    = lp.grid[l];
+        const uint32_t slot = ((x & 1) << 2) | ((y & 1) << 1) | (z & 1);
+        for (uint32_t k = 0; k < slot; ++k)
+        {
+            const uint32_t sx = (x & ~1u) + (k >> 2), sy = (y & ~1u) + ((k >> 1) & 1), sz = (z & ~1u) + (k & 1);
+            const uint32_t d = lp.offset[l] + sx + sy * g + sz * g * g;
+            if ((occ[d >> 5] >> (d & 31)) & 1u)
+                start += nodeCount[denseToSparse[d]];
+        }
+        x >>= 1;
+        y >>= 1;
+        z >>= 1;
+    }
+    return start + bucketStart[morton3(x, y, z) << (3 * (l - lc))];
+}
+
 // Node links and flags: kernelInitLeafNodes (octree_initialization.cuh:24-52) and the structural
 // part of kernelMergeHierarchical (hierarchical_merging.cuh:35-122):
 //   internal  = level >= 1 && count >= threshold
 //   finished  = parent is internal (the root is always finished, A13)
 //   pointCount = internal ? 0 : count
-// and the size of the leaf data block an internal node hands out to its leaf children.
+// For a leaf also its range of the sorted cloud, and for a level-0 node its leaf, over its cell's
+// count (nothing reads that again), so the distribution needs one lookup per point.
 __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, const uint32_t* __restrict__ nodeKey,
                                             const uint32_t* __restrict__ nodeCount,
                                             const int32_t* __restrict__ denseToSparse,
-                                            uint32_t* __restrict__ pointCount, uint64_t* __restrict__ dataIdx,
-                                            int32_t* __restrict__ parent, int32_t* __restrict__ children,
-                                            uint8_t* __restrict__ flags, uint32_t* __restrict__ blockSize,
-                                            uint32_t* __restrict__ subtree, const uint32_t* __restrict__ occ)
+                                            const uint32_t* __restrict__ occ, uint32_t* __restrict__ pointCount,
+                                            uint64_t* __restrict__ dataIdx, int32_t* __restrict__ parent,
+                                            int32_t* __restrict__ children, uint8_t* __restrict__ flags,
+                                            uint32_t* __restrict__ subtree, uint32_t lc,
+                                            const uint32_t* __restrict__ bucketStart,
+                                            uint32_t* __restrict__ sortedStart, uint32_t* __restrict__ cellLeaf)
 {
+    const uint32_t key = nodeKey[id];
+    const uint32_t l   = levelOfKey(key, lp);
+    const uint32_t g   = lp.grid[l];
+    const uint32_t lin = key - lp.offset[l];
+    const uint32_t x = lin % g, y = (lin / g) % g, z = lin / (g * g);
+    const uint32_t cnt  = nodeCount[id];
+    const bool internal = l >= 1 && cnt >= lp.threshold;
+
+    int32_t p = -1;
+    if (l < lp.depth)
     {
-        uint32_t key = nodeKey[id];
-        uint32_t l   = levelOfKey(key, lp);
-        uint32_t g   = lp.grid[l];
-        uint32_t lin = key - lp.offset[l];
-        uint32_t x = lin % g, y = (lin / g) % g, z = lin / (g * g);
-        uint32_t cnt  = nodeCount[id];
-        bool internal = l >= 1 && cnt >= lp.threshold;
+        const uint32_t pg = lp.grid[l + 1];  // the parent of an occupied cell is occupied
+        p                 = denseToSparse[lp.offset[l + 1] + (x >> 1) + (y >> 1) * pg + (z >> 1) * pg * pg];
+    }
+    const bool finished = (p < 0) ? true : (nodeCount[p] >= lp.threshold);
 
-        int32_t p = -1;
-        if (l < lp.depth)
-        {
-            uint32_t pg = lp.grid[l + 1];  // the parent of an occupied cell is occupied
-            p           = denseToSparse[lp.offset[l + 1] + (x >> 1) + (y >> 1) * pg + (z >> 1) * pg * pg];
-        }
-        bool finished = (p < 0) ? true : (nodeCount[p] >= lp.threshold);
-
-        uint32_t blk = 0;
+    for (int k = 0; k < 8; ++k)
+    {
+        int32_t c = -1;
         if (l >= 1)
         {
-            uint32_t cg = lp.grid[l - 1];
-            for (int k = 0; k < 8; ++k)
-            {
-                uint32_t cx = 2 * x + ((k >> 2) & 1), cy = 2 * y + ((k >> 1) & 1), cz = 2 * z + (k & 1);
-                const uint32_t cd = lp.offset[l - 1] + cx + cy * cg + cz * cg * cg;
-                // occupancy from the bitmap (the counts of empty cells of the lowest levels are not
-                // written); denseToSparse is set for occupied cells only
-                const bool occupied = ((occ[cd >> 5] >> (cd & 31)) & 1u) != 0;
-                int32_t c           = occupied ? denseToSparse[cd] : -1;
-                children[8 * static_cast<uint64_t>(id) + k] = c;
-                if (internal && c >= 0)
-                {
-                    uint32_t cc        = nodeCount[c];
-                    bool childInternal = (l - 1) >= 1 && cc >= lp.threshold;
-                    if (!childInternal)
-                        blk += cc;
-                }
-            }
+            const uint32_t cg = lp.grid[l - 1];
+            const uint32_t cx = 2 * x + ((k >> 2) & 1), cy = 2 * y + ((k >> 1) & 1), cz = 2 * z + (k & 1);
+            const uint32_t cd = lp.offset[l - 1] + cx + cy * cg + cz * cg * cg;
+            // occupancy from the bitmap (the counts of empty cells of the lowest levels are not
+            // written); denseToSparse is set for occupied cells only
+            if ((occ[cd >> 5] >> (cd & 31)) & 1u)
+                c = denseToSparse[cd];
         }
-        else
-        {
-            for (int k = 0; k < 8; ++k)
-                children[8 * static_cast<uint64_t>(id) + k] = -1;
-        }
-        pointCount[id] = internal ? 0u : cnt;
-        dataIdx[id]    = 0;
-        parent[id]     = p;
-        flags[id]      = static_cast<uint8_t>((finished ? NODE_FINISHED : 0) | (internal ? NODE_INTERNAL : 0));
-        blockSize[id]  = blk;
-        subtree[id]    = 0;
+        children[8 * static_cast<uint64_t>(id) + k] = c;
     }
+    pointCount[id] = internal ? 0u : cnt;
+    dataIdx[id]    = 0;
+    parent[id]     = p;
+    flags[id]      = static_cast<uint8_t>((finished ? NODE_FINISHED : 0) | (internal ? NODE_INTERNAL : 0));
+    subtree[id]    = 0;
+    if (finished && !internal)
+        sortedStart[id] = sortedStartOf(l, x, y, z, lc, lp, bucketStart, occ, denseToSparse, nodeCount);
+    if (l == 0)
+        cellLeaf[key] = leafOfCell(id, x, y, z, lp, nodeCount, denseToSparse);
 }
 
 static __global__ __launch_bounds__(BLOCK) void kNodeLinks(uint32_t m, LevelParams lp, const uint32_t* __restrict__ nodeKey,
                                                      const uint32_t* __restrict__ nodeCount,
                                                      const int32_t* __restrict__ denseToSparse,
+                                                     const uint32_t* __restrict__ occ,
                                                      uint32_t* __restrict__ pointCount, uint64_t* __restrict__ dataIdx,
-                                                     int32_t* __restrict__ parent,
-                                                     int32_t* __restrict__ children, uint8_t* __restrict__ flags,
-                                                     uint32_t* __restrict__ blockSize,
-                                                     uint32_t* __restrict__ subtree, const uint32_t* __restrict__ occ)
+                                                     int32_t* __restrict__ parent, int32_t* __restrict__ children,
+                                                     uint8_t* __restrict__ flags, uint32_t* __restrict__ subtree,
+                                                     uint32_t lc, const uint32_t* __restrict__ bucketStart,
+                                                     uint32_t* __restrict__ sortedStart, uint32_t* __restrict__ cellLeaf,
+                                                     uint64_t* __restrict__ cursor, uint32_t points)
 {
     for (uint64_t i = globalThread(); i < m; i += globalStride())
-        nodeLinksOf(static_cast<uint32_t>(i), lp, nodeKey, nodeCount, denseToSparse, pointCount, dataIdx,
-                    parent, children, flags, blockSize, subtree, occ);
+        nodeLinksOf(static_cast<uint32_t>(i), lp, nodeKey, nodeCount, denseToSparse, occ, pointCount, dataIdx, parent,
+                    children, flags, subtree, lc, bucketStart, sortedStart, cellLeaf);
+    if (globalThread() == 0)
+        *cursor = points;  // the output cursor before the first subsampling step
 }
+
+// Internal nodes (level >= 1 and at least `threshold` points), in id order.
+struct InternalNodeIn
+{
+    const uint32_t* nodeCount;
+    const uint32_t* levelStart;
+    uint32_t threshold;
+    __device__ uint32_t operator()(uint64_t i) const { return nodeCount[levelStart[1] + i] >= threshold ? 1u : 0u; }
+};
+
+struct InternalNodeOut
+{
+    uint32_t* list;
+    const uint32_t* levelStart;
+    __device__ void operator()(uint64_t i, uint32_t prefix, uint32_t v) const
+    {
+        if (v)
+            list[prefix] = levelStart[1] + static_cast<uint32_t>(i);
+    }
+};
 
 struct ArrayIn
 {
@@ -278,63 +397,47 @@ struct ExclusiveToArray
     __device__ void operator()(uint64_t i, uint32_t prefix, uint32_t) const { dst[i] = prefix; }
 };
 
-// Leaf data offsets (A4): an internal node's block starts at the exclusive scan of block sizes in
-// sparse-id order (= parent level, parent linear index); children follow in slot order.
-__device__ __forceinline__ void leafDataIdxOf(uint32_t id, uint32_t m, const uint32_t* __restrict__ blockStart,
-                                              const uint8_t* __restrict__ flags,
-                                              const int32_t* __restrict__ children,
-                                              const uint32_t* __restrict__ pointCount,
-                                              uint64_t* __restrict__ dataIdx)
+// Leaf data offsets (A4): an internal node's block of leaf children starts at the exclusive scan of
+// the block sizes in sparse-id order (= parent level, parent linear index), one item per node;
+// children follow in slot order.
+struct LeafBlockIn
 {
+    const uint8_t* flags;
+    const int32_t* children;
+    const uint32_t* pointCount;
+    __device__ uint32_t operator()(uint64_t id) const
     {
-        if (!(flags[id] & NODE_INTERNAL))
-        {
-            if (id == m - 1)
-                dataIdx[id] = 0;  // root as the only leaf (A13)
+        uint32_t block = 0;
+        if (flags[id] & NODE_INTERNAL)
+            for (int k = 0; k < 8; ++k)
+            {
+                const int32_t c = children[8 * id + k];
+                if (c >= 0 && !(flags[c] & NODE_INTERNAL))
+                    block += pointCount[c];
+            }
+        return block;
+    }
+};
+
+struct LeafBlockOut
+{
+    LeafBlockIn in;
+    uint64_t* dataIdx;
+    __device__ void operator()(uint64_t id, uint32_t prefix, uint32_t v) const
+    {
+        if (v == 0)
             return;
-        }
-        uint64_t r = blockStart[id];
+        uint64_t r = prefix;
         for (int k = 0; k < 8; ++k)
         {
-            int32_t c = children[8 * static_cast<uint64_t>(id) + k];
-            if (c >= 0 && !(flags[c] & NODE_INTERNAL))
+            const int32_t c = in.children[8 * id + k];
+            if (c >= 0 && !(in.flags[c] & NODE_INTERNAL))
             {
                 dataIdx[c] = r;
-                r += pointCount[c];
+                r += in.pointCount[c];
             }
         }
     }
-}
-
-static __global__ __launch_bounds__(BLOCK) void kLeafDataIdx(uint32_t m, uint32_t threshold,
-                                                       const uint32_t* __restrict__ blockStart,
-                                                       const uint8_t* __restrict__ flags,
-                                                       const int32_t* __restrict__ children,
-                                                       const uint32_t* __restrict__ pointCount,
-                                                       uint64_t* __restrict__ dataIdx)
-{
-    for (uint64_t i = globalThread(); i < m; i += globalStride())
-        leafDataIdxOf(static_cast<uint32_t>(i), m, blockStart, flags, children, pointCount, dataIdx);
-}
-
-// Level-0 cell -> its leaf (the first finished ancestor-or-self, point_distributing.cuh:56-60),
-// written over the level-0 counts so the distribution needs one lookup per point.
-__device__ __forceinline__ void cellLeafOf(uint32_t i, const uint32_t* __restrict__ nodeKey,
-                                           const uint8_t* __restrict__ flags, const int32_t* __restrict__ parent,
-                                           uint32_t* __restrict__ count)
-{
-    int32_t s = static_cast<int32_t>(i);
-    while (!(flags[s] & NODE_FINISHED))
-        s = parent[s];
-    count[nodeKey[i]] = static_cast<uint32_t>(s);
-}
-
-static __global__ __launch_bounds__(BLOCK) void kCellLeaf(uint32_t level0Nodes, const uint32_t* __restrict__ nodeKey,
-                                                    const uint8_t* __restrict__ flags,
-                                                    const int32_t* __restrict__ parent, uint32_t* __restrict__ count)
-{
-    for (uint64_t i = globalThread(); i < level0Nodes; i += globalStride())
-        cellLeafOf(static_cast<uint32_t>(i), nodeKey, flags, parent, count);
-}
+};
 
 }  // namespace oc

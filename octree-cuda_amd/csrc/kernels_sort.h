@@ -70,33 +70,6 @@ static_assert(sizeof(SortedPoint<double>) == 32, "double sorted point is 32 byte
 static_assert(sizeof(SortedPoint<float>) == 20, "float sorted point is 20 bytes");
 static_assert(STAGE_CHUNK <= 65535, "staged slots are 16-bit");
 
-// Bit interleaving for coordinates below 2^10 (part1by2 / compact1by2).
-__host__ __device__ __forceinline__ uint32_t spread3(uint32_t v)
-{
-    v &= 0x000003FFu;
-    v = (v ^ (v << 16)) & 0xFF0000FFu;
-    v = (v ^ (v << 8)) & 0x0300F00Fu;
-    v = (v ^ (v << 4)) & 0x030C30C3u;
-    v = (v ^ (v << 2)) & 0x09249249u;
-    return v;
-}
-
-__host__ __device__ __forceinline__ uint32_t compact3(uint32_t v)
-{
-    v &= 0x09249249u;
-    v = (v ^ (v >> 2)) & 0x030C30C3u;
-    v = (v ^ (v >> 4)) & 0x0300F00Fu;
-    v = (v ^ (v >> 8)) & 0xFF0000FFu;
-    v = (v ^ (v >> 16)) & 0x000003FFu;
-    return v;
-}
-
-// Morton code whose 3-bit groups are child slots (x -> 4, y -> 2, z -> 1).
-__host__ __device__ __forceinline__ uint32_t morton3(uint32_t x, uint32_t y, uint32_t z)
-{
-    return (spread3(x) << 2) | (spread3(y) << 1) | spread3(z);
-}
-
 // Exclusive scan over a 1024-thread workgroup; `total` receives the sum. Contains barriers.
 __device__ __forceinline__ uint32_t sortBlockExclusiveScan(uint32_t v, uint32_t& total, uint32_t* lds)
 {
@@ -768,50 +741,6 @@ static __global__ __launch_bounds__(BLOCK) void kGatherSorted(const SortedPoint<
         if (j < n)
             sorted[j] = bucketed[perm[j]];
     }
-}
-
-// Start of every leaf's range in the sorted cloud: the points of all nodes that precede it in
-// Morton order, i.e. of the lower-slot siblings of the leaf and of each of its ancestors.
-__device__ __forceinline__ void sortedStartOf(uint32_t id, const LevelParams& lp, const uint32_t* __restrict__ nodeKey,
-                                              const uint32_t* __restrict__ nodeCount,
-                                              const uint8_t* __restrict__ flags, const int32_t* __restrict__ parent,
-                                              const int32_t* __restrict__ children,
-                                              uint32_t* __restrict__ sortedStart)
-{
-    if ((flags[id] & (NODE_FINISHED | NODE_INTERNAL)) != NODE_FINISHED)
-        return;
-    uint32_t start = 0;
-    int32_t cur    = static_cast<int32_t>(id);
-    int32_t p      = parent[cur];
-    while (p >= 0)
-    {
-        const uint32_t key = nodeKey[cur];
-        const uint32_t l   = levelOfKey(key, lp);
-        const uint32_t g   = lp.grid[l];
-        const uint32_t lin = key - lp.offset[l];
-        const uint32_t x = lin % g, y = (lin / g) % g, z = lin / (g * g);
-        const int slot     = static_cast<int>(((x & 1) << 2) | ((y & 1) << 1) | (z & 1));
-        for (int k = 0; k < slot; ++k)
-        {
-            const int32_t c = children[8 * static_cast<uint64_t>(p) + k];
-            if (c >= 0)
-                start += nodeCount[c];
-        }
-        cur = p;
-        p   = parent[cur];
-    }
-    sortedStart[id] = start;
-}
-
-static __global__ __launch_bounds__(BLOCK) void kSortedStart(uint32_t m, LevelParams lp, const uint32_t* __restrict__ nodeKey,
-                                                       const uint32_t* __restrict__ nodeCount,
-                                                       const uint8_t* __restrict__ flags,
-                                                       const int32_t* __restrict__ parent,
-                                                       const int32_t* __restrict__ children,
-                                                       uint32_t* __restrict__ sortedStart)
-{
-    for (uint64_t i = globalThread(); i < m; i += globalStride())
-        sortedStartOf(static_cast<uint32_t>(i), lp, nodeKey, nodeCount, flags, parent, children, sortedStart);
 }
 
 // K5: kernelDistributePoints (point_distributing.cuh:31-76) over the sorted cloud. The leaf of a

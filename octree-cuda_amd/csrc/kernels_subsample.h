@@ -184,6 +184,20 @@ __device__ __forceinline__ Gridding nodeGridding(uint32_t lin, uint32_t gl, uint
     return Gridding{mx, my, mz, (mx + side) - mx, g};
 }
 
+// What one node's subsampling needs, from its key.
+__device__ __forceinline__ NodeGrid nodeGridOf(uint32_t id, uint32_t key, uint32_t levelOffset, uint32_t levelGrid,
+                                               uint32_t level, uint32_t depth, const double* cubicMin,
+                                               const double* sideHalf, double side, uint32_t g, uint64_t seed)
+{
+    NodeGrid ng;
+    ng.grid        = nodeGridding(key - levelOffset, levelGrid, level, depth, cubicMin, sideHalf, side, g);
+    const double t = ng.grid.bbSize / g;
+    ng.diag        = sqrt((t * 3) * (t * 3) * 3) / 2.0;
+    ng.salt        = nodeSalt(seed, key);
+    ng.id          = id;
+    return ng;
+}
+
 // Per internal node k of the level: its eight input segments (children in slot order, the leaf's
 // range of the sorted cloud or the child's staged subsample) and its gridding (nodeGridding).
 struct LevelTables
@@ -218,21 +232,8 @@ __device__ __forceinline__ void segmentsOf(uint64_t k, const SubsampleParams& sp
         lt.segCount[8 * k + s] = cnt;
         lt.segSrc[8 * k + s]   = src;
     }
-    const uint32_t key = lt.nodeKey[id];
-    NodeGrid ng;
-    ng.grid        = nodeGridding(key - sp.levelOffset, sp.levelGrid, sp.level, sp.depth, sp.cubicMin, sp.sideHalf,
-                                  sp.side, sp.g);
-    const double t = ng.grid.bbSize / sp.g;
-    ng.diag        = sqrt((t * 3) * (t * 3) * 3) / 2.0;
-    ng.salt        = nodeSalt(sp.seed, key);
-    ng.id          = id;
-    lt.nodeGrid[k] = ng;
-}
-
-static __global__ __launch_bounds__(BLOCK) void kSegments(uint32_t nodes, SubsampleParams sp, LevelTables lt)
-{
-    for (uint64_t k = globalThread(); k < nodes; k += globalStride())
-        segmentsOf(k, sp, lt);
+    lt.nodeGrid[k] = nodeGridOf(id, lt.nodeKey[id], sp.levelOffset, sp.levelGrid, sp.level, sp.depth, sp.cubicMin,
+                                sp.sideHalf, sp.side, sp.g, sp.seed);
 }
 
 // The sorted cloud in leaf and cell order. The fine sort's permutation puts the points in Morton
@@ -447,7 +448,8 @@ __device__ __forceinline__ void leafCellOrderChunk(uint64_t entry, const LeafOrd
 }
 
 template <typename T>
-static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrder(const uint64_t* __restrict__ chunkList, LeafOrderParams p,
+static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrder(const uint64_t* __restrict__ chunkList,
+                                                                const uint64_t* __restrict__ totals, LeafOrderParams p,
                                                                 const uint32_t* __restrict__ nodeKey,
                                                                 const int32_t* __restrict__ parent,
                                                                 const uint32_t* __restrict__ count,
@@ -457,6 +459,8 @@ static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrder(const uint
                                                                 SortedPoint<T>* __restrict__ out)
 {
     __shared__ LeafOrderLds lds;
+    if (blockIdx.x >= *totals >> 32)
+        return;  // the whole workgroup: the grid is an upper bound
     leafCellOrderChunk<T>(chunkList[blockIdx.x], leafOrderView(p), nodeKey, parent, count, sortedStart, bucketed, perm,
                           out, lds);
 }
@@ -492,45 +496,136 @@ __device__ __forceinline__ void tileListOf(uint64_t s, const uint32_t* __restric
         tileList[first + t] = static_cast<uint32_t>(s);
 }
 
-static __global__ __launch_bounds__(BLOCK) void kTileList(uint64_t segments, const uint32_t* __restrict__ segCount,
-                                                    const uint32_t* __restrict__ segTile, uint32_t* __restrict__ tileList)
+// Single cloud: the child slots of all internal nodes (8 k + slot, k in id order), one scan.
+// Item: chunks of a leaf child (high half; kLeafCellOrder) and its points (low half), so that the
+// prefix is its data offset (A4: blocks in parent-id order, children in slot order).
+struct ChildSlots
 {
-    for (uint64_t s = globalThread(); s < segments; s += globalStride())
-        tileListOf(s, segCount, segTile, tileList);
-}
-
-// A whole level's setup in one workgroup and one launch, for small levels (up to
-// SMALL_LEVEL_NODES nodes and SMALL_LEVEL_POINTS candidate inputs; a small build is bound by its
-// launch count): the internal nodes of the level, their segments and griddings, the segment scan
-// and the tile list. Writes K to *internalTotal and (tiles << 32 | inputs) to *segTotal.
-constexpr uint32_t SMALL_LEVEL_NODES  = 1u << 16;
-constexpr uint64_t SMALL_LEVEL_POINTS = 1u << 22;
-
-static __global__ __launch_bounds__(SCAN_THREADS) void kLevelSetup(uint32_t levelStart, uint32_t levelNodes,
-                                                            SubsampleParams sp, LevelTables lt,
-                                                            uint32_t* __restrict__ internalTotal,
-                                                            uint64_t* __restrict__ segTotal)
-{
-    __shared__ uint32_t lds32[SCAN_ITEMS * SCAN_WAVES];
-    __shared__ uint64_t lds64[SCAN_ITEMS * SCAN_WAVES];
-    blockScanAll<uint32_t>(InternalIn{lt.flags, levelStart}, InternalOut{lt.internalList, levelStart}, levelNodes,
-                           internalTotal, lds32);
-    __syncthreads();
-    const uint32_t K = *internalTotal;
-    for (uint32_t k = threadIdx.x; k < K; k += SCAN_THREADS)
-        segmentsOf(k, sp, lt);
-    __syncthreads();
-    const uint64_t segments = 8ull * K;
-    blockScanAll<uint64_t>(SegmentIn{lt.segCount}, SegmentOut{lt.segTile, lt.segInput}, segments, segTotal, lds64);
-    __syncthreads();
-    for (uint64_t s = threadIdx.x; s < segments; s += SCAN_THREADS)
+    const uint32_t* internal;  // ids of the internal nodes, ascending
+    const uint8_t* flags;
+    const int32_t* children;
+    const uint32_t* nodeCount;
+    __device__ __forceinline__ int32_t child(uint64_t s) const
     {
-        const uint32_t tiles = (lt.segCount[s] + TILE - 1) / TILE;
-        const uint32_t first = lt.segTile[s];
-        for (uint32_t t = 0; t < tiles; ++t)
-            lt.tileList[first + t] = static_cast<uint32_t>(s);
+        return children[8 * static_cast<uint64_t>(internal[s >> 3]) + (s & 7)];
     }
+};
+
+struct LeafSlotIn
+{
+    ChildSlots cs;
+    __device__ uint64_t operator()(uint64_t s) const
+    {
+        const int32_t c = cs.child(s);
+        if (c < 0 || (cs.flags[c] & NODE_INTERNAL))
+            return 0;
+        const uint32_t n = cs.nodeCount[c];
+        return (static_cast<uint64_t>((n + LEAF_CHUNK - 1) / LEAF_CHUNK) << 32) | n;
+    }
+};
+
+struct LeafSlotOut
+{
+    ChildSlots cs;
+    uint64_t* dataIdx;
+    uint64_t* chunkList;  // chunk number << 32 | leaf id
+    __device__ void operator()(uint64_t s, uint64_t prefix, uint64_t v) const
+    {
+        if (v == 0)
+            return;
+        const uint32_t c = static_cast<uint32_t>(cs.child(s));
+        dataIdx[c]       = static_cast<uint32_t>(prefix);
+        for (uint32_t k = 0; k < (v >> 32); ++k)
+            chunkList[(prefix >> 32) + k] = (static_cast<uint64_t>(k) << 32) | c;
+    }
+};
+
+// Input segments of one level: the child slots of its internal nodes (cs.internal is the level's part
+// of the list), scanned as (tiles << 32 | inputs).
+struct LevelSegmentIn
+{
+    ChildSlots cs;
+    const uint32_t* pointCount;
+    __device__ uint64_t operator()(uint64_t s) const
+    {
+        const int32_t c  = cs.child(s);
+        const uint64_t n = c >= 0 ? pointCount[c] : 0u;
+        return (((n + TILE - 1) / TILE) << 32) | n;
+    }
+};
+
+struct LevelSegmentOut
+{
+    ChildSlots cs;
+    const uint32_t* sortedStart;
+    const uint32_t* stage;
+    uint32_t *segCount, *segSrc, *segTile, *segInput;
+    __device__ void operator()(uint64_t s, uint64_t prefix, uint64_t v) const
+    {
+        const int32_t c = cs.child(s);
+        segCount[s]     = static_cast<uint32_t>(v);
+        segSrc[s]       = c < 0 ? 0u : (cs.flags[c] & NODE_INTERNAL) ? stage[c] : sortedStart[c];
+        segTile[s]      = static_cast<uint32_t>(prefix >> 32);
+        segInput[s]     = static_cast<uint32_t>(prefix);
+    }
+};
+
+// Before a level's first pass: the griddings of its nodes, the segment of every tile (a search per
+// tile, all of them in flight; a thread per segment wrote a large child's thousands of entries by
+// itself, 71 us of a 5.1M-point build) and a clear bitmap.
+static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, SubsampleParams sp,
+                                                        const uint32_t* __restrict__ internal,
+                                                        const uint32_t* __restrict__ nodeKey,
+                                                        NodeGrid* __restrict__ nodeGrid,
+                                                        const uint32_t* __restrict__ segTile,
+                                                        const uint64_t* __restrict__ segTotal,
+                                                        uint32_t* __restrict__ tileList, uint64_t words,
+                                                        uint32_t* __restrict__ bitmap)
+{
+    for (uint64_t k = globalThread(); k < nodes; k += globalStride())
+        nodeGrid[k] = nodeGridOf(internal[k], nodeKey[internal[k]], sp.levelOffset, sp.levelGrid, sp.level, sp.depth,
+                                 sp.cubicMin, sp.sideHalf, sp.side, sp.g, sp.seed);
+    const uint32_t tiles = static_cast<uint32_t>(*segTotal >> 32);
+    for (uint64_t t = globalThread(); t < tiles; t += globalStride())
+    {
+        // the last segment that starts at or before t; segments without tiles start where the next does
+        uint32_t lo = 0, hi = 8 * nodes;
+        while (hi - lo > 1)
+        {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (segTile[mid] <= t)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        tileList[t] = lo;
+    }
+    for (uint64_t w = globalThread(); w < words; w += globalStride())
+        bitmap[w] = 0;
 }
+
+// The tiles of a batch of a level's nodes: from *lo (null: 0) to *hi.
+struct TileRange
+{
+    const uint32_t* lo;
+    const uint32_t* hi;
+    __device__ __forceinline__ uint32_t first() const { return lo ? *lo : 0u; }
+    __device__ __forceinline__ uint32_t count() const { return *hi - first(); }
+};
+
+// One step of the subsampling (a batch of a level's nodes), with the sizes that only the device
+// knows: the output cursor before and after it and its occupied cells.
+struct StepSizes
+{
+    const uint64_t* cursor;  // N + points subsampled before this step
+    uint64_t* next;          // the same after it
+    const uint32_t* cells;   // occupied cells
+    uint64_t capacity;       // E
+    // false: the points do not fit the output (A14); nothing of this step or a later one is written
+    __device__ __forceinline__ bool fits() const { return *cursor + *cells <= capacity; }
+};
+
+constexpr uint64_t CURSOR_FULL = 1ull << 62;
 
 // Identifies the input of this thread: tile -> segment -> (node k, input position, input index q).
 struct InputRef
@@ -596,8 +691,7 @@ __device__ __forceinline__ void markTile(uint32_t tile, uint32_t nodeBase, uint6
 }
 
 template <typename T>
-static __global__ __launch_bounds__(TILE) void kMark(uint32_t tileBase, uint32_t tiles, uint32_t nodeBase,
-                                               uint64_t wordsPerNode,
+static __global__ __launch_bounds__(TILE) void kMark(TileRange range, uint32_t nodeBase, uint64_t wordsPerNode,
                                                const uint32_t* __restrict__ tileList,
                                                const uint32_t* __restrict__ segTile,
                                                const uint32_t* __restrict__ segCount,
@@ -609,10 +703,10 @@ static __global__ __launch_bounds__(TILE) void kMark(uint32_t tileBase, uint32_t
 {
     // consecutive tiles share bitmap words: runs of them per XCD
     const uint32_t t = xcdRunItem(blockIdx.x, XCD_TILE_RUN);
-    if (t >= tiles)
+    if (t >= range.count())
         return;
-    markTile<T>(tileBase + t, nodeBase, wordsPerNode, tileList, segTile, segCount, segSrc, segInput,
-                nodeGrid, ps, bitmap, cellOf, err);
+    markTile<T>(range.first() + t, nodeBase, wordsPerNode, tileList, segTile, segCount, segSrc, segInput, nodeGrid, ps,
+                bitmap, cellOf, err);
 }
 
 struct PopcountIn
@@ -628,37 +722,24 @@ __device__ __forceinline__ uint32_t cellRank(const uint32_t* bitmap, const uint3
     return prefix[word] + __popc(bitmap[word] & ((1u << bit) - 1u));
 }
 
-// Per node of the batch: subsample size (occupied cells), staging position, first dense index.
-__device__ __forceinline__ void batchNodeOf(uint64_t kl, uint32_t nodeBase, uint32_t nodes, uint64_t wordsPerNode,
+// Per node of the batch: subsample size (occupied cells) and staging position.
+__device__ __forceinline__ void batchNodeOf(uint64_t kl, uint32_t nodeBase, uint64_t wordsPerNode,
                                             const NodeGrid* __restrict__ nodeGrid,
                                             const uint32_t* __restrict__ prefix, uint32_t cursor,
-                                            uint32_t* __restrict__ pointCount, uint32_t* __restrict__ stage,
-                                            uint32_t* __restrict__ nodeFirst)
+                                            uint32_t* __restrict__ pointCount, uint32_t* __restrict__ stage)
 {
-    uint32_t b    = prefix[kl * wordsPerNode];
-    nodeFirst[kl] = b;
-    if (kl == nodes)
-        return;
-    uint32_t e     = prefix[(kl + 1) * wordsPerNode];
+    const uint32_t b = prefix[kl * wordsPerNode], e = prefix[(kl + 1) * wordsPerNode];
     uint32_t id    = nodeGrid[nodeBase + kl].id;
     pointCount[id] = e - b;
     stage[id]      = cursor + b;
 }
 
-static __global__ __launch_bounds__(BLOCK) void kBatchNodes(uint32_t nodeBase, uint32_t nodes, uint64_t wordsPerNode,
-                                                      const NodeGrid* __restrict__ nodeGrid,
-                                                      const uint32_t* __restrict__ prefix, uint32_t cursor,
-                                                      uint32_t* __restrict__ pointCount, uint32_t* __restrict__ stage,
-                                                      uint32_t* __restrict__ nodeFirst)
-{
-    for (uint64_t kl = globalThread(); kl <= nodes; kl += globalStride())
-        batchNodeOf(kl, nodeBase, nodes, wordsPerNode, nodeGrid, prefix, cursor, pointCount, stage, nodeFirst);
-}
-
-static __global__ __launch_bounds__(BLOCK) void kClearCompact(uint64_t n, uint64_t* __restrict__ win,
+// (n: the step's occupied cells, on the device)
+static __global__ __launch_bounds__(BLOCK) void kClearCompact(const uint32_t* __restrict__ n, uint64_t* __restrict__ win,
                                                         uint64_t* __restrict__ color, uint32_t* __restrict__ cellCnt)
 {
-    for (uint64_t i = globalThread(); i < n; i += globalStride())
+    const uint64_t cells = *n;
+    for (uint64_t i = globalThread(); i < cells; i += globalStride())
     {
         if (win)
             win[i] = ~0ull;
@@ -768,8 +849,27 @@ __device__ __forceinline__ void accumulateTile(uint32_t tile, uint32_t nodeBase,
     }
 }
 
+// Subsampled points of an internal node and all internal nodes below it (a leaf's: zero).
+__device__ __forceinline__ void subtreeOf(uint32_t id, const uint8_t* __restrict__ flags,
+                                          const int32_t* __restrict__ children, const uint32_t* pointCount,
+                                          uint32_t* subtree)
+{
+    if (!(flags[id] & NODE_INTERNAL))
+        return;
+    uint32_t s = pointCount[id];
+    for (int k = 0; k < 8; ++k)
+    {
+        const int32_t c = children[8 * static_cast<uint64_t>(id) + k];
+        if (c >= 0)
+            s += subtree[c];
+    }
+    subtree[id] = s;
+}
+
+// The nodes' subsample sizes, subtree sums and the next step's cursor go with it (one thread per node).
 template <typename T, uint32_t MODE, bool RANDOM>
-static __global__ __launch_bounds__(TILE) void kAccumulate(uint32_t tileBase, uint32_t nodeBase, uint64_t wordsPerNode,
+static __global__ __launch_bounds__(TILE) void kAccumulate(TileRange range, StepSizes step, uint32_t nodeBase,
+                                                     uint32_t nodes, uint64_t wordsPerNode,
                                                      const uint32_t* __restrict__ tileList,
                                                      const uint32_t* __restrict__ segTile,
                                                      const uint32_t* __restrict__ segCount,
@@ -782,12 +882,48 @@ static __global__ __launch_bounds__(TILE) void kAccumulate(uint32_t tileBase, ui
                                                      uint64_t* __restrict__ win,
                                                      uint64_t* __restrict__ color, uint32_t* __restrict__ cellCnt,
                                                      uint32_t* __restrict__ cellKey, uint32_t* __restrict__ cellNode,
-                                                     uint32_t* __restrict__ rankOf)
+                                                     uint32_t* __restrict__ rankOf, uint32_t* __restrict__ pointCount,
+                                                     uint32_t* __restrict__ stage, uint32_t* __restrict__ subtree,
+                                                     const uint8_t* __restrict__ flags,
+                                                     const int32_t* __restrict__ children, uint32_t* __restrict__ err)
 {
-    accumulateTile<T, MODE, RANDOM>(tileBase + blockIdx.x, nodeBase, wordsPerNode, tileList, segTile, segCount,
-                                    segSrc, segInput, nodeGrid, bitmap, prefix, cellOf, ps, win, color, cellCnt,
-                                    cellKey, cellNode, rankOf);
+    const bool fits       = step.fits();
+    const uint64_t cursor = *step.cursor;
+    if (globalThread() == 0)
+    {
+        *step.next = fits ? cursor + *step.cells : CURSOR_FULL;
+        if (!fits)
+            atomicOr(err, ERR_OVERFLOW);
+    }
+    for (uint64_t kl = globalThread(); kl < nodes; kl += globalStride())
+    {
+        const uint32_t id = nodeGrid[nodeBase + kl].id;
+        if (fits)
+            batchNodeOf(kl, nodeBase, wordsPerNode, nodeGrid, prefix, static_cast<uint32_t>(cursor), pointCount, stage);
+        else
+            pointCount[id] = 0;  // no input of a later step
+        subtreeOf(id, flags, children, pointCount, subtree);  // of the levels below: complete
+    }
+    if (!fits)
+        return;
+    if (blockIdx.x < range.count())
+        accumulateTile<T, MODE, RANDOM>(range.first() + blockIdx.x, nodeBase, wordsPerNode, tileList, segTile,
+                                        segCount, segSrc, segInput, nodeGrid, bitmap, prefix, cellOf, ps, win, color,
+                                        cellCnt, cellKey, cellNode, rankOf);
 }
+
+// exclusive prefix into an array, with the total behind it
+struct ExclusiveWithTotal
+{
+    uint32_t* dst;
+    const uint32_t* n;
+    __device__ void operator()(uint64_t i, uint32_t prefix, uint32_t v) const
+    {
+        dst[i] = prefix;
+        if (i + 1 == *n)
+            dst[i + 1] = prefix + v;
+    }
+};
 
 // Per-point data of the weighted filter, in cell order so that a cell's points are one contiguous
 // run (cellStart[cell] + arrival rank), in two arrays:
@@ -857,7 +993,7 @@ __device__ __forceinline__ void scatterPayloadTile(uint32_t tile, const uint32_t
 }
 
 template <typename T, bool RANDOM>
-static __global__ __launch_bounds__(TILE) void kScatterPayload(uint32_t tileBase, uint32_t tiles,
+static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, StepSizes step,
                                                          const uint32_t* __restrict__ tileList,
                                                          const uint32_t* __restrict__ segTile,
                                                          const uint32_t* __restrict__ segCount,
@@ -871,12 +1007,13 @@ static __global__ __launch_bounds__(TILE) void kScatterPayload(uint32_t tileBase
                                                          WeightPayload* __restrict__ payload,
                                                          uint64_t* __restrict__ winKey)
 {
+    if (!step.fits())
+        return;
     // consecutive tiles store to neighbouring payload slots: runs of them per XCD
     const uint32_t t = xcdRunItem(blockIdx.x, XCD_TILE_RUN);
-    if (t >= tiles)
-        return;
-    scatterPayloadTile<T, RANDOM>(tileBase + t, tileList, segTile, segCount, segSrc, segInput, nodeGrid,
-                                  cellKey, rankOf, cellStart, cellOf, ps, payload, winKey);
+    if (t < range.count())
+        scatterPayloadTile<T, RANDOM>(range.first() + t, tileList, segTile, segCount, segSrc, segInput, nodeGrid,
+                                      cellKey, rankOf, cellStart, cellOf, ps, payload, winKey);
 }
 
 // Select (rp_subsampling.cuh:70-321, fp_subsampling.cuh:30-306): one output record per occupied
@@ -963,8 +1100,8 @@ __device__ __forceinline__ void emitCell(uint32_t c, uint32_t nodeBase, uint64_t
 }
 
 template <typename T, uint32_t MODE>
-static __global__ __launch_bounds__(BLOCK) void kEmit(uint32_t cells, uint32_t nodeBase, uint64_t wordsPerNode,
-                                                uint32_t cursor, const NodeGrid* __restrict__ nodeGrid,
+static __global__ __launch_bounds__(BLOCK) void kEmit(StepSizes step, uint32_t nodeBase, uint64_t wordsPerNode,
+                                                const NodeGrid* __restrict__ nodeGrid,
                                                 const uint32_t* __restrict__ bitmap,
                                                 const uint32_t* __restrict__ prefix,
                                                 const uint32_t* __restrict__ cellKey,
@@ -972,6 +1109,9 @@ static __global__ __launch_bounds__(BLOCK) void kEmit(uint32_t cells, uint32_t n
                                                 const uint64_t* __restrict__ win, const uint64_t* __restrict__ color,
                                                 PointStore<T> ps)
 {
+    if (!step.fits())
+        return;
+    const uint32_t cells = *step.cells, cursor = static_cast<uint32_t>(*step.cursor);
     for (uint64_t ci = globalThread(); ci < cells; ci += globalStride())
         emitCell<T, MODE>(static_cast<uint32_t>(ci), nodeBase, wordsPerNode, cursor, nodeGrid, bitmap, prefix, cellKey,
                           cellNode, win, color, ps);
@@ -1134,8 +1274,8 @@ __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, 
 }
 
 template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kEmitWeighted(uint32_t cells, uint32_t nodeBase, uint64_t wordsPerNode,
-                                                        uint32_t cursor, const NodeGrid* __restrict__ nodeGrid,
+static __global__ __launch_bounds__(BLOCK) void kEmitWeighted(StepSizes step, uint32_t nodeBase, uint64_t wordsPerNode,
+                                                        const NodeGrid* __restrict__ nodeGrid,
                                                         const uint32_t* __restrict__ bitmap,
                                                         const uint32_t* __restrict__ prefix,
                                                         const uint32_t* __restrict__ cellKey,
@@ -1144,35 +1284,18 @@ static __global__ __launch_bounds__(BLOCK) void kEmitWeighted(uint32_t cells, ui
                                                         const WeightPayload* __restrict__ payload,
                                                         const uint64_t* __restrict__ winKey, PointStore<T> ps)
 {
-    // each XCD takes runs of EMIT_CHUNK consecutive cell blocks
-    const uint32_t c = xcdRunItem(blockIdx.x, EMIT_CHUNK) * BLOCK + threadIdx.x;
-    if (c >= cells)
+    if (!step.fits())
         return;
-    emitWeightedCell<T>(c, nodeBase, wordsPerNode, cursor, nodeGrid, bitmap, prefix, cellKey, cellNode, cellStart,
-                        payload, winKey, ps);
+    // each XCD takes runs of EMIT_CHUNK consecutive cell blocks
+    const uint64_t c = static_cast<uint64_t>(xcdRunItem(blockIdx.x, EMIT_CHUNK)) * BLOCK + threadIdx.x;
+    if (c < *step.cells)
+        emitWeightedCell<T>(static_cast<uint32_t>(c), nodeBase, wordsPerNode, static_cast<uint32_t>(*step.cursor),
+                            nodeGrid, bitmap, prefix, cellKey, cellNode, cellStart, payload, winKey, ps);
 }
 
 // DFS post-order placement (A6, kernel_helpers.cuh:55-59): subtree sums of subsample sizes
-// bottom-up, then region starts top-down; an internal node's data follows its children's
-// subtrees: dataIdx = N + regionStart + sum of its children's subtree sizes. kSubtree / kRegion
-// take one level per launch; kPlaceLevels does all levels in one workgroup for small trees (a
-// small build is bound by its launch count, not by these few thousand nodes).
-__device__ __forceinline__ void subtreeOf(uint32_t id, const uint8_t* __restrict__ flags,
-                                          const int32_t* __restrict__ children,
-                                          const uint32_t* __restrict__ pointCount, uint32_t* __restrict__ subtree)
-{
-    if (!(flags[id] & NODE_INTERNAL))
-        return;
-    uint32_t s = pointCount[id];
-    for (int k = 0; k < 8; ++k)
-    {
-        const int32_t c = children[8 * static_cast<uint64_t>(id) + k];
-        if (c >= 0)
-            s += subtree[c];
-    }
-    subtree[id] = s;
-}
-
+// bottom-up (with the levels), then region starts: an internal node's data follows its children's
+// subtrees: dataIdx = N + regionStart + sum of its children's subtree sizes.
 __device__ __forceinline__ void regionOf(uint32_t id, uint32_t root, uint32_t N, const uint8_t* __restrict__ flags,
                                          const int32_t* __restrict__ children, const uint32_t* __restrict__ subtree,
                                          uint32_t* __restrict__ region, uint64_t* __restrict__ dataIdx)
@@ -1192,57 +1315,36 @@ __device__ __forceinline__ void regionOf(uint32_t id, uint32_t root, uint32_t N,
     dataIdx[id] = static_cast<uint64_t>(N) + r;
 }
 
-static __global__ __launch_bounds__(BLOCK) void kSubtree(uint32_t levelStart, uint32_t nodes,
-                                                   const uint8_t* __restrict__ flags,
+// Single cloud: every internal node of the list on its own, its region from the subtrees of the
+// lower-slot siblings on its way up. No level waits for another (one workgroup going down level by
+// level took 105 us for 6600 nodes).
+static __global__ __launch_bounds__(64) void kPlaceNodes(const uint32_t* __restrict__ list, uint32_t nodes, uint32_t N,
+                                                   const int32_t* __restrict__ parent,
                                                    const int32_t* __restrict__ children,
                                                    const uint32_t* __restrict__ pointCount,
-                                                   uint32_t* __restrict__ subtree)
+                                                   const uint32_t* __restrict__ subtree, uint64_t* __restrict__ dataIdx)
 {
     for (uint64_t j = globalThread(); j < nodes; j += globalStride())
-        subtreeOf(levelStart + static_cast<uint32_t>(j), flags, children, pointCount, subtree);
-}
-
-static __global__ __launch_bounds__(BLOCK) void kRegion(uint32_t levelStart, uint32_t nodes, uint32_t root, uint32_t N,
-                                                  const uint8_t* __restrict__ flags,
-                                                  const int32_t* __restrict__ children,
-                                                  const uint32_t* __restrict__ subtree,
-                                                  uint32_t* __restrict__ region, uint64_t* __restrict__ dataIdx)
-{
-    for (uint64_t j = globalThread(); j < nodes; j += globalStride())
-        regionOf(levelStart + static_cast<uint32_t>(j), root, N, flags, children, subtree, region, dataIdx);
-}
-
-constexpr int PLACE_THREADS = 1024;
-
-struct PlaceParams
-{
-    uint32_t levelStart[MAX_LEVELS + 1];  // sparse ids of level l: [levelStart[l], levelStart[l + 1])
-    uint32_t depth, m, root, N;
-};
-
-// One workgroup: subtree sizes zeroed, then summed level by level bottom-up, then regions and data
-// offsets top-down, a barrier between levels (the workgroup's writes are visible to it after one).
-static __global__ __launch_bounds__(PLACE_THREADS) void kPlaceLevels(PlaceParams pp, const uint8_t* __restrict__ flags,
-                                                              const int32_t* __restrict__ children,
-                                                              const uint32_t* __restrict__ pointCount,
-                                                              uint32_t* __restrict__ subtree,
-                                                              uint32_t* __restrict__ region,
-                                                              uint64_t* __restrict__ dataIdx)
-{
-    for (uint32_t i = threadIdx.x; i < pp.m; i += PLACE_THREADS)
-        subtree[i] = 0;
-    __syncthreads();
-    for (uint32_t l = 1; l <= pp.depth; ++l)
     {
-        for (uint32_t id = pp.levelStart[l] + threadIdx.x; id < pp.levelStart[l + 1]; id += PLACE_THREADS)
-            subtreeOf(id, flags, children, pointCount, subtree);
-        __syncthreads();
-    }
-    for (uint32_t l = pp.depth; l >= 1; --l)
-    {
-        for (uint32_t id = pp.levelStart[l] + threadIdx.x; id < pp.levelStart[l + 1]; id += PLACE_THREADS)
-            regionOf(id, pp.root, pp.N, flags, children, subtree, region, dataIdx);
-        __syncthreads();
+        const uint32_t id = list[j];
+        uint32_t before   = subtree[id] - pointCount[id];  // its children's subtrees
+        int32_t cur       = static_cast<int32_t>(id);
+        for (int32_t p = parent[cur]; p >= 0; cur = p, p = parent[cur])
+        {
+            int32_t c[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                c[k] = children[8 * static_cast<uint64_t>(p) + k];
+            bool lower = true;  // slots before cur's
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+            {
+                lower = lower && c[k] != cur;
+                if (lower && c[k] >= 0)
+                    before += subtree[c[k]];
+            }
+        }
+        dataIdx[id] = static_cast<uint64_t>(N) + before;
     }
 }
 
@@ -1259,6 +1361,25 @@ struct PlacedChunksIn
     __device__ uint32_t operator()(uint64_t i) const
     {
         return (flags[i] & NODE_INTERNAL) ? (pointCount[i] + PLACE_CHUNK - 1) / PLACE_CHUNK : 0u;
+    }
+};
+
+// the same over a list of internal nodes
+struct PlacedListIn
+{
+    const uint32_t* list;
+    const uint32_t* pointCount;
+    __device__ uint32_t operator()(uint64_t j) const { return (pointCount[list[j]] + PLACE_CHUNK - 1) / PLACE_CHUNK; }
+};
+
+struct PlacedListOut
+{
+    const uint32_t* list;
+    uint64_t* chunks;  // chunk number << 32 | node id
+    __device__ void operator()(uint64_t j, uint32_t prefix, uint32_t v) const
+    {
+        for (uint32_t k = 0; k < v; ++k)
+            chunks[prefix + k] = (static_cast<uint64_t>(k) << 32) | list[j];
     }
 };
 
@@ -1292,7 +1413,8 @@ __device__ __forceinline__ void permuteChunk(uint64_t entry, uint32_t N, const u
 }
 
 template <typename T>
-static __global__ __launch_bounds__(BLOCK) void kPermute(const uint64_t* __restrict__ chunkList, uint32_t N,
+static __global__ __launch_bounds__(BLOCK) void kPermute(const uint64_t* __restrict__ chunkList,
+                                                   const uint32_t* __restrict__ chunks, uint32_t N,
                                                    const uint32_t* __restrict__ stage,
                                                    const uint64_t* __restrict__ dataIdx,
                                                    const uint32_t* __restrict__ pointCount,
@@ -1302,8 +1424,10 @@ static __global__ __launch_bounds__(BLOCK) void kPermute(const uint64_t* __restr
                                                    double sy, double sz, uint32_t* __restrict__ lut,
                                                    OutRecord* __restrict__ out)
 {
-    permuteChunk<T>(chunkList[blockIdx.x], N, stage, dataIdx, pointCount, stLut, stOut, stPts, stRgb, cubic, sx, sy,
-                    sz, lut, out);
+    const uint32_t all = *chunks;
+    for (uint32_t c = blockIdx.x; c < all; c += gridDim.x)
+        permuteChunk<T>(chunkList[c], N, stage, dataIdx, pointCount, stLut, stOut, stPts, stRgb, cubic, sx, sy, sz,
+                        lut, out);
 }
 
 }  // namespace oc

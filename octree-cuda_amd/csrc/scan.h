@@ -122,6 +122,20 @@ __device__ __forceinline__ T tileExclusiveScan(const T (&v)[SCAN_ITEMS], T (&pre
     return carry;
 }
 
+// The same where tiles of zeros are common (bitmaps): they need no scan.
+template <typename T>
+__device__ __forceinline__ T sparseTileScan(const T (&v)[SCAN_ITEMS], T (&pre)[SCAN_ITEMS], T* lds)
+{
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < SCAN_ITEMS; ++k)
+    {
+        any |= v[k] != 0;
+        pre[k] = 0;
+    }
+    return __syncthreads_or(any) ? tileExclusiveScan(v, pre, lds) : T(0);
+}
+
 // out(i, offset + exclusive prefix, value) for each item i of this thread in the tile (items past n
 // skipped).
 template <typename T, typename Out>
@@ -153,12 +167,32 @@ __device__ __forceinline__ void tileRange(uint64_t tiles, uint64_t& first, uint6
     last               = first + per < tiles ? first + per : tiles;
 }
 
-template <typename T, typename In>
-static __global__ __launch_bounds__(SCAN_THREADS) void kScanReduce(In in, uint64_t n, T* blockSums, uint64_t tiles)
+// The number of items: known to the host, or on the device as the difference of two words.
+struct HostCount
+{
+    uint64_t n;
+    __device__ uint64_t operator()() const { return n; }
+};
+
+struct DeviceCount
+{
+    const uint32_t* end;
+    const uint32_t* begin;  // may be null
+    __device__ uint64_t operator()() const { return *end - (begin ? *begin : 0u); }
+};
+
+__host__ __device__ inline uint64_t scanTiles(uint64_t n)
+{
+    return (n + SCAN_TILE - 1) / SCAN_TILE;
+}
+
+template <typename T, typename In, typename Size>
+static __global__ __launch_bounds__(SCAN_THREADS) void kScanReduce(In in, Size size, T* blockSums)
 {
     __shared__ T lds[SCAN_WAVES];
+    const uint64_t n = size();
     uint64_t first, last;
-    tileRange(tiles, first, last);
+    tileRange(scanTiles(n), first, last);
     T s = 0;
     for (uint64_t tile = first; tile < last; ++tile)
     {
@@ -183,22 +217,29 @@ __device__ __forceinline__ T blockSum(T v, T* lds)
     return total;
 }
 
-template <typename T, typename In, typename Out>
-static __global__ __launch_bounds__(SCAN_THREADS) void kScanDown(In in, Out out, uint64_t n, const T* blockSums,
-                                                          uint64_t tiles, T* total)
+// Sum of the range sums before this workgroup's range.
+template <typename T>
+__device__ __forceinline__ T sumBefore(const T* blockSums, T* lds)
 {
-    __shared__ T lds[SCAN_ITEMS * SCAN_WAVES];
-    uint64_t first, last;
-    tileRange(tiles, first, last);
     T before = 0;
     for (uint32_t b = threadIdx.x; b < blockIdx.x; b += SCAN_THREADS)
         before += blockSums[b];
-    T carry = blockSum(before, lds);
+    return blockSum(before, lds);
+}
+
+template <typename T, typename In, typename Out, typename Size>
+static __global__ __launch_bounds__(SCAN_THREADS) void kScanDown(In in, Out out, Size size, const T* blockSums, T* total)
+{
+    __shared__ T lds[SCAN_ITEMS * SCAN_WAVES];
+    const uint64_t n = size();
+    uint64_t first, last;
+    tileRange(scanTiles(n), first, last);
+    T carry = sumBefore(blockSums, lds);
     for (uint64_t tile = first; tile < last; ++tile)
     {
         T v[SCAN_ITEMS], pre[SCAN_ITEMS];
         loadTile<T>(in, tile * SCAN_TILE, n, v);
-        const T chunk = tileExclusiveScan(v, pre, lds);
+        const T chunk = sparseTileScan(v, pre, lds);
         storeTile<T>(out, tile * SCAN_TILE, n, v, pre, carry);
         carry += chunk;
     }
@@ -265,11 +306,6 @@ __device__ __forceinline__ void blockScanAll(In in, Out out, uint64_t n, T* tota
         *total = carry;
 }
 
-__host__ __device__ inline uint64_t scanTiles(uint64_t n)
-{
-    return (n + SCAN_TILE - 1) / SCAN_TILE;
-}
-
 // Out-of-place inputs up to this many tiles are scanned by kScanDirect: its last workgroup reads
 // all of them, SCAN_DIRECT_TILES / 2 dependent rounds of loads (16 tiles: ~6 us; one workgroup
 // walking them took ~25 us, two launches take ~9 us).
@@ -290,8 +326,19 @@ void scanExclusive(uint64_t n, In in, Out out, T* tileScratch, T* total, hipStre
         return;
     }
     const unsigned grid = static_cast<unsigned>(tiles < SCAN_GRID ? tiles : SCAN_GRID);
-    kScanReduce<T, In><<<grid, SCAN_THREADS, 0, stream>>>(in, n, tileScratch, tiles);
-    kScanDown<T, In, Out><<<grid, SCAN_THREADS, 0, stream>>>(in, out, n, tileScratch, tiles, total);
+    kScanReduce<T><<<grid, SCAN_THREADS, 0, stream>>>(in, HostCount{n}, tileScratch);
+    kScanDown<T><<<grid, SCAN_THREADS, 0, stream>>>(in, out, HostCount{n}, tileScratch, total);
+}
+
+// The same over a number of items that only the device knows; bound: the most it can be.
+// tileScratch must hold min(scanTiles(bound), SCAN_GRID) values.
+template <typename T, typename In, typename Out>
+void scanExclusive(DeviceCount n, uint64_t bound, In in, Out out, T* tileScratch, T* total, hipStream_t stream)
+{
+    const uint64_t tiles = scanTiles(bound);
+    const unsigned grid  = static_cast<unsigned>(tiles < SCAN_GRID ? (tiles ? tiles : 1) : SCAN_GRID);
+    kScanReduce<T><<<grid, SCAN_THREADS, 0, stream>>>(in, n, tileScratch);
+    kScanDown<T><<<grid, SCAN_THREADS, 0, stream>>>(in, out, n, tileScratch, total);
 }
 
 }  // namespace oc

@@ -127,8 +127,8 @@ EXPORTED int ocpi_copy_point_lut (void* session, uint32_t* destination, uint64_t
 /* Copies the first `count` 18-byte output records (int32 x, y, z; uint16 r, g, b). */
 EXPORTED int ocpi_copy_output (void* session, uint8_t* destination, uint64_t count);
 
-/* Device-side durations of the last ocpi_generate_octree, in milliseconds, measured with HIP
- * events on the session stream: [0] counting kernel, [1] merge (pyramid, nodes, leaf blocks),
+/* Device-side durations of the last ocpi_generate_octree, in milliseconds, between clock stamps that
+ * its kernels take as they start: [0] counting kernel, [1] merge (pyramid, nodes, leaf blocks),
  * [2] distribution kernel, [3] subsampling (all levels and the final placement), [4] whole
  * build, [5] summed subsampling insert kernels, [6] summed subsampling emit kernels. */
 EXPORTED int ocpi_get_stage_timings (void* session, float* milliseconds, uint32_t n);

@@ -77,10 +77,6 @@ public:
     void generate() override;
     const BuildResult& lastBuild() const override { return *this; }
     void setProgress(std::function<void()> hook) override { itsProgress = std::move(hook); }
-    // Per-batch subsampling events (the insert / emit split of the stage timings); off, a build
-    // makes fewer runtime calls, which matters when many builders share one process.
-    void setDetailedTimings(bool on) { itsDetailedTimings = on; }
-
     // Device bytes held by the arena, and its release (the next setup grows it again).
     uint64_t arenaBytes() const override;
     void releaseArena() override;
@@ -139,7 +135,6 @@ private:
     void subsampleLevels();
     void placeInternalNodes();
 
-    void syncStream();
     void progress();
     void waitForSnapshotOnStream();
     void waitMailbox(uint64_t seq);
@@ -155,8 +150,8 @@ private:
     // host memory and the host spins on the sequence (no staging copy, no blocking-sync wake-up).
     uint64_t* itsMailbox  = nullptr;
     uint64_t itsMailSeq   = 0;
+    int itsClockRate      = 0;  // kHz, of the stage timings' device clock
     bool itsReady         = false;  // setup() has run
-    bool itsDetailedTimings = true;
     std::function<void()> itsProgress;  // called between the stages of generate()
     CloudInfo itsCloud;
     ProcessingInfo itsProc;
@@ -203,7 +198,7 @@ private:
     // occupancy bitmaps with their popcount prefix, per-cell (dense index) state, per-input state
     DeviceBuffer itsLeafList, itsInternalList, itsSegCount, itsSegSrc, itsSegTile, itsSegInput, itsNodeGrid,
             itsTileList;
-    DeviceBuffer itsBitmap, itsPrefix, itsCursors;
+    DeviceBuffer itsBitmap, itsPrefix, itsCursors, itsStamps;
     DeviceBuffer itsWin, itsColor, itsCellCnt, itsCellStart, itsCellKey, itsCellNode;
     DeviceBuffer itsCellOf, itsRankOf, itsPayload;
 
@@ -211,23 +206,6 @@ private:
     DeviceBuffer itsScalars, itsScanScratch;
 
     std::vector<DeviceBuffer*> arena();
-
-    enum EventSlot
-    {
-        EV_START,
-        EV_COUNT_BEGIN,
-        EV_COUNT_END,
-        EV_MERGE_END,
-        EV_DIST_BEGIN,
-        EV_DIST_END,
-        EV_END,
-        EV_SLOTS
-    };
-    hipEvent_t itsEvents[EV_SLOTS] = {};
-    // per subsampling batch: evaluate begin/end, emit begin/end (when detailed timings are on)
-    std::vector<std::array<hipEvent_t, 4>> itsBatchEvents;
-    uint32_t itsBatchesRun = 0;
-    std::array<hipEvent_t, 4>& batchEvents();
 };
 
 }  // namespace oc

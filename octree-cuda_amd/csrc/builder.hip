@@ -123,7 +123,8 @@ enum MailSlot
     MAIL_INPUTS,
     MAIL_LEVEL = 8,                        // first node of every level
     MAIL_INNER = MAIL_LEVEL + MAX_LEVELS,  // first internal node of every level
-    MAIL_WORDS = MAIL_INNER + MAX_LEVELS
+    MAIL_TICKS = MAIL_INNER + MAX_LEVELS,  // stage durations
+    MAIL_WORDS = MAIL_TICKS + 7
 };
 
 static uint32_t octreeDepth(uint32_t grid)  // tools.cu:63-88
@@ -142,8 +143,7 @@ OctreeBuilder::OctreeBuilder(int device) : itsDevice(device)
     OC_HIP_CHECK(hipEventCreateWithFlags(&itsBuiltEvent, hipEventDisableTiming));
     OC_HIP_CHECK(hipEventCreateWithFlags(&itsCopiedEvent, hipEventDisableTiming));
     OC_HIP_CHECK(hipEventCreateWithFlags(&itsUploadedEvent, hipEventDisableTiming));
-    for (auto& ev : itsEvents)
-        OC_HIP_CHECK(hipEventCreate(&ev));
+    OC_HIP_CHECK(hipDeviceGetAttribute(&itsClockRate, hipDeviceAttributeWallClockRate, itsDevice));
     OC_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&itsMailbox), MAIL_WORDS * sizeof(uint64_t), hipHostMallocCoherent));
     std::fill(itsMailbox, itsMailbox + MAIL_WORDS, 0);
 }
@@ -262,7 +262,7 @@ std::vector<DeviceBuffer*> OctreeBuilder::arena()
             &itsBucketCount, &itsBucketStart, &itsBucketCursor,  &itsBucketList,  &itsLut,          &itsOut,
             &itsStLut,       &itsStOut,       &itsStPts,         &itsStRgb,        &itsInternalList, &itsSegCount,    &itsSegSrc,
             &itsSegTile,     &itsSegInput,    &itsNodeGrid,      &itsTileList,     &itsBitmap,      &itsPrefix,
-            &itsCursors,     &itsWin,         &itsColor,         &itsCellCnt,      &itsCellStart,   &itsCellKey,
+            &itsCursors,     &itsStamps,      &itsWin,         &itsColor,         &itsCellCnt,      &itsCellStart,   &itsCellKey,
             &itsCellNode,    &itsCellOf,      &itsRankOf,        &itsPayload,      &itsScalars,
             &itsScanScratch, &itsLeafList,   &itsSplitChunks,   &itsSplitHist};
 }
@@ -337,32 +337,8 @@ OctreeBuilder::~OctreeBuilder()
         (void)hipEventDestroy(itsCopiedEvent);
     if (itsUploadedEvent)
         (void)hipEventDestroy(itsUploadedEvent);
-    for (auto& ev : itsEvents)
-        if (ev)
-            (void)hipEventDestroy(ev);
-    for (auto& quad : itsBatchEvents)
-        for (auto& ev : quad)
-            if (ev)
-                (void)hipEventDestroy(ev);
     if (itsMailbox)
         (void)hipHostFree(itsMailbox);
-}
-
-std::array<hipEvent_t, 4>& OctreeBuilder::batchEvents()
-{
-    if (itsBatchesRun == itsBatchEvents.size())
-    {
-        std::array<hipEvent_t, 4> quad{};
-        for (auto& ev : quad)
-            OC_HIP_CHECK(hipEventCreate(&ev));
-        itsBatchEvents.push_back(quad);
-    }
-    return itsBatchEvents[itsBatchesRun++];
-}
-
-void OctreeBuilder::syncStream()
-{
-    OC_HIP_CHECK(hipStreamSynchronize(itsStream));
 }
 
 // The sizes after the merge, to the host mailbox: the nodes, the error flags, the internal nodes,
@@ -412,14 +388,32 @@ __global__ void kPublishInputs(const uint64_t* __restrict__ segTotal, uint64_t* 
     __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// The end of a build: the error flags and the used output records (the last cursor).
-__global__ void kPublishEnd(const uint64_t* __restrict__ sc, const uint64_t* __restrict__ cursor, uint64_t* box,
-                            uint64_t seq)
+// The end of a build: the error flags, the used output records (the last cursor) and the stage
+// durations from the clock stamps, in clock ticks.
+__global__ __launch_bounds__(64) void kPublishEnd(const uint64_t* __restrict__ sc, const uint64_t* __restrict__ cursors,
+                                                  const uint64_t* __restrict__ stamps, uint32_t steps, uint64_t* box,
+                                                  uint64_t seq)
 {
+    const uint64_t now = wall_clock64();
     if (threadIdx.x != 0)
         return;
-    __hip_atomic_store(box + MAIL_ERROR, sc[SC_ERROR], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(box + MAIL_USED, *cursor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    auto post = [&](uint32_t at, uint64_t v) {
+        __hip_atomic_store(box + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    };
+    const uint64_t start = sc[SC_STAMP], merge = sc[SC_STAMP + 1], dist = sc[SC_STAMP + 2];
+    const uint64_t levels = steps ? stamps[ST_BEGIN] : now;
+    uint64_t insert = 0, emit = 0;
+    for (uint32_t i = 0; i < steps; ++i)
+    {
+        const uint64_t* st = stamps + ST_STAMPS * i;
+        insert += st[ST_INSERT_END] - st[ST_INSERT_BEGIN];
+        emit += st[ST_STAMPS + ST_BEGIN] - st[ST_EMIT_BEGIN];
+    }
+    const uint64_t ticks[7] = {merge - start, dist - merge, levels - dist, now - levels, now - start, insert, emit};
+    for (uint32_t k = 0; k < 7; ++k)
+        post(MAIL_TICKS + k, ticks[k]);
+    post(MAIL_ERROR, sc[SC_ERROR]);
+    post(MAIL_USED, cursors[steps]);
     __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -459,25 +453,20 @@ void OctreeBuilder::generate()
 template <typename T>
 void OctreeBuilder::generateTyped()
 {
-    itsBatchesRun = 0;
-
-    OC_HIP_CHECK(hipEventRecord(itsEvents[EV_START], itsStream));
     countPoints<T>();  // writes nothing a snapshot reads, so it overlaps the previous one's copies
     progress();
     waitForSnapshotOnStream();
     mergeLevels();
     progress();
-    OC_HIP_CHECK(hipEventRecord(itsEvents[EV_MERGE_END], itsStream));
     distributePoints<T>();
     progress();
     subsampleLevels<T>();
     placeInternalNodes();
-    OC_HIP_CHECK(hipEventRecord(itsEvents[EV_END], itsStream));
     const uint64_t seq = ++itsMailSeq;
-    kPublishEnd<<<1, 64, 0, itsStream>>>(itsScalars.as<uint64_t>(), itsCursors.as<uint64_t>() + itsSteps, itsMailbox, seq);
+    kPublishEnd<<<1, 64, 0, itsStream>>>(itsScalars.as<uint64_t>(), itsCursors.as<uint64_t>(),
+                                         itsStamps.as<uint64_t>(), itsSteps, itsMailbox, seq);
     OC_LAUNCH_CHECK();
     waitMailbox(seq);
-    syncStream();
 
     const uint64_t err = itsMailbox[MAIL_ERROR];
     if (err & ERR_OVERFLOW)  // A14
@@ -486,28 +475,9 @@ void OctreeBuilder::generateTyped()
     if (err & ERR_OUTSIDE)
         throw std::runtime_error("a point lies outside the cubic bounding box");
     itsUsed = itsMailbox[MAIL_USED];
-    if (err & ERR_CAPACITY)
-        throw std::runtime_error("a node has more than 2^31 input points");
-
-    auto ms = [&](int a, int b) {
-        float v = 0.f;
-        OC_HIP_CHECK(hipEventElapsedTime(&v, itsEvents[a], itsEvents[b]));
-        return v;
-    };
     itsTimings.assign(7, 0.f);
-    itsTimings[0] = ms(EV_COUNT_BEGIN, EV_COUNT_END);
-    itsTimings[1] = ms(EV_COUNT_END, EV_MERGE_END);
-    itsTimings[2] = ms(EV_DIST_BEGIN, EV_DIST_END);
-    itsTimings[3] = ms(EV_DIST_END, EV_END);
-    itsTimings[4] = ms(EV_START, EV_END);
-    for (uint32_t i = 0; i < itsBatchesRun; ++i)
-    {
-        float a = 0.f, b = 0.f;
-        OC_HIP_CHECK(hipEventElapsedTime(&a, itsBatchEvents[i][0], itsBatchEvents[i][1]));
-        OC_HIP_CHECK(hipEventElapsedTime(&b, itsBatchEvents[i][2], itsBatchEvents[i][3]));
-        itsTimings[5] += a;
-        itsTimings[6] += b;
-    }
+    for (uint32_t k = 0; k < 7; ++k)
+        itsTimings[k] = static_cast<float>(static_cast<double>(itsMailbox[MAIL_TICKS + k]) / itsClockRate);
 }
 
 template <typename T>
@@ -527,7 +497,6 @@ void OctreeBuilder::countPoints()
     kBuildInit<<<gridFor(std::max<uint64_t>({nb, marked / 32, itsDense - marked}), 2048), BLOCK, 0, itsStream>>>(
             sc, bucketCount, nb + 1, occ, marked / 32, itsCount.as<uint32_t>(), marked, itsDense);
     OC_LAUNCH_CHECK();
-    OC_HIP_CHECK(hipEventRecord(itsEvents[EV_COUNT_BEGIN], itsStream));
 
     const unsigned histBlocks = static_cast<unsigned>(std::min<uint64_t>(2048, (n + 8191) / 8192));
     kBucketHist<T><<<histBlocks, HIST_THREADS, 0, itsStream>>>(itsCloudDevice, n, itsCloud.dataStride, g,
@@ -579,7 +548,6 @@ void OctreeBuilder::countPoints()
                                                              itsSplitHist.as<uint32_t>(), itsPerm.as<uint32_t>());
         OC_LAUNCH_CHECK();
     }
-    OC_HIP_CHECK(hipEventRecord(itsEvents[EV_COUNT_END], itsStream));  // the records move with the distribution
 }
 
 bool OctreeBuilder::fineSortBits() const
@@ -610,7 +578,8 @@ void OctreeBuilder::mergeLevels()
         lo.offset[l] = itsLevelOffset[l];
     lo.levels = itsDepth + 1;
     // levels 0..coarse come from the fine sort
-    kPropagateTop<<<1, TOP_THREADS, 0, itsStream>>>(count, lo, itsCoarse, itsProc.chunkingGrid);
+    kPropagateTop<<<1, TOP_THREADS, 0, itsStream>>>(count, lo, itsCoarse, itsProc.chunkingGrid,
+                                                      sc + SC_STAMP + 1);
     OC_LAUNCH_CHECK();
 
     // occupancy bits of the levels the fine sort has not marked, sparse ids (A2) + node keys / counts
@@ -671,6 +640,7 @@ void OctreeBuilder::mergeLevels()
     itsNodeStage.ensure(sizeof(uint32_t) * m);
     itsNodeSub.ensure(sizeof(uint32_t) * m);
     itsCursors.ensure(sizeof(uint64_t) * (planSteps() + 1));
+    itsStamps.ensure(sizeof(uint64_t) * (ST_STAMPS * itsSteps + 1));
     kNodeLinks<<<gridFor(m), BLOCK, 0, itsStream>>>(
             itsM, levelParams(), itsNodeKey.as<uint32_t>(), itsNodeCount.as<uint32_t>(),
             itsDenseToSparse.as<int32_t>(), occ, itsNodePoints.as<uint32_t>(), itsNodeData.as<uint64_t>(),
@@ -742,8 +712,8 @@ void OctreeBuilder::distributePoints()
                itsProc.chunkingGrid};
     // octree_chunking.cu:108-112
     double sx = 1.0 / itsCloud.scale[0], sy = 1.0 / itsCloud.scale[1], sz = 1.0 / itsCloud.scale[2];
-    OC_HIP_CHECK(hipEventRecord(itsEvents[EV_DIST_BEGIN], itsStream));
     const LeafOrderParams p = leafTables();
+    uint64_t* stamp         = itsScalars.as<uint64_t>() + SC_STAMP + 2;
     // the records move to the sorted cloud: leaf and cell order when there are internal nodes and
     // more than one cell to a node's grid, plain Morton order otherwise; then the leaf data blocks are
     // copied from it
@@ -752,17 +722,16 @@ void OctreeBuilder::distributePoints()
         kLeafCellOrder<T><<<static_cast<unsigned>(leafChunkBound()), LEAF_THREADS, 0, itsStream>>>(
                 itsLeafList.as<uint64_t>(), itsScalars.as<uint64_t>() + SC_LEAF_TOTAL, p, itsNodeKey.as<uint32_t>(),
                 itsNodeParent.as<int32_t>(), itsNodeCount.as<uint32_t>(), itsNodeSorted.as<uint32_t>(),
-                itsBucketed.as<SortedPoint<T>>(), itsPerm.as<uint32_t>(), itsSorted.as<SortedPoint<T>>());
+                itsBucketed.as<SortedPoint<T>>(), itsPerm.as<uint32_t>(), itsSorted.as<SortedPoint<T>>(), stamp);
     else
         kGatherSorted<T><<<gatherGrid(n), BLOCK, 0, itsStream>>>(itsBucketed.as<SortedPoint<T>>(),
                                                                      itsPerm.as<uint32_t>(), n,
-                                                                     itsSorted.as<SortedPoint<T>>());
+                                                                     itsSorted.as<SortedPoint<T>>(), stamp);
     OC_LAUNCH_CHECK();
     kDistributeSorted<T><<<gridFor(n, 16384), BLOCK, 0, itsStream>>>(
             itsSorted.as<SortedPoint<T>>(), n, g, itsCount.as<uint32_t>(), itsNodeSorted.as<uint32_t>(),
             itsNodeData.as<uint64_t>(), itsLut.as<uint32_t>(), itsOut.as<OutRecord>(), sx, sy, sz);
     OC_LAUNCH_CHECK();
-    OC_HIP_CHECK(hipEventRecord(itsEvents[EV_DIST_END], itsStream));
 }
 
 // Nodes of one subsampling step: their bitmaps and prefixes fit kBitmapBudget.
@@ -907,20 +876,17 @@ void OctreeBuilder::subsampleLevels()
                                   k1 < K ? itsSegTile.as<uint32_t>() + 8ull * k1
                                          : reinterpret_cast<uint32_t*>(sc + SC_SEG_TOTAL) + 1};
             const StepSizes step{cursors + stepAt, cursors + stepAt + 1, prefix + words, itsE};
+            uint64_t* stamps = itsStamps.as<uint64_t>() + ST_STAMPS * stepAt;
             ++stepAt;
-            std::array<hipEvent_t, 4> none{};
-            auto& ev         = itsDetailedTimings ? batchEvents() : none;
 
             kLevelPrepare<<<gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384), BLOCK, 0, itsStream>>>(
                     K, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
-                    sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap);
+                    sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, stamps + ST_BEGIN);
             OC_LAUNCH_CHECK();
-            if (itsDetailedTimings)
-                OC_HIP_CHECK(hipEventRecord(ev[0], itsStream));
             kMark<T><<<tileGrid, TILE, 0, itsStream>>>(
                     tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                     itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid, ps,
-                    bitmap, itsCellOf.as<uint32_t>(), err);
+                    bitmap, itsCellOf.as<uint32_t>(), err, stamps + ST_INSERT_BEGIN);
             OC_LAUNCH_CHECK();
             // per-cell state, reset for the occupied cells: by the scan itself on small levels, else
             // by kClearCompact
@@ -963,8 +929,6 @@ void OctreeBuilder::subsampleLevels()
                                   : kAccumulate<T, COLOR_INTER_WEIGHTED, false>);
                 break;
             }
-            if (itsDetailedTimings)
-                OC_HIP_CHECK(hipEventRecord(ev[1], itsStream));
 
             if (weighted)
             {
@@ -977,25 +941,24 @@ void OctreeBuilder::subsampleLevels()
                             tiles, step, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                             itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
                             itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(), itsCellStart.as<uint32_t>(),
-                            itsCellOf.as<uint32_t>(), ps, itsPayload.as<WeightPayload>(), winKey);
+                            itsCellOf.as<uint32_t>(), ps, itsPayload.as<WeightPayload>(), winKey,
+                            stamps + ST_INSERT_END);
                     OC_LAUNCH_CHECK();
                 };
                 scatter(random ? kScatterPayload<T, true> : kScatterPayload<T, false>);
             }
 
-            if (itsDetailedTimings)
-                OC_HIP_CHECK(hipEventRecord(ev[2], itsStream));
             if (weighted)
                 kEmitWeighted<T><<<xcdRunGrid((cellMost + BLOCK - 1) / BLOCK, EMIT_CHUNK), BLOCK, 0, itsStream>>>(
                         step, k0, wordsPerNode, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
                         itsCellNode.as<uint32_t>(), itsCellStart.as<uint32_t>(), itsPayload.as<WeightPayload>(), winKey,
-                        ps);
+                        ps, stamps + ST_EMIT_BEGIN);
             else
             {
                 auto emit = [&](auto kernel) {
                     kernel<<<gridFor(cellMost), BLOCK, 0, itsStream>>>(
                             step, k0, wordsPerNode, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
-                            itsCellNode.as<uint32_t>(), win, color, ps);
+                            itsCellNode.as<uint32_t>(), win, color, ps, stamps + ST_INSERT_END, stamps + ST_EMIT_BEGIN);
                 };
                 switch (itsColorMode)
                 {
@@ -1005,8 +968,6 @@ void OctreeBuilder::subsampleLevels()
                 }
             }
             OC_LAUNCH_CHECK();
-            if (itsDetailedTimings)
-                OC_HIP_CHECK(hipEventRecord(ev[3], itsStream));
         }
         progress();
     }
@@ -1021,7 +982,7 @@ void OctreeBuilder::placeInternalNodes()
     const uint32_t* list = itsInternalList.as<uint32_t>();
     kPlaceNodes<<<std::min<uint32_t>((nodes + 63) / 64, 4096), 64, 0, itsStream>>>(
             list, nodes, N, itsNodeParent.as<int32_t>(), itsNodeChild.as<int32_t>(), itsNodePoints.as<uint32_t>(),
-            itsNodeSub.as<uint32_t>(), itsNodeData.as<uint64_t>());
+            itsNodeSub.as<uint32_t>(), itsNodeData.as<uint64_t>(), itsStamps.as<uint64_t>() + ST_STAMPS * itsSteps);
     OC_LAUNCH_CHECK();
     // (internal node, chunk) work items; the leaf chunk list is free again after the distribution
     uint32_t* chunks = reinterpret_cast<uint32_t*>(itsScalars.as<uint64_t>() + SC_TABLE_TOTAL);
@@ -1096,9 +1057,7 @@ void OctreeBuilder::drainCopies() noexcept
 
 std::unique_ptr<SlotBuilder> makeSlotBuilder(int device)
 {
-    auto b = std::make_unique<OctreeBuilder>(device);
-    b->setDetailedTimings(false);
-    return b;
+    return std::make_unique<OctreeBuilder>(device);
 }
 
 uint64_t slotFootprint(const CloudInfo& cloud, const ProcessingInfo& proc, bool hostCloud)

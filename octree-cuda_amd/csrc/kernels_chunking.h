@@ -26,7 +26,8 @@ enum ScalarSlot : int
     SC_NEXT_BUCKET = 6,  // the fine sort's next occupied bucket
     SC_INTERNAL    = 7,  // internal nodes
     SC_LEVEL_START = 8,  // u32[MAX_LEVELS + 1] packed into the following slots
-    SC_COUNT       = 16
+    SC_STAMP       = 14,  // clock at the start of the build, of the merge and of the distribution
+    SC_COUNT       = 17
 };
 
 constexpr uint32_t ERR_OUTSIDE  = 1u;
@@ -51,7 +52,7 @@ static __global__ __launch_bounds__(BLOCK) void kBuildInit(uint64_t* __restrict_
 {
     const uint64_t i = globalThread();
     if (i < SC_COUNT)
-        sc[i] = 0;
+        sc[i] = i == SC_STAMP ? wall_clock64() : 0;
     for (uint64_t b = i; b < buckets; b += globalStride())
         bucketCount[b] = 0;
     for (uint64_t w = i; w < words; w += globalStride())
@@ -96,8 +97,9 @@ __device__ __forceinline__ void propagateTop(uint32_t* count, const LevelOffsets
 }
 
 static __global__ __launch_bounds__(TOP_THREADS) void kPropagateTop(uint32_t* count, LevelOffsets lo, uint32_t lc,
-                                                             uint32_t chunkingGrid)
+                                                             uint32_t chunkingGrid, uint64_t* stamp)
 {
+    stampStart(stamp);
     propagateTop(count, lo, lc, chunkingGrid);
 }
 

@@ -729,8 +729,9 @@ inline unsigned gatherGrid(uint32_t n)
 template <typename T>
 static __global__ __launch_bounds__(BLOCK) void kGatherSorted(const SortedPoint<T>* __restrict__ bucketed,
                                                         const uint32_t* __restrict__ perm, uint32_t n,
-                                                        SortedPoint<T>* __restrict__ sorted)
+                                                        SortedPoint<T>* __restrict__ sorted, uint64_t* stamp)
 {
+    stampStart(stamp);
     const uint32_t perXcd = gridDim.x / XCD_COUNT;
     const uint64_t tile   = static_cast<uint64_t>(blockIdx.x % XCD_COUNT) * perXcd + blockIdx.x / XCD_COUNT;
     const uint64_t base   = tile * GATHER_TILE + threadIdx.x;

@@ -456,9 +456,10 @@ static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrder(const uint
                                                                 const uint32_t* __restrict__ sortedStart,
                                                                 const SortedPoint<T>* __restrict__ bucketed,
                                                                 const uint32_t* __restrict__ perm,
-                                                                SortedPoint<T>* __restrict__ out)
+                                                                SortedPoint<T>* __restrict__ out, uint64_t* stamp)
 {
     __shared__ LeafOrderLds lds;
+    stampStart(stamp);
     if (blockIdx.x >= *totals >> 32)
         return;  // the whole workgroup: the grid is an upper bound
     leafCellOrderChunk<T>(chunkList[blockIdx.x], leafOrderView(p), nodeKey, parent, count, sortedStart, bucketed, perm,
@@ -580,8 +581,9 @@ static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, Su
                                                         const uint32_t* __restrict__ segTile,
                                                         const uint64_t* __restrict__ segTotal,
                                                         uint32_t* __restrict__ tileList, uint64_t words,
-                                                        uint32_t* __restrict__ bitmap)
+                                                        uint32_t* __restrict__ bitmap, uint64_t* stamp)
 {
+    stampStart(stamp);
     for (uint64_t k = globalThread(); k < nodes; k += globalStride())
         nodeGrid[k] = nodeGridOf(internal[k], nodeKey[internal[k]], sp.levelOffset, sp.levelGrid, sp.level, sp.depth,
                                  sp.cubicMin, sp.sideHalf, sp.side, sp.g, sp.seed);
@@ -611,6 +613,16 @@ struct TileRange
     const uint32_t* hi;
     __device__ __forceinline__ uint32_t first() const { return lo ? *lo : 0u; }
     __device__ __forceinline__ uint32_t count() const { return *hi - first(); }
+};
+
+// Clock stamps of a subsampling step, then one after the last step.
+enum StepStamp : uint32_t
+{
+    ST_BEGIN,
+    ST_INSERT_BEGIN,
+    ST_INSERT_END,
+    ST_EMIT_BEGIN,
+    ST_STAMPS
 };
 
 // One step of the subsampling (a batch of a level's nodes), with the sizes that only the device
@@ -699,8 +711,9 @@ static __global__ __launch_bounds__(TILE) void kMark(TileRange range, uint32_t n
                                                const uint32_t* __restrict__ segInput,
                                                const NodeGrid* __restrict__ nodeGrid, PointStore<T> ps,
                                                uint32_t* __restrict__ bitmap, uint32_t* __restrict__ cellOf,
-                                               uint32_t* __restrict__ err)
+                                               uint32_t* __restrict__ err, uint64_t* stamp)
 {
+    stampStart(stamp);
     // consecutive tiles share bitmap words: runs of them per XCD
     const uint32_t t = xcdRunItem(blockIdx.x, XCD_TILE_RUN);
     if (t >= range.count())
@@ -1005,8 +1018,9 @@ static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, 
                                                          const uint32_t* __restrict__ cellStart,
                                                          const uint32_t* __restrict__ cellOf, PointStore<T> ps,
                                                          WeightPayload* __restrict__ payload,
-                                                         uint64_t* __restrict__ winKey)
+                                                         uint64_t* __restrict__ winKey, uint64_t* stamp)
 {
+    stampStart(stamp);
     if (!step.fits())
         return;
     // consecutive tiles store to neighbouring payload slots: runs of them per XCD
@@ -1107,8 +1121,10 @@ static __global__ __launch_bounds__(BLOCK) void kEmit(StepSizes step, uint32_t n
                                                 const uint32_t* __restrict__ cellKey,
                                                 const uint32_t* __restrict__ cellNode,
                                                 const uint64_t* __restrict__ win, const uint64_t* __restrict__ color,
-                                                PointStore<T> ps)
+                                                PointStore<T> ps, uint64_t* insertEnd, uint64_t* stamp)
 {
+    stampStart(insertEnd);
+    stampStart(stamp);
     if (!step.fits())
         return;
     const uint32_t cells = *step.cells, cursor = static_cast<uint32_t>(*step.cursor);
@@ -1282,8 +1298,10 @@ static __global__ __launch_bounds__(BLOCK) void kEmitWeighted(StepSizes step, ui
                                                         const uint32_t* __restrict__ cellNode,
                                                         const uint32_t* __restrict__ cellStart,
                                                         const WeightPayload* __restrict__ payload,
-                                                        const uint64_t* __restrict__ winKey, PointStore<T> ps)
+                                                        const uint64_t* __restrict__ winKey, PointStore<T> ps,
+                                                        uint64_t* stamp)
 {
+    stampStart(stamp);
     if (!step.fits())
         return;
     // each XCD takes runs of EMIT_CHUNK consecutive cell blocks
@@ -1322,8 +1340,10 @@ static __global__ __launch_bounds__(64) void kPlaceNodes(const uint32_t* __restr
                                                    const int32_t* __restrict__ parent,
                                                    const int32_t* __restrict__ children,
                                                    const uint32_t* __restrict__ pointCount,
-                                                   const uint32_t* __restrict__ subtree, uint64_t* __restrict__ dataIdx)
+                                                   const uint32_t* __restrict__ subtree, uint64_t* __restrict__ dataIdx,
+                                                   uint64_t* stamp)
 {
+    stampStart(stamp);
     for (uint64_t j = globalThread(); j < nodes; j += globalStride())
     {
         const uint32_t id = list[j];

@@ -22,12 +22,9 @@ namespace oc {
 
 namespace {
 
-// Records are read straight from their places, 64 consecutive ones per load instruction. The pass is
-// bound by HBM (119.7M 27-byte records: 5.0 TB/s of their lines with one record in flight per thread
-// and half of the wave slots, see BB_ITEMS); a small cloud by the launch.
+// Bound by HBM (119.7M 27-byte records: 5.3 TB/s of their lines), a small cloud by the launch.
 constexpr int BB_THREADS = 512;
 constexpr int BB_BLOCKS  = 1024;
-constexpr int BB_ITEMS   = 4;  // records in flight per thread
 
 __device__ __forceinline__ void waveMinMax(double v[6])
 {
@@ -91,24 +88,8 @@ __global__ __launch_bounds__(BB_THREADS) void kBounds(const uint8_t* __restrict_
                                                       BoundsScratch* scratch, uint64_t* box, uint64_t seq)
 {
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    const uint64_t step = globalStride();
-    uint64_t i          = globalThread();
-    for (; i + (BB_ITEMS - 1) * step < n; i += BB_ITEMS * step)
-    {
-        double x[BB_ITEMS], y[BB_ITEMS], z[BB_ITEMS];
-#pragma unroll
-        for (int k = 0; k < BB_ITEMS; ++k)
-            loadXYZ<T>(cloud + (i + k * step) * stride, x[k], y[k], z[k]);
-#pragma unroll
-        for (int k = 0; k < BB_ITEMS; ++k)
-            include(v, x[k], y[k], z[k]);
-    }
-    for (; i < n; i += step)
-    {
-        double x, y, z;
-        loadXYZ<T>(cloud + i * stride, x, y, z);
-        include(v, x, y, z);
-    }
+    __shared__ RecordStage stages[BB_THREADS / 64];
+    forRecords<T, BB_THREADS>(cloud, n, stride, stages, [&v](double x, double y, double z) { include(v, x, y, z); });
     blockMinMax(v);
     __shared__ bool last;
     if (threadIdx.x == 0)

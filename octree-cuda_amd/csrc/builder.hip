@@ -498,7 +498,8 @@ void OctreeBuilder::countPoints()
             sc, bucketCount, nb + 1, occ, marked / 32, itsCount.as<uint32_t>(), marked, itsDense);
     OC_LAUNCH_CHECK();
 
-    const unsigned histBlocks = static_cast<unsigned>(std::min<uint64_t>(2048, (n + 8191) / 8192));
+    // four rounds of records or more per workgroup; at most twice the resident ones
+    const unsigned histBlocks = static_cast<unsigned>(std::min<uint64_t>(2048, (static_cast<uint64_t>(n) + 2047) / 2048));
     kBucketHist<T><<<histBlocks, HIST_THREADS, 0, itsStream>>>(itsCloudDevice, n, itsCloud.dataStride, g,
                                                                3 * itsCoarse, nb, bucketCount,
                                                                reinterpret_cast<uint32_t*>(sc + SC_ERROR));

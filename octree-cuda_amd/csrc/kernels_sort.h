@@ -135,18 +135,15 @@ static __global__ __launch_bounds__(HIST_THREADS) void kBucketHist(const uint8_t
         h[b] = 0;
     __syncthreads();
     bool outside = false;
-    for (uint64_t i = globalThread(); i < n; i += globalStride())
-    {
-        double x, y, z;
-        loadXYZ<T>(cloud + i * stride, x, y, z);
+    auto take    = [&](double x, double y, double z) {
         const uint32_t m = pointMorton(x, y, z, g);
         if (m == ~0u)
-        {
             outside = true;
-            continue;
-        }
-        atomicAdd(h + (m >> fineBits), 1u);
-    }
+        else
+            atomicAdd(h + (m >> fineBits), 1u);
+    };
+    __shared__ RecordStage stages[HIST_THREADS / 64];
+    forRecords<T, HIST_THREADS>(cloud, n, stride, stages, take);
     if (outside)
         atomicOr(err, ERR_OUTSIDE);
     __syncthreads();

@@ -816,6 +816,7 @@ void OctreeBuilder::subsampleLevels()
     itsTileList.ensure(sizeof(uint32_t) * tileMost);
     itsBitmap.ensure(sizeof(uint32_t) * wordMost);
     itsPrefix.ensure(sizeof(uint32_t) * (wordMost + 1));
+    itsScanScratch.ensure(sizeof(uint64_t) * SCAN_GRID + sizeof(uint32_t) * scanTiles(wordMost));  // range, tile sums
     itsCellOf.ensure(sizeof(uint32_t) * N);
     itsCellKey.ensure(sizeof(uint32_t) * N);
     itsCellNode.ensure(sizeof(uint32_t) * N);
@@ -892,12 +893,24 @@ void OctreeBuilder::subsampleLevels()
             // per-cell state, reset for the occupied cells: by the scan itself on small levels, else
             // by kClearCompact
             const bool clearInScan = words <= CLEAR_IN_SCAN_WORDS;
-            if (clearInScan)
-                scanExclusive<uint32_t>(words, PopcountIn{bitmap}, PrefixClearOut{prefix, win, color, cellCnt},
-                                        itsScanScratch.as<uint32_t>(), prefix + words, itsStream);
+            const PrefixClearOut clearing{prefix, win, color, cellCnt};
+            const uint64_t wordTiles = scanTiles(words);
+            uint32_t* rangeSums      = itsScanScratch.as<uint32_t>();
+            if (wordTiles <= SCAN_DIRECT_TILES)
+                scanExclusive<uint32_t>(words, PopcountIn{bitmap}, clearing, rangeSums, prefix + words, itsStream);
             else
-                scanExclusive<uint32_t>(words, PopcountIn{bitmap}, ExclusiveToArray{prefix},
-                                        itsScanScratch.as<uint32_t>(), prefix + words, itsStream);
+            {
+                const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(wordTiles, SCAN_GRID));
+                uint32_t* tileSums  = rangeSums + 2 * SCAN_GRID;
+                kWordReduce<<<grid, SCAN_THREADS, 0, itsStream>>>(bitmap, words, tileSums, rangeSums);
+                if (clearInScan)
+                    kWordPrefix<<<grid, SCAN_THREADS, 0, itsStream>>>(bitmap, words, wordsPerNode, clearing, tileSums,
+                                                                      rangeSums, prefix);
+                else
+                    kWordPrefix<<<grid, SCAN_THREADS, 0, itsStream>>>(bitmap, words, wordsPerNode,
+                                                                      ExclusiveToArray{prefix}, tileSums, rangeSums,
+                                                                      prefix);
+            }
             OC_LAUNCH_CHECK();
             if (!clearInScan)
             {

@@ -763,6 +763,68 @@ static __global__ __launch_bounds__(BLOCK) void kClearCompact(const uint32_t* __
     }
 }
 
+// Large levels, the popcount scan's first pass: occupied cells per tile of SCAN_TILE words and per
+// workgroup's range of tiles.
+static __global__ __launch_bounds__(SCAN_THREADS) void kWordReduce(const uint32_t* __restrict__ bitmap, uint64_t words,
+                                                            uint32_t* __restrict__ tileSums,
+                                                            uint32_t* __restrict__ rangeSums)
+{
+    __shared__ uint32_t lds[SCAN_WAVES];
+    uint64_t first, last;
+    tileRange(scanTiles(words), first, last);
+    uint32_t range = 0;
+    for (uint64_t tile = first; tile < last; ++tile)
+    {
+        uint32_t v[SCAN_ITEMS], s = 0;
+        loadTile<uint32_t>(PopcountIn{bitmap}, tile * SCAN_TILE, words, v);
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; ++k)
+            s += v[k];
+        const uint32_t sum = __syncthreads_or(s != 0) ? blockSum(s, lds) : 0u;
+        if (threadIdx.x == 0)
+            tileSums[tile] = sum;
+        range += sum;
+    }
+    if (threadIdx.x == 0)
+        rangeSums[blockIdx.x] = range;
+}
+
+// Second pass: the prefix of every word in the tiles that hold any occupied cell, and of every node's
+// first word (no other is read). The nodes' cells lie on surfaces, so most tiles (a slab of four cell
+// layers of a 128^3 grid) are empty: neither read nor written here.
+template <typename Out>
+static __global__ __launch_bounds__(SCAN_THREADS) void kWordPrefix(const uint32_t* __restrict__ bitmap, uint64_t words,
+                                                            uint64_t wordsPerNode, Out out,
+                                                            const uint32_t* __restrict__ tileSums,
+                                                            const uint32_t* __restrict__ rangeSums,
+                                                            uint32_t* __restrict__ prefix)
+{
+    __shared__ uint32_t lds[SCAN_ITEMS * SCAN_WAVES];
+    uint64_t first, last;
+    tileRange(scanTiles(words), first, last);
+    uint32_t carry = sumBefore(rangeSums, lds);
+    for (uint64_t tile = first; tile < last; ++tile)
+    {
+        const uint64_t base = tile * SCAN_TILE;
+        const uint32_t sum  = tileSums[tile];
+        if (sum == 0)
+        {
+            const uint64_t end = base + SCAN_TILE < words ? base + SCAN_TILE : words;
+            for (uint64_t w = ((base + wordsPerNode - 1) / wordsPerNode + threadIdx.x) * wordsPerNode; w < end;
+                 w += SCAN_THREADS * wordsPerNode)
+                prefix[w] = carry;
+            continue;
+        }
+        uint32_t v[SCAN_ITEMS], pre[SCAN_ITEMS];
+        loadTile<uint32_t>(PopcountIn{bitmap}, base, words, v);
+        (void)tileExclusiveScan(v, pre, lds);
+        storeTile<uint32_t>(out, base, words, v, pre, carry);
+        carry += sum;
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+        prefix[words] = carry;
+}
+
 // Output of the popcount scan for small levels (one launch less than a separate clear; on large
 // levels the per-word loops cost more than kClearCompact): the word's prefix, and the per-cell
 // state of the word's occupied

@@ -524,10 +524,9 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
         OC_LAUNCH_CHECK();
     }
     mark(1);
-    kPropagateTopB<T><<<B0, TOP_THREADS, 0, s>>>(ctx, L);
     const uint64_t words = (static_cast<uint64_t>(L.dense) + 31) / 32;
     const dim3 wordGrid(scanWidth(words), B0);
-    kScanReduceB<uint32_t><<<wordGrid, SCAN_THREADS, 0, s>>>(OccupancyJob<T>{ctx, L.marked, L.dense});
+    kOccupancyB<T><<<wordGrid, SCAN_THREADS, 0, s>>>(ctx, L);
     kOccupiedIdsB<T><<<wordGrid, SCAN_THREADS, 0, s>>>(ctx, L);
     OC_LAUNCH_CHECK();
     };

@@ -108,9 +108,9 @@ size_t DeviceBuffer::peakAllocated()
 // Bytes of bitmap + prefix the nodes of one subsampling batch may use.
 static constexpr uint64_t kBitmapBudget = 6ull << 30;
 
-// Bitmap words up to which the popcount scan also resets the cells (a launch less; its threads walk
-// the cells of their words, which costs more than a pass of its own on large levels).
-static constexpr uint64_t CLEAR_IN_SCAN_WORDS = 1u << 20;
+// Bitmap words up to which a level's cells are reset with its bitmap, one per input (a launch less; on
+// larger levels there are many more inputs than cells).
+static constexpr uint64_t RESET_INPUTS_WORDS = 1u << 20;
 
 // words of the host mailbox
 enum MailSlot
@@ -498,8 +498,11 @@ void OctreeBuilder::countPoints()
             sc, bucketCount, nb + 1, occ, marked / 32, itsCount.as<uint32_t>(), marked, itsDense);
     OC_LAUNCH_CHECK();
 
-    // four rounds of records or more per workgroup; at most twice the resident ones
-    const unsigned histBlocks = static_cast<unsigned>(std::min<uint64_t>(2048, (static_cast<uint64_t>(n) + 2047) / 2048));
+    // four rounds of records per workgroup until the chip is full, then sixteen: every workgroup adds its
+    // histogram to the global one at the end (5.1M points: 35 us, with four rounds 49)
+    const unsigned histBlocks = static_cast<unsigned>(std::min<uint64_t>(
+            2048, std::max<uint64_t>((static_cast<uint64_t>(n) + 8191) / 8192,
+                                     std::min<uint64_t>(COMPUTE_UNITS, (static_cast<uint64_t>(n) + 2047) / 2048))));
     kBucketHist<T><<<histBlocks, HIST_THREADS, 0, itsStream>>>(itsCloudDevice, n, itsCloud.dataStride, g,
                                                                3 * itsCoarse, nb, bucketCount,
                                                                reinterpret_cast<uint32_t*>(sc + SC_ERROR));
@@ -578,12 +581,8 @@ void OctreeBuilder::mergeLevels()
     for (uint32_t l = 0; l <= itsDepth; ++l)
         lo.offset[l] = itsLevelOffset[l];
     lo.levels = itsDepth + 1;
-    // levels 0..coarse come from the fine sort
-    kPropagateTop<<<1, TOP_THREADS, 0, itsStream>>>(count, lo, itsCoarse, itsProc.chunkingGrid,
-                                                      sc + SC_STAMP + 1);
-    OC_LAUNCH_CHECK();
-
-    // occupancy bits of the levels the fine sort has not marked, sparse ids (A2) + node keys / counts
+    // levels 0..coarse come from the fine sort: the counts of the levels above, the occupancy bits of the
+    // levels the fine sort has not marked, sparse ids (A2) + node keys / counts
     // + first id of every level by a scan over the bitmap's words, and the list of internal nodes
     uint32_t* occ         = itsOccupancy.as<uint32_t>();
     const uint64_t marked = fineSortBits() ? itsLevelOffset[BIT_LEVELS] / 32 : 0;
@@ -601,8 +600,8 @@ void OctreeBuilder::mergeLevels()
     itsScanScratch.ensure(sizeof(uint64_t) * SCAN_GRID);
     uint32_t* sums = itsScanScratch.as<uint32_t>();
     const unsigned wordGrid = static_cast<unsigned>(std::min<uint64_t>(scanTiles(words), SCAN_GRID));
-    kScanReduce<uint32_t><<<wordGrid, SCAN_THREADS, 0, itsStream>>>(OccupancyIn{occ, count, marked, itsDense},
-                                                                    HostCount{words}, sums);
+    kOccupancy<<<wordGrid, SCAN_THREADS, 0, itsStream>>>(occ, count, marked, itsDense, lo, itsCoarse,
+                                                         itsProc.chunkingGrid, sums, sc + SC_STAMP + 1);
     OC_LAUNCH_CHECK();
     const IdTables ids{occ, count, itsDenseToSparse.as<int32_t>(), itsNodeKey.as<uint32_t>(),
                        itsNodeCount.as<uint32_t>(), levelStart, lo};
@@ -838,6 +837,7 @@ void OctreeBuilder::subsampleLevels()
     uint32_t* cellCnt = weighted ? itsCellCnt.as<uint32_t>() : nullptr;
     uint32_t* bitmap  = itsBitmap.as<uint32_t>();
     uint32_t* prefix  = itsPrefix.as<uint32_t>();
+    const CellState cellState{win, color, cellCnt};
 
     uint32_t stepAt = 0;
     for (uint32_t l = 1; l <= itsDepth; ++l)
@@ -881,40 +881,34 @@ void OctreeBuilder::subsampleLevels()
             uint64_t* stamps = itsStamps.as<uint64_t>() + ST_STAMPS * stepAt;
             ++stepAt;
 
+            const bool resetInputs = words <= RESET_INPUTS_WORDS;
             kLevelPrepare<<<gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384), BLOCK, 0, itsStream>>>(
                     K, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
-                    sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, stamps + ST_BEGIN);
+                    sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs,
+                    stamps + ST_BEGIN);
             OC_LAUNCH_CHECK();
             kMark<T><<<tileGrid, TILE, 0, itsStream>>>(
                     tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                     itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid, ps,
                     bitmap, itsCellOf.as<uint32_t>(), err, stamps + ST_INSERT_BEGIN);
             OC_LAUNCH_CHECK();
-            // per-cell state, reset for the occupied cells: by the scan itself on small levels, else
-            // by kClearCompact
-            const bool clearInScan = words <= CLEAR_IN_SCAN_WORDS;
-            const PrefixClearOut clearing{prefix, win, color, cellCnt};
             const uint64_t wordTiles = scanTiles(words);
             uint32_t* rangeSums      = itsScanScratch.as<uint32_t>();
             if (wordTiles <= SCAN_DIRECT_TILES)
-                scanExclusive<uint32_t>(words, PopcountIn{bitmap}, clearing, rangeSums, prefix + words, itsStream);
+                scanExclusive<uint32_t>(words, PopcountIn{bitmap}, ExclusiveToArray{prefix}, rangeSums, prefix + words,
+                                        itsStream);
             else
             {
                 const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(wordTiles, SCAN_GRID));
                 uint32_t* tileSums  = rangeSums + 2 * SCAN_GRID;
                 kWordReduce<<<grid, SCAN_THREADS, 0, itsStream>>>(bitmap, words, tileSums, rangeSums);
-                if (clearInScan)
-                    kWordPrefix<<<grid, SCAN_THREADS, 0, itsStream>>>(bitmap, words, wordsPerNode, clearing, tileSums,
-                                                                      rangeSums, prefix);
-                else
-                    kWordPrefix<<<grid, SCAN_THREADS, 0, itsStream>>>(bitmap, words, wordsPerNode,
-                                                                      ExclusiveToArray{prefix}, tileSums, rangeSums,
-                                                                      prefix);
+                kWordPrefix<<<grid, SCAN_THREADS, 0, itsStream>>>(bitmap, words, wordsPerNode, tileSums, rangeSums,
+                                                                  prefix);
             }
             OC_LAUNCH_CHECK();
-            if (!clearInScan)
+            if (!resetInputs)
             {
-                kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(prefix + words, win, color, cellCnt);
+                kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(step.cells, cellState);
                 OC_LAUNCH_CHECK();
             }
 

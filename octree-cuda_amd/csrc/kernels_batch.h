@@ -310,20 +310,6 @@ __device__ __forceinline__ BoundScan<In, Out> bound(In in, Out out, uint64_t n, 
     return BoundScan<In, Out>{in, out, n, sums, total, total32};
 }
 
-// occupancy bits and their number per range of words, for the canonical sparse ids (kOccupiedIdsB)
-template <typename T>
-struct OccupancyJob
-{
-    const BatchCloud<T>* ctx;
-    uint64_t marked, dense;
-    __device__ auto bind(uint32_t c) const
-    {
-        const BatchCloud<T>& cc = ctx[c];
-        const OccupancyIn in{cc.occ, cc.count, marked / 32, dense};
-        return bound(in, 0, (dense + 31) / 32, cc.scanSums, cc.sc + BS_M);
-    }
-};
-
 // leaf data blocks (A4): scan of the block sizes in id order
 template <typename T>
 struct LeafBlockJob
@@ -648,14 +634,21 @@ __device__ __forceinline__ LevelOffsets levelOffsets(const BatchLevels& L)
     return lo;
 }
 
-// the levels above the bucket level, a workgroup per cloud
+// canonical sparse ids over the occupancy bitmap (A2), first pass: grid (scanWidth, B)
 template <typename T>
-static __global__ __launch_bounds__(TOP_THREADS) void kPropagateTopB(const BatchCloud<T>* __restrict__ ctx, BatchLevels L)
+static __global__ __launch_bounds__(SCAN_THREADS) void kOccupancyB(const BatchCloud<T>* __restrict__ ctx, BatchLevels L)
 {
-    propagateTop(ctx[blockIdx.x].count, levelOffsets(L), L.lc, L.grid[0]);
+    __shared__ uint32_t lds[SCAN_WAVES];
+    const BatchCloud<T>& cc = ctx[blockIdx.y];
+    uint64_t first, last;
+    tileRange(scanTiles((static_cast<uint64_t>(L.dense) + 31) / 32), first, last);
+    const uint32_t bits = occupancyTiles(cc.occ, cc.count, L.marked / 32, L.dense, levelOffsets(L), L.lc, L.grid[0],
+                                         first, last, lds);
+    if (threadIdx.x == 0)
+        reinterpret_cast<uint32_t*>(cc.scanSums)[blockIdx.x] = bits;
 }
 
-// canonical sparse ids over the occupancy bitmap (A2), second pass: grid (scanWidth, B)
+// second pass, the same grid
 template <typename T>
 static __global__ __launch_bounds__(SCAN_THREADS) void kOccupiedIdsB(const BatchCloud<T>* __restrict__ ctx, BatchLevels L)
 {

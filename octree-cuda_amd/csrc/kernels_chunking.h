@@ -81,59 +81,91 @@ struct LevelOffsets
     uint32_t levels;
 };
 
-// The levels above the bucket level, at most 8^3 + 4^3 + 2^3 + 1 cells: one workgroup, one launch.
-constexpr int TOP_THREADS = 512;
-
+// The levels above the bucket level, at most 8^3 + 4^3 + 2^3 + 1 cells: one workgroup.
 __device__ __forceinline__ void propagateTop(uint32_t* count, const LevelOffsets& lo, uint32_t lc,
                                              uint32_t chunkingGrid)
 {
     for (uint32_t l = lc + 1; l < lo.levels; ++l)
     {
         const uint32_t grid = chunkingGrid >> l;
-        for (uint32_t i = threadIdx.x; i < grid * grid * grid; i += TOP_THREADS)
+        for (uint32_t i = threadIdx.x; i < grid * grid * grid; i += blockDim.x)
             propagateOne(i, count, lo.offset[l], grid, lo.offset[l - 1], 2 * grid);
         __syncthreads();
     }
 }
 
-static __global__ __launch_bounds__(TOP_THREADS) void kPropagateTop(uint32_t* count, LevelOffsets lo, uint32_t lc,
-                                                             uint32_t chunkingGrid, uint64_t* stamp)
+// Occupancy bitmap (bit d: dense cell d holds points) of the 32 cells of word w, from their counts.
+__device__ __forceinline__ uint32_t occupancyWord(const uint32_t* count, uint64_t w, uint64_t dense)
 {
-    stampStart(stamp);
-    propagateTop(count, lo, lc, chunkingGrid);
+    uint32_t bits    = 0;
+    const uint64_t d = 32 * w;
+    if (d + 32 <= dense)
+    {
+        const uint4* c = reinterpret_cast<const uint4*>(count + d);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            const uint4 v = c[k];
+            bits |= ((v.x ? 1u : 0u) | (v.y ? 2u : 0u) | (v.z ? 4u : 0u) | (v.w ? 8u : 0u)) << (4 * k);
+        }
+    }
+    else
+        for (uint32_t k = 0; d + k < dense; ++k)
+            bits |= (count[d + k] ? 1u : 0u) << k;
+    return bits;
 }
 
-// Occupancy bitmap (bit d: dense cell d holds points), one scan item per word: the words of the
-// levels that the fine sort has marked as they are, the others made from their counts and stored.
-struct OccupancyIn
+// First pass of the id scan over the tiles [first, last) of the bitmap's words: the words from `marked`
+// on are made from their counts (the fine sort has marked the ones before), and the number of set bits
+// comes back in thread 0. All threads. The workgroups with words of the levels above the bucket level,
+// the last few words of all, first sum up those levels (twice if two workgroups share them: the same
+// values).
+__device__ __forceinline__ uint32_t occupancyTiles(uint32_t* occ, uint32_t* count, uint64_t marked, uint64_t dense,
+                                                   const LevelOffsets& lo, uint32_t lc, uint32_t chunkingGrid,
+                                                   uint64_t first, uint64_t last, uint32_t* lds)
 {
-    uint32_t* occ;
-    const uint32_t* count;
-    uint64_t marked;  // words
-    uint64_t dense;   // cells
-    __device__ uint32_t operator()(uint64_t w) const
+    const uint64_t words = (dense + 31) / 32;
+    if (lc + 1 < lo.levels && first < last && last * SCAN_TILE > lo.offset[lc + 1] / 32)
+        propagateTop(count, lo, lc, chunkingGrid);
+    uint32_t bits = 0;
+    for (uint64_t tile = first; tile < last; ++tile)
     {
-        if (w < marked)
-            return __popc(occ[w]);
-        uint32_t bits    = 0;
-        const uint64_t d = 32 * w;
-        if (d + 32 <= dense)
+        const uint64_t base = tile * SCAN_TILE;
+        if (base + SCAN_TILE <= marked)
         {
-            const uint4* c = reinterpret_cast<const uint4*>(count + d);
+            uint32_t v[SCAN_ITEMS];
+            loadTile<uint32_t>([occ](uint64_t w) { return occ[w]; }, base, words, v);
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-            {
-                const uint4 v = c[k];
-                bits |= ((v.x ? 1u : 0u) | (v.y ? 2u : 0u) | (v.z ? 4u : 0u) | (v.w ? 8u : 0u)) << (4 * k);
-            }
+            for (int k = 0; k < SCAN_ITEMS; ++k)
+                bits += __popc(v[k]);
         }
         else
-            for (uint32_t k = 0; k < dense - d; ++k)
-                bits |= (count[d + k] ? 1u : 0u) << k;
-        occ[w] = bits;
-        return __popc(bits);
+            for (uint64_t w = base + threadIdx.x; w < base + SCAN_TILE && w < words; w += SCAN_THREADS)
+            {
+                uint32_t v;
+                if (w < marked)
+                    v = occ[w];
+                else
+                    occ[w] = v = occupancyWord(count, w, dense);
+                bits += __popc(v);
+            }
     }
-};
+    return blockSum(bits, lds);
+}
+
+static __global__ __launch_bounds__(SCAN_THREADS) void kOccupancy(uint32_t* occ, uint32_t* count, uint64_t marked,
+                                                           uint64_t dense, LevelOffsets lo, uint32_t lc,
+                                                           uint32_t chunkingGrid, uint32_t* __restrict__ sums,
+                                                           uint64_t* stamp)
+{
+    __shared__ uint32_t lds[SCAN_WAVES];
+    stampStart(stamp);
+    uint64_t first, last;
+    tileRange(scanTiles((dense + 31) / 32), first, last);
+    const uint32_t bits = occupancyTiles(occ, count, marked, dense, lo, lc, chunkingGrid, first, last, lds);
+    if (threadIdx.x == 0)
+        sums[blockIdx.x] = bits;
+}
 
 // Sparse ids (A2): the exclusive rank of an occupied dense cell; its node key and dense count are
 // written in the same pass, and the first id of every level (ids ascend with the dense index and a
@@ -151,7 +183,8 @@ struct IdTables
 };
 
 // Set bits of a tile that are listed in LDS at a time.
-constexpr uint32_t ID_LIST = 8192;
+constexpr uint32_t ID_LIST  = 8192;
+constexpr uint32_t ID_ITEMS = 8;
 
 struct IdLds
 {
@@ -200,14 +233,27 @@ __device__ __forceinline__ uint32_t occupiedIds(const IdTables& t, uint64_t word
                                                              static_cast<uint32_t>(__builtin_ctz(bits)));
             }
             __syncthreads();
+            // a terrain's cells fill a few tiles: several counts in flight per thread
             const uint32_t n = ids - base < ID_LIST ? ids - base : ID_LIST;
-            for (uint32_t j = threadIdx.x; j < n; j += SCAN_THREADS)
+            for (uint32_t j0 = threadIdx.x; j0 < n; j0 += ID_ITEMS * SCAN_THREADS)
             {
-                const uint64_t d      = cell + lds.list[j];
-                const uint32_t id     = carry + base + j;
-                t.nodeKey[id]         = static_cast<uint32_t>(d);
-                t.nodeCount[id]       = t.count[d];
-                t.denseToSparse[d]    = static_cast<int32_t>(id);
+                uint32_t d[ID_ITEMS], c[ID_ITEMS];
+#pragma unroll
+                for (uint32_t k = 0; k < ID_ITEMS; ++k)
+                {
+                    const uint32_t j = j0 + k * SCAN_THREADS;
+                    d[k]             = static_cast<uint32_t>(cell) + lds.list[j < n ? j : j0];
+                    c[k]             = t.count[d[k]];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < ID_ITEMS; ++k)
+                    if (const uint32_t j = j0 + k * SCAN_THREADS; j < n)
+                    {
+                        const uint32_t id     = carry + base + j;
+                        t.nodeKey[id]         = d[k];
+                        t.nodeCount[id]       = c[k];
+                        t.denseToSparse[d[k]] = static_cast<int32_t>(id);
+                    }
             }
             __syncthreads();
         }

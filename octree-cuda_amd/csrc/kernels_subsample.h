@@ -571,9 +571,28 @@ struct LevelSegmentOut
     }
 };
 
+// Per-cell state of the accumulation, by dense index: no winner, no colour sum, no points. Arrays that
+// the colour mode does not use are null.
+struct CellState
+{
+    uint64_t* win;
+    uint64_t* color;
+    uint32_t* cellCnt;
+    __device__ __forceinline__ void reset(uint64_t c) const
+    {
+        if (win)
+            win[c] = ~0ull;
+        if (color)
+            color[c] = 0;
+        if (cellCnt)
+            cellCnt[c] = 0;
+    }
+};
+
 // Before a level's first pass: the griddings of its nodes, the segment of every tile (a search per
 // tile, all of them in flight; a thread per segment wrote a large child's thousands of entries by
-// itself, 71 us of a 5.1M-point build) and a clear bitmap.
+// itself, 71 us of a 5.1M-point build) and a clear bitmap. For a small level also the state of as many
+// cells as it has inputs (it has no more), which spares it kClearCompact.
 static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, SubsampleParams sp,
                                                         const uint32_t* __restrict__ internal,
                                                         const uint32_t* __restrict__ nodeKey,
@@ -581,7 +600,8 @@ static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, Su
                                                         const uint32_t* __restrict__ segTile,
                                                         const uint64_t* __restrict__ segTotal,
                                                         uint32_t* __restrict__ tileList, uint64_t words,
-                                                        uint32_t* __restrict__ bitmap, uint64_t* stamp)
+                                                        uint32_t* __restrict__ bitmap, CellState cells, bool reset,
+                                                        uint64_t* stamp)
 {
     stampStart(stamp);
     for (uint64_t k = globalThread(); k < nodes; k += globalStride())
@@ -604,6 +624,12 @@ static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, Su
     }
     for (uint64_t w = globalThread(); w < words; w += globalStride())
         bitmap[w] = 0;
+    if (reset)
+    {
+        const uint32_t inputs = static_cast<uint32_t>(*segTotal);
+        for (uint64_t c = globalThread(); c < inputs; c += globalStride())
+            cells.reset(c);
+    }
 }
 
 // The tiles of a batch of a level's nodes: from *lo (null: 0) to *hi.
@@ -747,20 +773,12 @@ __device__ __forceinline__ void batchNodeOf(uint64_t kl, uint32_t nodeBase, uint
     stage[id]      = cursor + b;
 }
 
-// (n: the step's occupied cells, on the device)
-static __global__ __launch_bounds__(BLOCK) void kClearCompact(const uint32_t* __restrict__ n, uint64_t* __restrict__ win,
-                                                        uint64_t* __restrict__ color, uint32_t* __restrict__ cellCnt)
+// the state of a large level's cells (n: how many, on the device)
+static __global__ __launch_bounds__(BLOCK) void kClearCompact(const uint32_t* __restrict__ n, CellState cells)
 {
-    const uint64_t cells = *n;
-    for (uint64_t i = globalThread(); i < cells; i += globalStride())
-    {
-        if (win)
-            win[i] = ~0ull;
-        if (color)
-            color[i] = 0;
-        if (cellCnt)
-            cellCnt[i] = 0;
-    }
+    const uint64_t count = *n;
+    for (uint64_t c = globalThread(); c < count; c += globalStride())
+        cells.reset(c);
 }
 
 // Large levels, the popcount scan's first pass: occupied cells per tile of SCAN_TILE words and per
@@ -792,9 +810,8 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kWordReduce(const uint32_
 // Second pass: the prefix of every word in the tiles that hold any occupied cell, and of every node's
 // first word (no other is read). The nodes' cells lie on surfaces, so most tiles (a slab of four cell
 // layers of a 128^3 grid) are empty: neither read nor written here.
-template <typename Out>
 static __global__ __launch_bounds__(SCAN_THREADS) void kWordPrefix(const uint32_t* __restrict__ bitmap, uint64_t words,
-                                                            uint64_t wordsPerNode, Out out,
+                                                            uint64_t wordsPerNode,
                                                             const uint32_t* __restrict__ tileSums,
                                                             const uint32_t* __restrict__ rangeSums,
                                                             uint32_t* __restrict__ prefix)
@@ -818,38 +835,12 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kWordPrefix(const uint32_
         uint32_t v[SCAN_ITEMS], pre[SCAN_ITEMS];
         loadTile<uint32_t>(PopcountIn{bitmap}, base, words, v);
         (void)tileExclusiveScan(v, pre, lds);
-        storeTile<uint32_t>(out, base, words, v, pre, carry);
+        storeTile<uint32_t>(ExclusiveToArray{prefix}, base, words, v, pre, carry);
         carry += sum;
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
         prefix[words] = carry;
 }
-
-// Output of the popcount scan for small levels (one launch less than a separate clear; on large
-// levels the per-word loops cost more than kClearCompact): the word's prefix, and the per-cell
-// state of the word's occupied
-// cells (dense indices prefix .. prefix + popcount - 1) reset for the accumulation: no winner,
-// no colour sum, no points. Arrays that the colour mode does not use are null.
-struct PrefixClearOut
-{
-    uint32_t* prefix;
-    uint64_t* win;
-    uint64_t* color;
-    uint32_t* cellCnt;
-    __device__ void operator()(uint64_t w, uint32_t p, uint32_t cells) const
-    {
-        prefix[w] = p;
-        for (uint32_t k = 0; k < cells; ++k)
-        {
-            if (win)
-                win[p + k] = ~0ull;
-            if (color)
-                color[p + k] = 0;
-            if (cellCnt)
-                cellCnt[p + k] = 0;
-        }
-    }
-};
 
 // Evaluate, part 2: winner (A7/A8: atomicMin of rank << 32 | input position, rank = point index
 // for the implicit method or the keyed bijective hash of it for the explicit one), the packed

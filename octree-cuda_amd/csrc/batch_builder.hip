@@ -84,7 +84,6 @@ BatchLevels levelsOf(uint32_t G)
     L.lc      = std::min<uint32_t>(MAX_COARSE_LEVEL, L.depth > 3 ? L.depth - 3 : 0);
     const uint32_t bg = G >> L.lc;
     L.buckets = bg * bg * bg;
-    L.marked  = L.lc == MAX_COARSE_LEVEL ? L.offset[BIT_LEVELS] : 0;
     return L;
 }
 
@@ -163,7 +162,7 @@ void carveCloud(Carver& cv, BatchCloud<T>& cc, const BatchRequest& r, const Clou
         cc.splitHist   = nullptr;
     }
     cv.take(cc.count, L.dense);
-    cv.take(cc.denseToSparse, L.dense);
+    cv.take(cc.idBase, (static_cast<uint64_t>(L.dense) + 31) / 32);
     cv.take(cc.occ, (static_cast<uint64_t>(L.dense) + 31) / 32);
     cv.take(cc.nodeKey, s.mBound);
     cv.take(cc.nodeCount, s.mBound);
@@ -512,14 +511,14 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
     OC_LAUNCH_CHECK();
     kBucketScatterB<T><<<LG.sortGrid, SCATTER_THREADS, 0, s>>>(ctx, B0, slot(P_SCATTER), fineBits);
     OC_LAUNCH_CHECK();
-    kFineSortB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, fp, L.buckets, L.marked != 0);
+    kFineSortB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, fp, L.buckets);
     OC_LAUNCH_CHECK();
     if (split)
     {
         kSplitChunksB<T><<<std::min<uint32_t>(B0, 1024), SCAN_THREADS, 0, s>>>(ctx, B0, L.buckets);
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(ScalarCount<T>{ctx, BS_SPLIT, false}, B0, slot(P_SPLIT));
         kFineChunkHistB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), L.lc);
-        kFineSplitScanB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), fp, L.marked != 0);
+        kFineSplitScanB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), fp);
         kFineChunkPermB<T><<<LG.sortGrid, SORT_THREADS, 0, s>>>(ctx, B0, slot(P_SPLIT), L.lc);
         OC_LAUNCH_CHECK();
     }

@@ -127,8 +127,6 @@ private:
     uint32_t planSteps();
     uint64_t leafChunkBound() const;
     uint64_t placeChunkBound() const;
-    // whether the fine sort writes the occupancy bits of the BIT_LEVELS lowest levels
-    bool fineSortBits() const;
     template <typename T>
     void distributePoints();
     template <typename T>
@@ -181,7 +179,7 @@ private:
     DeviceBuffer itsCloudOwned;
 
     // dense pyramid and sparse nodes
-    DeviceBuffer itsCount, itsDenseToSparse, itsOccupancy;  // dense counts, sparse ids, occupancy bits
+    DeviceBuffer itsCount, itsIdBase, itsOccupancy;  // dense counts, sparse ids by bitmap word, occupancy bits
     DeviceBuffer itsNodeKey, itsNodeCount, itsNodePoints, itsNodeData, itsNodeParent, itsNodeChild, itsNodeFlags,
             itsNodeSorted, itsNodeStage, itsNodeSub;
 

@@ -8,7 +8,7 @@
 //   sorted         the same records in level-0 Morton order: every node is one contiguous range;
 //                  the leaves' points are read from here by the subsampling
 //   count          D x u32 dense count pyramid; after the merge its level-0 part maps cell -> leaf
-//   denseToSparse  D x i32, set for occupied cells (non-zero dense count) only
+//   occupancy, id base  a bit per dense cell, a u32 per 32 cells: dense cell -> sparse id
 //   nodes (SoA)    key, dense count, pointCount, dataIdx (u64), parent, children[8], flags, ...
 //   output region  E records: lut (u32 point index), out (18-byte record). [0, N) holds the leaves,
 //                  [N, N + I) the subsampled points in DFS post-order
@@ -207,7 +207,7 @@ void OctreeBuilder::setup(const CloudInfo& cloud, const ProcessingInfo& proc, co
     // Fixed-size state: the dense pyramid, the node key/count arrays (bounded by min(D, levels*N))
     // and the output region.
     itsCount.ensure(sizeof(uint32_t) * static_cast<uint64_t>(itsDense));
-    itsDenseToSparse.ensure(sizeof(int32_t) * static_cast<uint64_t>(itsDense));
+    itsIdBase.ensure(sizeof(uint32_t) * ((static_cast<uint64_t>(itsDense) + 31) / 32));
     itsOccupancy.ensure(sizeof(uint32_t) * ((static_cast<uint64_t>(itsDense) + 31) / 32));
     const uint64_t mBound = nodeBound();
     // The previous build's snapshot copies may still read the node keys and counts, the LUT and
@@ -254,7 +254,7 @@ void OctreeBuilder::setup(const CloudInfo& cloud, const ProcessingInfo& proc, co
 
 std::vector<DeviceBuffer*> OctreeBuilder::arena()
 {
-    return {&itsCloudOwned,  &itsCount,       &itsDenseToSparse, &itsOccupancy,
+    return {&itsCloudOwned,  &itsCount,       &itsIdBase,       &itsOccupancy,
             &itsNodeKey,     &itsNodeCount,   &itsNodePoints,
             &itsNodeData,    &itsNodeParent,  &itsNodeChild,     &itsNodeFlags,    &itsNodeSorted,
             &itsNodeStage,   &itsNodeSub,     &itsBucketed,     &itsSorted,      &itsFineCode,
@@ -300,7 +300,7 @@ uint64_t OctreeBuilder::estimateFootprint(const CloudInfo& cloud, const Processi
     const uint64_t staged = e > n ? e - n : 1;
     const uint64_t mBound = std::min<uint64_t>(dense, (depth + 1) * n);
     uint64_t bytes        = hostCloud ? n * cloud.dataStride : 0;
-    bytes += 8 * dense + 4 * ((dense + 31) / 32);          // count pyramid, dense -> sparse, occupancy bits
+    bytes += 8 * dense + 4 * ((dense + 31) / 32);          // count pyramid; occupancy bits and id bases (at most a word a cell)
     bytes += 8 * mBound + 77 * mBound + n / 1024;           // node keys / counts, node arrays, leaf chunks
     bytes += 22 * e;                                        // lut + output records
     bytes += (2 * sortedPointBytes(cloud) + 2 + 4) * n;     // bucketed, sorted, fine codes, permutation
@@ -492,10 +492,11 @@ void OctreeBuilder::countPoints()
     Gridding g{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2], itsCloud.bbMax[0] - itsCloud.bbMin[0],
                itsProc.chunkingGrid};
     itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(nb) + 1));
-    uint32_t* occ = fineSortBits() ? itsOccupancy.as<uint32_t>() : nullptr;
-    const uint64_t marked = occ ? itsLevelOffset[BIT_LEVELS] : 0;
-    kBuildInit<<<gridFor(std::max<uint64_t>({nb, marked / 32, itsDense - marked}), 2048), BLOCK, 0, itsStream>>>(
-            sc, bucketCount, nb + 1, occ, marked / 32, itsCount.as<uint32_t>(), marked, itsDense);
+    uint32_t* occ         = itsOccupancy.as<uint32_t>();
+    const uint64_t words  = (static_cast<uint64_t>(itsDense) + 31) / 32;
+    const uint64_t counts = itsLevelOffset[itsCoarse];  // read for empty cells from here on
+    kBuildInit<<<gridFor(std::max<uint64_t>({nb, words, itsDense - counts}), 2048), BLOCK, 0, itsStream>>>(
+            sc, bucketCount, nb + 1, occ, words, itsCount.as<uint32_t>(), counts, itsDense);
     OC_LAUNCH_CHECK();
 
     // four rounds of records per workgroup until the chip is full, then sixteen: every workgroup adds its
@@ -554,12 +555,6 @@ void OctreeBuilder::countPoints()
     }
 }
 
-bool OctreeBuilder::fineSortBits() const
-{
-    // 32^3-cell buckets: chunking grids of 256 and 512, whose levels also start at multiples of 64
-    return itsCoarse == MAX_COARSE_LEVEL;
-}
-
 LevelParams OctreeBuilder::levelParams() const
 {
     LevelParams lp{};
@@ -581,11 +576,10 @@ void OctreeBuilder::mergeLevels()
     for (uint32_t l = 0; l <= itsDepth; ++l)
         lo.offset[l] = itsLevelOffset[l];
     lo.levels = itsDepth + 1;
-    // levels 0..coarse come from the fine sort: the counts of the levels above, the occupancy bits of the
-    // levels the fine sort has not marked, sparse ids (A2) + node keys / counts
+    // levels 0..coarse come from the fine sort: counts and occupancy bits of the levels above, sparse ids
+    // (A2) + node keys / counts
     // + first id of every level by a scan over the bitmap's words, and the list of internal nodes
     uint32_t* occ         = itsOccupancy.as<uint32_t>();
-    const uint64_t marked = fineSortBits() ? itsLevelOffset[BIT_LEVELS] / 32 : 0;
     uint32_t* levelStart  = reinterpret_cast<uint32_t*>(sc + SC_LEVEL_START);
     uint32_t* nodes       = reinterpret_cast<uint32_t*>(sc + SC_M);
     const uint64_t words  = (static_cast<uint64_t>(itsDense) + 31) / 32;
@@ -600,10 +594,10 @@ void OctreeBuilder::mergeLevels()
     itsScanScratch.ensure(sizeof(uint64_t) * SCAN_GRID);
     uint32_t* sums = itsScanScratch.as<uint32_t>();
     const unsigned wordGrid = static_cast<unsigned>(std::min<uint64_t>(scanTiles(words), SCAN_GRID));
-    kOccupancy<<<wordGrid, SCAN_THREADS, 0, itsStream>>>(occ, count, marked, itsDense, lo, itsCoarse,
+    kOccupancy<<<wordGrid, SCAN_THREADS, 0, itsStream>>>(occ, count, itsDense, lo, itsCoarse,
                                                          itsProc.chunkingGrid, sums, sc + SC_STAMP + 1);
     OC_LAUNCH_CHECK();
-    const IdTables ids{occ, count, itsDenseToSparse.as<int32_t>(), itsNodeKey.as<uint32_t>(),
+    const IdTables ids{occ, count, itsIdBase.as<uint32_t>(), itsNodeKey.as<uint32_t>(),
                        itsNodeCount.as<uint32_t>(), levelStart, lo};
     kOccupiedIds<<<wordGrid, SCAN_THREADS, 0, itsStream>>>(ids, words, sums, nodes);
     OC_LAUNCH_CHECK();
@@ -643,7 +637,7 @@ void OctreeBuilder::mergeLevels()
     itsStamps.ensure(sizeof(uint64_t) * (ST_STAMPS * itsSteps + 1));
     kNodeLinks<<<gridFor(m), BLOCK, 0, itsStream>>>(
             itsM, levelParams(), itsNodeKey.as<uint32_t>(), itsNodeCount.as<uint32_t>(),
-            itsDenseToSparse.as<int32_t>(), occ, itsNodePoints.as<uint32_t>(), itsNodeData.as<uint64_t>(),
+            IdMap{occ, itsIdBase.as<uint32_t>()}, itsNodePoints.as<uint32_t>(), itsNodeData.as<uint64_t>(),
             itsNodeParent.as<int32_t>(), itsNodeChild.as<int32_t>(), itsNodeFlags.as<uint8_t>(),
             itsNodeSub.as<uint32_t>(), itsCoarse, itsBucketStart.as<uint32_t>(), itsNodeSorted.as<uint32_t>(), count,
             itsCursors.as<uint64_t>(), itsCloud.pointAmount);

@@ -75,7 +75,7 @@ struct BatchCloud
     uint64_t* splitChunks;
     uint32_t* splitHist;
     uint32_t* count;
-    int32_t* denseToSparse;
+    uint32_t* idBase;
     uint32_t* occ;  // one bit per dense cell
     uint32_t *nodeKey, *nodeCount;  // bounded by min(D, (depth + 1) N)
     // nodes
@@ -130,7 +130,6 @@ struct BatchLevels
     uint32_t grid[MAX_LEVELS];
     uint32_t nodes[MAX_LEVELS];
     uint32_t dense;
-    uint32_t marked;  // cells of the levels whose occupancy bits the fine sort writes (0: none)
 };
 
 // The cloud of item i: the last c with prefix[c] <= i (prefix[B] = total > i).
@@ -431,13 +430,13 @@ struct PlacedChunkJob
 // Count stage
 // ------------------------------------------------------------------------------------------------
 
-// What every cloud starts from: zero scalars and bucket counts, and with the fine sort's occupancy
-// bits the bitmap of the levels it marks and the counts of the others (as kBuildInit).
+// What every cloud starts from: zero scalars, bucket counts, occupancy bitmap and counts of the bucket
+// level and above (as kBuildInit).
 template <typename T>
 static __global__ __launch_bounds__(BLOCK) void kBatchInit(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
                                                      BatchLevels L)
 {
-    const uint32_t words = L.marked / 32, counts = L.marked ? L.dense - L.marked : 0;
+    const uint32_t words = (L.dense + 31) / 32, counts = L.dense - L.offset[L.lc];
     const uint64_t per = BS_SLOTS + L.buckets + 1 + words + counts;
     for (uint64_t i = globalThread(); i < per * B; i += globalStride())
     {
@@ -458,7 +457,7 @@ static __global__ __launch_bounds__(BLOCK) void kBatchInit(const BatchCloud<T>* 
         if (k < words)
             cc.occ[k] = 0;
         else
-            cc.count[L.marked + (k - words)] = 0;
+            cc.count[L.offset[L.lc] + (k - words)] = 0;
     }
 }
 
@@ -537,7 +536,7 @@ static __global__ __launch_bounds__(SCATTER_THREADS) void kBucketScatterB(const 
 // items: (cloud, bucket)
 template <typename T>
 static __global__ __launch_bounds__(SORT_THREADS) void kFineSortB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                            FineSortParams fp, uint32_t buckets, bool bits)
+                                                            FineSortParams fp, uint32_t buckets)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS + 1];
     __shared__ uint32_t scratch[SORT_WAVES];
@@ -546,7 +545,7 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineSortB(const BatchClo
     {
         const BatchCloud<T>& cc = ctx[item / buckets];
         fineSortBucket(item % buckets, cc.fineCode, cc.bucketStart, fp, cc.count, cc.perm, h, scratch,
-                       bits ? cc.occ : nullptr);
+                       cc.occ);
         __syncthreads();
     }
 }
@@ -588,7 +587,7 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineChunkHistB(const Bat
 template <typename T>
 static __global__ __launch_bounds__(SORT_THREADS) void kFineSplitScanB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
                                                                  const uint32_t* __restrict__ prefix,
-                                                                 FineSortParams fp, bool bits)
+                                                                 FineSortParams fp)
 {
     __shared__ uint32_t h[MAX_FINE_CELLS + 1];
     __shared__ uint32_t scratch[SORT_WAVES];
@@ -601,7 +600,7 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineSplitScanB(const Bat
         if (static_cast<uint32_t>(cc.splitChunks[chunk]) != 0)
             continue;  // not the first chunk of its bucket (uniform over the workgroup)
         fineSplitScan(chunk, cc.bucketStart, cc.splitChunks, fp, cc.count, cc.splitHist, h, scratch,
-                      bits ? cc.occ : nullptr);
+                      cc.occ);
         __syncthreads();
     }
 }
@@ -642,7 +641,7 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kOccupancyB(const BatchCl
     const BatchCloud<T>& cc = ctx[blockIdx.y];
     uint64_t first, last;
     tileRange(scanTiles((static_cast<uint64_t>(L.dense) + 31) / 32), first, last);
-    const uint32_t bits = occupancyTiles(cc.occ, cc.count, L.marked / 32, L.dense, levelOffsets(L), L.lc, L.grid[0],
+    const uint32_t bits = occupancyTiles(cc.occ, cc.count, L.dense, levelOffsets(L), L.lc, L.grid[0],
                                          first, last, lds);
     if (threadIdx.x == 0)
         reinterpret_cast<uint32_t*>(cc.scanSums)[blockIdx.x] = bits;
@@ -654,7 +653,7 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kOccupiedIdsB(const Batch
 {
     __shared__ IdLds lds;
     const BatchCloud<T>& cc = ctx[blockIdx.y];
-    const IdTables t{cc.occ, cc.count, cc.denseToSparse, cc.nodeKey, cc.nodeCount, cc.levelStart(), levelOffsets(L)};
+    const IdTables t{cc.occ, cc.count, cc.idBase, cc.nodeKey, cc.nodeCount, cc.levelStart(), levelOffsets(L)};
     const uint64_t words = (static_cast<uint64_t>(L.dense) + 31) / 32;
     uint64_t first, last;
     tileRange(scanTiles(words), first, last);
@@ -692,7 +691,7 @@ static __global__ __launch_bounds__(BLOCK) void kNodeLinksB(const BatchCloud<T>*
         const uint32_t c        = findCloud(wp, B, static_cast<uint32_t>(i));
         const BatchCloud<T>& cc = ctx[c];
         const uint32_t id       = static_cast<uint32_t>(i) - wp[c];
-        nodeLinksOf(id, levelParams(L, cc.threshold), cc.nodeKey, cc.nodeCount, cc.denseToSparse, cc.occ, cc.nodePoints,
+        nodeLinksOf(id, levelParams(L, cc.threshold), cc.nodeKey, cc.nodeCount, IdMap{cc.occ, cc.idBase}, cc.nodePoints,
                     cc.nodeData, cc.nodeParent, cc.nodeChild, cc.nodeFlags, cc.nodeSub, L.lc, cc.bucketStart, cc.nodeSorted,
                     cc.count);
         cc.keyOut[id]   = cc.nodeKey[id];

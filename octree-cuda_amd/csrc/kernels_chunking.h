@@ -43,9 +43,8 @@ inline unsigned gridFor(uint64_t n, uint64_t cap = 65536)
 }
 
 
-// What a build starts from, cleared in one launch: the scalars, the bucket counts, the bitmap words
-// [0, words) of the levels whose occupancy bits the fine sort writes (none for small grids) and the
-// counts [first, last) of the other levels.
+// What a build starts from, cleared in one launch: the scalars, the bucket counts, the occupancy
+// bitmap and the counts [first, last) of the bucket level and the levels above.
 static __global__ __launch_bounds__(BLOCK) void kBuildInit(uint64_t* __restrict__ sc, uint32_t* __restrict__ bucketCount,
                                                      uint32_t buckets, uint32_t* __restrict__ occ, uint64_t words,
                                                      uint32_t* __restrict__ count, uint64_t first, uint64_t last)
@@ -115,17 +114,17 @@ __device__ __forceinline__ uint32_t occupancyWord(const uint32_t* count, uint64_
     return bits;
 }
 
-// First pass of the id scan over the tiles [first, last) of the bitmap's words: the words from `marked`
-// on are made from their counts (the fine sort has marked the ones before), and the number of set bits
-// comes back in thread 0. All threads. The workgroups with words of the levels above the bucket level,
-// the last few words of all, first sum up those levels (twice if two workgroups share them: the same
-// values).
-__device__ __forceinline__ uint32_t occupancyTiles(uint32_t* occ, uint32_t* count, uint64_t marked, uint64_t dense,
+// First pass of the id scan over the tiles [first, last) of the bitmap's words: the number of set bits,
+// in thread 0. All threads. The fine sort has marked the levels up to the bucket level; the workgroups
+// with words of the levels above, the last few of all, first sum up those levels (twice if two
+// workgroups share them: the same values) and make the words from the counts.
+__device__ __forceinline__ uint32_t occupancyTiles(uint32_t* occ, uint32_t* count, uint64_t dense,
                                                    const LevelOffsets& lo, uint32_t lc, uint32_t chunkingGrid,
                                                    uint64_t first, uint64_t last, uint32_t* lds)
 {
-    const uint64_t words = (dense + 31) / 32;
-    if (lc + 1 < lo.levels && first < last && last * SCAN_TILE > lo.offset[lc + 1] / 32)
+    const uint64_t words  = (dense + 31) / 32;
+    const uint64_t marked = lo.offset[lc + 1] / 32;  // the level above the buckets is never past the root
+    if (first < last && last * SCAN_TILE > marked)
         propagateTop(count, lo, lc, chunkingGrid);
     uint32_t bits = 0;
     for (uint64_t tile = first; tile < last; ++tile)
@@ -153,8 +152,8 @@ __device__ __forceinline__ uint32_t occupancyTiles(uint32_t* occ, uint32_t* coun
     return blockSum(bits, lds);
 }
 
-static __global__ __launch_bounds__(SCAN_THREADS) void kOccupancy(uint32_t* occ, uint32_t* count, uint64_t marked,
-                                                           uint64_t dense, LevelOffsets lo, uint32_t lc,
+static __global__ __launch_bounds__(SCAN_THREADS) void kOccupancy(uint32_t* occ, uint32_t* count, uint64_t dense,
+                                                           LevelOffsets lo, uint32_t lc,
                                                            uint32_t chunkingGrid, uint32_t* __restrict__ sums,
                                                            uint64_t* stamp)
 {
@@ -162,24 +161,43 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kOccupancy(uint32_t* occ,
     stampStart(stamp);
     uint64_t first, last;
     tileRange(scanTiles((dense + 31) / 32), first, last);
-    const uint32_t bits = occupancyTiles(occ, count, marked, dense, lo, lc, chunkingGrid, first, last, lds);
+    const uint32_t bits = occupancyTiles(occ, count, dense, lo, lc, chunkingGrid, first, last, lds);
     if (threadIdx.x == 0)
         sums[blockIdx.x] = bits;
 }
 
 // Sparse ids (A2): the exclusive rank of an occupied dense cell; its node key and dense count are
 // written in the same pass, and the first id of every level (ids ascend with the dense index and a
-// level is one dense range). denseToSparse is written for occupied cells only: an array of D
-// entries is never filled with -1.
+// level is one dense range).
 struct IdTables
 {
     const uint32_t* occ;
     const uint32_t* count;
-    int32_t* denseToSparse;
+    uint32_t* idBase;
     uint32_t* nodeKey;
     uint32_t* nodeCount;
     uint32_t* levelStart;
     LevelOffsets levels;
+};
+
+// The id of an occupied dense cell: the first id of its bitmap word (there for the words of the tiles
+// that hold any occupied cell) and the set bits below it. Bitmap and bases are 38 MB at a 512 grid and
+// stay in cache; an array of an id per dense cell was 613 MB.
+struct IdMap
+{
+    const uint32_t* occ;
+    const uint32_t* idBase;
+    // the cell is occupied
+    __device__ __forceinline__ uint32_t at(uint32_t d) const
+    {
+        return idBase[d >> 5] + __popc(occ[d >> 5] & ((1u << (d & 31)) - 1u));
+    }
+    // -1: it is not
+    __device__ __forceinline__ int32_t find(uint32_t d) const
+    {
+        const uint32_t w = occ[d >> 5];
+        return (w >> (d & 31)) & 1u ? static_cast<int32_t>(idBase[d >> 5] + __popc(w & ((1u << (d & 31)) - 1u))) : -1;
+    }
 };
 
 // Set bits of a tile that are listed in LDS at a time.
@@ -219,6 +237,11 @@ __device__ __forceinline__ uint32_t occupiedIds(const IdTables& t, uint64_t word
                 if (item == k * SCAN_THREADS + threadIdx.x)
                     t.levelStart[l] = carry + pre[k] + __popc(w[k] & ((1u << (d & 31)) - 1u));
         }
+        if (ids)
+#pragma unroll
+            for (int k = 0; k < SCAN_ITEMS; ++k)
+                if (const uint64_t i = tile * SCAN_TILE + k * SCAN_THREADS + threadIdx.x; i < words)
+                    t.idBase[i] = carry + pre[k];
         for (uint32_t base = 0; base < ids; base += ID_LIST)
         {
 #pragma unroll
@@ -249,10 +272,9 @@ __device__ __forceinline__ uint32_t occupiedIds(const IdTables& t, uint64_t word
                 for (uint32_t k = 0; k < ID_ITEMS; ++k)
                     if (const uint32_t j = j0 + k * SCAN_THREADS; j < n)
                     {
-                        const uint32_t id     = carry + base + j;
-                        t.nodeKey[id]         = d[k];
-                        t.nodeCount[id]       = c[k];
-                        t.denseToSparse[d[k]] = static_cast<int32_t>(id);
+                        const uint32_t id = carry + base + j;
+                        t.nodeKey[id]     = d[k];
+                        t.nodeCount[id]   = c[k];
                     }
             }
             __syncthreads();
@@ -294,13 +316,12 @@ __device__ __forceinline__ uint32_t levelOfKey(uint32_t key, const LevelParams& 
 // The leaf of a level-0 cell (the first finished ancestor-or-self, point_distributing.cuh:56-60): the
 // first node on the way up whose parent is internal, or the root.
 __device__ __forceinline__ uint32_t leafOfCell(uint32_t id, uint32_t x, uint32_t y, uint32_t z, const LevelParams& lp,
-                                               const uint32_t* __restrict__ nodeCount,
-                                               const int32_t* __restrict__ denseToSparse)
+                                               const uint32_t* __restrict__ nodeCount, const IdMap& ids)
 {
     for (uint32_t l = 1; l <= lp.depth; ++l)
     {
         const uint32_t g = lp.grid[l];
-        const uint32_t p = static_cast<uint32_t>(denseToSparse[lp.offset[l] + (x >> l) + (y >> l) * g + (z >> l) * g * g]);
+        const uint32_t p = ids.at(lp.offset[l] + (x >> l) + (y >> l) * g + (z >> l) * g * g);
         if (nodeCount[p] >= lp.threshold)
             return id;
         id = p;
@@ -313,9 +334,7 @@ __device__ __forceinline__ uint32_t leafOfCell(uint32_t id, uint32_t x, uint32_t
 // of the lower-slot siblings of the node and of its ancestors inside the bucket.
 __device__ __forceinline__ uint32_t sortedStartOf(uint32_t l, uint32_t x, uint32_t y, uint32_t z, uint32_t lc,
                                                   const LevelParams& lp, const uint32_t* __restrict__ bucketStart,
-                                                  const uint32_t* __restrict__ occ,
-                                                  const int32_t* __restrict__ denseToSparse,
-                                                  const uint32_t* __restrict__ nodeCount)
+                                                  const IdMap& ids, const uint32_t* __restrict__ nodeCount)
 {
     uint32_t start = 0;
     for (; l < lc; ++l)
@@ -325,9 +344,9 @@ __device__ __forceinline__ uint32_t sortedStartOf(uint32_t l, uint32_t x, uint32
         for (uint32_t k = 0; k < slot; ++k)
         {
             const uint32_t sx = (x & ~1u) + (k >> 2), sy = (y & ~1u) + ((k >> 1) & 1), sz = (z & ~1u) + (k & 1);
-            const uint32_t d = lp.offset[l] + sx + sy * g + sz * g * g;
-            if ((occ[d >> 5] >> (d & 31)) & 1u)
-                start += nodeCount[denseToSparse[d]];
+            const int32_t c = ids.find(lp.offset[l] + sx + sy * g + sz * g * g);
+            if (c >= 0)
+                start += nodeCount[c];
         }
         x >>= 1;
         y >>= 1;
@@ -344,9 +363,8 @@ __device__ __forceinline__ uint32_t sortedStartOf(uint32_t l, uint32_t x, uint32
 // For a leaf also its range of the sorted cloud, and for a level-0 node its leaf, over its cell's
 // count (nothing reads that again), so the distribution needs one lookup per point.
 __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, const uint32_t* __restrict__ nodeKey,
-                                            const uint32_t* __restrict__ nodeCount,
-                                            const int32_t* __restrict__ denseToSparse,
-                                            const uint32_t* __restrict__ occ, uint32_t* __restrict__ pointCount,
+                                            const uint32_t* __restrict__ nodeCount, const IdMap& ids,
+                                            uint32_t* __restrict__ pointCount,
                                             uint64_t* __restrict__ dataIdx, int32_t* __restrict__ parent,
                                             int32_t* __restrict__ children, uint8_t* __restrict__ flags,
                                             uint32_t* __restrict__ subtree, uint32_t lc,
@@ -365,7 +383,7 @@ __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, 
     if (l < lp.depth)
     {
         const uint32_t pg = lp.grid[l + 1];  // the parent of an occupied cell is occupied
-        p                 = denseToSparse[lp.offset[l + 1] + (x >> 1) + (y >> 1) * pg + (z >> 1) * pg * pg];
+        p = static_cast<int32_t>(ids.at(lp.offset[l + 1] + (x >> 1) + (y >> 1) * pg + (z >> 1) * pg * pg));
     }
     const bool finished = (p < 0) ? true : (nodeCount[p] >= lp.threshold);
 
@@ -376,11 +394,7 @@ __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, 
         {
             const uint32_t cg = lp.grid[l - 1];
             const uint32_t cx = 2 * x + ((k >> 2) & 1), cy = 2 * y + ((k >> 1) & 1), cz = 2 * z + (k & 1);
-            const uint32_t cd = lp.offset[l - 1] + cx + cy * cg + cz * cg * cg;
-            // occupancy from the bitmap (the counts of empty cells of the lowest levels are not
-            // written); denseToSparse is set for occupied cells only
-            if ((occ[cd >> 5] >> (cd & 31)) & 1u)
-                c = denseToSparse[cd];
+            c = ids.find(lp.offset[l - 1] + cx + cy * cg + cz * cg * cg);
         }
         children[8 * static_cast<uint64_t>(id) + k] = c;
     }
@@ -390,15 +404,13 @@ __device__ __forceinline__ void nodeLinksOf(uint32_t id, const LevelParams& lp, 
     flags[id]      = static_cast<uint8_t>((finished ? NODE_FINISHED : 0) | (internal ? NODE_INTERNAL : 0));
     subtree[id]    = 0;
     if (finished && !internal)
-        sortedStart[id] = sortedStartOf(l, x, y, z, lc, lp, bucketStart, occ, denseToSparse, nodeCount);
+        sortedStart[id] = sortedStartOf(l, x, y, z, lc, lp, bucketStart, ids, nodeCount);
     if (l == 0)
-        cellLeaf[key] = leafOfCell(id, x, y, z, lp, nodeCount, denseToSparse);
+        cellLeaf[key] = leafOfCell(id, x, y, z, lp, nodeCount, ids);
 }
 
 static __global__ __launch_bounds__(BLOCK) void kNodeLinks(uint32_t m, LevelParams lp, const uint32_t* __restrict__ nodeKey,
-                                                     const uint32_t* __restrict__ nodeCount,
-                                                     const int32_t* __restrict__ denseToSparse,
-                                                     const uint32_t* __restrict__ occ,
+                                                     const uint32_t* __restrict__ nodeCount, IdMap ids,
                                                      uint32_t* __restrict__ pointCount, uint64_t* __restrict__ dataIdx,
                                                      int32_t* __restrict__ parent, int32_t* __restrict__ children,
                                                      uint8_t* __restrict__ flags, uint32_t* __restrict__ subtree,
@@ -407,7 +419,7 @@ static __global__ __launch_bounds__(BLOCK) void kNodeLinks(uint32_t m, LevelPara
                                                      uint64_t* __restrict__ cursor, uint32_t points)
 {
     for (uint64_t i = globalThread(); i < m; i += globalStride())
-        nodeLinksOf(static_cast<uint32_t>(i), lp, nodeKey, nodeCount, denseToSparse, occ, pointCount, dataIdx, parent,
+        nodeLinksOf(static_cast<uint32_t>(i), lp, nodeKey, nodeCount, ids, pointCount, dataIdx, parent,
                     children, flags, subtree, lc, bucketStart, sortedStart, cellLeaf);
     if (globalThread() == 0)
         *cursor = points;  // the output cursor before the first subsampling step

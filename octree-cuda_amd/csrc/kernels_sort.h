@@ -342,20 +342,15 @@ __device__ __forceinline__ uint32_t fineSlot(uint32_t c)
     return c ^ (((c >> 5) ^ (c >> 10)) & 31u);
 }
 
-// Levels whose occupancy bits the fine sort writes when it gets the bitmap (lc = 5, chunking grid
-// >= 256): a bucket's rows of levels 0, 1 and 2 are 32, 16 and 8 cells from a multiple of that, one
-// word, half-word and byte of the bitmap, so each row is stored whole by one lane, no atomics.
-constexpr uint32_t BIT_LEVELS = 3;
-
 // Dense counts of bucket b's cells on levels 0..lc (kernelPropagatePointCounts,
 // point_count_propagation.cuh:34-86, as differences of the Morton prefix h over the bucket's
-// fine cells; h null: an empty bucket, all zero). With occ, the occupancy bits of levels 0..2 as
-// well, and only what is not zero: the bitmap of those levels and the counts of the others have
-// been cleared, and the later passes read the counts of levels 0..2 for occupied cells only
-// (storing those levels' zero counts was 77 MB per 512^3 build whatever the cloud's size: the fine
-// sort and kOccupancyBits took 147 + 35 us of a 200K-point build, now 60 + 4 after 6 us of clearing).
+// fine cells) and their occupancy bits. Only what is not zero is written: the bitmap is clear, and the
+// counts below level lc are read for occupied cells only (storing those levels' zero counts was 77 MB
+// per 512^3 build whatever the cloud's size: with a pass for the bits it took 147 + 35 us of a
+// 200K-point build). A row of a bucket's level is `side` cells from a multiple of `side`: a word, a
+// half-word or a byte of the bitmap is stored whole by one lane, shorter rows (20 a bucket) are ored.
 __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& fp, const uint32_t* h,
-                                             uint32_t* __restrict__ count, uint32_t* __restrict__ occ = nullptr)
+                                             uint32_t* __restrict__ count, uint32_t* __restrict__ occ)
 {
     const uint32_t bx = compact3(b >> 2), by = compact3(b >> 1), bz = compact3(b);
     for (uint32_t k = 0; k <= fp.lc; ++k)
@@ -367,29 +362,25 @@ __device__ __forceinline__ void bucketCounts(uint32_t b, const FineSortParams& f
         for (uint32_t j = threadIdx.x; j < n3; j += SORT_THREADS)
         {
             const uint32_t lx = j & (side - 1), ly = (j >> (fp.lc - k)) & (side - 1), lz = j >> (2 * (fp.lc - k));
-            uint32_t v = 0;
-            if (h)
-            {
-                const uint32_t m = morton3(lx, ly, lz);
-                v                = h[fineSlot((m + 1) << (3 * k))] - h[fineSlot(m << (3 * k))];
-            }
+            const uint32_t m  = morton3(lx, ly, lz);
+            const uint32_t v  = h[fineSlot((m + 1) << (3 * k))] - h[fineSlot(m << (3 * k))];
             const uint64_t gx = static_cast<uint64_t>(bx) * side + lx, gy = static_cast<uint64_t>(by) * side + ly,
                            gz = static_cast<uint64_t>(bz) * side + lz;
             const uint64_t d = offset + gx + gy * gk + gz * gk * gk;
-            if (!occ || v)
+            if (v)
                 count[d] = v;
-            if (occ && k < BIT_LEVELS)  // uniform; every lane of the wave is here (n3 is a multiple of 64)
+            // the lanes of a row are together here or none of them is (n3 is a multiple of side)
+            const uint64_t set = (__ballot(v != 0) >> (threadIdx.x & (64 - side) & 63)) & ((1ull << side) - 1);
+            if (lx == 0 && set)
             {
-                const uint64_t set = __ballot(v != 0) >> (threadIdx.x & (64 - side) & 63);
-                if (lx == 0 && (set & ((1ull << side) - 1)))
-                {
-                    if (k == 0)
-                        occ[d >> 5] = static_cast<uint32_t>(set);
-                    else if (k == 1)
-                        reinterpret_cast<uint16_t*>(occ)[d >> 4] = static_cast<uint16_t>(set);
-                    else
-                        reinterpret_cast<uint8_t*>(occ)[d >> 3] = static_cast<uint8_t>(set);
-                }
+                if (side == 32)
+                    occ[d >> 5] = static_cast<uint32_t>(set);
+                else if (side == 16)
+                    reinterpret_cast<uint16_t*>(occ)[d >> 4] = static_cast<uint16_t>(set);
+                else if (side == 8)
+                    reinterpret_cast<uint8_t*>(occ)[d >> 3] = static_cast<uint8_t>(set);
+                else
+                    atomicOr(occ + (d >> 5), static_cast<uint32_t>(set) << (d & 31));
             }
         }
     }
@@ -487,19 +478,14 @@ __device__ __forceinline__ void finePermute(const uint16_t* __restrict__ fineCod
 __device__ __forceinline__ void fineSortBucket(uint32_t b, const uint16_t* __restrict__ fineCode,
                                                const uint32_t* __restrict__ bucketStart, const FineSortParams& fp,
                                                uint32_t* __restrict__ count, uint32_t* __restrict__ perm, uint32_t* h,
-                                               uint32_t* scratch, uint32_t* __restrict__ occ = nullptr)
+                                               uint32_t* scratch, uint32_t* __restrict__ occ)
 {
     const uint32_t cells = 1u << (3 * fp.lc);
     const uint32_t lo = bucketStart[b], hi = bucketStart[b + 1];
     if (hi - lo > FINE_SPLIT)
         return;  // sorted by the split path
     if (lo == hi)
-    {
-        // an empty bucket (most of them in a sparse cloud): zero counts, no histogram, no scan
-        if (!occ)
-            bucketCounts(b, fp, nullptr, count);
-        return;
-    }
+        return;  // an empty bucket (most of them in a sparse cloud)
 
     for (uint32_t c = threadIdx.x; c <= cells; c += SORT_THREADS)
         h[c] = 0;
@@ -603,7 +589,7 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineChunkHist(const uint
 __device__ __forceinline__ void fineSplitScan(uint32_t chunk, const uint32_t* __restrict__ bucketStart,
                                               const uint64_t* __restrict__ chunks, const FineSortParams& fp,
                                               uint32_t* __restrict__ count, uint32_t* __restrict__ chunkHist,
-                                              uint32_t* h, uint32_t* scratch, uint32_t* __restrict__ occ = nullptr)
+                                              uint32_t* h, uint32_t* scratch, uint32_t* __restrict__ occ)
 {
     const uint32_t b     = static_cast<uint32_t>(chunks[chunk] >> 32);
     const uint32_t parts = (bucketStart[b + 1] - bucketStart[b] + FINE_SPLIT - 1) / FINE_SPLIT;

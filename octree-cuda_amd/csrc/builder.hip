@@ -583,7 +583,6 @@ void OctreeBuilder::mergeLevels()
     uint32_t* levelStart  = reinterpret_cast<uint32_t*>(sc + SC_LEVEL_START);
     uint32_t* nodes       = reinterpret_cast<uint32_t*>(sc + SC_M);
     const uint64_t words  = (static_cast<uint64_t>(itsDense) + 31) / 32;
-    const uint64_t bound  = nodeBound();
     // at most N / threshold internal nodes on a level (they hold disjoint point sets), and at most
     // as many as nodes above level 0
     uint64_t inner = 0;
@@ -602,7 +601,7 @@ void OctreeBuilder::mergeLevels()
     kOccupiedIds<<<wordGrid, SCAN_THREADS, 0, itsStream>>>(ids, words, sums, nodes);
     OC_LAUNCH_CHECK();
     uint32_t* internal = itsInternalList.as<uint32_t>();
-    scanExclusive<uint32_t>(DeviceCount{nodes, levelStart + 1}, bound,
+    scanExclusive<uint32_t>(DeviceCount{nodes, levelStart + 1}, nodeBound(),
                             InternalNodeIn{itsNodeCount.as<uint32_t>(), levelStart, itsProc.mergingThreshold},
                             InternalNodeOut{internal, levelStart}, sums, reinterpret_cast<uint32_t*>(sc + SC_INTERNAL),
                             itsStream);
@@ -841,12 +840,17 @@ void OctreeBuilder::subsampleLevels()
             continue;
         const ChildSlots cs        = childSlots(itsInner[l]);
         NodeGrid* nodeGrid         = itsNodeGrid.as<NodeGrid>();
-        scanExclusive<uint64_t>(8ull * K, LevelSegmentIn{cs, itsNodePoints.as<uint32_t>()},
-                                LevelSegmentOut{cs, itsNodeSorted.as<uint32_t>(), itsNodeStage.as<uint32_t>(),
-                                                itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(),
-                                                itsSegTile.as<uint32_t>(), itsSegInput.as<uint32_t>()},
-                                itsScanScratch.as<uint64_t>(), sc + SC_SEG_TOTAL, itsStream);
-        OC_LAUNCH_CHECK();
+        const LevelSegmentIn segIn{cs, itsNodePoints.as<uint32_t>()};
+        const LevelSegmentOut segOut{cs, itsNodeSorted.as<uint32_t>(), itsNodeStage.as<uint32_t>(),
+                                     itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                                     itsSegInput.as<uint32_t>()};
+        // in one launch with the level's other preparations, when it is one step sized without a readback
+        const bool oneLaunch = K <= START_NODES && K <= batchNodes && N < READ_INPUTS_POINTS;
+        if (!oneLaunch)
+        {
+            scanExclusive<uint64_t>(8ull * K, segIn, segOut, itsScanScratch.as<uint64_t>(), sc + SC_SEG_TOTAL, itsStream);
+            OC_LAUNCH_CHECK();
+        }
         uint64_t inputMost = N;
         if (N >= READ_INPUTS_POINTS)
         {
@@ -876,10 +880,16 @@ void OctreeBuilder::subsampleLevels()
             ++stepAt;
 
             const bool resetInputs = words <= RESET_INPUTS_WORDS;
-            kLevelPrepare<<<gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384), BLOCK, 0, itsStream>>>(
-                    K, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
-                    sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs,
-                    stamps + ST_BEGIN);
+            const unsigned prepareGrid = gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384);
+            if (oneLaunch)
+                kLevelStart<<<std::min(prepareGrid, 2048u), BLOCK, 0, itsStream>>>(
+                        K, sp, segIn, segOut, itsNodeKey.as<uint32_t>(), nodeGrid, sc + SC_SEG_TOTAL,
+                        itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs, stamps + ST_BEGIN);
+            else
+                kLevelPrepare<<<prepareGrid, BLOCK, 0, itsStream>>>(
+                        K, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
+                        sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs,
+                        stamps + ST_BEGIN);
             OC_LAUNCH_CHECK();
             kMark<T><<<tileGrid, TILE, 0, itsStream>>>(
                     tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
@@ -982,15 +992,11 @@ void OctreeBuilder::placeInternalNodes()
     if (nodes == 0)
         return;
     const uint32_t* list = itsInternalList.as<uint32_t>();
+    // (internal node, chunk) work items; the leaf chunk list is free again after the distribution
+    uint32_t* chunks = reinterpret_cast<uint32_t*>(itsScalars.as<uint64_t>() + SC_TABLE_TOTAL);  // zero so far
     kPlaceNodes<<<std::min<uint32_t>((nodes + 63) / 64, 4096), 64, 0, itsStream>>>(
             list, nodes, N, itsNodeParent.as<int32_t>(), itsNodeChild.as<int32_t>(), itsNodePoints.as<uint32_t>(),
-            itsNodeSub.as<uint32_t>(), itsNodeData.as<uint64_t>(), itsStamps.as<uint64_t>() + ST_STAMPS * itsSteps);
-    OC_LAUNCH_CHECK();
-    // (internal node, chunk) work items; the leaf chunk list is free again after the distribution
-    uint32_t* chunks = reinterpret_cast<uint32_t*>(itsScalars.as<uint64_t>() + SC_TABLE_TOTAL);
-    scanExclusive<uint32_t>(nodes, PlacedListIn{list, itsNodePoints.as<uint32_t>()},
-                            PlacedListOut{list, itsLeafList.as<uint64_t>()}, itsScanScratch.as<uint32_t>(), chunks,
-                            itsStream);
+            itsNodeSub.as<uint32_t>(), itsNodeData.as<uint64_t>(), itsLeafList.as<uint64_t>(), chunks, itsStamps.as<uint64_t>() + ST_STAMPS * itsSteps);
     OC_LAUNCH_CHECK();
     const Gridding cubic{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
                          itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid};

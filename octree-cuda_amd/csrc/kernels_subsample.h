@@ -593,21 +593,17 @@ struct CellState
 // tile, all of them in flight; a thread per segment wrote a large child's thousands of entries by
 // itself, 71 us of a 5.1M-point build) and a clear bitmap. For a small level also the state of as many
 // cells as it has inputs (it has no more), which spares it kClearCompact.
-static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, SubsampleParams sp,
-                                                        const uint32_t* __restrict__ internal,
-                                                        const uint32_t* __restrict__ nodeKey,
-                                                        NodeGrid* __restrict__ nodeGrid,
-                                                        const uint32_t* __restrict__ segTile,
-                                                        const uint64_t* __restrict__ segTotal,
-                                                        uint32_t* __restrict__ tileList, uint64_t words,
-                                                        uint32_t* __restrict__ bitmap, CellState cells, bool reset,
-                                                        uint64_t* stamp)
+__device__ __forceinline__ void levelPrepare(uint32_t nodes, const SubsampleParams& sp,
+                                             const uint32_t* __restrict__ internal,
+                                             const uint32_t* __restrict__ nodeKey, NodeGrid* __restrict__ nodeGrid,
+                                             const uint32_t* segTile, uint64_t segTotal,
+                                             uint32_t* __restrict__ tileList, uint64_t words,
+                                             uint32_t* __restrict__ bitmap, const CellState& cells, bool reset)
 {
-    stampStart(stamp);
     for (uint64_t k = globalThread(); k < nodes; k += globalStride())
         nodeGrid[k] = nodeGridOf(internal[k], nodeKey[internal[k]], sp.levelOffset, sp.levelGrid, sp.level, sp.depth,
                                  sp.cubicMin, sp.sideHalf, sp.side, sp.g, sp.seed);
-    const uint32_t tiles = static_cast<uint32_t>(*segTotal >> 32);
+    const uint32_t tiles = static_cast<uint32_t>(segTotal >> 32);
     for (uint64_t t = globalThread(); t < tiles; t += globalStride())
     {
         // the last segment that starts at or before t; segments without tiles start where the next does
@@ -626,10 +622,57 @@ static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, Su
         bitmap[w] = 0;
     if (reset)
     {
-        const uint32_t inputs = static_cast<uint32_t>(*segTotal);
+        const uint32_t inputs = static_cast<uint32_t>(segTotal);
         for (uint64_t c = globalThread(); c < inputs; c += globalStride())
             cells.reset(c);
     }
+}
+
+static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, SubsampleParams sp,
+                                                        const uint32_t* __restrict__ internal,
+                                                        const uint32_t* __restrict__ nodeKey,
+                                                        NodeGrid* __restrict__ nodeGrid,
+                                                        const uint32_t* __restrict__ segTile,
+                                                        const uint64_t* __restrict__ segTotal,
+                                                        uint32_t* __restrict__ tileList, uint64_t words,
+                                                        uint32_t* __restrict__ bitmap, CellState cells, bool reset,
+                                                        uint64_t* stamp)
+{
+    stampStart(stamp);
+    levelPrepare(nodes, sp, internal, nodeKey, nodeGrid, segTile, *segTotal, tileList, words, bitmap, cells, reset);
+}
+
+// Levels of up to START_NODES nodes: the segment scan and kLevelPrepare in one launch. Every workgroup
+// scans the (at most SCAN_TILE) segments into its LDS, so none waits for another; the first one writes
+// them out.
+constexpr uint32_t START_NODES = SCAN_TILE / 8;
+static_assert(BLOCK == SCAN_THREADS, "kLevelStart scans with one workgroup's threads");
+
+static __global__ __launch_bounds__(BLOCK) void kLevelStart(uint32_t nodes, SubsampleParams sp, LevelSegmentIn in,
+                                                      LevelSegmentOut out, const uint32_t* __restrict__ nodeKey,
+                                                      NodeGrid* __restrict__ nodeGrid, uint64_t* __restrict__ segTotal,
+                                                      uint32_t* __restrict__ tileList, uint64_t words,
+                                                      uint32_t* __restrict__ bitmap, CellState cells, bool reset,
+                                                      uint64_t* stamp)
+{
+    __shared__ uint64_t lds[SCAN_ITEMS * SCAN_WAVES];
+    __shared__ uint32_t segTile[SCAN_TILE];
+    stampStart(stamp);
+    const uint32_t segments = 8 * nodes;
+    uint64_t v[SCAN_ITEMS], pre[SCAN_ITEMS];
+    loadTile<uint64_t>(in, 0, segments, v);
+    const uint64_t total = tileExclusiveScan(v, pre, lds);
+#pragma unroll
+    for (int k = 0; k < SCAN_ITEMS; ++k)
+        segTile[k * SCAN_THREADS + threadIdx.x] = static_cast<uint32_t>(pre[k] >> 32);
+    __syncthreads();
+    if (blockIdx.x == 0)
+    {
+        storeTile<uint64_t>(out, 0, segments, v, pre, 0);
+        if (threadIdx.x == 0)
+            *segTotal = total;
+    }
+    levelPrepare(nodes, sp, in.cs.internal, nodeKey, nodeGrid, segTile, total, tileList, words, bitmap, cells, reset);
 }
 
 // The tiles of a batch of a level's nodes: from *lo (null: 0) to *hi.
@@ -1386,14 +1429,20 @@ __device__ __forceinline__ void regionOf(uint32_t id, uint32_t root, uint32_t N,
     dataIdx[id] = static_cast<uint64_t>(N) + r;
 }
 
+// Placement of the subsampled records: the staged records of an internal node are one contiguous
+// range, and so is its final range [dataIdx, dataIdx + pointCount), so every (node, chunk of
+// PLACE_CHUNK records) work item is a contiguous copy.
+constexpr uint32_t PLACE_CHUNK = 4096;
+
 // Single cloud: every internal node of the list on its own, its region from the subtrees of the
 // lower-slot siblings on its way up. No level waits for another (one workgroup going down level by
-// level took 105 us for 6600 nodes).
+// level took 105 us for 6600 nodes). Its chunks go to the work list in no particular order.
 static __global__ __launch_bounds__(64) void kPlaceNodes(const uint32_t* __restrict__ list, uint32_t nodes, uint32_t N,
                                                    const int32_t* __restrict__ parent,
                                                    const int32_t* __restrict__ children,
                                                    const uint32_t* __restrict__ pointCount,
                                                    const uint32_t* __restrict__ subtree, uint64_t* __restrict__ dataIdx,
+                                                   uint64_t* __restrict__ chunkList, uint32_t* __restrict__ chunks,
                                                    uint64_t* stamp)
 {
     stampStart(stamp);
@@ -1417,14 +1466,13 @@ static __global__ __launch_bounds__(64) void kPlaceNodes(const uint32_t* __restr
                     before += subtree[c[k]];
             }
         }
-        dataIdx[id] = static_cast<uint64_t>(N) + before;
+        dataIdx[id]       = static_cast<uint64_t>(N) + before;
+        const uint32_t n  = (pointCount[id] + PLACE_CHUNK - 1) / PLACE_CHUNK;
+        const uint32_t at = atomicAdd(chunks, n);
+        for (uint32_t k = 0; k < n; ++k)
+            chunkList[at + k] = (static_cast<uint64_t>(k) << 32) | id;
     }
 }
-
-// Placement of the subsampled records: the staged records of an internal node are one contiguous
-// range, and so is its final range [dataIdx, dataIdx + pointCount), so every (node, chunk of
-// PLACE_CHUNK records) work item is a contiguous copy.
-constexpr uint32_t PLACE_CHUNK = 4096;
 
 // chunks of an internal node's placement
 struct PlacedChunksIn
@@ -1434,25 +1482,6 @@ struct PlacedChunksIn
     __device__ uint32_t operator()(uint64_t i) const
     {
         return (flags[i] & NODE_INTERNAL) ? (pointCount[i] + PLACE_CHUNK - 1) / PLACE_CHUNK : 0u;
-    }
-};
-
-// the same over a list of internal nodes
-struct PlacedListIn
-{
-    const uint32_t* list;
-    const uint32_t* pointCount;
-    __device__ uint32_t operator()(uint64_t j) const { return (pointCount[list[j]] + PLACE_CHUNK - 1) / PLACE_CHUNK; }
-};
-
-struct PlacedListOut
-{
-    const uint32_t* list;
-    uint64_t* chunks;  // chunk number << 32 | node id
-    __device__ void operator()(uint64_t j, uint32_t prefix, uint32_t v) const
-    {
-        for (uint32_t k = 0; k < v; ++k)
-            chunks[prefix + k] = (static_cast<uint64_t>(k) << 32) | list[j];
     }
 };
 

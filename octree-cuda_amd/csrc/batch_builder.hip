@@ -610,7 +610,7 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
     // ---- distribution: leaf and cell order of the sorted clouds, then the leaf blocks ----------
     scanBatch<uint32_t>(LeafChunkJob<T>{ctx}, B, maxM, s);
     kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(ScalarCount<T>{ctx, BS_TABLE_TOTAL, false}, B, slot(P_LEAFCHUNK));
-    kLeafCellOrderB<T><<<LG.sortGrid, LEAF_THREADS, 0, s>>>(ctx, B, slot(P_LEAFCHUNK), L);
+    kLeafCellOrderB<T><<<LG.sortGrid, LEAF_THREADS, 0, s>>>(ctx, B, slot(P_LEAFCHUNK), L, mode);
     kGatherSortedB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_POINTS));
     kDistributeSortedB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_DIST));
     OC_LAUNCH_CHECK();
@@ -768,7 +768,7 @@ void BatchBuilder::subsampleGroup(uint32_t B, const BatchLevels& L, const BatchB
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(TileCount<T>{ctx}, B, slot(P_TILES));
         kWorkPrefix<<<1, SCAN_THREADS, 0, s>>>(WordCount<T>{ctx}, B, slot(P_WORDS));
         kClearBitmapsB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_WORDS));
-        kMarkB<T><<<LG.tileGrid, TILE, 0, s>>>(ctx, B, slot(P_TILES));
+        kMarkB<T><<<LG.tileGrid, TILE, 0, s>>>(ctx, B, slot(P_TILES), MODE);
         scanBatch<uint32_t>(PopcountJob<T>{ctx}, B, bounds.words, s);
         kLevelCellsB<T><<<(B + 255) / 256, 256, 0, s>>>(ctx, B);
         kBatchNodesB<T><<<LG.threadGrid, BLOCK, 0, s>>>(ctx, B, slot(P_K));

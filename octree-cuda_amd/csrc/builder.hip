@@ -670,6 +670,7 @@ LeafOrderParams OctreeBuilder::leafTables()
     }
     p.lp                = levelParams();
     p.g                 = itsProc.subsamplingGrid;
+    p.order             = cellOrderOf(itsColorMode, p.g);
     const uint32_t h    = p.g > 1 ? p.g / 2 : 1;  // cells per axis of a leaf's octant, as kLeafCellOrder
     const uint64_t keys = rowsPerNode(h) * ((h + 31) / 32);
     while (((keys - 1) >> p.keyShift) >= LEAF_KEYS)
@@ -894,7 +895,7 @@ void OctreeBuilder::subsampleLevels()
             kMark<T><<<tileGrid, TILE, 0, itsStream>>>(
                     tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                     itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid, ps,
-                    bitmap, itsCellOf.as<uint32_t>(), err, stamps + ST_INSERT_BEGIN);
+                    cellOrderOf(itsColorMode, g), bitmap, itsCellOf.as<uint32_t>(), err, stamps + ST_INSERT_BEGIN);
             OC_LAUNCH_CHECK();
             const uint64_t wordTiles = scanTiles(words);
             uint32_t* rangeSums      = itsScanScratch.as<uint32_t>();

@@ -706,7 +706,8 @@ static __global__ __launch_bounds__(BLOCK) void kNodeLinksB(const BatchCloud<T>*
 // items: leaf chunks of all clouds (prefix over the clouds' chunk counts)
 template <typename T>
 static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrderB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                                 const uint32_t* __restrict__ prefix, BatchLevels L)
+                                                                 const uint32_t* __restrict__ prefix, BatchLevels L,
+                                                                 uint32_t mode)
 {
     __shared__ LeafOrderLds lds;
     const uint32_t total = prefix[B];
@@ -715,7 +716,8 @@ static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrderB(const Bat
         const uint32_t c        = findCloud(prefix, B, item);
         const BatchCloud<T>& cc = ctx[c];
         // the cubic minimum is Gridding's first three members
-        const LeafOrderView p{&cc.grid.minX, cc.sideHalf, cc.side, L.offset, L.grid, L.depth, cc.g, cc.keyShift};
+        const LeafOrderView p{&cc.grid.minX, cc.sideHalf, cc.side, L.offset, L.grid, L.depth, cc.g, cc.keyShift,
+                              cellOrderOf(mode, cc.g)};
         leafCellOrderChunk<T>(cc.chunkList[item - prefix[c]], p, cc.nodeKey, cc.nodeParent, cc.nodeCount,
                               cc.nodeSorted, cc.bucketed, cc.perm, cc.sorted, lds);
     }
@@ -856,7 +858,7 @@ static __global__ __launch_bounds__(BLOCK) void kClearBitmapsB(const BatchCloud<
 // items: tiles (one per workgroup and step)
 template <typename T>
 static __global__ __launch_bounds__(TILE) void kMarkB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
-                                                const uint32_t* __restrict__ prefix)
+                                                const uint32_t* __restrict__ prefix, uint32_t mode)
 {
     const uint32_t total = prefix[B];
     for (uint32_t item = blockIdx.x; item < total; item += gridDim.x)
@@ -864,7 +866,7 @@ static __global__ __launch_bounds__(TILE) void kMarkB(const BatchCloud<T>* __res
         const uint32_t c        = findCloud(prefix, B, item);
         const BatchCloud<T>& cc = ctx[c];
         markTile<T>(item - prefix[c], 0, cc.wordsPerNode, cc.tileList, cc.segTile, cc.segCount, cc.segSrc,
-                    cc.segInput, cc.nodeGrid, cc.store(), cc.bitmap, cc.cellOf,
+                    cc.segInput, cc.nodeGrid, cc.store(), cellOrderOf(mode, cc.g), cc.bitmap, cc.cellOf,
                     reinterpret_cast<uint32_t*>(cc.sc + BS_ERROR));
     }
 }

@@ -420,8 +420,8 @@ void BatchBuilder::buildGroup(const std::vector<uint32_t>& members, const std::v
         const double cubicSize  = r.cloud.bbMax[0] - r.cloud.bbMin[0];  // metadata.cuh:66-69
         cc.n                    = r.cloud.pointAmount;
         cc.stride               = r.cloud.dataStride;
-        cc.grid                 = Gridding{r.cloud.bbMin[0], r.cloud.bbMin[1], r.cloud.bbMin[2], cubicSize,
-                                           r.proc.chunkingGrid};
+        cc.grid                 = gridding(r.cloud.bbMin[0], r.cloud.bbMin[1], r.cloud.bbMin[2], cubicSize,
+                                           r.proc.chunkingGrid);
         cc.sx                   = 1.0 / r.cloud.scale[0];  // octree_chunking.cu:108-112
         cc.sy                   = 1.0 / r.cloud.scale[1];
         cc.sz                   = 1.0 / r.cloud.scale[2];

@@ -489,8 +489,8 @@ void OctreeBuilder::countPoints()
     uint32_t* bucketCount  = itsBucketCount.as<uint32_t>();
     uint32_t* bucketStart  = itsBucketStart.as<uint32_t>();
     uint32_t* bucketCursor = itsBucketCursor.as<uint32_t>();
-    Gridding g{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2], itsCloud.bbMax[0] - itsCloud.bbMin[0],
-               itsProc.chunkingGrid};
+    const Gridding g = gridding(itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
+                                itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid);
     itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(nb) + 1));
     uint32_t* occ         = itsOccupancy.as<uint32_t>();
     const uint64_t words  = (static_cast<uint64_t>(itsDense) + 31) / 32;
@@ -702,8 +702,8 @@ uint64_t OctreeBuilder::placeChunkBound() const
 template <typename T>
 void OctreeBuilder::distributePoints()
 {
-    Gridding g{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2], itsCloud.bbMax[0] - itsCloud.bbMin[0],
-               itsProc.chunkingGrid};
+    const Gridding g = gridding(itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
+                                itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid);
     // octree_chunking.cu:108-112
     double sx = 1.0 / itsCloud.scale[0], sy = 1.0 / itsCloud.scale[1], sz = 1.0 / itsCloud.scale[2];
     const LeafOrderParams p = leafTables();
@@ -777,7 +777,7 @@ void OctreeBuilder::subsampleLevels()
     ps.stPts  = itsStPts.as<T>();
     ps.stRgb  = weighted ? itsStRgb.as<uint32_t>() : nullptr;
     ps.N      = N;
-    ps.cubic  = Gridding{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2], cubicSize, itsProc.chunkingGrid};
+    ps.cubic  = gridding(itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2], cubicSize, itsProc.chunkingGrid);
     ps.sx     = 1.0 / itsCloud.scale[0];
     ps.sy     = 1.0 / itsCloud.scale[1];
     ps.sz     = 1.0 / itsCloud.scale[2];
@@ -999,8 +999,8 @@ void OctreeBuilder::placeInternalNodes()
             list, nodes, N, itsNodeParent.as<int32_t>(), itsNodeChild.as<int32_t>(), itsNodePoints.as<uint32_t>(),
             itsNodeSub.as<uint32_t>(), itsNodeData.as<uint64_t>(), itsLeafList.as<uint64_t>(), chunks, itsStamps.as<uint64_t>() + ST_STAMPS * itsSteps);
     OC_LAUNCH_CHECK();
-    const Gridding cubic{itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
-                         itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid};
+    const Gridding cubic = gridding(itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
+                                    itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid);
     const double sx = 1.0 / itsCloud.scale[0], sy = 1.0 / itsCloud.scale[1], sz = 1.0 / itsCloud.scale[2];
     const uint32_t* rgb = itsColorMode == COLOR_INTER_WEIGHTED ? itsStRgb.as<uint32_t>() : nullptr;
     const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(placeChunkBound(), 1u << 20));

@@ -133,25 +133,38 @@ __device__ __forceinline__ void forRecords(const uint8_t* cloud, uint32_t n, uin
 
 // Cell coordinates of a point in a grid, with the reference's exact expression order
 // (kernel_helpers.cuh:11-25): t = bbSize / G; u = (p - min) / t; clamp to G - 1 with fmin;
-// truncate to int64, then reinterpret as uint64.
-__device__ __forceinline__ void gridCoords(double px, double py, double pz, const Gridding& g, uint64_t& ix,
-                                           uint64_t& iy, uint64_t& iz)
+// truncate to int64, then reinterpret as uint64. Returned in 32 bits: a coordinate outside the grid is
+// any value >= G.
+//
+// Four divisions and three 64-bit conversions are ~150 instructions (without them, 25.8M points: kMark
+// 506 -> 478 us, kDistributeSorted 278 -> 257; 119.7M: kDistributeSorted 1421 -> 1357). The product q = (p - min) * inv has three roundings where u has two, so
+// |u - q| <= 2^-50 |q| < 2^-30 for |q| < 2^20: unless q lies within 2^-30 of a whole number, u and q
+// truncate (and clamp) alike. A wave takes the divisions only where one of its points lies that close
+// to a cell face, far outside, or is not a number.
+__device__ __forceinline__ void gridCoords(double px, double py, double pz, const Gridding& g, uint32_t& ix,
+                                           uint32_t& iy, uint32_t& iz)
 {
-    double t  = g.bbSize / g.gridSize;
-    double uX = (px - g.minX) / t;
-    double uY = (py - g.minY) / t;
-    double uZ = (pz - g.minZ) / t;
-    t         = g.gridSize - 1.0;
-    ix        = static_cast<uint64_t>(static_cast<int64_t>(fmin(uX, t)));
-    iy        = static_cast<uint64_t>(static_cast<int64_t>(fmin(uY, t)));
-    iz        = static_cast<uint64_t>(static_cast<int64_t>(fmin(uZ, t)));
-}
-
-__device__ __forceinline__ uint32_t mapPointToGrid(double px, double py, double pz, const Gridding& g)
-{
-    uint64_t ix, iy, iz;
-    gridCoords(px, py, pz, g, ix, iy, iz);
-    return static_cast<uint32_t>(ix + iy * g.gridSize + iz * g.gridSize * g.gridSize);
+    constexpr double NEAR = 1.0 / (1u << 30), FAR = 1u << 20;
+    const double top = g.gridSize - 1.0;
+    const double dx = px - g.minX, dy = py - g.minY, dz = pz - g.minZ;
+    const double qx = dx * g.inv, qy = dy * g.inv, qz = dz * g.inv;
+    const double fx = qx - floor(qx), fy = qy - floor(qy), fz = qz - floor(qz);
+    // the sum is not below FAR where any of them is not a number
+    if (fabs(qx) + fabs(qy) + fabs(qz) < FAR && fmin(fmin(fx, fy), fz) > NEAR && fmax(fmax(fx, fy), fz) < 1.0 - NEAR)
+    {
+        ix = static_cast<uint32_t>(static_cast<int32_t>(fmin(qx, top)));
+        iy = static_cast<uint32_t>(static_cast<int32_t>(fmin(qy, top)));
+        iz = static_cast<uint32_t>(static_cast<int32_t>(fmin(qz, top)));
+        return;
+    }
+    const double t = g.bbSize / g.gridSize;
+    auto coord     = [&](double d) {
+        const uint64_t i = static_cast<uint64_t>(static_cast<int64_t>(fmin(d / t, top)));
+        return i < g.gridSize ? static_cast<uint32_t>(i) : ~0u;
+    };
+    ix = coord(dx);
+    iy = coord(dy);
+    iz = coord(dz);
 }
 
 // Packed colour (kernel_helpers.cuh:49-53): 18-bit r, g, b fields and a 10-bit count; sums wrap

@@ -757,11 +757,11 @@ static __global__ __launch_bounds__(BLOCK) void kDistributeSortedB(const BatchCl
         for (uint64_t s = lo + threadIdx.x; s < hi; s += BLOCK)
         {
             const SortedPoint<T> p = cc.sorted[s];
-            uint64_t ix, iy, iz;
+            uint32_t ix, iy, iz;
             gridCoords(static_cast<double>(p.x), static_cast<double>(p.y), static_cast<double>(p.z), g, ix, iy, iz);
             if (ix >= g.gridSize || iy >= g.gridSize || iz >= g.gridSize)
                 continue;  // only in-grid points are sorted
-            const uint32_t cell = static_cast<uint32_t>(ix + iy * g.gridSize + iz * g.gridSize * g.gridSize);
+            const uint32_t cell = ix + iy * g.gridSize + iz * g.gridSize * g.gridSize;
             const uint32_t leaf = cc.count[cell];
             const uint64_t pos  = cc.nodeData[leaf] + (s - cc.nodeSorted[leaf]);
             cc.lut[pos]         = p.idx;

@@ -117,11 +117,11 @@ __device__ __forceinline__ uint32_t sortBlockExclusiveScanN(uint32_t v, uint32_t
 // Level-0 Morton code of a point, or ~0u when it lies outside the grid.
 __device__ __forceinline__ uint32_t pointMorton(double x, double y, double z, const Gridding& g)
 {
-    uint64_t ix, iy, iz;
+    uint32_t ix, iy, iz;
     gridCoords(x, y, z, g, ix, iy, iz);
     if (ix >= g.gridSize || iy >= g.gridSize || iz >= g.gridSize)
         return ~0u;
-    return morton3(static_cast<uint32_t>(ix), static_cast<uint32_t>(iy), static_cast<uint32_t>(iz));
+    return morton3(ix, iy, iz);
 }
 
 template <typename T>
@@ -744,9 +744,9 @@ static __global__ __launch_bounds__(BLOCK) void kDistributeSorted(const SortedPo
     // the leaf's placement) issued for all of them before the next
     const uint64_t stride = globalStride();
     auto cellOf = [&](const SortedPoint<T>& p, uint32_t& cell) {
-        uint64_t ix, iy, iz;
+        uint32_t ix, iy, iz;
         gridCoords(static_cast<double>(p.x), static_cast<double>(p.y), static_cast<double>(p.z), g, ix, iy, iz);
-        cell = static_cast<uint32_t>(ix + iy * g.gridSize + iz * g.gridSize * g.gridSize);
+        cell = ix + iy * g.gridSize + iz * g.gridSize * g.gridSize;
         return ix < g.gridSize && iy < g.gridSize && iz < g.gridSize;  // only in-grid points are sorted
     };
     for (uint64_t s0 = globalThread(); s0 < n; s0 += stride * DIST_ITEMS)

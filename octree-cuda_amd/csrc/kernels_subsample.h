@@ -204,7 +204,7 @@ __device__ __forceinline__ Gridding nodeGridding(uint32_t lin, uint32_t gl, uint
         if ((z >> b) & 1)
             mz = mz + sideHalf[L];
     }
-    return Gridding{mx, my, mz, (mx + side) - mx, g};
+    return gridding(mx, my, mz, (mx + side) - mx, g);
 }
 
 // What one node's subsampling needs, from its key.
@@ -347,9 +347,9 @@ __device__ __forceinline__ uint32_t leafSlot(uint32_t key)
     return key + (key >> 5);
 }
 
-__device__ __forceinline__ uint32_t leafLocal(uint64_t i, uint32_t origin, uint32_t h)
+__device__ __forceinline__ uint32_t leafLocal(uint32_t i, uint32_t origin, uint32_t h)
 {
-    return i < origin ? 0u : static_cast<uint32_t>(i - origin < h ? i - origin : h - 1);
+    return i < origin ? 0u : i - origin < h ? i - origin : h - 1;
 }
 
 // Word key of a point: its cell in the parent grid (multiplied by 1 / t instead of divided by t:
@@ -359,15 +359,14 @@ __device__ __forceinline__ uint32_t leafLocal(uint64_t i, uint32_t origin, uint3
 struct LeafKeyer
 {
     Gridding grid;
-    double inv;  // gridSize / bbSize
     uint32_t ox, oy, oz, h, wordsPerRow, shift;
     CellOrder order;
     __device__ __forceinline__ uint32_t operator()(double x, double y, double z) const
     {
         const double top = grid.gridSize - 1.0;
-        const uint64_t ix = static_cast<uint64_t>(static_cast<int64_t>(fmin((x - grid.minX) * inv, top)));
-        const uint64_t iy = static_cast<uint64_t>(static_cast<int64_t>(fmin((y - grid.minY) * inv, top)));
-        const uint64_t iz = static_cast<uint64_t>(static_cast<int64_t>(fmin((z - grid.minZ) * inv, top)));
+        const uint32_t ix = static_cast<uint32_t>(static_cast<int32_t>(fmin((x - grid.minX) * grid.inv, top)));
+        const uint32_t iy = static_cast<uint32_t>(static_cast<int32_t>(fmin((y - grid.minY) * grid.inv, top)));
+        const uint32_t iz = static_cast<uint32_t>(static_cast<int32_t>(fmin((z - grid.minZ) * grid.inv, top)));
         const uint32_t lx = leafLocal(ix, ox, h), ly = leafLocal(iy, oy, h), lz = leafLocal(iz, oz, h);
         const uint32_t word = order == CELLS_MORTON ? morton3(lx, ly, lz) >> 5 : rowIndex(ly, lz, h) * wordsPerRow + (lx >> 5);
         return word >> shift;
@@ -405,7 +404,6 @@ __device__ __forceinline__ void leafCellOrderChunk(uint64_t entry, const LeafOrd
             pl = k;
     LeafKeyer keyer;
     keyer.grid = nodeGridding(pkey - p.offset[pl], p.grid[pl], pl, p.depth, p.cubicMin, p.sideHalf, p.side[pl], p.g);
-    keyer.inv  = keyer.grid.gridSize / keyer.grid.bbSize;
     // the leaf's octant of the parent grid: the low bit of its coordinates one level down
     const uint32_t ll = pl - 1, lgl = p.grid[ll], llin = nodeKey[leaf] - p.offset[ll];
     keyer.h           = p.g > 1 ? p.g / 2 : 1;  // cells per axis of the leaf's octant (1 for a 1-cell grid)
@@ -778,7 +776,7 @@ __device__ __forceinline__ void markTile(uint32_t tile, uint32_t nodeBase, uint6
         const NodeGrid ng = nodeGrid[in.k];
         T px, py, pz;
         ps.xyz(in.pos, px, py, pz);
-        uint64_t ix, iy, iz;
+        uint32_t ix, iy, iz;
         gridCoords(static_cast<double>(px), static_cast<double>(py), static_cast<double>(pz), ng.grid, ix, iy, iz);
         const uint32_t gs = ng.grid.gridSize;
         if (ix >= gs || iy >= gs || iz >= gs)
@@ -789,7 +787,7 @@ __device__ __forceinline__ void markTile(uint32_t tile, uint32_t nodeBase, uint6
         }
         else
         {
-            cell = cellIndex(static_cast<uint32_t>(ix), static_cast<uint32_t>(iy), static_cast<uint32_t>(iz), gs, order);
+            cell         = cellIndex(ix, iy, iz, gs, order);
             cellOf[in.q] = cell;
         }
     }

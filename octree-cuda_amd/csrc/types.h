@@ -40,7 +40,13 @@ struct Gridding
     double minX, minY, minZ;
     double bbSize;
     uint32_t gridSize;
+    double inv;  // gridSize / bbSize, rounded
 };
+
+constexpr Gridding gridding(double minX, double minY, double minZ, double bbSize, uint32_t gridSize)
+{
+    return Gridding{minX, minY, minZ, bbSize, gridSize, gridSize / bbSize};
+}
 static_assert(offsetof(Gridding, minY) == sizeof(double) && offsetof(Gridding, minZ) == 2 * sizeof(double),
               "the cubic minimum is read as three consecutive doubles");
 

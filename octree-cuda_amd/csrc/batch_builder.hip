@@ -170,12 +170,12 @@ void carveCloud(Carver& cv, BatchCloud<T>& cc, const BatchRequest& r, const Clou
     cv.take(cc.lut, s.E);
     cv.take(cc.out, s.E);
     cv.take(cc.stLut, s.staged);
-    cv.take(cc.stOut, s.staged);
     cv.take(cc.stPts, 3 * s.staged);
-    if (mode == COLOR_INTER_WEIGHTED)
-        cv.take(cc.stRgb, s.staged);
+    cc.staged = StagedColors{};
+    if (packedColors(mode))
+        cv.take(cc.staged.packed, s.staged);
     else
-        cc.stRgb = nullptr;
+        cv.take(cc.staged.rgb, s.staged);
     cv.take(cc.internalList, s.kBound);
     cv.take(cc.segCount, 8 * s.kBound);
     cv.take(cc.segSrc, 8 * s.kBound);
@@ -339,6 +339,8 @@ uint64_t BatchBuilder::estimateFootprint(const std::vector<BatchRequest>& reques
             carveCloud(cv, cc, r, s, L, mode, &copy);
             carveNodes(cv, cc, std::min<uint64_t>(s.mBound, 2 * s.n + 16), s);
         }
+        // admission charges a staged point its whole record (and the weighted filter's colour)
+        bytes += s.staged * (sizeof(OutRecord) - (packedColors(mode) ? 8 : mode == COLOR_NONE ? 4 : 0));
         bytes += cv.off + BS_SLOTS * 8 + 4096;
     }
     return bytes;

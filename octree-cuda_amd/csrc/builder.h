@@ -123,6 +123,7 @@ private:
     struct LevelParams levelParams() const;
     struct ChildSlots childSlots(uint32_t firstInternal) const;
     struct LeafOrderParams leafTables();
+    struct StagedColors stagedColors() const;
     uint32_t stepNodes() const;
     uint32_t planSteps();
     uint64_t leafChunkBound() const;
@@ -190,7 +191,7 @@ private:
     // output region [0, E) (lut: point index, out: 18-byte record): leaf points at [0, N), internal
     // subsamples at [N, N + I) after the final placement. Staging (st*): subsampled points in
     // level order, read by the next level, placed at the end.
-    DeviceBuffer itsLut, itsOut, itsStLut, itsStOut, itsStPts, itsStRgb;
+    DeviceBuffer itsLut, itsOut, itsStLut, itsStPts, itsStColor;
 
     // per-level subsampling workspace: internal node list, input segments and tiles, per-node
     // occupancy bitmaps with their popcount prefix, per-cell (dense index) state, per-input state

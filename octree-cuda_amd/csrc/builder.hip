@@ -235,10 +235,8 @@ void OctreeBuilder::setup(const CloudInfo& cloud, const ProcessingInfo& proc, co
     itsBucketCursor.ensure(sizeof(uint32_t) * (itsBuckets + 1));
     itsBucketList.ensure(sizeof(uint32_t) * itsBuckets);
     itsStLut.ensure(sizeof(uint32_t) * stagedCap);
-    itsStOut.ensure(sizeof(OutRecord) * stagedCap);
     itsStPts.ensure(coordBytes * stagedCap);
-    if (itsColorMode == COLOR_INTER_WEIGHTED)
-        itsStRgb.ensure(sizeof(uint32_t) * stagedCap);
+    itsStColor.ensure(sizeof(OutRecord) * stagedCap);  // what the footprint charges a staged point
     itsScalars.ensure(sizeof(uint64_t) * SC_COUNT);
     // The output starts zeroed (the tail past N + I stays zero, A15). The fill goes on the copy
     // stream, behind the previous build's snapshot copies that still read the output; the build
@@ -260,7 +258,7 @@ std::vector<DeviceBuffer*> OctreeBuilder::arena()
             &itsNodeStage,   &itsNodeSub,     &itsBucketed,     &itsSorted,      &itsFineCode,
             &itsPerm,
             &itsBucketCount, &itsBucketStart, &itsBucketCursor,  &itsBucketList,  &itsLut,          &itsOut,
-            &itsStLut,       &itsStOut,       &itsStPts,         &itsStRgb,        &itsInternalList, &itsSegCount,    &itsSegSrc,
+            &itsStLut,       &itsStPts,       &itsStColor,       &itsInternalList, &itsSegCount,    &itsSegSrc,
             &itsSegTile,     &itsSegInput,    &itsNodeGrid,      &itsTileList,     &itsBitmap,      &itsPrefix,
             &itsCursors,     &itsStamps,      &itsWin,         &itsColor,         &itsCellCnt,      &itsCellStart,   &itsCellKey,
             &itsCellNode,    &itsCellOf,      &itsRankOf,        &itsPayload,      &itsScalars,
@@ -728,6 +726,12 @@ void OctreeBuilder::distributePoints()
     OC_LAUNCH_CHECK();
 }
 
+StagedColors OctreeBuilder::stagedColors() const
+{
+    const bool packed = packedColors(itsColorMode);
+    return StagedColors{packed ? nullptr : itsStColor.as<uint32_t>(), packed ? itsStColor.as<uint64_t>() : nullptr};
+}
+
 // Nodes of one subsampling step: their bitmaps and prefixes fit kBitmapBudget.
 uint32_t OctreeBuilder::stepNodes() const
 {
@@ -768,19 +772,14 @@ void OctreeBuilder::subsampleLevels()
     const uint64_t cellsPerNode = rowsPerNode(g) * g;
     const uint64_t wordsPerNode = (cellsPerNode + 31) / 32;
     const uint32_t batchNodes   = stepNodes();
-    const bool packed   = itsColorMode == COLOR_INTRA || itsColorMode == COLOR_INTER;
+    const bool packed   = packedColors(itsColorMode);
     const bool weighted = itsColorMode == COLOR_INTER_WEIGHTED;
     PointStore<T> ps{};
     ps.sorted = itsSorted.as<SortedPoint<T>>();
     ps.stLut  = itsStLut.as<uint32_t>();
-    ps.stOut  = itsStOut.as<OutRecord>();
     ps.stPts  = itsStPts.as<T>();
-    ps.stRgb  = weighted ? itsStRgb.as<uint32_t>() : nullptr;
+    ps.staged = stagedColors();
     ps.N      = N;
-    ps.cubic  = gridding(itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2], cubicSize, itsProc.chunkingGrid);
-    ps.sx     = 1.0 / itsCloud.scale[0];
-    ps.sy     = 1.0 / itsCloud.scale[1];
-    ps.sz     = 1.0 / itsCloud.scale[2];
 
     SubsampleParams sp{};
     for (int a = 0; a < 3; ++a)
@@ -1002,18 +1001,17 @@ void OctreeBuilder::placeInternalNodes()
     const Gridding cubic = gridding(itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
                                     itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid);
     const double sx = 1.0 / itsCloud.scale[0], sy = 1.0 / itsCloud.scale[1], sz = 1.0 / itsCloud.scale[2];
-    const uint32_t* rgb = itsColorMode == COLOR_INTER_WEIGHTED ? itsStRgb.as<uint32_t>() : nullptr;
     const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(placeChunkBound(), 1u << 20));
     if (itsCloud.cloudType == CLOUD_FLOAT_UINT8_T)
         kPermute<float><<<grid, BLOCK, 0, itsStream>>>(
                 itsLeafList.as<uint64_t>(), chunks, N, itsNodeStage.as<uint32_t>(), itsNodeData.as<uint64_t>(),
-                itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(), itsStOut.as<OutRecord>(),
-                itsStPts.as<float>(), rgb, cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
+                itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(),
+                itsStPts.as<float>(), stagedColors(), cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
     else
         kPermute<double><<<grid, BLOCK, 0, itsStream>>>(
                 itsLeafList.as<uint64_t>(), chunks, N, itsNodeStage.as<uint32_t>(), itsNodeData.as<uint64_t>(),
-                itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(), itsStOut.as<OutRecord>(),
-                itsStPts.as<double>(), rgb, cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
+                itsNodePoints.as<uint32_t>(), itsStLut.as<uint32_t>(),
+                itsStPts.as<double>(), stagedColors(), cubic, sx, sy, sz, itsLut.as<uint32_t>(), itsOut.as<OutRecord>());
     OC_LAUNCH_CHECK();
 }
 

@@ -237,11 +237,53 @@ __device__ __forceinline__ void storeRecord(OutRecord* dst, const OutRecord& r)
     __builtin_memcpy(dst, &r, sizeof(OutRecord));
 }
 
-__device__ __forceinline__ OutRecord loadRecord(const OutRecord* src)
+// Output records of a wave, put in place through LDS: stored by their own lanes they are 18 bytes apart,
+// and each of the five stores of a lane touches the same ten lines again.
+struct OutStage
 {
-    OutRecord r;
-    __builtin_memcpy(&r, src, sizeof(OutRecord));
-    return r;
+    uint32_t word[64 * sizeof(OutRecord) / 4 + 1];
+};
+
+// Lane i's record to dst[i], i < count <= 64, dst at an even address: every lane writes its record at its
+// place of the wave's stage (as four words and a half, whichever comes first at its alignment), then the
+// wave stores consecutive words. All lanes of the wave take part.
+__device__ __forceinline__ void storeRecords(OutRecord* dst, const OutRecord& r, uint32_t count, OutStage& stage)
+{
+    const uint32_t lane  = threadIdx.x & 63;
+    const uint64_t begin = reinterpret_cast<uint64_t>(dst);
+    const uint32_t skip  = static_cast<uint32_t>(begin & 2);
+    const uint32_t end   = skip + count * static_cast<uint32_t>(sizeof(OutRecord));
+    uint16_t* halves     = reinterpret_cast<uint16_t*>(stage.word);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < count)
+    {
+        const uint32_t at   = skip + lane * static_cast<uint32_t>(sizeof(OutRecord));
+        const bool half     = (at & 2) != 0;  // the record starts with the second half of a word
+        const uint32_t v[5] = {static_cast<uint32_t>(r.x), static_cast<uint32_t>(r.y), static_cast<uint32_t>(r.z),
+                               r.r | (static_cast<uint32_t>(r.g) << 16), r.b};
+        uint32_t* w         = stage.word + ((at + 2) >> 2);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            w[k] = half ? __builtin_amdgcn_alignbyte(v[k + 1], v[k], 2) : v[k];
+        halves[(at >> 1) + (half ? 0 : 8)] = static_cast<uint16_t>(half ? v[0] : v[4]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t* out = reinterpret_cast<uint32_t*>(begin - skip);
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+    {
+        const uint32_t i = lane + 64 * k;
+        if (4 * i >= skip && 4 * i + 4 <= end)
+            out[i] = stage.word[i];
+    }
+    if (count && lane == 0)  // halves of words that other records share
+    {
+        if (skip)
+            reinterpret_cast<uint16_t*>(out)[1] = halves[1];
+        if (end & 2)
+            reinterpret_cast<uint16_t*>(out)[(end >> 1) - 1] = halves[(end >> 1) - 1];
+    }
 }
 
 // Wave-level runs: consecutive lanes holding equal keys (inputs arrive spatially sorted, so lanes

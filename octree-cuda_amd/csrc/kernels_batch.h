@@ -90,9 +90,8 @@ struct BatchCloud
     uint32_t* lut;
     OutRecord* out;
     uint32_t* stLut;
-    OutRecord* stOut;
     T* stPts;
-    uint32_t* stRgb;
+    StagedColors staged;
     // per-level work
     uint32_t *internalList, *segCount, *segSrc, *segTile, *segInput, *tileList;
     NodeGrid* nodeGrid;
@@ -110,14 +109,9 @@ struct BatchCloud
         PointStore<T> ps;
         ps.sorted = sorted;
         ps.stLut  = stLut;
-        ps.stOut  = stOut;
         ps.stPts  = stPts;
-        ps.stRgb  = stRgb;
+        ps.staged = staged;
         ps.N      = n;
-        ps.cubic  = grid;
-        ps.sx     = sx;
-        ps.sy     = sy;
-        ps.sz     = sz;
         return ps;
     }
 };
@@ -1050,13 +1044,14 @@ template <typename T>
 static __global__ __launch_bounds__(BLOCK) void kPermuteB(const BatchCloud<T>* __restrict__ ctx, uint32_t B,
                                                     const uint32_t* __restrict__ prefix)
 {
+    __shared__ OutStage lds[BLOCK / 64];
     const uint32_t total = prefix[B];
     for (uint32_t item = blockIdx.x; item < total; item += gridDim.x)
     {
         const uint32_t c        = findCloud(prefix, B, item);
         const BatchCloud<T>& cc = ctx[c];
         permuteChunk<T>(cc.chunkList[item - prefix[c]], cc.n, cc.nodeStage, cc.nodeData, cc.nodePoints, cc.stLut,
-                        cc.stOut, cc.stPts, cc.stRgb, cc.grid, cc.sx, cc.sy, cc.sz, cc.lut, cc.out);
+                        cc.stPts, cc.staged, cc.grid, cc.sx, cc.sy, cc.sz, cc.lut, cc.out, lds[threadIdx.x >> 6]);
     }
 }
 

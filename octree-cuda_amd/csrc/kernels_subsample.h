@@ -100,40 +100,44 @@ __device__ __forceinline__ uint32_t cellIndex(uint32_t x, uint32_t y, uint32_t z
     return order == CELLS_MORTON ? morton3(x, y, z) : rowIndex(y, z, g) * g + x;
 }
 
+// Colours of the staged points. An average of packed sums can take 16 bits (their fields wrap), so the
+// filters on packed sums keep the packed form; no filter and the distance-weighted one keep 8 bits each.
+struct StagedColors
+{
+    uint32_t* rgb;     // r | g << 8 | b << 16, or null
+    uint64_t* packed;  // encodeColors, or null
+};
+
 // The points a subsampling level reads: leaf points at positions [0, N) of the sorted cloud (a
 // leaf's points are one contiguous range there) and already subsampled points of lower
 // levels at positions [N, N + I) (staging, in level order until the final DFS post-order
-// placement). A leaf point's output record is derived from its sorted record exactly as the
-// distribution writes it.
+// placement). A staged point is its index, exact coordinates and colour; its output record is derived
+// from them by the placement exactly as a leaf point's is by the distribution (kept as records of 18
+// bytes beside the coordinates, a level wrote 34 bytes per float point instead of 20 to 24).
 template <typename T>
 struct PointStore
 {
     const SortedPoint<T>* sorted;
     uint32_t* stLut;
-    OutRecord* stOut;
     T* stPts;
-    uint32_t* stRgb;  // distance-weighted filter: staged colours r | g << 8 | b << 16 (8 bits each)
+    StagedColors staged;
     uint32_t N;
-    Gridding cubic;
-    double sx, sy, sz;
     __device__ __forceinline__ uint32_t index(uint32_t pos) const
     {
         return pos < N ? sorted[pos].idx : stLut[pos - N];
     }
-    __device__ __forceinline__ OutRecord record(uint32_t pos) const
-    {
-        if (pos < N)
-        {
-            const SortedPoint<T>& p = sorted[pos];
-            return quantizePoint(p.x, p.y, p.z, p.rgb, cubic, sx, sy, sz);
-        }
-        return loadRecord(stOut + (pos - N));
-    }
-    // the point's colour r | g << 8 | b << 16, the low 8 bits of each channel (distance-weighted
-    // filter only: a staged point's colour comes from stRgb, 4 bytes instead of its 18-byte record)
+    // r | g << 8 | b << 16 (no filter, distance-weighted filter)
     __device__ __forceinline__ uint32_t rgb(uint32_t pos) const
     {
-        return pos < N ? sorted[pos].rgb : stRgb[pos - N];
+        return pos < N ? sorted[pos].rgb : staged.rgb[pos - N];
+    }
+    // encodeColors (filters on packed sums)
+    __device__ __forceinline__ uint64_t packed(uint32_t pos) const
+    {
+        if (pos >= N)
+            return staged.packed[pos - N];
+        const uint32_t c = sorted[pos].rgb;
+        return encodeColors(c & 0xFF, (c >> 8) & 0xFF, (c >> 16) & 0xFF);
     }
     __device__ __forceinline__ void xyz(uint32_t pos, T& x, T& y, T& z) const
     {
@@ -970,10 +974,7 @@ __device__ __forceinline__ void accumulateTile(uint32_t tile, uint32_t nodeBase,
         const uint32_t rank = RANDOM ? fmix32(idx ^ nodeGrid[in.k].salt) : idx;
         key                 = (static_cast<uint64_t>(rank) << 32) | in.pos;
         if (MODE == COLOR_INTRA || MODE == COLOR_INTER)
-        {
-            const OutRecord r = ps.record(in.pos);
-            col               = encodeColors(r.r, r.g, r.b);
-        }
+            col = ps.packed(in.pos);
     }
     key = runScan<uint64_t>(key, run, [](uint64_t x, uint64_t y) { return x < y ? x : y; });
     if (MODE == COLOR_INTRA || MODE == COLOR_INTER)
@@ -1171,12 +1172,10 @@ __device__ __forceinline__ void emitCell(uint32_t c, uint32_t nodeBase, uint64_t
     {
         const uint32_t kl = cellNode[c];
         const NodeGrid ng = nodeGrid[nodeBase + kl];
-        OutRecord rec{};
+        uint64_t sum      = 0;  // packed colours
 
         if (MODE == COLOR_INTRA)
-        {
-            decodeColors(color[c], rec.r, rec.g, rec.b);
-        }
+            sum = color[c];
         else if (MODE == COLOR_INTER)
         {
             const uint32_t key    = cellKey[c];
@@ -1189,7 +1188,6 @@ __device__ __forceinline__ void emitCell(uint32_t c, uint32_t nodeBase, uint64_t
             const int32_t x0 = cx > 0 ? cx - 1 : 0;
             const int32_t x1 = cx + 1 < static_cast<int32_t>(gs) ? cx + 1 : cx;
             const uint32_t span = static_cast<uint32_t>(x1 - x0 + 1);
-            uint64_t sum        = 0;
 #pragma unroll
             for (int r = 0; r < 9; ++r)
             {
@@ -1215,22 +1213,17 @@ __device__ __forceinline__ void emitCell(uint32_t c, uint32_t nodeBase, uint64_t
                 if (n > 2)
                     sum += color[first + 2];
             }
-            decodeColors(sum, rec.r, rec.g, rec.b);
         }
         const uint32_t wpos = static_cast<uint32_t>(win[c] & 0xFFFFFFFFull);
-        OutRecord wrec      = ps.record(wpos);
+        const uint32_t st   = cursor - ps.N + c;  // staging index
         if (MODE == COLOR_NONE)
-        {
-            rec = wrec;
-        }
+            ps.staged.rgb[st] = ps.rgb(wpos);
         else
         {
-            rec.x = wrec.x;
-            rec.y = wrec.y;
-            rec.z = wrec.z;
+            uint16_t r, g, b;
+            decodeColors(sum, r, g, b);
+            ps.staged.packed[st] = encodeColors(r, g, b);
         }
-        const uint32_t st = cursor - ps.N + c;  // staging index
-        storeRecord(ps.stOut + st, rec);
         ps.stLut[st] = ps.index(wpos);
         T* d         = ps.stPts + 3 * static_cast<uint64_t>(st);
         ps.xyz(wpos, d[0], d[1], d[2]);
@@ -1406,7 +1399,7 @@ __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, 
     const uint32_t cb = static_cast<uint16_t>(acc[2] / acc[3]);
     const uint32_t st = cursor - ps.N + c;  // staging index
     ps.stLut[st] = bestIdx;
-    ps.stRgb[st] = (cr & 0xFF) | ((cg & 0xFF) << 8) | ((cb & 0xFF) << 16);
+    ps.staged.rgb[st] = (cr & 0xFF) | ((cg & 0xFF) << 8) | ((cb & 0xFF) << 16);
     T* d         = ps.stPts + 3 * static_cast<uint64_t>(st);
     d[0]         = bx;
     d[1]         = by;
@@ -1517,10 +1510,9 @@ template <typename T>
 __device__ __forceinline__ void permuteChunk(uint64_t entry, uint32_t N, const uint32_t* __restrict__ stage,
                                              const uint64_t* __restrict__ dataIdx,
                                              const uint32_t* __restrict__ pointCount,
-                                             const uint32_t* __restrict__ stLut, const OutRecord* __restrict__ stOut,
-                                             const T* __restrict__ stPts, const uint32_t* __restrict__ stRgb,
-                                             const Gridding& cubic, double sx, double sy, double sz,
-                                             uint32_t* __restrict__ lut, OutRecord* __restrict__ out)
+                                             const uint32_t* __restrict__ stLut, const T* __restrict__ stPts,
+                                             const StagedColors& staged, const Gridding& cubic, double sx, double sy, double sz,
+                                             uint32_t* __restrict__ lut, OutRecord* __restrict__ out, OutStage& lds)
 {
     const uint32_t id    = static_cast<uint32_t>(entry);
     const uint32_t first = static_cast<uint32_t>(entry >> 32) * PLACE_CHUNK;
@@ -1528,17 +1520,26 @@ __device__ __forceinline__ void permuteChunk(uint64_t entry, uint32_t N, const u
     const uint32_t cnt   = total - first < PLACE_CHUNK ? total - first : PLACE_CHUNK;
     const uint64_t src   = static_cast<uint64_t>(stage[id]) - N + first;  // staging index of the chunk
     const uint64_t dst   = dataIdx[id] + first;
-    for (uint32_t j = threadIdx.x; j < cnt; j += BLOCK)
+    const uint32_t lane  = threadIdx.x & 63;
+    for (uint32_t base = threadIdx.x - lane; base < cnt; base += BLOCK)
     {
-        const uint64_t s = src + j;
-        lut[dst + j]     = stLut[s];
-        if (stRgb)  // distance-weighted filter: the record from the staged coordinates and colour
+        const uint32_t count = cnt - base < 64 ? cnt - base : 64u;
+        OutRecord r{};
+        if (lane < count)
         {
-            const T* q = stPts + 3 * s;
-            storeRecord(out + dst + j, quantizePoint(q[0], q[1], q[2], stRgb[s], cubic, sx, sy, sz));
+            const uint64_t s     = src + base + lane;
+            lut[dst + base + lane] = stLut[s];
+            const T* q           = stPts + 3 * s;
+            r                    = quantizePoint(q[0], q[1], q[2], staged.rgb ? staged.rgb[s] : 0u, cubic, sx, sy, sz);
+            if (staged.packed)
+            {
+                const uint64_t c = staged.packed[s];
+                r.r              = static_cast<uint16_t>(c >> 46);
+                r.g              = static_cast<uint16_t>(c >> 28);
+                r.b              = static_cast<uint16_t>(c >> 10);
+            }
         }
-        else
-            storeRecord(out + dst + j, loadRecord(stOut + s));
+        storeRecords(out + dst + base, r, count, lds);
     }
 }
 
@@ -1549,15 +1550,15 @@ static __global__ __launch_bounds__(BLOCK) void kPermute(const uint64_t* __restr
                                                    const uint64_t* __restrict__ dataIdx,
                                                    const uint32_t* __restrict__ pointCount,
                                                    const uint32_t* __restrict__ stLut,
-                                                   const OutRecord* __restrict__ stOut, const T* __restrict__ stPts,
-                                                   const uint32_t* __restrict__ stRgb, Gridding cubic, double sx,
-                                                   double sy, double sz, uint32_t* __restrict__ lut,
+                                                   const T* __restrict__ stPts, StagedColors staged, Gridding cubic,
+                                                   double sx, double sy, double sz, uint32_t* __restrict__ lut,
                                                    OutRecord* __restrict__ out)
 {
+    __shared__ OutStage lds[BLOCK / 64];
     const uint32_t all = *chunks;
     for (uint32_t c = blockIdx.x; c < all; c += gridDim.x)
-        permuteChunk<T>(chunkList[c], N, stage, dataIdx, pointCount, stLut, stOut, stPts, stRgb, cubic, sx, sy, sz,
-                        lut, out);
+        permuteChunk<T>(chunkList[c], N, stage, dataIdx, pointCount, stLut, stPts, staged, cubic, sx, sy, sz, lut, out,
+                        lds[threadIdx.x >> 6]);
 }
 
 }  // namespace oc

@@ -73,6 +73,12 @@ enum ColorMode : uint32_t
     COLOR_INTER_WEIGHTED = 3
 };
 
+// filters on packed colour sums per cell
+constexpr bool packedColors(ColorMode mode)
+{
+    return mode == COLOR_INTRA || mode == COLOR_INTER;
+}
+
 constexpr uint32_t MAX_LEVELS = 10;  // chunking grid 512 -> depth 9 -> levels 0..9
 
 }  // namespace oc

@@ -832,6 +832,10 @@ void OctreeBuilder::subsampleLevels()
     uint32_t* prefix  = itsPrefix.as<uint32_t>();
     const CellState cellState{win, color, cellCnt};
 
+    // tiles combined in LDS, where there are enough points for them and the flag bit is free
+    const bool large          = N >= LARGE_POINTS && N < NOT_OWNED && 32 * wordsPerNode < NOT_OWNED;
+    const uint32_t tileInputs = large ? LARGE_TILE : TILE;
+    const int tileThreads     = large ? LARGE_THREADS : static_cast<int>(TILE);
     uint32_t stepAt = 0;
     for (uint32_t l = 1; l <= itsDepth; ++l)
     {
@@ -840,7 +844,7 @@ void OctreeBuilder::subsampleLevels()
             continue;
         const ChildSlots cs        = childSlots(itsInner[l]);
         NodeGrid* nodeGrid         = itsNodeGrid.as<NodeGrid>();
-        const LevelSegmentIn segIn{cs, itsNodePoints.as<uint32_t>()};
+        const LevelSegmentIn segIn{cs, itsNodePoints.as<uint32_t>(), tileInputs};
         const LevelSegmentOut segOut{cs, itsNodeSorted.as<uint32_t>(), itsNodeStage.as<uint32_t>(),
                                      itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                                      itsSegInput.as<uint32_t>()};
@@ -860,7 +864,8 @@ void OctreeBuilder::subsampleLevels()
             waitMailbox(seq);
             inputMost = itsMailbox[MAIL_INPUTS];
         }
-        const uint32_t tileGrid = xcdRunGrid(inputMost / TILE + 8ull * K, XCD_TILE_RUN);
+        const uint32_t parts    = tileInputs / TILE;
+        const uint32_t tileGrid = xcdRunGrid(inputMost / tileInputs + 8ull * K, XCD_TILE_RUN / parts);
         sp.level       = l;
         sp.levelOffset = itsLevelOffset[l];
         sp.levelGrid   = itsLevelGrid[l];
@@ -879,7 +884,7 @@ void OctreeBuilder::subsampleLevels()
             uint64_t* stamps = itsStamps.as<uint64_t>() + ST_STAMPS * stepAt;
             ++stepAt;
 
-            const bool resetInputs = words <= RESET_INPUTS_WORDS;
+            const bool resetInputs = !large && words <= RESET_INPUTS_WORDS;
             const unsigned prepareGrid = gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384);
             if (oneLaunch)
                 kLevelStart<<<std::min(prepareGrid, 2048u), BLOCK, 0, itsStream>>>(
@@ -891,11 +896,14 @@ void OctreeBuilder::subsampleLevels()
                         sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs,
                         stamps + ST_BEGIN);
             OC_LAUNCH_CHECK();
-            kMark<T><<<tileGrid, TILE, 0, itsStream>>>(
-                    tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                    itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid, ps,
-                    cellOrderOf(itsColorMode, g), bitmap, itsCellOf.as<uint32_t>(), err, stamps + ST_INSERT_BEGIN);
-            OC_LAUNCH_CHECK();
+            auto mark = [&](auto kernel) {
+                kernel<<<tileGrid, tileThreads, 0, itsStream>>>(
+                        tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                        itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid, ps,
+                        cellOrderOf(itsColorMode, g), bitmap, itsCellOf.as<uint32_t>(), err, stamps + ST_INSERT_BEGIN);
+                OC_LAUNCH_CHECK();
+            };
+            mark(large ? kMarkLarge<T> : kMark<T>);
             const uint64_t wordTiles = scanTiles(words);
             uint32_t* rangeSums      = itsScanScratch.as<uint32_t>();
             if (wordTiles <= SCAN_DIRECT_TILES)
@@ -910,14 +918,14 @@ void OctreeBuilder::subsampleLevels()
                                                                   prefix);
             }
             OC_LAUNCH_CHECK();
-            if (!resetInputs)
+            if (!large && !resetInputs)
             {
                 kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(step.cells, cellState);
                 OC_LAUNCH_CHECK();
             }
 
             auto accumulate = [&](auto kernel) {
-                kernel<<<tileGrid, TILE, 0, itsStream>>>(
+                kernel<<<tileGrid, tileThreads, 0, itsStream>>>(
                         tiles, step, k0, Kb, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                         itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
                         bitmap, prefix, itsCellOf.as<uint32_t>(), ps, win, color, cellCnt, itsCellKey.as<uint32_t>(),
@@ -926,20 +934,34 @@ void OctreeBuilder::subsampleLevels()
                         itsNodeFlags.as<uint8_t>(), itsNodeChild.as<int32_t>(), err);
                 OC_LAUNCH_CHECK();
             };
+            auto rest = [&](auto kernel) {
+                kernel<<<tileGrid, tileThreads, 0, itsStream>>>(
+                        tiles, step, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                        itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
+                        bitmap, prefix, itsCellOf.as<uint32_t>(), ps, win, color, cellCnt,
+                        weighted ? itsRankOf.as<uint32_t>() : nullptr);
+                OC_LAUNCH_CHECK();
+            };
+            auto accumulateMode = [&](auto mode, auto random) {
+                constexpr uint32_t M = decltype(mode)::value;
+                constexpr bool R     = decltype(random)::value;
+                accumulate(large ? kAccumulateLarge<T, M, R> : kAccumulate<T, M, R>);
+                if (large)
+                    rest(kAccumulateRest<T, M, R>);
+            };
+            auto accumulateAll = [&](auto mode) {
+                if (itsProc.useRandomSubsampling)
+                    accumulateMode(mode, std::true_type{});
+                else
+                    accumulateMode(mode, std::false_type{});
+            };
             const bool random = itsProc.useRandomSubsampling;
             switch (itsColorMode)
             {
-            case COLOR_NONE: accumulate(random ? kAccumulate<T, COLOR_NONE, true> : kAccumulate<T, COLOR_NONE, false>); break;
-            case COLOR_INTRA:
-                accumulate(random ? kAccumulate<T, COLOR_INTRA, true> : kAccumulate<T, COLOR_INTRA, false>);
-                break;
-            case COLOR_INTER:
-                accumulate(random ? kAccumulate<T, COLOR_INTER, true> : kAccumulate<T, COLOR_INTER, false>);
-                break;
-            default:
-                accumulate(random ? kAccumulate<T, COLOR_INTER_WEIGHTED, true>
-                                  : kAccumulate<T, COLOR_INTER_WEIGHTED, false>);
-                break;
+            case COLOR_NONE: accumulateAll(std::integral_constant<uint32_t, COLOR_NONE>{}); break;
+            case COLOR_INTRA: accumulateAll(std::integral_constant<uint32_t, COLOR_INTRA>{}); break;
+            case COLOR_INTER: accumulateAll(std::integral_constant<uint32_t, COLOR_INTER>{}); break;
+            default: accumulateAll(std::integral_constant<uint32_t, COLOR_INTER_WEIGHTED>{}); break;
             }
 
             if (weighted)
@@ -949,11 +971,11 @@ void OctreeBuilder::subsampleLevels()
                                         itsScanScratch.as<uint32_t>(), static_cast<uint32_t*>(nullptr), itsStream);
                 OC_LAUNCH_CHECK();
                 auto scatter = [&](auto kernel) {
-                    kernel<<<tileGrid, TILE, 0, itsStream>>>(
+                    kernel<<<tileGrid * parts, TILE, 0, itsStream>>>(
                             tiles, step, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                             itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
                             itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(), itsCellStart.as<uint32_t>(),
-                            itsCellOf.as<uint32_t>(), ps, itsPayload.as<WeightPayload>(), winKey,
+                            itsCellOf.as<uint32_t>(), ps, itsPayload.as<WeightPayload>(), winKey, parts,
                             stamps + ST_INSERT_END);
                     OC_LAUNCH_CHECK();
                 };

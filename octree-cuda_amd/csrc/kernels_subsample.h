@@ -10,6 +10,7 @@
 //   prefix scan  popcounts of all bitmap words -> dense index of every occupied cell
 //   kAccumulate  winner per cell (atomicMin of rank<<32 | input position), packed colour sums,
 //                per-cell point counts for the weighted filter
+//   (kMarkLarge, kAccumulateLarge and kAccumulateRest in large builds)
 //   kScatterPayload (weighted only) each point's offset from its cell centre + colour, and its
 //                winner key, in cell order
 //   kEmit        one output record per occupied cell, in ascending cell order per node
@@ -579,11 +580,12 @@ struct LevelSegmentIn
 {
     ChildSlots cs;
     const uint32_t* pointCount;
+    uint32_t tile;  // inputs per tile
     __device__ uint64_t operator()(uint64_t s) const
     {
         const int32_t c  = cs.child(s);
         const uint64_t n = c >= 0 ? pointCount[c] : 0u;
-        return (((n + TILE - 1) / TILE) << 32) | n;
+        return (((n + tile - 1) / tile) << 32) | n;
     }
 };
 
@@ -740,7 +742,8 @@ struct StepSizes
 
 constexpr uint64_t CURSOR_FULL = 1ull << 62;
 
-// Identifies the input of this thread: tile -> segment -> (node k, input position, input index q).
+// Identifies the input of this thread: tile -> segment -> (node k, input position, input index q). Large
+// tiles are read in parts of TILE inputs; `tile` then counts the parts.
 struct InputRef
 {
     uint32_t seg, local, k, pos, q;
@@ -749,11 +752,11 @@ struct InputRef
 
 __device__ __forceinline__ InputRef inputOf(uint32_t tile, const uint32_t* tileList, const uint32_t* segTile,
                                             const uint32_t* segCount, const uint32_t* segSrc,
-                                            const uint32_t* segInput)
+                                            const uint32_t* segInput, uint32_t parts = 1)
 {
     InputRef r;
-    r.seg   = tileList[tile];
-    r.local = (tile - segTile[r.seg]) * TILE + threadIdx.x;
+    r.seg   = tileList[tile / parts];
+    r.local = (tile - segTile[r.seg] * parts) * TILE + threadIdx.x;
     r.valid = r.local < segCount[r.seg];
     r.k     = r.seg >> 3;
     r.pos   = segSrc[r.seg] + r.local;
@@ -821,6 +824,151 @@ static __global__ __launch_bounds__(TILE) void kMark(TileRange range, uint32_t n
         return;
     markTile<T>(range.first() + t, nodeBase, wordsPerNode, tileList, segTile, segCount, segSrc, segInput, nodeGrid, ps,
                 order, bitmap, cellOf, err);
+}
+
+// Large builds: tiles of LARGE_TILE inputs, combined in LDS before anything goes to memory.
+//
+// What bounds the passes over the inputs there is the number of their atomics: the XCDs' L2s are not
+// coherent with each other, so every global atomic is carried out in memory, some 20 requests per ns on
+// the whole chip whatever their kind (measured from 5.1M to 119.7M points), and a level's inputs come in
+// the order of their children's grids, in which the points of one cell are mostly close together but not
+// consecutive. So a tile first combines its points per bitmap word (kMarkLarge) and per cell
+// (kAccumulateLarge) in a hash table in LDS. Of the tiles that meet in a cell the one whose bit was set
+// first owns it: kMarkLarge takes the old bits from its atomics and flags the cell index of every other
+// tile's inputs (NOT_OWNED). The owner stores the cell's state without reading it, so it needs no reset,
+// and kAccumulateRest then adds the flagged inputs with atomics. Mark + accumulate (+ reset of the cells):
+//   25.8M points, intra-cell   478 + 984 + 82 -> 468 + 560 + 119 us
+//   119.7M, distance-weighted  2122 + 3150 + 87 -> 1930 + 1798 + 623 us
+//   5.1M, inter-cell           143 + 345 -> 144 + 185 + 51 us
+//   1.5M, no filter            54 + 66 -> 77 + 68 + 27 us
+// so from LARGE_POINTS on (below, a level has too few tiles to hide their barriers and one launch more).
+constexpr uint32_t LARGE_POINTS = 3u << 20;
+constexpr int LARGE_THREADS     = 256;
+constexpr int LARGE_ITEMS       = 4;  // per thread
+constexpr uint32_t LARGE_TILE   = LARGE_THREADS * LARGE_ITEMS;
+constexpr uint32_t NOT_OWNED    = 1u << 31;  // cell and dense indices are below
+
+// Hash table in LDS of the at most LARGE_TILE distinct keys of a tile: key << 32 | the input that put it
+// there, whose number is also that of the key's values. Open addressing from a multiplicative hash: the
+// keys come in runs of consecutive ones, which would pile up in consecutive slots (5.1M points, rows in
+// pencils: accumulating them took 1380 instead of 182 us). The size is a compromise between probes and workgroups
+// per CU.
+constexpr uint32_t TABLE_SLOTS          = LARGE_TILE * 3 / 2;
+constexpr unsigned long long TABLE_FREE = ~0ull;
+
+// The input that put `key` into the table; `input` itself if it is the first one with it.
+__device__ __forceinline__ uint32_t tableInput(unsigned long long* table, uint32_t key, uint32_t input)
+{
+    uint32_t s                   = __umulhi(key * 2654435769u, TABLE_SLOTS);
+    const unsigned long long own = (static_cast<unsigned long long>(key) << 32) | input;
+    for (;;)  // ends: there are fewer keys than slots
+    {
+        const unsigned long long was = atomicCAS(table + s, TABLE_FREE, own);
+        if (was == TABLE_FREE)
+            return input;
+        if (was >> 32 == key)
+            return static_cast<uint32_t>(was);
+        s = s + 1 < TABLE_SLOTS ? s + 1 : 0;
+    }
+}
+
+// The inputs of a workgroup's tile: LARGE_ITEMS per thread, a wave's inputs of one item consecutive.
+struct LargeTile
+{
+    uint32_t k, pos, q, count;  // node of the level, position and index of the first input, inputs
+    __device__ __forceinline__ uint32_t at(int item) const { return LARGE_THREADS * item + threadIdx.x; }
+    __device__ __forceinline__ bool has(int item) const { return at(item) < count; }
+};
+
+__device__ __forceinline__ LargeTile largeTile(uint32_t tile, const uint32_t* tileList, const uint32_t* segTile,
+                                               const uint32_t* segCount, const uint32_t* segSrc,
+                                               const uint32_t* segInput)
+{
+    const uint32_t seg   = tileList[tile];
+    const uint32_t first = (tile - segTile[seg]) * LARGE_TILE;
+    const uint32_t left  = segCount[seg] - first;
+    return LargeTile{seg >> 3, segSrc[seg] + first, segInput[seg] + first, left < LARGE_TILE ? left : LARGE_TILE};
+}
+
+template <typename T>
+static __global__ __launch_bounds__(LARGE_THREADS) void kMarkLarge(TileRange range, uint32_t nodeBase, uint64_t wordsPerNode,
+                                                    const uint32_t* __restrict__ tileList,
+                                                    const uint32_t* __restrict__ segTile,
+                                                    const uint32_t* __restrict__ segCount,
+                                                    const uint32_t* __restrict__ segSrc,
+                                                    const uint32_t* __restrict__ segInput,
+                                                    const NodeGrid* __restrict__ nodeGrid, PointStore<T> ps,
+                                                    CellOrder order, uint32_t* __restrict__ bitmap,
+                                                    uint32_t* __restrict__ cellOf, uint32_t* __restrict__ err,
+                                                    uint64_t* stamp)
+{
+    __shared__ unsigned long long table[TABLE_SLOTS];
+    __shared__ uint32_t bits[LARGE_TILE];
+    stampStart(stamp);
+    // consecutive tiles share bitmap words: runs of them per XCD
+    const uint32_t t = xcdRunItem(blockIdx.x, XCD_TILE_RUN * TILE / LARGE_TILE);
+    if (t >= range.count())
+        return;  // the whole workgroup
+    const LargeTile in  = largeTile(range.first() + t, tileList, segTile, segCount, segSrc, segInput);
+    const Gridding grid = nodeGrid[in.k].grid;
+    T px[LARGE_ITEMS], py[LARGE_ITEMS], pz[LARGE_ITEMS];
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+        if (in.has(i))
+            ps.xyz(in.pos + in.at(i), px[i], py[i], pz[i]);
+    for (uint32_t s = threadIdx.x; s < TABLE_SLOTS; s += LARGE_THREADS)
+        table[s] = TABLE_FREE;
+    for (uint32_t s = threadIdx.x; s < LARGE_TILE; s += LARGE_THREADS)
+        bits[s] = 0;
+    __syncthreads();
+
+    uint32_t cell[LARGE_ITEMS], slot[LARGE_ITEMS];
+    bool created[LARGE_ITEMS];
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+    {
+        cell[i] = ~0u;
+        if (in.has(i))
+        {
+            uint32_t ix, iy, iz;
+            gridCoords(static_cast<double>(px[i]), static_cast<double>(py[i]), static_cast<double>(pz[i]), grid, ix,
+                       iy, iz);
+            const uint32_t gs = grid.gridSize;
+            if (ix >= gs || iy >= gs || iz >= gs)
+                atomicOr(err, ERR_OUTSIDE);  // skipped by the later passes; the build reports the error
+            else
+                cell[i] = cellIndex(ix, iy, iz, gs, order);
+        }
+        // one insertion per run of lanes in the same word; all lanes take part
+        const bool valid  = cell[i] != ~0u;
+        const WaveRun run = waveRun(valid ? cell[i] >> 5 : ~0ull - threadIdx.x);
+        slot[i]           = 0;
+        if (valid && run.lane == run.start)
+            slot[i] = tableInput(table, cell[i] >> 5, in.at(i));
+        slot[i]    = __shfl(slot[i], run.start, 64);
+        created[i] = valid && slot[i] == in.at(i);
+        if (valid)
+            atomicOr(bits + slot[i], 1u << (cell[i] & 31));
+    }
+    __syncthreads();
+    uint32_t* words = bitmap + (in.k - nodeBase) * wordsPerNode;
+    uint32_t old[LARGE_ITEMS];
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+        if (created[i])
+            old[i] = atomicOr(words + (cell[i] >> 5), bits[slot[i]]);
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+        if (created[i])
+            bits[slot[i]] &= ~old[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+        if (in.has(i))
+        {
+            const bool owned = cell[i] == ~0u || ((bits[slot[i]] >> (cell[i] & 31)) & 1u) != 0;
+            cellOf[in.q + in.at(i)] = owned ? cell[i] : cell[i] | NOT_OWNED;
+        }
 }
 
 struct PopcountIn
@@ -1005,6 +1153,33 @@ __device__ __forceinline__ void subtreeOf(uint32_t id, const uint8_t* __restrict
 }
 
 // The nodes' subsample sizes, subtree sums and the next step's cursor go with it (one thread per node).
+__device__ __forceinline__ bool accumulateNodes(const StepSizes& step, uint32_t nodeBase, uint32_t nodes,
+                                                uint64_t wordsPerNode, const NodeGrid* __restrict__ nodeGrid,
+                                                const uint32_t* __restrict__ prefix, uint32_t* __restrict__ pointCount,
+                                                uint32_t* __restrict__ stage, uint32_t* __restrict__ subtree,
+                                                const uint8_t* __restrict__ flags,
+                                                const int32_t* __restrict__ children, uint32_t* __restrict__ err)
+{
+    const bool fits       = step.fits();
+    const uint64_t cursor = *step.cursor;
+    if (globalThread() == 0)
+    {
+        *step.next = fits ? cursor + *step.cells : CURSOR_FULL;
+        if (!fits)
+            atomicOr(err, ERR_OVERFLOW);
+    }
+    for (uint64_t kl = globalThread(); kl < nodes; kl += globalStride())
+    {
+        const uint32_t id = nodeGrid[nodeBase + kl].id;
+        if (fits)
+            batchNodeOf(kl, nodeBase, wordsPerNode, nodeGrid, prefix, static_cast<uint32_t>(cursor), pointCount, stage);
+        else
+            pointCount[id] = 0;  // no input of a later step
+        subtreeOf(id, flags, children, pointCount, subtree);  // of the levels below: complete
+    }
+    return fits;
+}
+
 template <typename T, uint32_t MODE, bool RANDOM>
 static __global__ __launch_bounds__(TILE) void kAccumulate(TileRange range, StepSizes step, uint32_t nodeBase,
                                                      uint32_t nodes, uint64_t wordsPerNode,
@@ -1025,29 +1200,178 @@ static __global__ __launch_bounds__(TILE) void kAccumulate(TileRange range, Step
                                                      const uint8_t* __restrict__ flags,
                                                      const int32_t* __restrict__ children, uint32_t* __restrict__ err)
 {
-    const bool fits       = step.fits();
-    const uint64_t cursor = *step.cursor;
-    if (globalThread() == 0)
-    {
-        *step.next = fits ? cursor + *step.cells : CURSOR_FULL;
-        if (!fits)
-            atomicOr(err, ERR_OVERFLOW);
-    }
-    for (uint64_t kl = globalThread(); kl < nodes; kl += globalStride())
-    {
-        const uint32_t id = nodeGrid[nodeBase + kl].id;
-        if (fits)
-            batchNodeOf(kl, nodeBase, wordsPerNode, nodeGrid, prefix, static_cast<uint32_t>(cursor), pointCount, stage);
-        else
-            pointCount[id] = 0;  // no input of a later step
-        subtreeOf(id, flags, children, pointCount, subtree);  // of the levels below: complete
-    }
-    if (!fits)
+    if (!accumulateNodes(step, nodeBase, nodes, wordsPerNode, nodeGrid, prefix, pointCount, stage, subtree, flags,
+                         children, err))
         return;
     if (blockIdx.x < range.count())
         accumulateTile<T, MODE, RANDOM>(range.first() + blockIdx.x, nodeBase, wordsPerNode, tileList, segTile,
                                         segCount, segSrc, segInput, nodeGrid, bitmap, prefix, cellOf, ps, win, color,
                                         cellCnt, cellKey, cellNode, rankOf);
+}
+
+// A large tile's points per cell: the cells that the tile owns get their state from it.
+template <uint32_t MODE>
+struct CellTable
+{
+    static constexpr bool WEIGHTED = MODE == COLOR_INTER_WEIGHTED;
+    static constexpr bool COLOR    = MODE == COLOR_INTRA || MODE == COLOR_INTER;
+    unsigned long long cells[TABLE_SLOTS];
+    unsigned long long color[COLOR ? LARGE_TILE : 0];
+    uint32_t value[LARGE_TILE];  // least rank; points
+};
+
+template <typename T, uint32_t MODE, bool RANDOM>
+static __global__ __launch_bounds__(LARGE_THREADS) void kAccumulateLarge(
+        TileRange range, StepSizes step, uint32_t nodeBase, uint32_t nodes, uint64_t wordsPerNode,
+        const uint32_t* __restrict__ tileList, const uint32_t* __restrict__ segTile,
+        const uint32_t* __restrict__ segCount, const uint32_t* __restrict__ segSrc,
+        const uint32_t* __restrict__ segInput, const NodeGrid* __restrict__ nodeGrid,
+        const uint32_t* __restrict__ bitmap, const uint32_t* __restrict__ prefix, uint32_t* __restrict__ cellOf,
+        PointStore<T> ps, uint64_t* __restrict__ win, uint64_t* __restrict__ color, uint32_t* __restrict__ cellCnt,
+        uint32_t* __restrict__ cellKey, uint32_t* __restrict__ cellNode, uint32_t* __restrict__ rankOf,
+        uint32_t* __restrict__ pointCount, uint32_t* __restrict__ stage, uint32_t* __restrict__ subtree,
+        const uint8_t* __restrict__ flags, const int32_t* __restrict__ children, uint32_t* __restrict__ err)
+{
+    using Table = CellTable<MODE>;
+    __shared__ Table table;
+    if (!accumulateNodes(step, nodeBase, nodes, wordsPerNode, nodeGrid, prefix, pointCount, stage, subtree, flags,
+                         children, err))
+        return;
+    if (blockIdx.x >= range.count())
+        return;  // the whole workgroup
+    const LargeTile in  = largeTile(range.first() + blockIdx.x, tileList, segTile, segCount, segSrc, segInput);
+    const uint32_t kl   = in.k - nodeBase;
+    const uint64_t base = kl * wordsPerNode;
+    uint32_t cell[LARGE_ITEMS], c[LARGE_ITEMS], idx[LARGE_ITEMS];
+    uint64_t col[LARGE_ITEMS];
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+    {
+        cell[i] = in.has(i) ? cellOf[in.q + in.at(i)] : ~0u;
+        if (!Table::WEIGHTED && in.has(i))
+        {
+            idx[i] = ps.index(in.pos + in.at(i));
+            if (Table::COLOR)
+                col[i] = ps.packed(in.pos + in.at(i));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+        if ((cell[i] & NOT_OWNED) == 0)
+            c[i] = cellRank(bitmap, prefix, base + (cell[i] >> 5), cell[i] & 31);
+    for (uint32_t s = threadIdx.x; s < TABLE_SLOTS; s += LARGE_THREADS)
+        table.cells[s] = TABLE_FREE;
+    for (uint32_t s = threadIdx.x; s < LARGE_TILE; s += LARGE_THREADS)
+    {
+        table.value[s] = Table::WEIGHTED ? 0u : ~0u;
+        if (Table::COLOR)
+            table.color[s] = 0;
+    }
+    const uint32_t salt = RANDOM && !Table::WEIGHTED ? nodeGrid[in.k].salt : 0u;
+    __syncthreads();
+    uint32_t slot[LARGE_ITEMS], rank[LARGE_ITEMS];
+    bool created[LARGE_ITEMS];
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+    {
+        created[i] = false;
+        if (cell[i] & NOT_OWNED)
+            continue;
+        slot[i]    = tableInput(table.cells, c[i], in.at(i));
+        created[i] = slot[i] == in.at(i);
+        if (Table::WEIGHTED)
+        {
+            // the winner is taken from the cell's payload run in the emit; the input's cell index is
+            // replaced by the cell's dense index (the payload scatter reads the cell back from cellKey)
+            cellOf[in.q + in.at(i)] = c[i];
+            rankOf[in.q + in.at(i)] = atomicAdd(table.value + slot[i], 1u);
+            continue;
+        }
+        rank[i] = RANDOM ? fmix32(idx[i] ^ salt) : idx[i];
+        atomicMin(table.value + slot[i], rank[i]);
+        if (Table::COLOR)
+            atomicAdd(table.color + slot[i], static_cast<unsigned long long>(col[i]));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+    {
+        if (created[i])
+        {
+            cellKey[c[i]]  = cell[i];
+            cellNode[c[i]] = kl;
+            if (Table::WEIGHTED)
+                cellCnt[c[i]] = table.value[slot[i]];
+            if (Table::COLOR)
+                color[c[i]] = table.color[slot[i]];
+        }
+        // the winner itself: no two points have the same rank
+        if (!Table::WEIGHTED && (cell[i] & NOT_OWNED) == 0 && table.value[slot[i]] == rank[i])
+            win[c[i]] = (static_cast<uint64_t>(rank[i]) << 32) | (in.pos + in.at(i));
+    }
+}
+
+// The inputs in cells that another tile owns, after kAccumulateLarge: one atomic per run of lanes.
+template <typename T, uint32_t MODE, bool RANDOM>
+static __global__ __launch_bounds__(LARGE_THREADS) void kAccumulateRest(
+        TileRange range, StepSizes step, uint32_t nodeBase, uint64_t wordsPerNode,
+        const uint32_t* __restrict__ tileList, const uint32_t* __restrict__ segTile,
+        const uint32_t* __restrict__ segCount, const uint32_t* __restrict__ segSrc,
+        const uint32_t* __restrict__ segInput, const NodeGrid* __restrict__ nodeGrid,
+        const uint32_t* __restrict__ bitmap, const uint32_t* __restrict__ prefix, uint32_t* __restrict__ cellOf,
+        PointStore<T> ps, uint64_t* __restrict__ win, uint64_t* __restrict__ color, uint32_t* __restrict__ cellCnt,
+        uint32_t* __restrict__ rankOf)
+{
+    if (!step.fits() || blockIdx.x >= range.count())
+        return;
+    const LargeTile in  = largeTile(range.first() + blockIdx.x, tileList, segTile, segCount, segSrc, segInput);
+    const uint64_t base = (in.k - nodeBase) * wordsPerNode;
+    uint32_t cells[LARGE_ITEMS];
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+        cells[i] = in.has(i) ? cellOf[in.q + in.at(i)] : ~0u;
+#pragma unroll
+    for (int i = 0; i < LARGE_ITEMS; ++i)
+    {
+        const bool rest = (cells[i] & NOT_OWNED) != 0 && cells[i] != ~0u;
+        if (!__any(rest))
+            continue;  // the whole wave
+        const uint32_t cell = cells[i] & ~NOT_OWNED;
+        const uint32_t c    = rest ? cellRank(bitmap, prefix, base + (cell >> 5), cell & 31) : 0u;
+        const WaveRun run   = waveRun(rest ? c : ~0ull - threadIdx.x);
+        const bool last     = rest && run.lane == run.end;
+        if (MODE == COLOR_INTER_WEIGHTED)
+        {
+            uint32_t first = 0;
+            if (last)
+                first = atomicAdd(cellCnt + c, static_cast<uint32_t>(run.end - run.start + 1));
+            first = __shfl(first, run.end, 64);
+            if (rest)
+            {
+                cellOf[in.q + in.at(i)] = c;
+                rankOf[in.q + in.at(i)] = first + static_cast<uint32_t>(run.lane - run.start);
+            }
+            continue;
+        }
+        uint64_t key = ~0ull, col = 0;
+        if (rest)
+        {
+            const uint32_t idx  = ps.index(in.pos + in.at(i));
+            const uint32_t rank = RANDOM ? fmix32(idx ^ nodeGrid[in.k].salt) : idx;
+            key                 = (static_cast<uint64_t>(rank) << 32) | (in.pos + in.at(i));
+            if (MODE == COLOR_INTRA || MODE == COLOR_INTER)
+                col = ps.packed(in.pos + in.at(i));
+        }
+        key = runScan<uint64_t>(key, run, [](uint64_t x, uint64_t y) { return x < y ? x : y; });
+        if (MODE == COLOR_INTRA || MODE == COLOR_INTER)
+            col = runScan<uint64_t>(col, run, [](uint64_t x, uint64_t y) { return x + y; });
+        if (last)
+        {
+            atomicMin(reinterpret_cast<unsigned long long*>(win + c), static_cast<unsigned long long>(key));
+            if (MODE == COLOR_INTRA || MODE == COLOR_INTER)
+                atomicAdd(reinterpret_cast<unsigned long long*>(color + c), static_cast<unsigned long long>(col));
+        }
+    }
 }
 
 // exclusive prefix into an array, with the total behind it
@@ -1100,9 +1424,10 @@ __device__ __forceinline__ void scatterPayloadTile(uint32_t tile, const uint32_t
                                                    const uint32_t* __restrict__ rankOf,
                                                    const uint32_t* __restrict__ cellStart,
                                                    const uint32_t* __restrict__ cellOf, const PointStore<T>& ps,
-                                                   WeightPayload* __restrict__ payload, uint64_t* __restrict__ winKey)
+                                                   WeightPayload* __restrict__ payload, uint64_t* __restrict__ winKey,
+                                                   uint32_t parts = 1)
 {
-    InputRef in = inputOf(tile, tileList, segTile, segCount, segSrc, segInput);
+    InputRef in = inputOf(tile, tileList, segTile, segCount, segSrc, segInput, parts);
     if (!in.valid)
         return;
     const uint32_t c = cellOf[in.q];  // the dense index kAccumulate left there
@@ -1143,16 +1468,17 @@ static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, 
                                                          const uint32_t* __restrict__ cellStart,
                                                          const uint32_t* __restrict__ cellOf, PointStore<T> ps,
                                                          WeightPayload* __restrict__ payload,
-                                                         uint64_t* __restrict__ winKey, uint64_t* stamp)
+                                                         uint64_t* __restrict__ winKey, uint32_t parts,
+                                                         uint64_t* stamp)
 {
     stampStart(stamp);
     if (!step.fits())
         return;
     // consecutive tiles store to neighbouring payload slots: runs of them per XCD
     const uint32_t t = xcdRunItem(blockIdx.x, XCD_TILE_RUN);
-    if (t < range.count())
-        scatterPayloadTile<T, RANDOM>(range.first() + t, tileList, segTile, segCount, segSrc, segInput, nodeGrid,
-                                      cellKey, rankOf, cellStart, cellOf, ps, payload, winKey);
+    if (t < range.count() * parts)
+        scatterPayloadTile<T, RANDOM>(range.first() * parts + t, tileList, segTile, segCount, segSrc, segInput, nodeGrid,
+                                      cellKey, rankOf, cellStart, cellOf, ps, payload, winKey, parts);
 }
 
 // Select (rp_subsampling.cuh:70-321, fp_subsampling.cuh:30-306): one output record per occupied

@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "device_common.h"
 #include "kernels_chunking.h"
@@ -285,32 +286,46 @@ __device__ __forceinline__ void bucketScatterChunk(uint32_t chunk, const uint8_t
         off += cnt[k];
     }
     __syncthreads();
-    // records into LDS in bucket order; the fine code straight to its final place (this lane
-    // already has the point's Morton code)
+    // records into LDS in bucket order
     const uint32_t fineMask = (1u << fineBits) - 1u;
 #pragma unroll
     for (int j = 0; j < STAGE_ITEMS; ++j)
         if (code[j] != ~0u)
-        {
-            const uint32_t b    = code[j] >> fineBits;
-            const uint32_t slot = localStart[b] + rank[j];
-            stage[slot]         = p[j];
-            const uint32_t d    = slot + delta[b];
-            if (d < n)
-                fineCode[d] = static_cast<uint16_t>(code[j] & fineMask);
-        }
+            stage[localStart[code[j] >> fineBits] + rank[j]] = p[j];
     __syncthreads();
 
     // a staged record's bucket is recomputed from its coordinates (a few FP64 operations) rather
-    // than searched for among the buckets' first slots (a dozen dependent LDS reads)
-    for (uint32_t j = threadIdx.x; j < total; j += SCATTER_THREADS)
+    // than searched for among the buckets' first slots (a dozen dependent LDS reads). The records of a
+    // wave go out word by word, consecutive lanes storing consecutive words: a record stored by its own
+    // lane, and a fine code from the unsorted points, were a request of the L2 each (float points, 25.8M /
+    // 5.1M: 660 -> 608 / 134 -> 118 us; 119.7M double points 2.5 ms either way).
+    using Word              = std::conditional_t<sizeof(T) == 8, uint4, uint32_t>;
+    constexpr uint32_t W    = sizeof(SortedPoint<T>) / sizeof(Word);
+    const uint32_t lane     = threadIdx.x & 63;
+    for (uint32_t j0 = threadIdx.x - lane; j0 < total; j0 += SCATTER_THREADS)
     {
-        const SortedPoint<T> r = stage[j];
-        const uint32_t m       = pointMorton(static_cast<double>(r.x), static_cast<double>(r.y),
-                                             static_cast<double>(r.z), g);  // in the grid: it was staged
-        const uint32_t d       = j + delta[m >> fineBits];
-        if (d < n)  // always: the histogram and this pass compute the same codes
-            dst[d] = r;
+        const uint32_t j = j0 + lane;
+        uint32_t d       = ~0u;
+        if (j < total)
+        {
+            const uint32_t m  = pointMorton(static_cast<double>(stage[j].x), static_cast<double>(stage[j].y),
+                                            static_cast<double>(stage[j].z), g);  // in the grid: it was staged
+            const uint32_t at = j + delta[m >> fineBits];
+            if (at < n)  // always: the histogram and this pass compute the same codes
+            {
+                d           = at;
+                fineCode[d] = static_cast<uint16_t>(m & fineMask);
+            }
+        }
+        const Word* src = reinterpret_cast<const Word*>(stage + j0);
+#pragma unroll
+        for (uint32_t r = 0; r < W; ++r)
+        {
+            const uint32_t w  = 64 * r + lane, rec = w / W;
+            const uint32_t at = __shfl(d, static_cast<int>(rec), 64);
+            if (at != ~0u)
+                reinterpret_cast<Word*>(dst)[static_cast<uint64_t>(at) * W + (w - rec * W)] = src[w];
+        }
     }
     __syncthreads();
 }

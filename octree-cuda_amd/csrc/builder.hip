@@ -972,7 +972,7 @@ void OctreeBuilder::subsampleLevels()
                 OC_LAUNCH_CHECK();
                 auto scatter = [&](auto kernel) {
                     kernel<<<tileGrid * parts, TILE, 0, itsStream>>>(
-                            tiles, step, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                            tiles, step, g, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                             itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
                             itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(), itsCellStart.as<uint32_t>(),
                             itsCellOf.as<uint32_t>(), ps, itsPayload.as<WeightPayload>(), winKey, parts,
@@ -984,14 +984,14 @@ void OctreeBuilder::subsampleLevels()
 
             if (weighted)
                 kEmitWeighted<T><<<xcdRunGrid((cellMost + BLOCK - 1) / BLOCK, EMIT_CHUNK), BLOCK, 0, itsStream>>>(
-                        step, k0, wordsPerNode, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
+                        step, k0, wordsPerNode, g, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
                         itsCellNode.as<uint32_t>(), itsCellStart.as<uint32_t>(), itsPayload.as<WeightPayload>(), winKey,
                         ps, stamps + ST_EMIT_BEGIN);
             else
             {
                 auto emit = [&](auto kernel) {
                     kernel<<<gridFor(cellMost), BLOCK, 0, itsStream>>>(
-                            step, k0, wordsPerNode, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
+                            step, wordsPerNode, g, bitmap, prefix, itsCellKey.as<uint32_t>(),
                             itsCellNode.as<uint32_t>(), win, color, ps, stamps + ST_INSERT_END, stamps + ST_EMIT_BEGIN);
                 };
                 switch (itsColorMode)

@@ -952,7 +952,7 @@ static __global__ __launch_bounds__(TILE) void kScatterPayloadB(const BatchCloud
     {
         const uint32_t c        = findCloud(prefix, B, item);
         const BatchCloud<T>& cc = ctx[c];
-        scatterPayloadTile<T, RANDOM>(item - prefix[c], cc.tileList, cc.segTile, cc.segCount, cc.segSrc,
+        scatterPayloadTile<T, RANDOM>(item - prefix[c], cc.g, cc.tileList, cc.segTile, cc.segCount, cc.segSrc,
                                       cc.segInput, cc.nodeGrid, cc.cellKey, cc.rankOf, cc.cellStart, cc.cellOf,
                                       cc.store(), cc.payload, cc.winKey);
     }
@@ -972,10 +972,10 @@ static __global__ __launch_bounds__(BLOCK) void kEmitB(const BatchCloud<T>* __re
         const uint32_t k        = static_cast<uint32_t>(i) - wp[c];
         const uint32_t cursor   = static_cast<uint32_t>(cc.sc[BS_CURSOR]);
         if constexpr (MODE == COLOR_INTER_WEIGHTED)
-            emitWeightedCell<T>(k, 0, cc.wordsPerNode, cursor, cc.nodeGrid, cc.bitmap, cc.prefix, cc.cellKey,
+            emitWeightedCell<T>(k, 0, cc.wordsPerNode, cursor, cc.g, cc.nodeGrid, cc.bitmap, cc.prefix, cc.cellKey,
                                 cc.cellNode, cc.cellStart, cc.payload, cc.winKey, cc.store());
         else
-            emitCell<T, MODE>(k, 0, cc.wordsPerNode, cursor, cc.nodeGrid, cc.bitmap, cc.prefix, cc.cellKey,
+            emitCell<T, MODE>(k, cc.wordsPerNode, cursor, cc.g, cc.bitmap, cc.prefix, cc.cellKey,
                               cc.cellNode, cc.win, cc.color, cc.store());
     }
 }

@@ -78,6 +78,46 @@ __host__ __device__ __forceinline__ void rowCoords(uint32_t row, uint32_t g, uin
     z = (pencil / p) * PENCIL + inside / PENCIL;
 }
 
+// A cell's coordinates from its index, g the same for all cells of a build: shifts where it is a power of
+// two, integer divisions (some 25 instructions each) where not.
+__device__ __forceinline__ void cellCoords(uint32_t cell, uint32_t g, uint32_t& x, uint32_t& y, uint32_t& z)
+{
+    if (g >= PENCIL && (g & (g - 1)) == 0)
+    {
+        const uint32_t s = static_cast<uint32_t>(__builtin_ctz(g)), p = g / PENCIL;
+        const uint32_t row = cell >> s, pencil = row / (PENCIL * PENCIL), inside = row % (PENCIL * PENCIL);
+        x = cell & (g - 1);
+        y = (pencil & (p - 1)) * PENCIL + inside % PENCIL;
+        z = (pencil >> __builtin_ctz(p)) * PENCIL + inside / PENCIL;
+        return;
+    }
+    x = cell % g;
+    rowCoords(cell / g, g, y, z);
+}
+
+// The 3 x 3 x-rows around a cell: rowIndex is a sum of a part in y and one in z, so the first cells of
+// the nine rows are nine sums.
+struct CellRows
+{
+    uint32_t y[3], z[3];  // the parts, in cells
+    bool inY[3], inZ[3];  // in the grid
+    __device__ __forceinline__ CellRows(uint32_t cy, uint32_t cz, uint32_t g)
+    {
+        const uint32_t p = pencilsPerAxis(g);
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k)
+        {
+            const uint32_t ny = cy + k - 1, nz = cz + k - 1;  // below zero: above any g
+            inY[k] = ny < g;
+            inZ[k] = nz < g;
+            y[k]   = (ny / PENCIL * (PENCIL * PENCIL) + ny % PENCIL) * g;
+            z[k]   = (nz / PENCIL * p * (PENCIL * PENCIL) + nz % PENCIL * PENCIL) * g;
+        }
+    }
+    __device__ __forceinline__ bool has(int r) const { return inY[r / 3] && inZ[r % 3]; }
+    __device__ __forceinline__ uint32_t start(int r) const { return y[r / 3] + z[r % 3]; }
+};
+
 // Order of a node grid's cells in its bitmap, and so of a node's staged points and of the leaf points
 // that the node reads: rows in pencils where the colour filter walks neighbourhoods, Morton order
 // (child-slot groups, as the octree's) where it does not. Then the up to eight cells of a child that
@@ -220,7 +260,9 @@ __device__ __forceinline__ NodeGrid nodeGridOf(uint32_t id, uint32_t key, uint32
     NodeGrid ng;
     ng.grid        = nodeGridding(key - levelOffset, levelGrid, level, depth, cubicMin, sideHalf, side, g);
     const double t = ng.grid.bbSize / g;
-    ng.diag        = sqrt((t * 3) * (t * 3) * 3) / 2.0;
+    const double d = sqrt((t * 3) * (t * 3) * 3) / 2.0;
+    ng.cell        = static_cast<float>(t);
+    ng.weight      = static_cast<float>((-10.0 * 1.4426950408889634) / (d * d));
     ng.salt        = nodeSalt(seed, key);
     ng.id          = id;
     return ng;
@@ -1414,7 +1456,7 @@ __device__ __forceinline__ void cellCentre(const Gridding& g, uint32_t ix, uint3
 }
 
 template <typename T, bool RANDOM>
-__device__ __forceinline__ void scatterPayloadTile(uint32_t tile, const uint32_t* __restrict__ tileList,
+__device__ __forceinline__ void scatterPayloadTile(uint32_t tile, uint32_t g, const uint32_t* __restrict__ tileList,
                                                    const uint32_t* __restrict__ segTile,
                                                    const uint32_t* __restrict__ segCount,
                                                    const uint32_t* __restrict__ segSrc,
@@ -1435,10 +1477,8 @@ __device__ __forceinline__ void scatterPayloadTile(uint32_t tile, const uint32_t
         return;
     const uint32_t cell = cellKey[c];
     const NodeGrid ng   = nodeGrid[in.k];
-    const uint32_t gs   = ng.grid.gridSize;
-    uint32_t iy, iz;
-    rowCoords(cell / gs, gs, iy, iz);
-    const uint32_t ix = cell % gs;
+    uint32_t ix, iy, iz;
+    cellCoords(cell, g, ix, iy, iz);
     double cx, cy, cz;
     cellCentre(ng.grid, ix, iy, iz, cx, cy, cz);
     T px, py, pz;
@@ -1456,7 +1496,7 @@ __device__ __forceinline__ void scatterPayloadTile(uint32_t tile, const uint32_t
 }
 
 template <typename T, bool RANDOM>
-static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, StepSizes step,
+static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, StepSizes step, uint32_t g,
                                                          const uint32_t* __restrict__ tileList,
                                                          const uint32_t* __restrict__ segTile,
                                                          const uint32_t* __restrict__ segCount,
@@ -1477,7 +1517,7 @@ static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, 
     // consecutive tiles store to neighbouring payload slots: runs of them per XCD
     const uint32_t t = xcdRunItem(blockIdx.x, XCD_TILE_RUN);
     if (t < range.count() * parts)
-        scatterPayloadTile<T, RANDOM>(range.first() * parts + t, tileList, segTile, segCount, segSrc, segInput, nodeGrid,
+        scatterPayloadTile<T, RANDOM>(range.first() * parts + t, g, tileList, segTile, segCount, segSrc, segInput, nodeGrid,
                                       cellKey, rankOf, cellStart, cellOf, ps, payload, winKey, parts);
 }
 
@@ -1489,46 +1529,38 @@ static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, 
 // neighbourhood is walked as 9 x-rows: the occupied cells among x-1..x+1 of one row have
 // consecutive dense indices, so each row is one contiguous run of per-cell sums.
 template <typename T, uint32_t MODE>
-__device__ __forceinline__ void emitCell(uint32_t c, uint32_t nodeBase, uint64_t wordsPerNode, uint32_t cursor,
-                                         const NodeGrid* __restrict__ nodeGrid, const uint32_t* __restrict__ bitmap,
+__device__ __forceinline__ void emitCell(uint32_t c, uint64_t wordsPerNode, uint32_t cursor, uint32_t g,
+                                         const uint32_t* __restrict__ bitmap,
                                          const uint32_t* __restrict__ prefix, const uint32_t* __restrict__ cellKey,
                                          const uint32_t* __restrict__ cellNode, const uint64_t* __restrict__ win,
                                          const uint64_t* __restrict__ color, const PointStore<T>& ps)
 {
     {
-        const uint32_t kl = cellNode[c];
-        const NodeGrid ng = nodeGrid[nodeBase + kl];
-        uint64_t sum      = 0;  // packed colours
+        uint64_t sum = 0;  // packed colours
 
         if (MODE == COLOR_INTRA)
             sum = color[c];
         else if (MODE == COLOR_INTER)
         {
-            const uint32_t key    = cellKey[c];
-            const uint32_t gs     = ng.grid.gridSize;
-            const uint64_t words  = static_cast<uint64_t>(kl) * wordsPerNode;
-            uint32_t ry, rz;
-            rowCoords(key / gs, gs, ry, rz);
-            const int32_t cx = static_cast<int32_t>(key % gs), cy = static_cast<int32_t>(ry),
-                          cz = static_cast<int32_t>(rz);
-            const int32_t x0 = cx > 0 ? cx - 1 : 0;
-            const int32_t x1 = cx + 1 < static_cast<int32_t>(gs) ? cx + 1 : cx;
-            const uint32_t span = static_cast<uint32_t>(x1 - x0 + 1);
+            const uint64_t words = cellNode[c] * wordsPerNode;
+            uint32_t cx, cy, cz;
+            cellCoords(cellKey[c], g, cx, cy, cz);
+            const uint32_t x0 = cx > 0 ? cx - 1 : 0;
+            const uint32_t x1 = cx + 1 < g ? cx + 1 : cx;
+            const uint32_t span = x1 - x0 + 1;
+            const CellRows rows(cy, cz, g);
+            const uint32_t *nodeBits = bitmap + words, *nodePrefix = prefix + words;
 #pragma unroll
             for (int r = 0; r < 9; ++r)
             {
-                const int32_t ny = cy + (r / 3) - 1, nz = cz + (r % 3) - 1;
-                if (ny < 0 || nz < 0 || ny >= static_cast<int32_t>(gs) || nz >= static_cast<int32_t>(gs))
+                if (!rows.has(r))
                     continue;
-                const uint64_t L0 = static_cast<uint64_t>(x0) +
-                                    static_cast<uint64_t>(rowIndex(static_cast<uint32_t>(ny), static_cast<uint32_t>(nz), gs)) * gs;
-                const uint64_t w0 = words + (L0 >> 5);
-                const uint32_t b0 = static_cast<uint32_t>(L0 & 31);
-                uint64_t v        = bitmap[w0];
+                const uint32_t L0 = rows.start(r) + x0, w0 = L0 >> 5, b0 = L0 & 31;
+                uint64_t v        = nodeBits[w0];
                 if (b0 + span > 32)
-                    v |= static_cast<uint64_t>(bitmap[w0 + 1]) << 32;
+                    v |= static_cast<uint64_t>(nodeBits[w0 + 1]) << 32;
                 const uint32_t m     = static_cast<uint32_t>(v >> b0) & ((1u << span) - 1u);
-                const uint32_t first = prefix[w0] + __popc(static_cast<uint32_t>(v) & ((1u << b0) - 1u));
+                const uint32_t first = nodePrefix[w0] + __popc(static_cast<uint32_t>(v) & ((1u << b0) - 1u));
                 // at most 3 occupied cells (x - 1 .. x + 1): predicated loads, no loop, so the
                 // rows' loads are all in flight together
                 const uint32_t n = __popc(m);
@@ -1557,8 +1589,7 @@ __device__ __forceinline__ void emitCell(uint32_t c, uint32_t nodeBase, uint64_t
 }
 
 template <typename T, uint32_t MODE>
-static __global__ __launch_bounds__(BLOCK) void kEmit(StepSizes step, uint32_t nodeBase, uint64_t wordsPerNode,
-                                                const NodeGrid* __restrict__ nodeGrid,
+static __global__ __launch_bounds__(BLOCK) void kEmit(StepSizes step, uint64_t wordsPerNode, uint32_t g,
                                                 const uint32_t* __restrict__ bitmap,
                                                 const uint32_t* __restrict__ prefix,
                                                 const uint32_t* __restrict__ cellKey,
@@ -1572,8 +1603,8 @@ static __global__ __launch_bounds__(BLOCK) void kEmit(StepSizes step, uint32_t n
         return;
     const uint32_t cells = *step.cells, cursor = static_cast<uint32_t>(*step.cursor);
     for (uint64_t ci = globalThread(); ci < cells; ci += globalStride())
-        emitCell<T, MODE>(static_cast<uint32_t>(ci), nodeBase, wordsPerNode, cursor, nodeGrid, bitmap, prefix, cellKey,
-                          cellNode, win, color, ps);
+        emitCell<T, MODE>(static_cast<uint32_t>(ci), wordsPerNode, cursor, g, bitmap, prefix, cellKey, cellNode, win, color,
+                          ps);
 }
 
 // Select with the distance-weighted inter-cell filter (kernel_inter_cell_filtering.cuh:109-194,
@@ -1592,7 +1623,7 @@ static __global__ __launch_bounds__(BLOCK) void kEmit(StepSizes step, uint32_t n
 // atomics). Two records per step, both loads in flight before either is weighed.
 template <typename T>
 __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, uint64_t wordsPerNode,
-                                                 uint32_t cursor, const NodeGrid* __restrict__ nodeGrid,
+                                                 uint32_t cursor, uint32_t g, const NodeGrid* __restrict__ nodeGrid,
                                                  const uint32_t* __restrict__ bitmap,
                                                  const uint32_t* __restrict__ prefix,
                                                  const uint32_t* __restrict__ cellKey,
@@ -1602,37 +1633,33 @@ __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, 
                                                  const uint64_t* __restrict__ winKey, const PointStore<T>& ps)
 {
     const uint32_t kl    = cellNode[c];
-    const NodeGrid ng    = nodeGrid[nodeBase + kl];
-    const uint32_t key   = cellKey[c];
-    const uint32_t gs    = ng.grid.gridSize;
-    const uint64_t words = static_cast<uint64_t>(kl) * wordsPerNode;
-    uint32_t ry, rz;
-    rowCoords(key / gs, gs, ry, rz);
-    const int32_t cx = static_cast<int32_t>(key % gs), cy = static_cast<int32_t>(ry), cz = static_cast<int32_t>(rz);
-    const int32_t x0 = cx > 0 ? cx - 1 : 0;
-    const int32_t x1 = cx + 1 < static_cast<int32_t>(gs) ? cx + 1 : cx;
-    const uint32_t span = static_cast<uint32_t>(x1 - x0 + 1);
+    const float tf       = nodeGrid[nodeBase + kl].cell;
+    const float kexp     = nodeGrid[nodeBase + kl].weight;
+    const uint64_t words = kl * wordsPerNode;
+    uint32_t cx, cy, cz;
+    cellCoords(cellKey[c], g, cx, cy, cz);
+    const uint32_t x0 = cx > 0 ? cx - 1 : 0;
+    const uint32_t x1 = cx + 1 < g ? cx + 1 : cx;
+    const uint32_t span = x1 - x0 + 1;
+    const CellRows rows(cy, cz, g);
+    const uint32_t *nodeBits = bitmap + words, *nodePrefix = prefix + words;
 
     // first dense index and number of occupied cells of every row
     uint32_t first[9], count[9];
 #pragma unroll
     for (int r = 0; r < 9; ++r)
     {
-        const int32_t ny = cy + (r / 3) - 1, nz = cz + (r % 3) - 1;
         count[r] = 0;
         first[r] = 0;
-        if (ny < 0 || nz < 0 || ny >= static_cast<int32_t>(gs) || nz >= static_cast<int32_t>(gs))
+        if (!rows.has(r))
             continue;
-        const uint64_t L0 = static_cast<uint64_t>(x0) +
-                            static_cast<uint64_t>(rowIndex(static_cast<uint32_t>(ny), static_cast<uint32_t>(nz), gs)) * gs;
-        const uint64_t w0 = words + (L0 >> 5);
-        const uint32_t b0 = static_cast<uint32_t>(L0 & 31);
-        uint64_t v        = bitmap[w0];
+        const uint32_t L0 = rows.start(r) + x0, w0 = L0 >> 5, b0 = L0 & 31;
+        uint64_t v        = nodeBits[w0];
         if (b0 + span > 32)
-            v |= static_cast<uint64_t>(bitmap[w0 + 1]) << 32;
+            v |= static_cast<uint64_t>(nodeBits[w0 + 1]) << 32;
         const uint32_t m = static_cast<uint32_t>(v >> b0) & ((1u << span) - 1u);
         count[r]         = __popc(m);
-        first[r]         = prefix[w0] + __popc(static_cast<uint32_t>(v) & ((1u << b0) - 1u));
+        first[r]         = nodePrefix[w0] + __popc(static_cast<uint32_t>(v) & ((1u << b0) - 1u));
     }
     uint32_t lo[9], hi[9];
 #pragma unroll
@@ -1654,10 +1681,7 @@ __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, 
     ps.xyz(wpos, bx, by, bz);
     const uint32_t bestIdx = ps.index(wpos);
 
-    const double t     = ng.grid.bbSize / gs;
-    const float tf     = static_cast<float>(t);
-    const float kexp   = static_cast<float>((-10.0 * 1.4426950408889634) / (ng.diag * ng.diag));
-    const uint32_t cxm = (static_cast<uint32_t>(cx) + 3u) & 3u;  // (c.x - 1) mod 4: d.x = ((m.x - cxm) & 3) - 1
+    const uint32_t cxm = (cx + 3u) & 3u;  // (c.x - 1) mod 4: d.x = ((m.x - cxm) & 3) - 1
     float acc[4]       = {0.f, 0.f, 0.f, 0.f};
     // payloads as 16-byte vectors (they stay in registers under conditional loads)
     const uint4* pv = reinterpret_cast<const uint4*>(payload);
@@ -1734,6 +1758,7 @@ __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, 
 
 template <typename T>
 static __global__ __launch_bounds__(BLOCK) void kEmitWeighted(StepSizes step, uint32_t nodeBase, uint64_t wordsPerNode,
+                                                        uint32_t g,
                                                         const NodeGrid* __restrict__ nodeGrid,
                                                         const uint32_t* __restrict__ bitmap,
                                                         const uint32_t* __restrict__ prefix,
@@ -1751,7 +1776,7 @@ static __global__ __launch_bounds__(BLOCK) void kEmitWeighted(StepSizes step, ui
     const uint64_t c = static_cast<uint64_t>(xcdRunItem(blockIdx.x, EMIT_CHUNK)) * BLOCK + threadIdx.x;
     if (c < *step.cells)
         emitWeightedCell<T>(static_cast<uint32_t>(c), nodeBase, wordsPerNode, static_cast<uint32_t>(*step.cursor),
-                            nodeGrid, bitmap, prefix, cellKey, cellNode, cellStart, payload, winKey, ps);
+                            g, nodeGrid, bitmap, prefix, cellKey, cellNode, cellStart, payload, winKey, ps);
 }
 
 // DFS post-order placement (A6, kernel_helpers.cuh:55-59): subtree sums of subsample sizes

@@ -54,7 +54,8 @@ static_assert(offsetof(Gridding, minY) == sizeof(double) && offsetof(Gridding, m
 struct NodeGrid
 {
     Gridding grid;
-    double diag;     // half diagonal of 3x3x3 cells (rp_subsampling.cu:55-60)
+    float cell;      // side of a cell
+    float weight;    // -10 log2(e) / diag^2, diag: half diagonal of 3x3x3 cells (rp_subsampling.cu:55-60)
     uint32_t salt;   // explicit-random rank salt
     uint32_t id;     // sparse node id
 };

@@ -964,6 +964,7 @@ static __global__ __launch_bounds__(BLOCK) void kEmitB(const BatchCloud<T>* __re
                                                  const uint32_t* __restrict__ prefix)
 {
     __shared__ uint32_t wp[MAX_BATCH + 1];
+    __shared__ uint2 lds[MODE == COLOR_INTER_WEIGHTED ? WEIGHT_LDS : 1];
     loadPrefix(prefix, B, wp);
     for (uint64_t i = globalThread(); i < wp[B]; i += globalStride())
     {
@@ -973,7 +974,7 @@ static __global__ __launch_bounds__(BLOCK) void kEmitB(const BatchCloud<T>* __re
         const uint32_t cursor   = static_cast<uint32_t>(cc.sc[BS_CURSOR]);
         if constexpr (MODE == COLOR_INTER_WEIGHTED)
             emitWeightedCell<T>(k, 0, cc.wordsPerNode, cursor, cc.g, cc.nodeGrid, cc.bitmap, cc.prefix, cc.cellKey,
-                                cc.cellNode, cc.cellStart, cc.payload, cc.winKey, cc.store());
+                                cc.cellNode, cc.cellStart, cc.payload, cc.winKey, cc.store(), lds);
         else
             emitCell<T, MODE>(k, cc.wordsPerNode, cursor, cc.g, cc.bitmap, cc.prefix, cc.cellKey,
                               cc.cellNode, cc.win, cc.color, cc.store());

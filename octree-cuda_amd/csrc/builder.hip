@@ -515,12 +515,19 @@ void OctreeBuilder::countPoints()
                                             itsSplitChunks.as<uint64_t>(), nb},
                             itsScanScratch.as<uint64_t>(), sc + SC_BUCKETS, itsStream);
     OC_LAUNCH_CHECK();
-    const unsigned scatterBlocks = static_cast<unsigned>((static_cast<uint64_t>(n) + STAGE_CHUNK - 1) / STAGE_CHUNK);
-    kBucketScatter<T><<<scatterBlocks, SCATTER_THREADS, 0, itsStream>>>(itsCloudDevice, n, itsCloud.dataStride, g,
-                                                                     3 * itsCoarse, nb, bucketCursor,
-                                                                     itsBucketed.as<SortedPoint<T>>(),
-                                                                     itsFineCode.as<uint16_t>());
-    OC_LAUNCH_CHECK();
+    auto scatter = [&](auto kernel, uint32_t items) {
+        const uint64_t chunk = static_cast<uint64_t>(SCATTER_THREADS) * items;
+        kernel<<<static_cast<unsigned>((n + chunk - 1) / chunk), SCATTER_THREADS, 0, itsStream>>>(
+                itsCloudDevice, n, itsCloud.dataStride, g, 3 * itsCoarse, nb, bucketCursor,
+                itsBucketed.as<SortedPoint<T>>(), itsFineCode.as<uint16_t>());
+        OC_LAUNCH_CHECK();
+    };
+    if (n <= SCATTER_ONE_POINTS)
+        scatter(kBucketScatter<T, 1>, 1);
+    else if (n <= SCATTER_TWO_POINTS)
+        scatter(kBucketScatter<T, 2>, 2);
+    else
+        scatter(kBucketScatter<T, LARGE_STAGE_ITEMS<T>>, LARGE_STAGE_ITEMS<T>);
     FineSortParams fp{};
     fp.lc         = itsCoarse;
     fp.bucketGrid = itsProc.chunkingGrid >> itsCoarse;

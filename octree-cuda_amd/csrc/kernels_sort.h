@@ -210,26 +210,26 @@ struct BucketTablesOut
     }
 };
 
-// Each workgroup takes a chunk of STAGE_CHUNK consecutive points, ranks them per bucket in LDS,
+// Each workgroup takes a chunk of ITEMS consecutive points per thread, ranks them per bucket in LDS,
 // reserves one range per occupied bucket with a single global atomic, stages the records in LDS
 // in bucket order and writes them out so that consecutive lanes write consecutive records of one
 // bucket.
 // LDS of one bucket-scatter workgroup
-template <typename T>
+template <typename T, int ITEMS = STAGE_ITEMS>
 struct ScatterLds
 {
-    SortedPoint<T> stage[STAGE_CHUNK];
+    SortedPoint<T> stage[SCATTER_THREADS * ITEMS];
     uint32_t delta[MAX_BUCKETS];           // counts, then global start - local start
     uint16_t localStart[MAX_BUCKETS];      // first staged slot of every bucket
     uint32_t scratch[SCATTER_THREADS / 64];
 };
 
-// One chunk of STAGE_CHUNK points (all threads of the workgroup; ends with the LDS free again).
-template <typename T>
+// One chunk (all threads of the workgroup; ends with the LDS free again).
+template <typename T, int ITEMS = STAGE_ITEMS>
 __device__ __forceinline__ void bucketScatterChunk(uint32_t chunk, const uint8_t* __restrict__ cloud, uint32_t n,
                                                    uint32_t stride, const Gridding& g, uint32_t fineBits,
                                                    uint32_t* __restrict__ cursor, SortedPoint<T>* __restrict__ dst,
-                                                   uint16_t* __restrict__ fineCode, ScatterLds<T>& lds)
+                                                   uint16_t* __restrict__ fineCode, ScatterLds<T, ITEMS>& lds)
 {
     SortedPoint<T>* stage = lds.stage;
     uint32_t* delta       = lds.delta;
@@ -239,11 +239,11 @@ __device__ __forceinline__ void bucketScatterChunk(uint32_t chunk, const uint8_t
         delta[b] = 0;
     __syncthreads();
 
-    const uint64_t base = static_cast<uint64_t>(chunk) * STAGE_CHUNK;
-    uint32_t code[STAGE_ITEMS], rank[STAGE_ITEMS];
-    SortedPoint<T> p[STAGE_ITEMS];
+    const uint64_t base = static_cast<uint64_t>(chunk) * (SCATTER_THREADS * ITEMS);
+    uint32_t code[ITEMS], rank[ITEMS];
+    SortedPoint<T> p[ITEMS];
 #pragma unroll
-    for (int j = 0; j < STAGE_ITEMS; ++j)
+    for (int j = 0; j < ITEMS; ++j)
     {
         const uint64_t i = base + static_cast<uint64_t>(j) * SCATTER_THREADS + threadIdx.x;
         code[j]          = ~0u;
@@ -289,7 +289,7 @@ __device__ __forceinline__ void bucketScatterChunk(uint32_t chunk, const uint8_t
     // records into LDS in bucket order
     const uint32_t fineMask = (1u << fineBits) - 1u;
 #pragma unroll
-    for (int j = 0; j < STAGE_ITEMS; ++j)
+    for (int j = 0; j < ITEMS; ++j)
         if (code[j] != ~0u)
             stage[localStart[code[j] >> fineBits] + rank[j]] = p[j];
     __syncthreads();
@@ -297,8 +297,8 @@ __device__ __forceinline__ void bucketScatterChunk(uint32_t chunk, const uint8_t
     // a staged record's bucket is recomputed from its coordinates (a few FP64 operations) rather
     // than searched for among the buckets' first slots (a dozen dependent LDS reads). The records of a
     // wave go out word by word, consecutive lanes storing consecutive words: a record stored by its own
-    // lane, and a fine code from the unsorted points, were a request of the L2 each (float points, 25.8M /
-    // 5.1M: 660 -> 608 / 134 -> 118 us; 119.7M double points 2.5 ms either way).
+    // lane, and a fine code from the unsorted points, were a request of the L2 each (chunks of 4 float points
+    // per thread, 25.8M / 5.1M: 660 -> 608 / 134 -> 118 us; 119.7M double points 2.5 ms either way).
     using Word              = std::conditional_t<sizeof(T) == 8, uint4, uint32_t>;
     constexpr uint32_t W    = sizeof(SortedPoint<T>) / sizeof(Word);
     const uint32_t lane     = threadIdx.x & 63;
@@ -330,15 +330,23 @@ __device__ __forceinline__ void bucketScatterChunk(uint32_t chunk, const uint8_t
     __syncthreads();
 }
 
+// Points per thread of a single cloud's scatter. A workgroup's runs in the buckets are the longer the more
+// points it stages, and it takes a global atomic for each: as many as a CU's LDS holds (25.8M float points
+// with 2 / 4 / 6 per thread: 965 / 608 / 495 us). Clouds that would leave most CUs without a chunk take
+// smaller ones (50K points with 1 / 2 / 4: 8.3 / 9.9 / 13.6 us; 200K with 1 / 2: 17.3 / 15.2 us).
 template <typename T>
+constexpr int LARGE_STAGE_ITEMS = sizeof(T) == 4 ? 6 : STAGE_ITEMS;
+constexpr uint32_t SCATTER_ONE_POINTS = 1u << 17, SCATTER_TWO_POINTS = 1u << 19;
+
+template <typename T, int ITEMS>
 static __global__ __launch_bounds__(SCATTER_THREADS) void kBucketScatter(const uint8_t* __restrict__ cloud, uint32_t n,
                                                                 uint32_t stride, Gridding g, uint32_t fineBits,
                                                                 uint32_t buckets, uint32_t* __restrict__ cursor,
                                                                 SortedPoint<T>* __restrict__ dst,
                                                                 uint16_t* __restrict__ fineCode)
 {
-    __shared__ ScatterLds<T> lds;
-    bucketScatterChunk<T>(blockIdx.x, cloud, n, stride, g, fineBits, cursor, dst, fineCode, lds);
+    __shared__ ScatterLds<T, ITEMS> lds;
+    bucketScatterChunk<T, ITEMS>(blockIdx.x, cloud, n, stride, g, fineBits, cursor, dst, fineCode, lds);
 }
 
 struct FineSortParams

@@ -305,7 +305,7 @@ uint64_t OctreeBuilder::estimateFootprint(const CloudInfo& cloud, const Processi
     if (n > FINE_SPLIT)                                     // split buckets of the fine sort
         bytes += (2 * n / FINE_SPLIT + 1) * (8 + 4ull * MAX_FINE_CELLS);
     bytes += (4 + 18 + coordinateBytes(cloud)) * staged;     // staging
-    bytes += 8 * (staged / PLACE_CHUNK + 1);                // placement work list
+    bytes += 8 * (staged / 4096 + 1);                       // placement work list (the rest of it from the staging)
     if (proc.useInterCellAvg && proc.useWeightingFunction && !proc.useIntraCellAvg)
         bytes += 4 * staged;                                // staged colours of the weighted filter
     // per-level work: inputs (cell, then its dense index; rank; payload) and cells (winner, colour sum,

@@ -8,8 +8,8 @@ morrowbay-sized cloud: 119,701,547 points, 27-byte records (3 x float64 + RGB, c
 by 1e6), grids 512/128, merge threshold 10000, implicit subsampling with distance-weighted
 inter-cell colour filtering, output factor 2.2.
 
-Prints one JSON line. `roofline` is for the dominant kernel class, timed with HIP events on the
-session stream by the library; `cpu_baseline` times the CPU oracle on the same cloud on this host.
+Prints one JSON line. `roofline` is for the dominant kernel class, timed with device clock
+stamps by the library; `cpu_baseline` times the CPU oracle on the same cloud on this host.
 `host_to_host` is one cloud from host memory to results in host memory (never `value`);
 `other_workloads` the device-resident rate of the other named single-cloud shapes. `batched` is the
 batched-build workload (256 clouds of 10K-2M points) through the batched pipeline (one launch per
@@ -325,7 +325,7 @@ def main():
     ms = float(np.mean(step_ms))
     avg = {k: float(np.mean([t[k] for t in timings])) for k in timings[0]}
 
-    # roofline of the dominant stage (device time from HIP events on the session stream)
+    # roofline of the dominant stage (device time from clock stamps of the session's kernels)
     stage_ms = {"count": avg["count_ms"], "distribute": avg["distribute_ms"], "subsample": avg["subsample_ms"]}
     grid = wl.build.chunking_grid
 

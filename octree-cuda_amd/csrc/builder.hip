@@ -12,8 +12,8 @@
 //   nodes (SoA)    key, dense count, pointCount, dataIdx (u64), parent, children[8], flags, ...
 //   output region  E records: lut (u32 point index), out (18-byte record). [0, N) holds the leaves,
 //                  [N, N + I) the subsampled points in DFS post-order
-//   staging        subsampled points in level order (index, record, coordinates), read by the
-//                  next level and permuted into the output region at the end
+//   staging        subsampled points in level order (index, coordinates, colour), read by the
+//                  next level; their records go to the output region at the end
 #include "builder.h"
 
 #include <hip/hip_runtime.h>

@@ -6,10 +6,10 @@
 // cell instead (child slot order: x bit 4, y bit 2, z bit 1, as point_count_propagation.cuh:62-70),
 // in two passes that only use LDS atomics per point:
 //   kBucketHist     per-workgroup LDS histogram of coarse buckets (level-lc cells) -> bucket sizes
-//   kBucketScatter  each workgroup ranks its chunk of 4096 points per bucket in LDS, reserves one
+//   kBucketScatter  each workgroup ranks its chunk of points per bucket in LDS, reserves one
 //                   range per bucket with a single global atomic, stages the chunk in bucket order
-//                   in LDS and writes 32-byte sorted-point records (coordinates, point index,
-//                   colour) plus the 3*lc-bit fine code as contiguous runs
+//                   in LDS and writes sorted-point records (coordinates, point index, colour) plus
+//                   the 3*lc-bit fine code as contiguous runs
 //   kFineSort       one workgroup per bucket: LDS histogram over the bucket's (2^lc)^3 level-0
 //                   cells, exclusive scan, dense counts of levels 0..lc of the count pyramid,
 //                   then the permutation into full Morton order (4-byte indices)

@@ -4,7 +4,7 @@
 // nodes). Each node of a batch owns an occupancy bitmap over its g^3 subsampling grid and the
 // exclusive popcount prefix of that bitmap's words, i.e. a rank dictionary: the occupied cells of
 // the batch get dense indices in (node, cell index) order; the cell index groups the grid's x-rows
-// into 4 x 4 pencils (rowIndex). Per batch:
+// into 4 x 4 pencils or is a Morton code (CellOrder). Per batch:
 //   kMark        input point -> cell (the reference's mapPointToGrid with the node's gridding),
 //                set the cell's bit
 //   prefix scan  popcounts of all bitmap words -> dense index of every occupied cell
@@ -13,8 +13,9 @@
 //   (kMarkLarge, kAccumulateLarge and kAccumulateRest in large builds)
 //   kScatterPayload (weighted only) each point's offset from its cell centre + colour, and its
 //                winner key, in cell order
-//   kEmit        one output record per occupied cell, in ascending cell order per node
+//   kEmit        one staged point per occupied cell, in ascending cell order per node
 //                (kEmitWeighted for the distance-weighted filter)
+// and after the last level kPlaceNodes and kPermute, which write the staged points' records.
 // Leaf points come from the sorted cloud, whose leaf ranges kLeafCellOrder has put in the cell
 // order of each leaf's parent grid, so a level's first reads of them follow the bitmap.
 #pragma once
@@ -1521,9 +1522,9 @@ static __global__ __launch_bounds__(TILE) void kScatterPayload(TileRange range, 
                                       cellKey, rankOf, cellStart, cellOf, ps, payload, winKey, parts);
 }
 
-// Select (rp_subsampling.cuh:70-321, fp_subsampling.cuh:30-306): one output record per occupied
-// cell, written to staging at its dense index (node by node, cells ascending). The record keeps the
-// winner's global quantised position; the colour is the winner's (no filter), the decoded intra
+// Select (rp_subsampling.cuh:70-321, fp_subsampling.cuh:30-306): one point per occupied
+// cell, written to staging at its dense index (node by node, cells ascending). The point keeps the
+// winner's position; the colour is the winner's (no filter), the decoded intra
 // sum, or the decoded sum of the per-cell sums over the 3x3x3 neighbourhood (inter; equal to the
 // reference's per-point scatter into occupied neighbours because integer sums commute). The
 // neighbourhood is walked as 9 x-rows: the occupied cells among x-1..x+1 of one row have

@@ -87,7 +87,7 @@ void writeJsonReport(const std::string& filename, const BuildResult& b, const Ho
     j["pointDistribution"]["minPointsPerNode"]       = Json::u(s.minPointsPerNode);
     j["pointDistribution"]["maxPointsPerNode"]       = Json::u(s.maxPointsPerNode);
 
-    // device-side stage durations of the last build (HIP events on the session stream)
+    // device-side stage durations of the last build (clock stamps of its kernels)
     const auto& t             = b.stageTimings();
     const char* names[]       = {"pointCounting", "merging", "pointDistribution", "subsampling"};
     float accumulated         = 0.f;

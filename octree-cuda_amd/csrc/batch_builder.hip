@@ -339,8 +339,13 @@ uint64_t BatchBuilder::estimateFootprint(const std::vector<BatchRequest>& reques
             carveCloud(cv, cc, r, s, L, mode, &copy);
             carveNodes(cv, cc, std::min<uint64_t>(s.mBound, 2 * s.n + 16), s);
         }
-        // admission charges a staged point its whole record (and the weighted filter's colour)
+        // A budget admits the same requests as it did for a larger arena: admission charges a staged point
+        // its whole record (and the weighted filter's colour), a dense cell an id of its own, a node its
+        // block size, and the placement list chunks of 4096 records.
+        const uint64_t words = (static_cast<uint64_t>(L.dense) + 31) / 32;
         bytes += s.staged * (sizeof(OutRecord) - (packedColors(mode) ? 8 : mode == COLOR_NONE ? 4 : 0));
+        bytes += sizeof(uint32_t) * (L.dense - 2 * words + std::min<uint64_t>(s.mBound, 2 * s.n + 16));
+        bytes -= sizeof(uint64_t) * (s.staged / PLACE_CHUNK - s.staged / 4096);
         bytes += cv.off + BS_SLOTS * 8 + 4096;
     }
     return bytes;

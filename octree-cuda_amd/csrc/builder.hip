@@ -312,7 +312,10 @@ uint64_t OctreeBuilder::estimateFootprint(const CloudInfo& cloud, const Processi
     // count, start, key, node), both bounded by N and with it by E; the occupancy bitmaps and their prefix
     const uint64_t wordsPerNode = (rowsPerNode(proc.subsamplingGrid) * proc.subsamplingGrid + 31) / 32;
     const uint64_t levelNodes   = std::min<uint64_t>(mBound, n / std::max<uint32_t>(1, proc.mergingThreshold) + 8);
-    bytes += std::max<uint64_t>((8 + sizeof(WeightPayload) + sizeof(uint64_t)) * e + 32 * staged, 48 * n);
+    // for E next to N they take more than is charged by E, less what is charged above for an id per cell
+    const uint64_t spare = 4 * (dense - (dense + 31) / 32);
+    bytes += std::max<uint64_t>((8 + sizeof(WeightPayload) + sizeof(uint64_t)) * e + 32 * staged,
+                                48 * n > spare ? 48 * n - spare : 0);
     bytes += std::min<uint64_t>(kBitmapBudget, 8 * wordsPerNode * levelNodes);
     return bytes;
 }

@@ -183,7 +183,7 @@ void OctreeBuilder::setup(const CloudInfo& cloud, const ProcessingInfo& proc, co
         itsLevelNodes[l]    = g * g * g;
         itsDense += g * g * g;
     }
-    itsCoarse  = std::min<uint32_t>(MAX_COARSE_LEVEL, itsDepth > 3 ? itsDepth - 3 : 0);
+    itsCoarse  = coarseLevel(itsDepth);
     itsBuckets = (proc.chunkingGrid >> itsCoarse) * (proc.chunkingGrid >> itsCoarse) * (proc.chunkingGrid >> itsCoarse);
     itsColorMode = proc.useIntraCellAvg ? COLOR_INTRA
                                         : (proc.useInterCellAvg ? (proc.useWeightingFunction ? COLOR_INTER_WEIGHTED
@@ -539,11 +539,17 @@ void OctreeBuilder::countPoints()
         fp.levelOffset[l] = itsLevelOffset[l];
         fp.levelGrid[l]   = itsLevelGrid[l];
     }
-    kFineSort<<<std::min<uint32_t>(nb, COMPUTE_UNITS), SORT_THREADS, 0, itsStream>>>(
-            itsFineCode.as<uint16_t>(), bucketStart, itsBucketList.as<uint32_t>(), totals,
-            reinterpret_cast<uint32_t*>(sc + SC_NEXT_BUCKET), fp, itsCount.as<uint32_t>(), itsPerm.as<uint32_t>(),
-            occ);
-    OC_LAUNCH_CHECK();
+    auto fineSort = [&](auto kernel, uint32_t perUnit) {
+        kernel<<<std::min<uint32_t>(nb, perUnit * COMPUTE_UNITS), SORT_THREADS, 0, itsStream>>>(
+                itsFineCode.as<uint16_t>(), bucketStart, itsBucketList.as<uint32_t>(), totals,
+                reinterpret_cast<uint32_t*>(sc + SC_NEXT_BUCKET), fp, itsCount.as<uint32_t>(),
+                itsPerm.as<uint32_t>(), occ);
+        OC_LAUNCH_CHECK();
+    };
+    if (itsCoarse < MAX_COARSE_LEVEL)
+        fineSort(kFineSort<SMALL_FINE_CELLS>, 2);
+    else
+        fineSort(kFineSort<MAX_FINE_CELLS>, 1);
     if (n > FINE_SPLIT)
     {
         itsSplitHist.ensure(sizeof(uint32_t) * MAX_FINE_CELLS * chunkBound);

@@ -35,6 +35,18 @@ namespace oc {
 
 constexpr uint32_t MAX_COARSE_LEVEL = 5;                               // (2^5)^3 level-0 cells per bucket
 constexpr uint32_t MAX_FINE_CELLS   = 1u << (3 * MAX_COARSE_LEVEL);    // 32768
+constexpr uint32_t SMALL_FINE_CELLS = 1u << (3 * (MAX_COARSE_LEVEL - 1));
+
+// Bucket level of a single cloud's sort. A 256^3 grid has 16^3 buckets, as a 512^3 one: with 8^3 it had
+// fewer occupied ones than compute units, each with a histogram eight times as large (1.5M points:
+// kFineSort 73 -> 46 us, kLeafCellOrder 41 -> 36, kBucketScatter 41 -> 47). Smaller grids keep 8^3, whose
+// cells are few (64^3 grid, 50K points: kFineSort 9.2 us, 12.3 with 16^3).
+constexpr uint32_t coarseLevel(uint32_t depth)
+{
+    const uint32_t above = depth >= 8 ? 4 : 3;
+    const uint32_t level = depth > above ? depth - above : 0;
+    return level < MAX_COARSE_LEVEL ? level : MAX_COARSE_LEVEL;
+}
 constexpr uint32_t MAX_BUCKETS      = 4096;                            // (512 >> 5)^3
 constexpr int SORT_THREADS          = 1024;
 constexpr int SORT_WAVES            = SORT_THREADS / 64;
@@ -523,9 +535,10 @@ __device__ __forceinline__ void fineSortBucket(uint32_t b, const uint16_t* __res
     finePermute(fineCode, lo, hi, h, lo, perm);
 }
 
-// The occupied buckets (list of `totals` bits 32-47), a workgroup per compute unit taking the next
-// one from a counter: with its 132 KB of LDS one workgroup fits a compute unit, and a grid over all
+// The occupied buckets (list of `totals` bits 32-47), one or two workgroups per compute unit taking the
+// next one from a counter: with the 132 KB of LDS of 32^3 cells one fits, and a grid over all
 // buckets spent 16 rounds of launches on the empty ones (512^3 grid: 4096, a few hundred occupied).
+template <uint32_t CELLS>
 static __global__ __launch_bounds__(SORT_THREADS) void kFineSort(const uint16_t* __restrict__ fineCode,
                                                            const uint32_t* __restrict__ bucketStart,
                                                            const uint32_t* __restrict__ occupied,
@@ -534,7 +547,7 @@ static __global__ __launch_bounds__(SORT_THREADS) void kFineSort(const uint16_t*
                                                            uint32_t* __restrict__ count, uint32_t* __restrict__ perm,
                                                            uint32_t* __restrict__ occ)
 {
-    __shared__ uint32_t h[MAX_FINE_CELLS + 1];
+    __shared__ uint32_t h[CELLS + 32];  // fineSlot moves an entry by up to 31, the total's too
     __shared__ uint32_t scratch[SORT_WAVES];
     __shared__ uint32_t mine;
     const uint32_t buckets = static_cast<uint32_t>(*totals >> 32) & 0xFFFF;

@@ -24,6 +24,7 @@
 
 #include <cstdint>
 
+#include "cell_order.h"
 #include "device_common.h"
 #include "kernels_chunking.h"
 #include "kernels_sort.h"
@@ -33,11 +34,6 @@ namespace oc {
 
 constexpr uint32_t TILE = 256;  // inputs per workgroup in the per-input kernels
 
-// Cell index of a node grid. The x-rows (fixed y, z) are grouped into 4 x 4 pencils, pencils in
-// (z / 4, y / 4) order and rows inside a pencil in (z % 4, y % 4) order; a cell is row * g + x.
-// A row stays one contiguous run of bits (and of dense ranks), and the 9 rows a cell's 3x3x3
-// neighbourhood touches lie a few rows apart instead of a whole z-plane apart.
-constexpr uint32_t PENCIL = 4;
 constexpr uint32_t EMIT_CHUNK = 32;  // consecutive cell blocks of the weighted emit per XCD turn
 constexpr uint32_t XCD_TILE_RUN = 32;  // consecutive input tiles of kMark / kScatterPayload per XCD turn
 
@@ -54,70 +50,6 @@ __host__ __forceinline__ uint32_t xcdRunGrid(uint64_t items, uint32_t run)
     const uint64_t round = static_cast<uint64_t>(XCD_COUNT) * run;
     return static_cast<uint32_t>((items + round - 1) / round * round);
 }
-
-__host__ __device__ __forceinline__ uint32_t pencilsPerAxis(uint32_t g)
-{
-    return (g + PENCIL - 1) / PENCIL;
-}
-
-__host__ __device__ __forceinline__ uint64_t rowsPerNode(uint32_t g)
-{
-    const uint64_t p = pencilsPerAxis(g);
-    return p * p * PENCIL * PENCIL;
-}
-
-__host__ __device__ __forceinline__ uint32_t rowIndex(uint32_t y, uint32_t z, uint32_t g)
-{
-    const uint32_t p = pencilsPerAxis(g);
-    return (((z / PENCIL) * p + (y / PENCIL)) * PENCIL + (z % PENCIL)) * PENCIL + (y % PENCIL);
-}
-
-__host__ __device__ __forceinline__ void rowCoords(uint32_t row, uint32_t g, uint32_t& y, uint32_t& z)
-{
-    const uint32_t p = pencilsPerAxis(g), pencil = row / (PENCIL * PENCIL), inside = row % (PENCIL * PENCIL);
-    y = (pencil % p) * PENCIL + inside % PENCIL;
-    z = (pencil / p) * PENCIL + inside / PENCIL;
-}
-
-// A cell's coordinates from its index, g the same for all cells of a build: shifts where it is a power of
-// two, integer divisions (some 25 instructions each) where not.
-__device__ __forceinline__ void cellCoords(uint32_t cell, uint32_t g, uint32_t& x, uint32_t& y, uint32_t& z)
-{
-    if (g >= PENCIL && (g & (g - 1)) == 0)
-    {
-        const uint32_t s = static_cast<uint32_t>(__builtin_ctz(g)), p = g / PENCIL;
-        const uint32_t row = cell >> s, pencil = row / (PENCIL * PENCIL), inside = row % (PENCIL * PENCIL);
-        x = cell & (g - 1);
-        y = (pencil & (p - 1)) * PENCIL + inside % PENCIL;
-        z = (pencil >> __builtin_ctz(p)) * PENCIL + inside / PENCIL;
-        return;
-    }
-    x = cell % g;
-    rowCoords(cell / g, g, y, z);
-}
-
-// The 3 x 3 x-rows around a cell: rowIndex is a sum of a part in y and one in z, so the first cells of
-// the nine rows are nine sums.
-struct CellRows
-{
-    uint32_t y[3], z[3];  // the parts, in cells
-    bool inY[3], inZ[3];  // in the grid
-    __device__ __forceinline__ CellRows(uint32_t cy, uint32_t cz, uint32_t g)
-    {
-        const uint32_t p = pencilsPerAxis(g);
-#pragma unroll
-        for (uint32_t k = 0; k < 3; ++k)
-        {
-            const uint32_t ny = cy + k - 1, nz = cz + k - 1;  // below zero: above any g
-            inY[k] = ny < g;
-            inZ[k] = nz < g;
-            y[k]   = (ny / PENCIL * (PENCIL * PENCIL) + ny % PENCIL) * g;
-            z[k]   = (nz / PENCIL * p * (PENCIL * PENCIL) + nz % PENCIL * PENCIL) * g;
-        }
-    }
-    __device__ __forceinline__ bool has(int r) const { return inY[r / 3] && inZ[r % 3]; }
-    __device__ __forceinline__ uint32_t start(int r) const { return y[r / 3] + z[r % 3]; }
-};
 
 // Order of a node grid's cells in its bitmap, and so of a node's staged points and of the leaf points
 // that the node reads: rows in pencils where the colour filter walks neighbourhoods, Morton order
@@ -1073,9 +1005,9 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kWordReduce(const uint32_
         rangeSums[blockIdx.x] = range;
 }
 
-// Second pass: the prefix of every word in the tiles that hold any occupied cell, and of every node's
-// first word (no other is read). The nodes' cells lie on surfaces, so most tiles (a slab of four cell
-// layers of a 128^3 grid) are empty: neither read nor written here.
+// Second pass: the prefix of every word in the tiles that hold any occupied cell, and of the words of the
+// others that are read (emptyWordPrefixes). The nodes' cells lie on surfaces, so most tiles (a slab of four
+// cell layers of a 128^3 grid) are empty: not read here, and next to nothing written.
 static __global__ __launch_bounds__(SCAN_THREADS) void kWordPrefix(const uint32_t* __restrict__ bitmap, uint64_t words,
                                                             uint64_t wordsPerNode,
                                                             const uint32_t* __restrict__ tileSums,
@@ -1093,9 +1025,7 @@ static __global__ __launch_bounds__(SCAN_THREADS) void kWordPrefix(const uint32_
         if (sum == 0)
         {
             const uint64_t end = base + SCAN_TILE < words ? base + SCAN_TILE : words;
-            for (uint64_t w = ((base + wordsPerNode - 1) / wordsPerNode + threadIdx.x) * wordsPerNode; w < end;
-                 w += SCAN_THREADS * wordsPerNode)
-                prefix[w] = carry;
+            emptyWordPrefixes(base, end, wordsPerNode, threadIdx.x, SCAN_THREADS, [=](uint64_t w) { prefix[w] = carry; });
             continue;
         }
         uint32_t v[SCAN_ITEMS], pre[SCAN_ITEMS];
@@ -1556,15 +1486,10 @@ __device__ __forceinline__ void emitCell(uint32_t c, uint64_t wordsPerNode, uint
             {
                 if (!rows.has(r))
                     continue;
-                const uint32_t L0 = rows.start(r) + x0, w0 = L0 >> 5, b0 = L0 & 31;
-                uint64_t v        = nodeBits[w0];
-                if (b0 + span > 32)
-                    v |= static_cast<uint64_t>(nodeBits[w0 + 1]) << 32;
-                const uint32_t m     = static_cast<uint32_t>(v >> b0) & ((1u << span) - 1u);
-                const uint32_t first = nodePrefix[w0] + __popc(static_cast<uint32_t>(v) & ((1u << b0) - 1u));
+                const RowRun run = rowRun(nodeBits, nodePrefix, rows.start(r) + x0, span);
                 // at most 3 occupied cells (x - 1 .. x + 1): predicated loads, no loop, so the
                 // rows' loads are all in flight together
-                const uint32_t n = __popc(m);
+                const uint32_t n = run.count, first = run.first;
                 if (n > 0)
                     sum += color[first];
                 if (n > 1)
@@ -1658,13 +1583,9 @@ __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, 
         first[r] = 0;
         if (!rows.has(r))
             continue;
-        const uint32_t L0 = rows.start(r) + x0, w0 = L0 >> 5, b0 = L0 & 31;
-        uint64_t v        = nodeBits[w0];
-        if (b0 + span > 32)
-            v |= static_cast<uint64_t>(nodeBits[w0 + 1]) << 32;
-        const uint32_t m = static_cast<uint32_t>(v >> b0) & ((1u << span) - 1u);
-        count[r]         = __popc(m);
-        first[r]         = nodePrefix[w0] + __popc(static_cast<uint32_t>(v) & ((1u << b0) - 1u));
+        const RowRun run = rowRun(nodeBits, nodePrefix, rows.start(r) + x0, span);
+        count[r]         = run.count;
+        first[r]         = run.first;
     }
     // the payload runs of the non-empty rows, in order, through LDS: the loop below takes them by number
     uint32_t lo[9], hi[9];

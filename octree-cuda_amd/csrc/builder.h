@@ -127,6 +127,7 @@ private:
     uint32_t stepNodes() const;
     uint32_t planSteps();
     uint64_t leafChunkBound() const;
+    const uint64_t* readSteps(const uint64_t* total, uint32_t nodes, uint32_t stepNodes, uint32_t first);
     uint64_t placeChunkBound() const;
     template <typename T>
     void distributePoints();

@@ -108,9 +108,18 @@ size_t DeviceBuffer::peakAllocated()
 // Bytes of bitmap + prefix the nodes of one subsampling batch may use.
 static constexpr uint64_t kBitmapBudget = 6ull << 30;
 
-// Bitmap words up to which a level's cells are reset with its bitmap, one per input (a launch less; on
-// larger levels there are many more inputs than cells).
+// Bitmap words up to which a level's cells are reset with its bitmap, one per input (a launch less: 2M points
+// at grids 256 / 64 904 us, 922 with a launch of its own). On larger levels there are many more inputs than
+// cells; up to 3M points it makes no more than 2 % there, either way.
 static constexpr uint64_t RESET_INPUTS_WORDS = 1u << 20;
+
+// Points, and children of a level's nodes, from which the host reads a level's tiles and inputs back to size
+// its launches (subsampleLevels). Points: 4M 1168 us with readbacks, 1129 without; 8M 1779 / 1747; 30M 5191
+// / 5250, the weighted filter 9382 / 9545; 14M to 20M alike. Children (4M points, threshold 20, g = 8, 800K
+// children on the lowest level): 10.7 ms with them, 11.3 without; 1M points 3.01 / 3.13; from 4096 children
+// on instead of 131072 alike.
+static constexpr uint32_t READ_INPUTS_POINTS   = 1u << 24;
+static constexpr uint32_t READ_INPUTS_CHILDREN = 1u << 17;
 
 // words of the host mailbox
 enum MailSlot
@@ -120,12 +129,13 @@ enum MailSlot
     MAIL_NODES,
     MAIL_INTERNAL,
     MAIL_USED,
-    MAIL_INPUTS,
     MAIL_LEVEL = 8,                        // first node of every level
     MAIL_INNER = MAIL_LEVEL + MAX_LEVELS,  // first internal node of every level
     MAIL_TICKS = MAIL_INNER + MAX_LEVELS,  // stage durations
-    MAIL_WORDS = MAIL_TICKS + 7
+    MAIL_STEPS = MAIL_TICKS + 7,           // tiles and inputs before a level's steps, and after the last one
+    MAIL_WORDS = MAIL_STEPS + 64
 };
+constexpr uint32_t PUBLISHED_STEPS = MAIL_WORDS - MAIL_STEPS - 1;
 
 static uint32_t octreeDepth(uint32_t grid)  // tools.cu:63-88
 {
@@ -380,13 +390,22 @@ __global__ __launch_bounds__(64) void kPublishMerge(const uint64_t* __restrict__
         __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// (tiles << 32 | inputs) of a level
-__global__ void kPublishInputs(const uint64_t* __restrict__ segTotal, uint64_t* box, uint64_t seq)
+// (tiles << 32 | inputs) of a level before its step `first` and the PUBLISHED_STEPS after it, a step being
+// stepNodes of the level's `nodes`; past the last one: all of the level. segTile, segInput: the segment scan.
+__global__ __launch_bounds__(64) void kPublishSteps(const uint64_t* __restrict__ segTotal,
+                                                    const uint32_t* __restrict__ segTile,
+                                                    const uint32_t* __restrict__ segInput, uint32_t nodes,
+                                                    uint32_t stepNodes, uint32_t first, uint64_t* box, uint64_t seq)
 {
-    if (threadIdx.x != 0)
-        return;
-    __hip_atomic_store(box + MAIL_INPUTS, *segTotal & 0xFFFFFFFFull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    const uint64_t node = (static_cast<uint64_t>(first) + threadIdx.x) * stepNodes;
+    const uint64_t v =
+            node < nodes ? (static_cast<uint64_t>(segTile[8 * node]) << 32) | segInput[8 * node] : *segTotal;
+    if (threadIdx.x <= PUBLISHED_STEPS)
+        __hip_atomic_store(box + MAIL_STEPS + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The end of a build: the error flags, the used output records (the last cursor) and the stage
@@ -713,6 +732,17 @@ uint64_t OctreeBuilder::placeChunkBound() const
     return (itsE - itsCloud.pointAmount) / PLACE_CHUNK + itsInner[itsDepth + 1];
 }
 
+// The host's copy of the totals before the steps of a level from step `first` on (kPublishSteps).
+const uint64_t* OctreeBuilder::readSteps(const uint64_t* total, uint32_t nodes, uint32_t stepNodes, uint32_t first)
+{
+    const uint64_t seq = ++itsMailSeq;
+    kPublishSteps<<<1, 64, 0, itsStream>>>(total, itsSegTile.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodes, stepNodes,
+                                           first, itsMailbox, seq);
+    OC_LAUNCH_CHECK();
+    waitMailbox(seq);
+    return itsMailbox + MAIL_STEPS;
+}
+
 template <typename T>
 void OctreeBuilder::distributePoints()
 {
@@ -727,10 +757,21 @@ void OctreeBuilder::distributePoints()
     // copied from it
     const uint32_t n = itsCloud.pointAmount;
     if (itsInner[itsDepth + 1] > 0 && p.g >= 2)
-        kLeafCellOrder<T><<<static_cast<unsigned>(leafChunkBound()), LEAF_THREADS, 0, itsStream>>>(
-                itsLeafList.as<uint64_t>(), itsScalars.as<uint64_t>() + SC_LEAF_TOTAL, p, itsNodeKey.as<uint32_t>(),
-                itsNodeParent.as<int32_t>(), itsNodeCount.as<uint32_t>(), itsNodeSorted.as<uint32_t>(),
-                itsBucketed.as<SortedPoint<T>>(), itsPerm.as<uint32_t>(), itsSorted.as<SortedPoint<T>>(), stamp);
+    {
+        uint64_t chunks = leafChunkBound();
+        if (std::min<uint64_t>(8ull * itsInner[itsDepth + 1], itsM) >= READ_INPUTS_CHILDREN)
+            chunks = readSteps(itsScalars.as<uint64_t>() + SC_LEAF_TOTAL, 0, 0, 0)[0] >> 32;
+        for (uint64_t first = 0; first == 0 || first < chunks; first += LEAF_LAUNCH_CHUNKS)
+        {
+            const uint64_t some = std::min<uint64_t>(chunks - first, LEAF_LAUNCH_CHUNKS);
+            kLeafCellOrder<T><<<static_cast<unsigned>(std::max<uint64_t>(1, some)), LEAF_THREADS, 0, itsStream>>>(
+                    itsLeafList.as<uint64_t>(), static_cast<uint32_t>(first),
+                    itsScalars.as<uint64_t>() + SC_LEAF_TOTAL, p, itsNodeKey.as<uint32_t>(),
+                    itsNodeParent.as<int32_t>(), itsNodeCount.as<uint32_t>(), itsNodeSorted.as<uint32_t>(),
+                    itsBucketed.as<SortedPoint<T>>(), itsPerm.as<uint32_t>(), itsSorted.as<SortedPoint<T>>(),
+                    first == 0 ? stamp : nullptr);
+        }
+    }
     else
         kGatherSorted<T><<<gatherGrid(n), BLOCK, 0, itsStream>>>(itsBucketed.as<SortedPoint<T>>(),
                                                                      itsPerm.as<uint32_t>(), n,
@@ -764,17 +805,16 @@ uint32_t OctreeBuilder::planSteps()
     return itsSteps;
 }
 
-// Points from which the host reads a level's inputs back to size its launches.
-static constexpr uint32_t READ_INPUTS_POINTS = 1u << 24;
-
 // The levels bottom-up, a step per batch of a level's nodes. The merge has told the host the internal
 // nodes of every level; inputs, tiles, occupied cells and the output cursor stay on the device, the
 // launches are sized by bounds (a level's inputs are distinct points, so there are at most N of them,
-// and no more cells than inputs), and a step that does not fit the output leaves itself and the later
-// ones without work. So the host waits for nothing: with two readbacks a level, each of which drains
-// the GPU for ~15 us, small builds spent a third of their time waiting. From READ_INPUTS_POINTS points
-// on, one readback a level costs less than the empty workgroups of the upper levels (a 120M-point
-// bound is 470K of them, ~30 us a launch, three or four launches a level). Grids that stride over
+// and no more cells than inputs; only children that there are can have tiles), and a step that does not fit
+// the output leaves itself and the later ones without work. So the host waits for nothing: with two
+// readbacks a level, each of which drains the GPU for ~15 us, small builds spent a third of their time
+// waiting. From READ_INPUTS_POINTS points or READ_INPUTS_CHILDREN children on, one readback a level costs
+// less than the empty workgroups (a 120M-point bound is 470K of them, ~30 us a launch, three or four
+// launches a level), and a level of several steps reads the sizes of each: the level's bound would be
+// launched again for every step. Grids that stride over
 // the work instead were slower on large levels (payload scatter 3.9 -> 4.9 ms, emit 11.0 -> 11.9 ms at
 // 119.7M points): workgroups drift apart and no longer share cache lines while they are in L2.
 template <typename T>
@@ -814,14 +854,13 @@ void OctreeBuilder::subsampleLevels()
     if (levelMost == 0)
         return;
     const uint64_t segMost  = 8ull * levelMost;
-    const uint64_t tileMost = N / TILE + segMost;
     const uint64_t wordMost = std::min(levelMost, batchNodes) * wordsPerNode;
     itsSegCount.ensure(sizeof(uint32_t) * segMost);
     itsSegSrc.ensure(sizeof(uint32_t) * segMost);
     itsSegTile.ensure(sizeof(uint32_t) * segMost);
     itsSegInput.ensure(sizeof(uint32_t) * segMost);
     itsNodeGrid.ensure(sizeof(NodeGrid) * levelMost);
-    itsTileList.ensure(sizeof(uint32_t) * tileMost);
+    itsTileList.ensure(sizeof(uint32_t) * (N / TILE + segMost));
     itsBitmap.ensure(sizeof(uint32_t) * wordMost);
     itsPrefix.ensure(sizeof(uint32_t) * (wordMost + 1));
     itsScanScratch.ensure(sizeof(uint64_t) * SCAN_GRID + sizeof(uint32_t) * scanTiles(wordMost));  // range, tile sums
@@ -848,40 +887,36 @@ void OctreeBuilder::subsampleLevels()
     uint32_t* prefix  = itsPrefix.as<uint32_t>();
     const CellState cellState{win, color, cellCnt};
 
-    // tiles combined in LDS, where there are enough points for them and the flag bit is free
-    const bool large          = N >= LARGE_POINTS && N < NOT_OWNED && 32 * wordsPerNode < NOT_OWNED;
-    const uint32_t tileInputs = large ? LARGE_TILE : TILE;
-    const int tileThreads     = large ? LARGE_THREADS : static_cast<int>(TILE);
     uint32_t stepAt = 0;
     for (uint32_t l = 1; l <= itsDepth; ++l)
     {
         const uint32_t K = itsInner[l + 1] - itsInner[l];
         if (K == 0)
             continue;
+        // the segments that can hold inputs: children of the level's nodes
+        const uint64_t children = std::min<uint64_t>(8ull * K, itsLevelStart[l] - itsLevelStart[l - 1]);
+        // tiles combined in LDS, where there are enough points for them and the flag bit is free
+        const bool large = N >= LARGE_POINTS && N / children >= LARGE_CHILD && N < NOT_OWNED &&
+                           32 * wordsPerNode < NOT_OWNED;
+        const uint32_t tileInputs  = large ? LARGE_TILE : TILE;
+        const int tileThreads      = large ? LARGE_THREADS : static_cast<int>(TILE);
         const ChildSlots cs        = childSlots(itsInner[l]);
         NodeGrid* nodeGrid         = itsNodeGrid.as<NodeGrid>();
         const LevelSegmentIn segIn{cs, itsNodePoints.as<uint32_t>(), tileInputs};
         const LevelSegmentOut segOut{cs, itsNodeSorted.as<uint32_t>(), itsNodeStage.as<uint32_t>(),
                                      itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegTile.as<uint32_t>(),
                                      itsSegInput.as<uint32_t>()};
+        const bool readBack     = N >= READ_INPUTS_POINTS || K > batchNodes || children >= READ_INPUTS_CHILDREN;
         // in one launch with the level's other preparations, when it is one step sized without a readback
-        const bool oneLaunch = K <= START_NODES && K <= batchNodes && N < READ_INPUTS_POINTS;
+        const bool oneLaunch = K <= START_NODES && !readBack;
         if (!oneLaunch)
         {
             scanExclusive<uint64_t>(8ull * K, segIn, segOut, itsScanScratch.as<uint64_t>(), sc + SC_SEG_TOTAL, itsStream);
             OC_LAUNCH_CHECK();
         }
-        uint64_t inputMost = N;
-        if (N >= READ_INPUTS_POINTS)
-        {
-            const uint64_t seq = ++itsMailSeq;
-            kPublishInputs<<<1, 64, 0, itsStream>>>(sc + SC_SEG_TOTAL, itsMailbox, seq);
-            OC_LAUNCH_CHECK();
-            waitMailbox(seq);
-            inputMost = itsMailbox[MAIL_INPUTS];
-        }
         const uint32_t parts    = tileInputs / TILE;
-        const uint32_t tileGrid = xcdRunGrid(inputMost / tileInputs + 8ull * K, XCD_TILE_RUN / parts);
+        const uint64_t* totals  = nullptr;  // read back, from step stepAt - firstStep on
+        const uint32_t firstStep = stepAt;
         sp.level       = l;
         sp.levelOffset = itsLevelOffset[l];
         sp.levelGrid   = itsLevelGrid[l];
@@ -892,10 +927,29 @@ void OctreeBuilder::subsampleLevels()
             const uint32_t k1 = std::min<uint32_t>(K, k0 + batchNodes);
             const uint32_t Kb = k1 - k0;
             const uint64_t words = static_cast<uint64_t>(Kb) * wordsPerNode;
+            uint64_t inputMost = N, tileMost = N / tileInputs + std::min<uint64_t>(children, 8ull * Kb);
+            if (readBack)
+            {
+                const uint32_t at = (stepAt - firstStep) % PUBLISHED_STEPS;
+                if (at == 0)
+                    totals = readSteps(sc + SC_SEG_TOTAL, K, batchNodes, stepAt - firstStep);
+                inputMost = static_cast<uint32_t>(totals[at + 1] - totals[at]);
+                tileMost  = (totals[at + 1] >> 32) - (totals[at] >> 32);
+            }
             const uint64_t cellMost = std::min<uint64_t>(inputMost, 32 * words);
-            const TileRange tiles{k0 > 0 ? itsSegTile.as<uint32_t>() + 8ull * k0 : nullptr,
-                                  k1 < K ? itsSegTile.as<uint32_t>() + 8ull * k1
-                                         : reinterpret_cast<uint32_t*>(sc + SC_SEG_TOTAL) + 1};
+            const uint32_t* tilesLo = k0 > 0 ? itsSegTile.as<uint32_t>() + 8ull * k0 : nullptr;
+            const uint32_t* tilesHi = k1 < K ? itsSegTile.as<uint32_t>() + 8ull * k1
+                                             : reinterpret_cast<uint32_t*>(sc + SC_SEG_TOTAL) + 1;
+            // launch(tiles, workgroups, first launch) until all tiles of the step are taken
+            auto overTiles = [&](auto launch) {
+                for (uint64_t skip = 0; skip == 0 || skip < tileMost; skip += LAUNCH_TILES)
+                {
+                    const uint64_t some = std::max<uint64_t>(1, std::min<uint64_t>(tileMost - skip, LAUNCH_TILES));
+                    launch(TileRange{tilesLo, tilesHi, static_cast<uint32_t>(skip)},
+                           xcdRunGrid(some, XCD_TILE_RUN / parts), skip == 0);
+                    OC_LAUNCH_CHECK();
+                }
+            };
             const StepSizes step{cursors + stepAt, cursors + stepAt + 1, prefix + words, itsE};
             uint64_t* stamps = itsStamps.as<uint64_t>() + ST_STAMPS * stepAt;
             ++stepAt;
@@ -908,16 +962,18 @@ void OctreeBuilder::subsampleLevels()
                         itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs, stamps + ST_BEGIN);
             else
                 kLevelPrepare<<<prepareGrid, BLOCK, 0, itsStream>>>(
-                        K, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
+                        k0 == 0 ? K : 0, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
                         sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs,
                         stamps + ST_BEGIN);
             OC_LAUNCH_CHECK();
             auto mark = [&](auto kernel) {
-                kernel<<<tileGrid, tileThreads, 0, itsStream>>>(
-                        tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                        itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid, ps,
-                        cellOrderOf(itsColorMode, g), bitmap, itsCellOf.as<uint32_t>(), err, stamps + ST_INSERT_BEGIN);
-                OC_LAUNCH_CHECK();
+                overTiles([&](const TileRange& tiles, uint32_t grid, bool begin) {
+                    kernel<<<grid, tileThreads, 0, itsStream>>>(
+                            tiles, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                            itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
+                            ps, cellOrderOf(itsColorMode, g), bitmap, itsCellOf.as<uint32_t>(), err,
+                            begin ? stamps + ST_INSERT_BEGIN : nullptr);
+                });
             };
             mark(large ? kMarkLarge<T> : kMark<T>);
             const uint64_t wordTiles = scanTiles(words);
@@ -941,22 +997,25 @@ void OctreeBuilder::subsampleLevels()
             }
 
             auto accumulate = [&](auto kernel) {
-                kernel<<<tileGrid, tileThreads, 0, itsStream>>>(
-                        tiles, step, k0, Kb, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                        itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
-                        bitmap, prefix, itsCellOf.as<uint32_t>(), ps, win, color, cellCnt, itsCellKey.as<uint32_t>(),
-                        itsCellNode.as<uint32_t>(), weighted ? itsRankOf.as<uint32_t>() : nullptr,
-                        itsNodePoints.as<uint32_t>(), itsNodeStage.as<uint32_t>(), itsNodeSub.as<uint32_t>(),
-                        itsNodeFlags.as<uint8_t>(), itsNodeChild.as<int32_t>(), err);
-                OC_LAUNCH_CHECK();
+                overTiles([&](const TileRange& tiles, uint32_t grid, bool begin) {
+                    kernel<<<grid, tileThreads, 0, itsStream>>>(
+                            tiles, step, k0, begin ? Kb : 0, wordsPerNode, itsTileList.as<uint32_t>(),
+                            itsSegTile.as<uint32_t>(), itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(),
+                            itsSegInput.as<uint32_t>(), nodeGrid, bitmap, prefix, itsCellOf.as<uint32_t>(), ps, win,
+                            color, cellCnt, itsCellKey.as<uint32_t>(), itsCellNode.as<uint32_t>(),
+                            weighted ? itsRankOf.as<uint32_t>() : nullptr, itsNodePoints.as<uint32_t>(),
+                            itsNodeStage.as<uint32_t>(), itsNodeSub.as<uint32_t>(), itsNodeFlags.as<uint8_t>(),
+                            itsNodeChild.as<int32_t>(), err);
+                });
             };
             auto rest = [&](auto kernel) {
-                kernel<<<tileGrid, tileThreads, 0, itsStream>>>(
-                        tiles, step, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                        itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
-                        bitmap, prefix, itsCellOf.as<uint32_t>(), ps, win, color, cellCnt,
-                        weighted ? itsRankOf.as<uint32_t>() : nullptr);
-                OC_LAUNCH_CHECK();
+                overTiles([&](const TileRange& tiles, uint32_t grid, bool) {
+                    kernel<<<grid, tileThreads, 0, itsStream>>>(
+                            tiles, step, k0, wordsPerNode, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                            itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
+                            bitmap, prefix, itsCellOf.as<uint32_t>(), ps, win, color, cellCnt,
+                            weighted ? itsRankOf.as<uint32_t>() : nullptr);
+                });
             };
             auto accumulateMode = [&](auto mode, auto random) {
                 constexpr uint32_t M = decltype(mode)::value;
@@ -987,19 +1046,20 @@ void OctreeBuilder::subsampleLevels()
                                         itsScanScratch.as<uint32_t>(), static_cast<uint32_t*>(nullptr), itsStream);
                 OC_LAUNCH_CHECK();
                 auto scatter = [&](auto kernel) {
-                    kernel<<<tileGrid * parts, TILE, 0, itsStream>>>(
-                            tiles, step, g, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
-                            itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(), nodeGrid,
-                            itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(), itsCellStart.as<uint32_t>(),
-                            itsCellOf.as<uint32_t>(), ps, itsPayload.as<WeightPayload>(), winKey, parts,
-                            stamps + ST_INSERT_END);
-                    OC_LAUNCH_CHECK();
+                    overTiles([&](const TileRange& tiles, uint32_t grid, bool begin) {
+                        kernel<<<grid * parts, TILE, 0, itsStream>>>(
+                                tiles, step, g, itsTileList.as<uint32_t>(), itsSegTile.as<uint32_t>(),
+                                itsSegCount.as<uint32_t>(), itsSegSrc.as<uint32_t>(), itsSegInput.as<uint32_t>(),
+                                nodeGrid, itsCellKey.as<uint32_t>(), itsRankOf.as<uint32_t>(),
+                                itsCellStart.as<uint32_t>(), itsCellOf.as<uint32_t>(), ps,
+                                itsPayload.as<WeightPayload>(), winKey, parts, begin ? stamps + ST_INSERT_END : nullptr);
+                    });
                 };
                 scatter(random ? kScatterPayload<T, true> : kScatterPayload<T, false>);
             }
 
             if (weighted)
-                kEmitWeighted<T><<<xcdRunGrid((cellMost + BLOCK - 1) / BLOCK, EMIT_CHUNK), BLOCK, 0, itsStream>>>(
+                kEmitWeighted<T><<<xcdRunGrid(std::max<uint64_t>(1, (cellMost + BLOCK - 1) / BLOCK), EMIT_CHUNK), BLOCK, 0, itsStream>>>(
                         step, k0, wordsPerNode, g, nodeGrid, bitmap, prefix, itsCellKey.as<uint32_t>(),
                         itsCellNode.as<uint32_t>(), itsCellStart.as<uint32_t>(), itsPayload.as<WeightPayload>(), winKey,
                         ps, stamps + ST_EMIT_BEGIN);

@@ -10,7 +10,7 @@
 //   prefix scan  popcounts of all bitmap words -> dense index of every occupied cell
 //   kAccumulate  winner per cell (atomicMin of rank<<32 | input position), packed colour sums,
 //                per-cell point counts for the weighted filter
-//   (kMarkLarge, kAccumulateLarge and kAccumulateRest in large builds)
+//   (kMarkLarge, kAccumulateLarge and kAccumulateRest on the levels of large builds)
 //   kScatterPayload (weighted only) each point's offset from its cell centre + colour, and its
 //                winner key, in cell order
 //   kEmit        one staged point per occupied cell, in ascending cell order per node
@@ -255,6 +255,7 @@ constexpr int LEAF_THREADS    = 1024;
 constexpr int LEAF_ITEMS      = 4;                          // points per thread, held in registers
 constexpr uint32_t LEAF_KEYS  = 8192;                       // word keys (histogram entries)
 constexpr uint32_t LEAF_CHUNK = LEAF_THREADS * LEAF_ITEMS;  // points per workgroup
+constexpr uint32_t LEAF_LAUNCH_CHUNKS = 1u << 21;           // of one launch (fewer than 2^32 work-items)
 
 struct LeafOrderParams
 {
@@ -456,7 +457,7 @@ __device__ __forceinline__ void leafCellOrderChunk(uint64_t entry, const LeafOrd
 }
 
 template <typename T>
-static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrder(const uint64_t* __restrict__ chunkList,
+static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrder(const uint64_t* __restrict__ chunkList, uint32_t first,
                                                                 const uint64_t* __restrict__ totals, LeafOrderParams p,
                                                                 const uint32_t* __restrict__ nodeKey,
                                                                 const int32_t* __restrict__ parent,
@@ -468,9 +469,10 @@ static __global__ __launch_bounds__(LEAF_THREADS) void kLeafCellOrder(const uint
 {
     __shared__ LeafOrderLds lds;
     stampStart(stamp);
-    if (blockIdx.x >= *totals >> 32)
+    const uint32_t chunk = first + blockIdx.x;
+    if (chunk >= *totals >> 32)
         return;  // the whole workgroup: the grid is an upper bound
-    leafCellOrderChunk<T>(chunkList[blockIdx.x], leafOrderView(p), nodeKey, parent, count, sortedStart, bucketed, perm,
+    leafCellOrderChunk<T>(chunkList[chunk], leafOrderView(p), nodeKey, parent, count, sortedStart, bucketed, perm,
                           out, lds);
 }
 
@@ -600,8 +602,9 @@ struct CellState
 
 // Before a level's first pass: the griddings of its nodes, the segment of every tile (a search per
 // tile, all of them in flight; a thread per segment wrote a large child's thousands of entries by
-// itself, 71 us of a 5.1M-point build) and a clear bitmap. For a small level also the state of as many
-// cells as it has inputs (it has no more), which spares it kClearCompact.
+// itself, 71 us of a 5.1M-point build) and a clear bitmap. nodes = 0: only the bitmap and the cells (a later
+// step of the same level). For a small level also the state of as many cells as it has inputs (it has no
+// more), which spares it kClearCompact.
 __device__ __forceinline__ void levelPrepare(uint32_t nodes, const SubsampleParams& sp,
                                              const uint32_t* __restrict__ internal,
                                              const uint32_t* __restrict__ nodeKey, NodeGrid* __restrict__ nodeGrid,
@@ -612,7 +615,7 @@ __device__ __forceinline__ void levelPrepare(uint32_t nodes, const SubsamplePara
     for (uint64_t k = globalThread(); k < nodes; k += globalStride())
         nodeGrid[k] = nodeGridOf(internal[k], nodeKey[internal[k]], sp.levelOffset, sp.levelGrid, sp.level, sp.depth,
                                  sp.cubicMin, sp.sideHalf, sp.side, sp.g, sp.seed);
-    const uint32_t tiles = static_cast<uint32_t>(segTotal >> 32);
+    const uint32_t tiles = nodes ? static_cast<uint32_t>(segTotal >> 32) : 0u;
     for (uint64_t t = globalThread(); t < tiles; t += globalStride())
     {
         // the last segment that starts at or before t; segments without tiles start where the next does
@@ -684,13 +687,23 @@ static __global__ __launch_bounds__(BLOCK) void kLevelStart(uint32_t nodes, Subs
     levelPrepare(nodes, sp, in.cs.internal, nodeKey, nodeGrid, segTile, total, tileList, words, bitmap, cells, reset);
 }
 
-// The tiles of a batch of a level's nodes: from *lo (null: 0) to *hi.
+// Tiles that one launch takes: a launch holds fewer than 2^32 work-items, kScatterPayload's 256 for each of
+// up to four parts of a tile.
+constexpr uint32_t LAUNCH_TILES = 1u << 21;
+
+// The tiles of a batch of a level's nodes, from *lo (null: 0) to *hi, without the `skip` first ones (of
+// earlier launches): as many of them as one launch takes.
 struct TileRange
 {
     const uint32_t* lo;
     const uint32_t* hi;
-    __device__ __forceinline__ uint32_t first() const { return lo ? *lo : 0u; }
-    __device__ __forceinline__ uint32_t count() const { return *hi - first(); }
+    uint32_t skip;
+    __device__ __forceinline__ uint32_t first() const { return (lo ? *lo : 0u) + skip; }
+    __device__ __forceinline__ uint32_t count() const
+    {
+        const uint32_t from = first(), to = *hi;
+        return to <= from ? 0u : to - from < LAUNCH_TILES ? to - from : LAUNCH_TILES;
+    }
 };
 
 // Clock stamps of a subsampling step, then one after the last step.
@@ -801,7 +814,7 @@ static __global__ __launch_bounds__(TILE) void kMark(TileRange range, uint32_t n
                 order, bitmap, cellOf, err);
 }
 
-// Large builds: tiles of LARGE_TILE inputs, combined in LDS before anything goes to memory.
+// Levels of large builds: tiles of LARGE_TILE inputs, combined in LDS before anything goes to memory.
 //
 // What bounds the passes over the inputs there is the number of their atomics: the XCDs' L2s are not
 // coherent with each other, so every global atomic is carried out in memory, some 20 requests per ns on
@@ -816,8 +829,14 @@ static __global__ __launch_bounds__(TILE) void kMark(TileRange range, uint32_t n
 //   119.7M, distance-weighted  2122 + 3150 + 87 -> 1930 + 1798 + 623 us
 //   5.1M, inter-cell           143 + 345 -> 144 + 185 + 51 us
 //   1.5M, no filter            54 + 66 -> 77 + 68 + 27 us
-// so from LARGE_POINTS on (below, a level has too few tiles to hide their barriers and one launch more).
+// so from LARGE_POINTS on (below, a level has too few tiles to hide their barriers and one launch more; whole
+// builds with / without, intra-cell and weighted: 2M points 791 / 770 and 1366 / 1323 us, 3.2M 958 / 973 and
+// 1539 / 1528, 4M 1136 / 1164, 8M 1753 / 1886 and 2969 / 3050), on the levels whose children can have
+// LARGE_CHILD points each: a tile holds inputs of one child, and one that is nearly empty clears its table for
+// a few of them. 8M points at threshold 20, a dozen inputs a child: 17.7 ms with large tiles, 15.3 without;
+// threshold 60: 10.6 / 9.3; threshold 1000, about 200 a child: 4.05 / 4.15. (512 instead of 256: alike.)
 constexpr uint32_t LARGE_POINTS = 3u << 20;
+constexpr uint32_t LARGE_CHILD  = 256;
 constexpr int LARGE_THREADS     = 256;
 constexpr int LARGE_ITEMS       = 4;  // per thread
 constexpr uint32_t LARGE_TILE   = LARGE_THREADS * LARGE_ITEMS;

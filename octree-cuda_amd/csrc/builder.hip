@@ -511,7 +511,7 @@ void OctreeBuilder::countPoints()
     uint32_t* bucketCursor = itsBucketCursor.as<uint32_t>();
     const Gridding g = gridding(itsCloud.bbMin[0], itsCloud.bbMin[1], itsCloud.bbMin[2],
                                 itsCloud.bbMax[0] - itsCloud.bbMin[0], itsProc.chunkingGrid);
-    itsScanScratch.ensure(sizeof(uint64_t) * (scanTiles(nb) + 1));
+    itsScanScratch.ensure(sizeof(uint64_t) * scanTiles(nb));
     uint32_t* occ         = itsOccupancy.as<uint32_t>();
     const uint64_t words  = (static_cast<uint64_t>(itsDense) + 31) / 32;
     const uint64_t counts = itsLevelOffset[itsCoarse];  // read for empty cells from here on

@@ -296,13 +296,6 @@ __device__ __forceinline__ uint64_t shflUp64(uint64_t v, int delta)
     return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
-__device__ __forceinline__ uint64_t shfl64(uint64_t v, int lane)
-{
-    const uint32_t lo = __shfl(static_cast<uint32_t>(v), lane, 64);
-    const uint32_t hi = __shfl(static_cast<uint32_t>(v >> 32), lane, 64);
-    return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-
 struct WaveRun
 {
     int lane, start, end;

@@ -143,23 +143,12 @@ struct SubsampleParams
     uint64_t seed;
 };
 
-// internal nodes of a level -> compact list
+// internal nodes of a level (batched builds)
 struct InternalIn
 {
     const uint8_t* flags;
     uint32_t levelStart;
     __device__ uint32_t operator()(uint64_t i) const { return (flags[levelStart + i] & NODE_INTERNAL) ? 1u : 0u; }
-};
-
-struct InternalOut
-{
-    uint32_t* list;
-    uint32_t levelStart;
-    __device__ void operator()(uint64_t i, uint32_t prefix, uint32_t v) const
-    {
-        if (v)
-            list[prefix] = levelStart + static_cast<uint32_t>(i);
-    }
 };
 
 // Subsampling grid of the node with linear index lin at level `level` (grid gl per axis): the

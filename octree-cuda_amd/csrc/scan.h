@@ -11,10 +11,9 @@
 // the SCAN_THREADS items k * SCAN_THREADS ..): a wave64 shuffle scan per row, the wave totals of
 // all rows through LDS, one barrier. Inputs and outputs are functors so the flags / values are
 // generated and consumed in the same pass as the scan (e.g. occupancy flags straight from the
-// counting grid); an output functor is called once per item, in no particular order, and may
-// write the item's own input (in-place scans). Out-of-place scans of at most SCAN_DIRECT_TILES tiles
-// take one launch (small builds make many small scans): one workgroup per tile, which reduces the
-// tiles before its own by itself.
+// counting grid); an output functor is called once per item, in no particular order. Scans of at
+// most SCAN_DIRECT_TILES tiles take one launch (small builds make many small scans): one workgroup
+// per tile, which reduces the tiles before its own by itself.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -306,20 +305,20 @@ __device__ __forceinline__ void blockScanAll(In in, Out out, uint64_t n, T* tota
         *total = carry;
 }
 
-// Out-of-place inputs up to this many tiles are scanned by kScanDirect: its last workgroup reads
+// Inputs up to this many tiles are scanned by kScanDirect: its last workgroup reads
 // all of them, SCAN_DIRECT_TILES / 2 dependent rounds of loads (16 tiles: ~6 us; one workgroup
 // walking them took ~25 us, two launches take ~9 us).
 constexpr uint64_t SCAN_DIRECT_TILES = 16;
 // Workgroups of a two-launch scan: eight of 256 threads fill each of 256 compute units.
 constexpr uint64_t SCAN_GRID = 2048;
 
-// Exclusive scan of in(0..n-1); out(i, prefix, value) for each i; *total (device) = sum.
-// tileScratch must hold scanTiles(n) values. inPlace: out writes what in reads.
+// Exclusive scan of in(0..n-1); out(i, prefix, value) for each i; *total (device) = sum. out must not write
+// what in reads. tileScratch must hold min(scanTiles(n), SCAN_GRID) values.
 template <typename T, typename In, typename Out>
-void scanExclusive(uint64_t n, In in, Out out, T* tileScratch, T* total, hipStream_t stream, bool inPlace = false)
+void scanExclusive(uint64_t n, In in, Out out, T* tileScratch, T* total, hipStream_t stream)
 {
     const uint64_t tiles = scanTiles(n);
-    if (tiles <= (inPlace ? 1 : SCAN_DIRECT_TILES))
+    if (tiles <= SCAN_DIRECT_TILES)
     {
         kScanDirect<T, In, Out><<<static_cast<unsigned>(tiles ? tiles : 1), SCAN_THREADS, 0, stream>>>(in, out, n,
                                                                                                        total);

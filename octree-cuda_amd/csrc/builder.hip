@@ -318,14 +318,12 @@ uint64_t OctreeBuilder::estimateFootprint(const CloudInfo& cloud, const Processi
     bytes += 8 * (staged / 4096 + 1);                       // placement work list (the rest of it from the staging)
     if (proc.useInterCellAvg && proc.useWeightingFunction && !proc.useIntraCellAvg)
         bytes += 4 * staged;                                // staged colours of the weighted filter
-    // per-level work: inputs (cell, then its dense index; rank; payload) and cells (winner, colour sum,
-    // count, start, key, node), both bounded by N and with it by E; the occupancy bitmaps and their prefix
+    // per-level work: inputs (cell, then its dense index; rank; payload), at most N and with it E, and cells
+    // (winner, colour sum, count, start, key, node), at most as many as are staged; the occupancy bitmaps
+    // and their prefix
     const uint64_t wordsPerNode = (rowsPerNode(proc.subsamplingGrid) * proc.subsamplingGrid + 31) / 32;
     const uint64_t levelNodes   = std::min<uint64_t>(mBound, n / std::max<uint32_t>(1, proc.mergingThreshold) + 8);
-    // for E next to N they take more than is charged by E, less what is charged above for an id per cell
-    const uint64_t spare = 4 * (dense - (dense + 31) / 32);
-    bytes += std::max<uint64_t>((8 + sizeof(WeightPayload) + sizeof(uint64_t)) * e + 32 * staged,
-                                48 * n > spare ? 48 * n - spare : 0);
+    bytes += (8 + sizeof(WeightPayload) + sizeof(uint64_t)) * e + 32 * staged;
     bytes += std::min<uint64_t>(kBitmapBudget, 8 * wordsPerNode * levelNodes);
     return bytes;
 }
@@ -865,19 +863,21 @@ void OctreeBuilder::subsampleLevels()
     itsPrefix.ensure(sizeof(uint32_t) * (wordMost + 1));
     itsScanScratch.ensure(sizeof(uint64_t) * SCAN_GRID + sizeof(uint32_t) * scanTiles(wordMost));  // range, tile sums
     itsCellOf.ensure(sizeof(uint32_t) * N);
-    itsCellKey.ensure(sizeof(uint32_t) * N);
-    itsCellNode.ensure(sizeof(uint32_t) * N);
+    // a step that fits the output (no other one touches the cells' arrays) has no more cells than are staged
+    const uint32_t cellCap = static_cast<uint32_t>(std::min<uint64_t>(N, std::max<uint64_t>(1, itsE - N)));
+    itsCellKey.ensure(sizeof(uint32_t) * cellCap);
+    itsCellNode.ensure(sizeof(uint32_t) * cellCap);
     if (weighted)
     {
         itsRankOf.ensure(sizeof(uint32_t) * N);
         itsPayload.ensure((sizeof(WeightPayload) + sizeof(uint64_t)) * N);  // payloads, then winner keys
-        itsCellCnt.ensure(sizeof(uint32_t) * N);
-        itsCellStart.ensure(sizeof(uint32_t) * (static_cast<uint64_t>(N) + 1));
+        itsCellCnt.ensure(sizeof(uint32_t) * cellCap);
+        itsCellStart.ensure(sizeof(uint32_t) * (static_cast<uint64_t>(cellCap) + 1));
     }
     else  // the weighted filter takes its winners from the payload keys
-        itsWin.ensure(sizeof(uint64_t) * N);
+        itsWin.ensure(sizeof(uint64_t) * cellCap);
     if (packed)
-        itsColor.ensure(sizeof(uint64_t) * N);
+        itsColor.ensure(sizeof(uint64_t) * cellCap);
     uint64_t* winKey =
             weighted ? reinterpret_cast<uint64_t*>(itsPayload.as<uint8_t>() + sizeof(WeightPayload) * N) : nullptr;
     uint64_t* win     = weighted ? nullptr : itsWin.as<uint64_t>();
@@ -936,7 +936,7 @@ void OctreeBuilder::subsampleLevels()
                 inputMost = static_cast<uint32_t>(totals[at + 1] - totals[at]);
                 tileMost  = (totals[at + 1] >> 32) - (totals[at] >> 32);
             }
-            const uint64_t cellMost = std::min<uint64_t>(inputMost, 32 * words);
+            const uint64_t cellMost = std::min<uint64_t>({inputMost, 32 * words, cellCap});
             const uint32_t* tilesLo = k0 > 0 ? itsSegTile.as<uint32_t>() + 8ull * k0 : nullptr;
             const uint32_t* tilesHi = k1 < K ? itsSegTile.as<uint32_t>() + 8ull * k1
                                              : reinterpret_cast<uint32_t*>(sc + SC_SEG_TOTAL) + 1;
@@ -955,15 +955,16 @@ void OctreeBuilder::subsampleLevels()
             ++stepAt;
 
             const bool resetInputs = !large && words <= RESET_INPUTS_WORDS;
+            const uint32_t reset   = resetInputs ? cellCap : 0;
             const unsigned prepareGrid = gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384);
             if (oneLaunch)
                 kLevelStart<<<std::min(prepareGrid, 2048u), BLOCK, 0, itsStream>>>(
                         K, sp, segIn, segOut, itsNodeKey.as<uint32_t>(), nodeGrid, sc + SC_SEG_TOTAL,
-                        itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs, stamps + ST_BEGIN);
+                        itsTileList.as<uint32_t>(), words, bitmap, cellState, reset, stamps + ST_BEGIN);
             else
                 kLevelPrepare<<<prepareGrid, BLOCK, 0, itsStream>>>(
                         k0 == 0 ? K : 0, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
-                        sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, resetInputs,
+                        sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, reset,
                         stamps + ST_BEGIN);
             OC_LAUNCH_CHECK();
             auto mark = [&](auto kernel) {
@@ -992,7 +993,7 @@ void OctreeBuilder::subsampleLevels()
             OC_LAUNCH_CHECK();
             if (!large && !resetInputs)
             {
-                kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(step.cells, cellState);
+                kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(step, cellState);
                 OC_LAUNCH_CHECK();
             }
 
@@ -1041,7 +1042,7 @@ void OctreeBuilder::subsampleLevels()
 
             if (weighted)
             {
-                scanExclusive<uint32_t>(DeviceCount{step.cells, nullptr}, cellMost, ArrayIn{cellCnt},
+                scanExclusive<uint32_t>(step, cellMost, ArrayIn{cellCnt},
                                         ExclusiveWithTotal{itsCellStart.as<uint32_t>(), step.cells},
                                         itsScanScratch.as<uint32_t>(), static_cast<uint32_t*>(nullptr), itsStream);
                 OC_LAUNCH_CHECK();

@@ -593,13 +593,13 @@ struct CellState
 // tile, all of them in flight; a thread per segment wrote a large child's thousands of entries by
 // itself, 71 us of a 5.1M-point build) and a clear bitmap. nodes = 0: only the bitmap and the cells (a later
 // step of the same level). For a small level also the state of as many cells as it has inputs (it has no
-// more), which spares it kClearCompact.
+// more, and no more than `reset`, the ones that the cell arrays hold), which spares it kClearCompact.
 __device__ __forceinline__ void levelPrepare(uint32_t nodes, const SubsampleParams& sp,
                                              const uint32_t* __restrict__ internal,
                                              const uint32_t* __restrict__ nodeKey, NodeGrid* __restrict__ nodeGrid,
                                              const uint32_t* segTile, uint64_t segTotal,
                                              uint32_t* __restrict__ tileList, uint64_t words,
-                                             uint32_t* __restrict__ bitmap, const CellState& cells, bool reset)
+                                             uint32_t* __restrict__ bitmap, const CellState& cells, uint32_t reset)
 {
     for (uint64_t k = globalThread(); k < nodes; k += globalStride())
         nodeGrid[k] = nodeGridOf(internal[k], nodeKey[internal[k]], sp.levelOffset, sp.levelGrid, sp.level, sp.depth,
@@ -623,8 +623,8 @@ __device__ __forceinline__ void levelPrepare(uint32_t nodes, const SubsamplePara
         bitmap[w] = 0;
     if (reset)
     {
-        const uint32_t inputs = static_cast<uint32_t>(segTotal);
-        for (uint64_t c = globalThread(); c < inputs; c += globalStride())
+        const uint32_t inputs = static_cast<uint32_t>(segTotal), most = inputs < reset ? inputs : reset;
+        for (uint64_t c = globalThread(); c < most; c += globalStride())
             cells.reset(c);
     }
 }
@@ -636,7 +636,7 @@ static __global__ __launch_bounds__(BLOCK) void kLevelPrepare(uint32_t nodes, Su
                                                         const uint32_t* __restrict__ segTile,
                                                         const uint64_t* __restrict__ segTotal,
                                                         uint32_t* __restrict__ tileList, uint64_t words,
-                                                        uint32_t* __restrict__ bitmap, CellState cells, bool reset,
+                                                        uint32_t* __restrict__ bitmap, CellState cells, uint32_t reset,
                                                         uint64_t* stamp)
 {
     stampStart(stamp);
@@ -653,7 +653,7 @@ static __global__ __launch_bounds__(BLOCK) void kLevelStart(uint32_t nodes, Subs
                                                       LevelSegmentOut out, const uint32_t* __restrict__ nodeKey,
                                                       NodeGrid* __restrict__ nodeGrid, uint64_t* __restrict__ segTotal,
                                                       uint32_t* __restrict__ tileList, uint64_t words,
-                                                      uint32_t* __restrict__ bitmap, CellState cells, bool reset,
+                                                      uint32_t* __restrict__ bitmap, CellState cells, uint32_t reset,
                                                       uint64_t* stamp)
 {
     __shared__ uint64_t lds[SCAN_ITEMS * SCAN_WAVES];
@@ -715,6 +715,8 @@ struct StepSizes
     uint64_t capacity;       // E
     // false: the points do not fit the output (A14); nothing of this step or a later one is written
     __device__ __forceinline__ bool fits() const { return *cursor + *cells <= capacity; }
+    // the cells to work on (the cell arrays hold no more than the output has room for)
+    __device__ uint64_t operator()() const { return fits() ? *cells : 0u; }
 };
 
 constexpr uint64_t CURSOR_FULL = 1ull << 62;
@@ -979,10 +981,10 @@ __device__ __forceinline__ void batchNodeOf(uint64_t kl, uint32_t nodeBase, uint
     stage[id]      = cursor + b;
 }
 
-// the state of a large level's cells (n: how many, on the device)
-static __global__ __launch_bounds__(BLOCK) void kClearCompact(const uint32_t* __restrict__ n, CellState cells)
+// the state of a large level's cells
+static __global__ __launch_bounds__(BLOCK) void kClearCompact(StepSizes step, CellState cells)
 {
-    const uint64_t count = *n;
+    const uint64_t count = step();
     for (uint64_t c = globalThread(); c < count; c += globalStride())
         cells.reset(c);
 }

@@ -176,8 +176,8 @@ struct HostCount
 struct DeviceCount
 {
     const uint32_t* end;
-    const uint32_t* begin;  // may be null
-    __device__ uint64_t operator()() const { return *end - (begin ? *begin : 0u); }
+    const uint32_t* begin;
+    __device__ uint64_t operator()() const { return *end - *begin; }
 };
 
 __host__ __device__ inline uint64_t scanTiles(uint64_t n)
@@ -329,10 +329,10 @@ void scanExclusive(uint64_t n, In in, Out out, T* tileScratch, T* total, hipStre
     kScanDown<T><<<grid, SCAN_THREADS, 0, stream>>>(in, out, HostCount{n}, tileScratch, total);
 }
 
-// The same over a number of items that only the device knows; bound: the most it can be.
+// The same over a number of items that only the device knows, n(); bound: the most it can be.
 // tileScratch must hold min(scanTiles(bound), SCAN_GRID) values.
-template <typename T, typename In, typename Out>
-void scanExclusive(DeviceCount n, uint64_t bound, In in, Out out, T* tileScratch, T* total, hipStream_t stream)
+template <typename T, typename Size, typename In, typename Out>
+void scanExclusive(Size n, uint64_t bound, In in, Out out, T* tileScratch, T* total, hipStream_t stream)
 {
     const uint64_t tiles = scanTiles(bound);
     const unsigned grid  = static_cast<unsigned>(tiles < SCAN_GRID ? (tiles ? tiles : 1) : SCAN_GRID);

@@ -121,6 +121,13 @@ static constexpr uint64_t RESET_INPUTS_WORDS = 1u << 20;
 static constexpr uint32_t READ_INPUTS_POINTS   = 1u << 24;
 static constexpr uint32_t READ_INPUTS_CHILDREN = 1u << 17;
 
+// Points from which the arrays of a level's inputs and cells are sized by what the host reads back, as each
+// level turns out (a readback more per step), instead of by the most that they can be: those bounds take up
+// to 8 % of a build's memory (40M points, grids 64 / 32: 10.6 GB instead of 9.8), which matters where a
+// build takes a good part of the card's 288 GB and costs nothing to speak of there.
+static constexpr uint32_t EXACT_ARRAYS_POINTS = 1u << 27;
+static_assert(EXACT_ARRAYS_POINTS >= READ_INPUTS_POINTS, "their levels' inputs are read back");
+
 // words of the host mailbox
 enum MailSlot
 {
@@ -132,10 +139,11 @@ enum MailSlot
     MAIL_LEVEL = 8,                        // first node of every level
     MAIL_INNER = MAIL_LEVEL + MAX_LEVELS,  // first internal node of every level
     MAIL_TICKS = MAIL_INNER + MAX_LEVELS,  // stage durations
-    MAIL_STEPS = MAIL_TICKS + 7,           // tiles and inputs before a level's steps, and after the last one
-    MAIL_WORDS = MAIL_STEPS + 64
+    MAIL_STEPS = MAIL_TICKS + 7,           // tiles and inputs before a level's steps and after the last of them
+    MAIL_TOTAL = MAIL_STEPS + 63,          // and of the whole level
+    MAIL_WORDS
 };
-constexpr uint32_t PUBLISHED_STEPS = MAIL_WORDS - MAIL_STEPS - 1;
+constexpr uint32_t PUBLISHED_STEPS = MAIL_TOTAL - MAIL_STEPS - 1;
 
 static uint32_t octreeDepth(uint32_t grid)  // tools.cu:63-88
 {
@@ -389,21 +397,31 @@ __global__ __launch_bounds__(64) void kPublishMerge(const uint64_t* __restrict__
 }
 
 // (tiles << 32 | inputs) of a level before its step `first` and the PUBLISHED_STEPS after it, a step being
-// stepNodes of the level's `nodes`; past the last one: all of the level. segTile, segInput: the segment scan.
+// stepNodes of the level's `nodes`; past the last one, and behind them (MAIL_TOTAL): all of the level.
+// segTile, segInput: the segment scan.
 __global__ __launch_bounds__(64) void kPublishSteps(const uint64_t* __restrict__ segTotal,
                                                     const uint32_t* __restrict__ segTile,
                                                     const uint32_t* __restrict__ segInput, uint32_t nodes,
                                                     uint32_t stepNodes, uint32_t first, uint64_t* box, uint64_t seq)
 {
     const uint64_t node = (static_cast<uint64_t>(first) + threadIdx.x) * stepNodes;
-    const uint64_t v =
-            node < nodes ? (static_cast<uint64_t>(segTile[8 * node]) << 32) | segInput[8 * node] : *segTotal;
-    if (threadIdx.x <= PUBLISHED_STEPS)
-        __hip_atomic_store(box + MAIL_STEPS + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    const uint64_t v    = threadIdx.x <= PUBLISHED_STEPS && node < nodes
+                                  ? (static_cast<uint64_t>(segTile[8 * node]) << 32) | segInput[8 * node]
+                                  : *segTotal;
+    __hip_atomic_store(box + MAIL_STEPS + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x == 0)
         __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The cells that a step works on.
+__global__ void kPublishCells(StepSizes step, uint64_t* box, uint64_t seq)
+{
+    if (threadIdx.x != 0)
+        return;
+    __hip_atomic_store(box + MAIL_USED, step(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(box + MAIL_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The end of a build: the error flags, the used output records (the last cursor) and the stage
@@ -862,31 +880,48 @@ void OctreeBuilder::subsampleLevels()
     itsBitmap.ensure(sizeof(uint32_t) * wordMost);
     itsPrefix.ensure(sizeof(uint32_t) * (wordMost + 1));
     itsScanScratch.ensure(sizeof(uint64_t) * SCAN_GRID + sizeof(uint32_t) * scanTiles(wordMost));  // range, tile sums
-    itsCellOf.ensure(sizeof(uint32_t) * N);
-    // a step that fits the output (no other one touches the cells' arrays) has no more cells than are staged
+    // Arrays for the inputs of a level and for the cells of a step. A step that fits the output (no other one
+    // touches the cells' arrays) has no more cells than are staged.
     const uint32_t cellCap = static_cast<uint32_t>(std::min<uint64_t>(N, std::max<uint64_t>(1, itsE - N)));
-    itsCellKey.ensure(sizeof(uint32_t) * cellCap);
-    itsCellNode.ensure(sizeof(uint32_t) * cellCap);
-    if (weighted)
+    const bool exactArrays = N >= EXACT_ARRAYS_POINTS;
+    uint64_t *winKey = nullptr, *win = nullptr, *color = nullptr;
+    uint32_t* cellCnt = nullptr;
+    auto sizeInputs   = [&](uint64_t inputs) {
+        itsCellOf.ensure(sizeof(uint32_t) * inputs);
+        if (weighted)
+        {
+            itsRankOf.ensure(sizeof(uint32_t) * inputs);
+            itsPayload.ensure((sizeof(WeightPayload) + sizeof(uint64_t)) * inputs);  // payloads, then winner keys
+            winKey = reinterpret_cast<uint64_t*>(itsPayload.as<uint8_t>() + sizeof(WeightPayload) * inputs);
+        }
+    };
+    auto sizeCells = [&](uint64_t cells) {
+        itsCellKey.ensure(sizeof(uint32_t) * cells);
+        itsCellNode.ensure(sizeof(uint32_t) * cells);
+        if (weighted)  // takes its winners from the payload keys
+        {
+            itsCellCnt.ensure(sizeof(uint32_t) * cells);
+            itsCellStart.ensure(sizeof(uint32_t) * (cells + 1));
+            cellCnt = itsCellCnt.as<uint32_t>();
+        }
+        else
+        {
+            itsWin.ensure(sizeof(uint64_t) * cells);
+            win = itsWin.as<uint64_t>();
+        }
+        if (packed)
+        {
+            itsColor.ensure(sizeof(uint64_t) * cells);
+            color = itsColor.as<uint64_t>();
+        }
+    };
+    if (!exactArrays)
     {
-        itsRankOf.ensure(sizeof(uint32_t) * N);
-        itsPayload.ensure((sizeof(WeightPayload) + sizeof(uint64_t)) * N);  // payloads, then winner keys
-        itsCellCnt.ensure(sizeof(uint32_t) * cellCap);
-        itsCellStart.ensure(sizeof(uint32_t) * (static_cast<uint64_t>(cellCap) + 1));
+        sizeInputs(N);
+        sizeCells(cellCap);
     }
-    else  // the weighted filter takes its winners from the payload keys
-        itsWin.ensure(sizeof(uint64_t) * cellCap);
-    if (packed)
-        itsColor.ensure(sizeof(uint64_t) * cellCap);
-    uint64_t* winKey =
-            weighted ? reinterpret_cast<uint64_t*>(itsPayload.as<uint8_t>() + sizeof(WeightPayload) * N) : nullptr;
-    uint64_t* win     = weighted ? nullptr : itsWin.as<uint64_t>();
-    uint64_t* color   = packed ? itsColor.as<uint64_t>() : nullptr;
-    uint32_t* cellCnt = weighted ? itsCellCnt.as<uint32_t>() : nullptr;
     uint32_t* bitmap  = itsBitmap.as<uint32_t>();
     uint32_t* prefix  = itsPrefix.as<uint32_t>();
-    const CellState cellState{win, color, cellCnt};
-
     uint32_t stepAt = 0;
     for (uint32_t l = 1; l <= itsDepth; ++l)
     {
@@ -933,6 +968,8 @@ void OctreeBuilder::subsampleLevels()
                 const uint32_t at = (stepAt - firstStep) % PUBLISHED_STEPS;
                 if (at == 0)
                     totals = readSteps(sc + SC_SEG_TOTAL, K, batchNodes, stepAt - firstStep);
+                if (exactArrays && k0 == 0)
+                    sizeInputs(std::max<uint32_t>(1, static_cast<uint32_t>(itsMailbox[MAIL_TOTAL])));
                 inputMost = static_cast<uint32_t>(totals[at + 1] - totals[at]);
                 tileMost  = (totals[at + 1] >> 32) - (totals[at] >> 32);
             }
@@ -954,18 +991,19 @@ void OctreeBuilder::subsampleLevels()
             uint64_t* stamps = itsStamps.as<uint64_t>() + ST_STAMPS * stepAt;
             ++stepAt;
 
-            const bool resetInputs = !large && words <= RESET_INPUTS_WORDS;
+            const bool resetInputs = !exactArrays && !large && words <= RESET_INPUTS_WORDS;
             const uint32_t reset   = resetInputs ? cellCap : 0;
             const unsigned prepareGrid = gridFor(std::max<uint64_t>(words, inputMost / TILE), 16384);
             if (oneLaunch)
                 kLevelStart<<<std::min(prepareGrid, 2048u), BLOCK, 0, itsStream>>>(
                         K, sp, segIn, segOut, itsNodeKey.as<uint32_t>(), nodeGrid, sc + SC_SEG_TOTAL,
-                        itsTileList.as<uint32_t>(), words, bitmap, cellState, reset, stamps + ST_BEGIN);
+                        itsTileList.as<uint32_t>(), words, bitmap, CellState{win, color, cellCnt}, reset,
+                        stamps + ST_BEGIN);
             else
                 kLevelPrepare<<<prepareGrid, BLOCK, 0, itsStream>>>(
                         k0 == 0 ? K : 0, sp, cs.internal, itsNodeKey.as<uint32_t>(), nodeGrid, itsSegTile.as<uint32_t>(),
-                        sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, cellState, reset,
-                        stamps + ST_BEGIN);
+                        sc + SC_SEG_TOTAL, itsTileList.as<uint32_t>(), words, bitmap, CellState{win, color, cellCnt},
+                        reset, stamps + ST_BEGIN);
             OC_LAUNCH_CHECK();
             auto mark = [&](auto kernel) {
                 overTiles([&](const TileRange& tiles, uint32_t grid, bool begin) {
@@ -991,9 +1029,17 @@ void OctreeBuilder::subsampleLevels()
                                                                   prefix);
             }
             OC_LAUNCH_CHECK();
+            if (exactArrays)
+            {
+                const uint64_t seq = ++itsMailSeq;
+                kPublishCells<<<1, 64, 0, itsStream>>>(step, itsMailbox, seq);
+                OC_LAUNCH_CHECK();
+                waitMailbox(seq);
+                sizeCells(std::max<uint64_t>(1, itsMailbox[MAIL_USED]));
+            }
             if (!large && !resetInputs)
             {
-                kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(step, cellState);
+                kClearCompact<<<gridFor(cellMost, 16384), BLOCK, 0, itsStream>>>(step, CellState{win, color, cellCnt});
                 OC_LAUNCH_CHECK();
             }
 

@@ -1650,12 +1650,26 @@ __device__ __forceinline__ void emitWeightedCell(uint32_t c, uint32_t nodeBase, 
     // Every lane walks its own runs one after the other, WEIGHT_LOADS payloads in flight: a wave then
     // takes as many steps as its fullest neighbourhood has points, and not in every one of the nine rows
     // as many as the fullest of that row (119.7M points: 75 payload loads a wave -> 45, 11.1 -> 10.8 ms; two
-    // or three in flight 11.5 ms).
+    // or three in flight 11.5 ms). Lanes that are all well inside a run take its next payloads without
+    // looking for its end: the last lanes around a cell that holds a good part of the cloud walk nothing else
+    // (three quarters of 5M points in one cell: 842 -> 705 ms, row by row 744; 119.7M points 30.9 / 30.4 ms).
     uint32_t run = 0, q = 0, e = 0;
     float uyc = 0.f, uzc = 0.f;
     while (points > 0)
     {
         uint4 pl[WEIGHT_LOADS];
+        if (__all(e - q >= WEIGHT_LOADS))
+        {
+#pragma unroll
+            for (uint32_t k = 0; k < WEIGHT_LOADS; ++k)
+                pl[k] = pv[q + k];
+#pragma unroll
+            for (uint32_t k = 0; k < WEIGHT_LOADS; ++k)
+                weigh(pl[k], uyc, uzc);
+            q += WEIGHT_LOADS;
+            points -= WEIGHT_LOADS;
+            continue;
+        }
         float uy[WEIGHT_LOADS], uz[WEIGHT_LOADS];
 #pragma unroll
         for (uint32_t k = 0; k < WEIGHT_LOADS; ++k)

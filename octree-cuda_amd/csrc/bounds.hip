@@ -1,6 +1,6 @@
 // Bounding box of a device-resident cloud: the caller-side step of the reference CLI
 // (calculateRealBB, src/boundingbox.h:10-33: per-axis fmin / fmax of the coordinates widened to
-// double) as a min/max reduction in one launch, and calculateCubicBB (:35-52) on the host.
+// double) as a two-pass min/max reduction, and calculateCubicBB (:35-52) on the host.
 #include "bounds.h"
 
 #include <hip/hip_runtime.h>
@@ -22,8 +22,11 @@ namespace oc {
 
 namespace {
 
-// Bound by HBM (119.7M 27-byte records: 5.3 TB/s of their lines), a small cloud by the launch.
-constexpr int BB_THREADS = 512;
+// Bound by HBM (40M 15-byte records 108 us, 5.6 TB/s), a small cloud by the launches. In one launch, whose last
+// workgroup reduced the others' results, every workgroup's release to the device cost more than the second
+// launch (~6 us, mostly under the first one's enqueueing): 1M 15-byte records 37 us a call instead of 19, 10M
+// 59 / 37, 40M 170 / 120; records staged through LDS or 512 threads a workgroup gained nothing there.
+constexpr int BB_THREADS = 256;
 constexpr int BB_BLOCKS  = 1024;
 
 __device__ __forceinline__ void waveMinMax(double v[6])
@@ -46,7 +49,6 @@ __device__ __forceinline__ void blockMinMax(double v[6])
     __shared__ double lds[BB_THREADS / 64][6];
     waveMinMax(v);
     const int w = threadIdx.x >> 6;
-    __syncthreads();
     if ((threadIdx.x & 63) == 0)
         for (int k = 0; k < 6; ++k)
             lds[w][k] = v[k];
@@ -70,64 +72,52 @@ __device__ __forceinline__ void include(double v[6], double x, double y, double 
     v[5] = fmax(v[5], z);
 }
 
-// Device memory of one reduction: the workgroups' minima and maxima, the final ones, and how many
-// workgroups are done (zero between reductions: the last workgroup resets it).
+// Device memory of one reduction: the workgroups' minima and maxima, and the final ones.
 struct BoundsScratch
 {
     double partial[6 * BB_BLOCKS];
     double result[6];
-    uint32_t done;
-    uint32_t pad;
 };
 
-// The workgroup that finishes last reduces the others' results (a second launch took 5 us and read
-// what the first had just written). box: null, or a coherent host mailbox of 6 values and a
-// sequence number, so that the caller needs no copy.
+// Minima and maxima of each workgroup.
 template <typename T>
-__global__ __launch_bounds__(BB_THREADS) void kBounds(const uint8_t* __restrict__ cloud, uint32_t n, uint32_t stride,
-                                                      BoundsScratch* scratch, uint64_t* box, uint64_t seq)
+__global__ __launch_bounds__(BB_THREADS) void kBoundsPartial(const uint8_t* __restrict__ cloud, uint32_t n,
+                                                             uint32_t stride, BoundsScratch* __restrict__ scratch)
 {
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    __shared__ RecordStage stages[BB_THREADS / 64];
-    forRecords<T, BB_THREADS>(cloud, n, stride, stages, [&v](double x, double y, double z) { include(v, x, y, z); });
+    for (uint64_t i = globalThread(); i < n; i += globalStride())
+    {
+        double x, y, z;
+        loadXYZ<T>(cloud + i * stride, x, y, z);
+        include(v, x, y, z);
+    }
     blockMinMax(v);
-    __shared__ bool last;
     if (threadIdx.x == 0)
-    {
         for (int k = 0; k < 6; ++k)
-            __hip_atomic_store(scratch->partial + 6 * blockIdx.x + k, v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = __hip_atomic_fetch_add(&scratch->done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x;
-    }
-    __syncthreads();
-    if (!last)
-        return;
-    for (int k = 0; k < 3; ++k)
-    {
-        v[k]     = INFINITY;
-        v[3 + k] = -INFINITY;
-    }
-    for (uint32_t b = threadIdx.x; b < gridDim.x; b += BB_THREADS)
-    {
-        double p[6];
-        for (int k = 0; k < 6; ++k)
-            p[k] = __hip_atomic_load(scratch->partial + 6 * b + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            scratch->partial[6 * blockIdx.x + k] = v[k];
+}
+
+// The final ones, from those of `blocks` workgroups. box: null, or a coherent host mailbox of 6 values and a
+// sequence number, so that the caller needs no copy.
+__global__ __launch_bounds__(BB_THREADS) void kBoundsFinal(BoundsScratch* scratch, uint32_t blocks, uint64_t* box,
+                                                           uint64_t seq)
+{
+    double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    for (uint32_t b = threadIdx.x; b < blocks; b += BB_THREADS)
         for (int a = 0; a < 3; ++a)
         {
-            v[a]     = fmin(v[a], p[a]);
-            v[3 + a] = fmax(v[3 + a], p[3 + a]);
+            v[a]     = fmin(v[a], scratch->partial[6 * b + a]);
+            v[3 + a] = fmax(v[3 + a], scratch->partial[6 * b + 3 + a]);
         }
-    }
     blockMinMax(v);
     if (threadIdx.x != 0)
         return;
-    scratch->done = 0;
     for (int k = 0; k < 6; ++k)
-    {
-        scratch->result[k] = v[k];
         if (box)
             __hip_atomic_store(box + k, static_cast<uint64_t>(__double_as_longlong(v[k])), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+        else
+            scratch->result[k] = v[k];
     if (box)
         __hip_atomic_store(box + 6, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -152,14 +142,15 @@ void launchBounds(const uint8_t* cloud, uint32_t n, uint32_t stride, uint8_t clo
     const uint32_t blocks =
             static_cast<uint32_t>(std::min<uint64_t>(BB_BLOCKS, (static_cast<uint64_t>(n) + BB_THREADS - 1) / BB_THREADS));
     if (cloudType == CLOUD_FLOAT_UINT8_T)
-        kBounds<float><<<blocks, BB_THREADS, 0, stream>>>(cloud, n, stride, scratch, box, seq);
+        kBoundsPartial<float><<<blocks, BB_THREADS, 0, stream>>>(cloud, n, stride, scratch);
     else
-        kBounds<double><<<blocks, BB_THREADS, 0, stream>>>(cloud, n, stride, scratch, box, seq);
+        kBoundsPartial<double><<<blocks, BB_THREADS, 0, stream>>>(cloud, n, stride, scratch);
+    kBoundsFinal<<<1, BB_THREADS, 0, stream>>>(scratch, blocks, box, seq);
 }
 
 // What one reduction uses: a stream of its own, scratch memory and a mailbox. A call takes one from the
 // device's pool and gives it back, so calls on several threads run side by side as before, and a call
-// alone creates nothing (stream, allocation, free and copy were 60 of 80 us for 200K points).
+// alone creates nothing (200K points: 18 us, of 73 with a stream, an allocation and a copy of its own).
 struct BoundsContext
 {
     hipStream_t stream     = nullptr;
@@ -188,7 +179,6 @@ struct BoundsContext
         check(hipHostMalloc(reinterpret_cast<void**>(&box), 7 * sizeof(uint64_t), hipHostMallocCoherent),
               "hipHostMalloc of the bounding-box mailbox");
         std::fill(box, box + 7, 0);
-        check(hipMemsetAsync(scratch, 0, sizeof(BoundsScratch), stream), "hipMemset of the bounding-box scratch");
     }
 };
 
@@ -211,7 +201,7 @@ std::vector<std::unique_ptr<BoundsContext>>* idleContexts()
 // The scratch of the allocation-free variant, one per device. In host code this name only stands for
 // the object; its device address comes from hipGetSymbolAddress, once per device.
 static __device__ __align__(256) BoundsScratch scratch;
-static_assert(sizeof(BoundsScratch) <= 49208, "the documented size of the static scratch");
+static_assert(sizeof(BoundsScratch) == 49200, "the documented size of the static scratch");
 
 void realBoundingBox(const uint8_t* deviceCloud, uint32_t n, uint32_t stride, uint8_t cloudType, int device,
                      double real[6])
@@ -234,7 +224,7 @@ void realBoundingBox(const uint8_t* deviceCloud, uint32_t n, uint32_t stride, ui
         ctx = std::make_unique<BoundsContext>();
         ctx->create();
     }
-    // on an error the context goes with its stream drained; its counter may not be zero
+    // on an error the context goes, its stream drained
     const uint64_t seq = ++ctx->seq;
     launchBounds(deviceCloud, n, stride, cloudType, ctx->scratch, ctx->box, seq, ctx->stream);
     check(hipGetLastError(), "bounding box reduction");
